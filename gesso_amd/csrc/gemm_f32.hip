@@ -1,0 +1,316 @@
+// y = x W^T (+ bias), everything float32, on the matrix cores: the true 32-bit path's product.
+//
+// v_mfma_f32_16x16x4_f32 multiplies float32 operands without rounding them and adds its four products to the accumulator
+// one after the other in ascending k, each with one rounding: a chain of FMAs.  So an output here is summed in the order of
+// the tiled FMA kernel (gemm_tiled.hip): k in chunks of GS_SUM_CHUNK = 64, each from zero in ascending k, the chunks' sums
+// added in ascending order.  Its value depends neither on which kernel computed it nor on the rows beside it.
+//
+// The instruction wants row l % 16 and k = l / 16 of a tile in lane l.  Loaded like that from rows in memory, sixteen lanes
+// in a row of the wavefront ask sixteen lines at a time, and a compute unit gets some 8 bytes a cycle whatever it loads
+// (2048 x 8192 weights, 6 rows: 28 us, of which the weights alone 21); so a wavefront loads whole runs of a row, sixteen
+// lanes 256 bytes, and puts them in order through LDS (rows 4 numbers further apart than their length: no bank twice).
+//
+// Few rows (up to 64): gemm_f32_rows_kernel.  The weights bind, so each is read once: a block owns 8 or 16 rows of W and
+// its eight wavefronts take the chunks in turns, D chunks in flight each; the chunk sums go to LDS, and one thread an output
+// adds them in order.
+//
+// Many rows: gemm_f32_tiles_kernel.  The matrix cores bind (157 TFLOP/s): a block owns 32 MT x 32 NT outputs, its four
+// wavefronts (two by two) MT x NT tiles of 16 x 16 each; the operands of the next 32 k are loaded under the products of
+// these.
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(4))) float gf_f32x4_t;
+
+#define GF_WAVES 8
+
+// Four values from k on of a row of K (K a multiple of 4); nothing beyond K is read.  TAIL: k may lie beyond K (zeros).
+template <bool TAIL>
+__device__ __forceinline__ gf_f32x4_t gf_load(const float* __restrict__ row, int k, int K) {
+  if (!TAIL) return *reinterpret_cast<const gf_f32x4_t*>(row + k);
+  gf_f32x4_t v = *reinterpret_cast<const gf_f32x4_t*>(row + (k < K ? k : 0));
+  return k < K ? v : gf_f32x4_t{0.f, 0.f, 0.f, 0.f};
+}
+
+// WR: rows of W a block owns (8 or 16), XR: rows of X (4, 8, or tiles of 16), D: chunks a wavefront holds in flight.
+template <int WR, int XR, int D, bool TAIL, typename TO>
+__global__ __launch_bounds__(GF_WAVES * 64) void gemm_f32_rows_kernel(const float* __restrict__ X, int ldx,
+                                                                      const float* __restrict__ W,
+                                                                      const float* __restrict__ bias, TO* __restrict__ Y,
+                                                                      int ldy, int M, int N, int K, int room) {
+  constexpr int MT = XR > 16 ? XR / 16 : 1, XT = XR < 16 ? XR : 16;       // tiles of X, rows used of each
+  constexpr int OUT = MT * 16 * WR, PER = (OUT + GF_WAVES * 64 - 1) / (GF_WAVES * 64);
+  constexpr int LD = GS_SUM_CHUNK + 4;
+  extern __shared__ float sums[];                                         // chunk sums of a pass: `room` of OUT numbers
+  __shared__ float order[GF_WAVES][16 * LD];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * WR;
+  // lane l loads the four k at 4 (l % 16) of row l / 16 of four
+  const float* wp[WR / 4];
+  const float* xp[MT][XT / 4];
+#pragma unroll
+  for (int j = 0; j < WR / 4; ++j) wp[j] = W + (size_t)(n0 + 4 * j + g < N ? n0 + 4 * j + g : N - 1) * K;
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < XT / 4; ++j) xp[i][j] = X + (size_t)(16 * i + 4 * j + g < M ? 16 * i + 4 * j + g : M - 1) * ldx;
+  const int chunks = (K + GS_SUM_CHUNK - 1) / GS_SUM_CHUNK;
+
+  struct Chunk {
+    gf_f32x4_t w[WR / 4], x[MT][XT / 4];
+  };
+  auto load = [&](Chunk& b, int c) __attribute__((always_inline)) {
+    const int k = c * GS_SUM_CHUNK + 4 * r16;
+#pragma unroll
+    for (int j = 0; j < WR / 4; ++j) b.w[j] = gf_load<TAIL>(wp[j], k, K);
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < XT / 4; ++j) b.x[i][j] = gf_load<TAIL>(xp[i][j], k, K);
+  };
+  float* mine = order[wave];
+  float* put = mine + g * LD + 4 * r16;           // where a lane leaves what it loaded, four rows a load
+  const float* get = mine + r16 * LD + g;         // and where it finds its operands, four numbers apart
+  // (a tile of fewer rows than sixteen leaves the others as they are: they end in outputs nobody keeps)
+  auto multiply = [&](Chunk& b, int c, bool keep) __attribute__((always_inline)) {
+    float w[16];
+#pragma unroll
+    for (int j = 0; j < WR / 4; ++j) *reinterpret_cast<gf_f32x4_t*>(put + 4 * j * LD) = b.w[j];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) w[q] = get[4 * q];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      float x[16];
+#pragma unroll
+      for (int j = 0; j < XT / 4; ++j) *reinterpret_cast<gf_f32x4_t*>(put + 4 * j * LD) = b.x[i][j];
+#pragma unroll
+      for (int q = 0; q < 16; ++q) x[q] = get[4 * q];
+      gf_f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int q = 0; q < 16; ++q) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[q], x[q], acc, 0, 0, 0);
+      // element e of lane l: row 4 (l / 16) + e of W, row l % 16 of X: X's row after X's row, WR numbers each
+      if (keep && 4 * g < WR) *reinterpret_cast<gf_f32x4_t*>(sums + c * OUT + (i * 16 + r16) * WR + 4 * g) = acc;
+    }
+  };
+  float tot[PER];
+#pragma unroll
+  for (int p = 0; p < PER; ++p) tot[p] = 0.f;
+  for (int c0 = 0; c0 < chunks; c0 += room) {     // (one pass where LDS holds all chunks' sums)
+    // the wavefront's chunks: c0 + wave, + GF_WAVES, ...; as many rounds for every wavefront, D chunks in flight, no load
+    // behind a branch (a round beyond the last chunk loads that chunk again and leaves nothing)
+    const int held = chunks - c0 < room ? chunks - c0 : room, n = (held + GF_WAVES - 1) / GF_WAVES;
+    auto chunk = [&](int i) __attribute__((always_inline)) { return wave + i * GF_WAVES < held ? wave + i * GF_WAVES : held - 1; };
+    Chunk b[D];
+#pragma unroll
+    for (int d = 0; d < D; ++d) load(b[d], c0 + chunk(d));
+    int i = 0;
+    for (; i + D < n; i += D)
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        multiply(b[d], chunk(i + d), true);
+        load(b[d], c0 + chunk(i + d + D));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+      if (i + d < n) multiply(b[d], chunk(i + d), wave + (i + d) * GF_WAVES < held);
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+      const int o = threadIdx.x + p * GF_WAVES * 64;
+      if (o < OUT) {
+#pragma unroll 8
+        for (int c = 0; c < held; ++c) tot[p] += sums[c * OUT + o];
+      }
+    }
+    if (c0 + room < chunks) __syncthreads();
+  }
+#pragma unroll
+  for (int p = 0; p < PER; ++p) {
+    const int o = threadIdx.x + p * GF_WAVES * 64;
+    if (o >= OUT) continue;
+    const int n = n0 + o % WR, m = o / WR;
+    if (n < N && m < M) {
+      float t = tot[p];
+      if (bias) t += bias[n];
+      Y[(size_t)m * ldy + n] = from_f32<TO>(t);
+    }
+  }
+}
+
+template <int MT, int NT, bool TAIL, typename TO>
+__global__ __launch_bounds__(256) void gemm_f32_tiles_kernel(const float* __restrict__ X, int ldx,
+                                                             const float* __restrict__ W,
+                                                             const float* __restrict__ bias, TO* __restrict__ Y, int ldy,
+                                                             int M, int N, int K) {
+  constexpr int KS = 32, LD = KS + 4, BM = 32 * MT, BN = 32 * NT;
+  __shared__ float xs[2][BM * LD], ws[2][BN * LD];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, g = lane >> 4;
+  const int mb = blockIdx.x * BM, nb = blockIdx.y * BN, mw = (wave & 1) * 16 * MT, nw = (wave >> 1) * 16 * NT;
+  // thread t loads the four k at 4 (t % 8) of row t / 8, 32 rows a load
+  const int lr = threadIdx.x >> 3, lk = 4 * (threadIdx.x & 7);
+  const float* xp[MT];
+  const float* wp[NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) xp[i] = X + (size_t)(mb + 32 * i + lr < M ? mb + 32 * i + lr : M - 1) * ldx;
+#pragma unroll
+  for (int j = 0; j < NT; ++j) wp[j] = W + (size_t)(nb + 32 * j + lr < N ? nb + 32 * j + lr : N - 1) * K;
+  gf_f32x4_t xr[MT], wr[NT];
+  auto load = [&](int k) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) xr[i] = gf_load<TAIL>(xp[i], k + lk, K);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) wr[j] = gf_load<TAIL>(wp[j], k + lk, K);
+  };
+  auto put = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) *reinterpret_cast<gf_f32x4_t*>(&xs[s][(32 * i + lr) * LD + lk]) = xr[i];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) *reinterpret_cast<gf_f32x4_t*>(&ws[s][(32 * j + lr) * LD + lk]) = wr[j];
+  };
+  gf_f32x4_t acc[MT][NT], tot[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) tot[i][j] = gf_f32x4_t{0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](int s, bool first) __attribute__((always_inline)) {
+    const float* x = &xs[s][(mw + r16) * LD + g];
+    const float* w = &ws[s][(nw + r16) * LD + g];
+#pragma unroll
+    for (int q = 0; q < KS / 4; ++q) {
+      float a[MT], b[NT];
+#pragma unroll
+      for (int i = 0; i < MT; ++i) a[i] = x[16 * i * LD + 4 * q];
+#pragma unroll
+      for (int j = 0; j < NT; ++j) b[j] = w[16 * j * LD + 4 * q];
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          const gf_f32x4_t c = first && q == 0 ? gf_f32x4_t{0.f, 0.f, 0.f, 0.f} : acc[i][j];
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[j], a[i], c, 0, 0, 0);
+        }
+    }
+  };
+  load(0);
+  put(0);
+  __syncthreads();
+  for (int k = 0; k < K; k += GS_SUM_CHUNK) {     // a chunk: two steps of 32 k (beyond K: zeros)
+    load(TAIL || k + KS < K ? k + KS : k);
+    multiply(0, true);
+    put(1);
+    __syncthreads();
+    load(TAIL || k + 2 * KS < K ? k + 2 * KS : k);    // (after the last chunk: loaded and not used)
+    multiply(1, false);
+    put(0);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) tot[i][j][e] += acc[i][j][e];
+  }
+  // element e of lane l: row 4 (l / 16) + e of W, row l % 16 of X
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int m = mb + mw + 16 * i + r16;
+    if (m >= M) continue;
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int n = nb + nw + 16 * j + 4 * g + e;
+        if (n >= N) continue;
+        float t = tot[i][j][e];
+        if (bias) t += bias[n];
+        Y[(size_t)m * ldy + n] = from_f32<TO>(t);
+      }
+  }
+}
+
+// Whether the matrix-core kernels take the operands: K and the row stride in whole pieces of 16 bytes, both aligned.
+extern "C" int gs_gemm_f32_supports(int M, int K, int ldx, const void* X, const void* W) {
+  return M >= 1 && K > 0 && K % 4 == 0 && (M == 1 || ldx % 4 == 0) && ((uintptr_t)X & 15) == 0 && ((uintptr_t)W & 15) == 0;
+}
+
+template <int WR, int XR, int D, typename TO>
+static void run_rows(const float* X, int ldx, const float* W, const float* bias, TO* Y, int ldy, int M, int N, int K,
+                     hipStream_t stream) {
+  constexpr int out = (XR > 16 ? XR : 16) * WR, most = 7168 / out;         // 28 KB of LDS for the sums, beside 34 KB
+  const int blocks = gs_ceil_div(N, WR), chunks = gs_ceil_div(K, GS_SUM_CHUNK), room = chunks < most ? chunks : most;
+  const size_t lds = (size_t)room * out * sizeof(float);
+  if (K % GS_SUM_CHUNK == 0)
+    gemm_f32_rows_kernel<WR, XR, D, false, TO><<<blocks, GF_WAVES * 64, lds, stream>>>(X, ldx, W, bias, Y, ldy, M, N, K, room);
+  else
+    gemm_f32_rows_kernel<WR, XR, D, true, TO><<<blocks, GF_WAVES * 64, lds, stream>>>(X, ldx, W, bias, Y, ldy, M, N, K, room);
+}
+
+template <int MT, int NT, typename TO>
+static void run_tiles(const float* X, int ldx, const float* W, const float* bias, TO* Y, int ldy, int M, int N, int K,
+                      hipStream_t stream) {
+  const dim3 grid(gs_ceil_div(M, 32 * MT), gs_ceil_div(N, 32 * NT));
+  if (K % GS_SUM_CHUNK == 0)
+    gemm_f32_tiles_kernel<MT, NT, false, TO><<<grid, 256, 0, stream>>>(X, ldx, W, bias, Y, ldy, M, N, K);
+  else
+    gemm_f32_tiles_kernel<MT, NT, true, TO><<<grid, 256, 0, stream>>>(X, ldx, W, bias, Y, ldy, M, N, K);
+}
+
+// Which kernel, by sizes (microseconds on cold weights, one MI355X; the FMA kernels that ran before: 63 on average for the
+// products of a decode step of 6 rows, 729 for those of a prompt portion of 900 tokens, 2048 x 2048 to 16384 x 2048).
+// Up to 16 rows: blocks of 8 rows of W up to N = 8192, which then still are no more than four a compute unit (6 rows,
+//   2048 x 8192: 21.8, blocks of 16 rows 30.7; 6144 x 2048: 15.1 and 17.2); of 16 rows beyond (65536 x 2048: 118 and 121;
+//   16 rows: 129 and 135).
+// Up to 64 rows: every block of the rows kernel reads all rows of X for its few of W, so wide weights go to the tiles (40 rows,
+//   16384 x 2048: tiles of 32 x 32 70, rows 112; 65536: tiles of 64 x 64 178, rows 432), narrow ones do not fill the chip
+//   there (2048 x 8192: rows 70, tiles of 32 x 32 195).
+// More: the largest tiles that make two blocks a compute unit (680 rows: 2048 x 8192 by 64 x 64 333, 32 x 64 280; 16384 x 2048
+//   442 and 475; 300 rows, 2048 x 2048: 64 x 64 79, 32 x 64 67, 32 x 32 55; larger ones than 64 x 64 were slower everywhere,
+//   2,048 rows included).
+template <typename TO>
+static void run(const float* X, int ldx, const float* W, const float* bias, TO* Y, int ldy, int M, int N, int K,
+                hipStream_t stream) {
+#define GF_ROWS(WR, XR) return run_rows<WR, XR, 2, TO>(X, ldx, W, bias, Y, ldy, M, N, K, stream)
+#define GF_TILES(MT, NT) return run_tiles<MT, NT, TO>(X, ldx, W, bias, Y, ldy, M, N, K, stream)
+  const long by64 = (long)gs_ceil_div(M, 64) * gs_ceil_div(N, 64), by32x64 = (long)gs_ceil_div(M, 32) * gs_ceil_div(N, 64);
+  if (M <= 16) {
+    if (N <= 8192) {
+      if (M <= 4) GF_ROWS(8, 4);
+      if (M <= 8) GF_ROWS(8, 8);
+      GF_ROWS(8, 16);
+    }
+    if (M <= 4) GF_ROWS(16, 4);
+    if (M <= 8) GF_ROWS(16, 8);
+    GF_ROWS(16, 16);
+  }
+  if (M <= 64) {
+    if (by64 >= 1024) GF_TILES(2, 2);
+    if (N > 8192) GF_TILES(1, 1);
+    if (N <= 2048) {
+      if (M <= 32) GF_ROWS(8, 32);
+      if (M <= 48) GF_ROWS(8, 48);
+      GF_ROWS(8, 64);
+    }
+    if (M <= 32) GF_ROWS(16, 32);
+    if (M <= 48) GF_ROWS(16, 48);
+    GF_ROWS(16, 64);
+  }
+  if (by64 >= 512) GF_TILES(2, 2);
+  if (by32x64 >= 512) GF_TILES(1, 2);
+  GF_TILES(1, 1);
+#undef GF_ROWS
+#undef GF_TILES
+}
+
+extern "C" int gs_gemm_f32(const float* X, int ldx, const float* W, const float* bias, void* Y, int y_dtype, int ldy,
+                           int M, int N, int K, hipStream_t stream) {
+  GS_REQUIRE(N > 0 && K > 0 && ldy >= N && (M <= 1 || ldx >= K), "gemm_f32: bad sizes N=%d K=%d ldx=%d ldy=%d", N, K, ldx, ldy);
+  GS_REQUIRE(gs_gemm_f32_supports(M, K, ldx, X, W), "gemm_f32: needs rows, K and strides a multiple of 4, aligned operands (M=%d K=%d)", M, K);
+  GS_REQUIRE(gs_ceil_div(N, 32) <= 65535, "gemm_f32: N=%d too large for one launch", N);
+  GS_REQUIRE(y_dtype == GS_F32 || y_dtype == GS_BF16, "gemm_f32: unknown output dtype %d", y_dtype);
+  if (y_dtype == GS_F32)
+    run<float>(X, ldx, W, bias, (float*)Y, ldy, M, N, K, stream);
+  else
+    run<bf16>(X, ldx, W, bias, (bf16*)Y, ldy, M, N, K, stream);
+  GS_LAUNCH_CHECK("gemm_f32");
+  return 0;
+}

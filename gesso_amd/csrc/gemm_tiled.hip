@@ -4,8 +4,8 @@
 // storage for X, W and Y.  Products and sums are float32 FMAs: with float32 storage this is the
 // true 32-bit path (no matrix-core input rounding).  Each output element is summed in one fixed order,
 // so its value does not depend on M or on which rows share the launch: k in chunks of 64, each chunk
-// from zero in ascending k, the chunks' sums added in ascending order.  (The streaming kernel for few
-// rows, gemv_f32.hip, adds in the same order; a chunk is what one of its lanes takes.)
+// from zero in ascending k, the chunks' sums added in ascending order.  (The matrix-core kernels for
+// aligned float32 operands, gemm_f32.hip, add in the same order.)
 //
 // 64 x 64 tile per block of 256 threads, 4 x 4 outputs per thread, k in steps of 16 through LDS.
 #include "common.h"

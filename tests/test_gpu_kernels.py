@@ -409,6 +409,24 @@ def test_float32_product_of_few_rows_streams_the_weights_and_adds_in_the_same_or
     close(ops.gemm_tiled(x.to(DEV), w.to(DEV), out_dtype=torch.bfloat16), x.double() @ w.double().T, torch.bfloat16)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 9, 4), (2, 8193, 64), (4, 17, 8192), (8, 8200, 132), (9, 33, 68), (16, 50, 9000), (17, 2049, 516), (32, 40, 8196),
+                                   (33, 8200, 60), (49, 2056, 1024), (64, 100, 260), (64, 65536, 64), (65, 33, 96), (200, 4100, 100), (513, 4100, 36)])
+def test_float32_product_on_the_matrix_cores_adds_in_the_tiled_kernels_order(ops, M, N, K):
+    """Every branch of the choice by sizes, at the edges of its tiles and with chunks cut short, against the FMA kernel
+    (which takes the same rows when they lie at an odd stride): the same bits, and every bias and row in its place."""
+    g = gen(M + 3 * N + K)
+    wide = torch.randn(M + 1, K + 1, generator=g).to(DEV)
+    x, w, b = wide[:M, :K], torch.randn(N, K, generator=g).to(DEV), torch.randn(N, generator=g).to(DEV)
+    if M == 1:
+        x = wide.reshape(-1)[1:K + 1].reshape(1, K)            # (one row has no stride: at an odd address instead)
+    want = ops.gemm_tiled(x, w, b)
+    close(want, x.double().cpu() @ w.double().cpu().T + b.double().cpu(), torch.float32, scale=math.sqrt(K) / 4)
+    assert torch.equal(ops.gemm_tiled(x.contiguous().clone(), w, b), want)
+    room = torch.full((M + 2, N), 7.0, device=DEV)
+    ops.gemm_tiled(x.contiguous().clone(), w, b, out=room[1:M + 1])
+    assert torch.equal(room[1:M + 1], want) and bool((room[0] == 7).all() and (room[M + 1] == 7).all())
+
+
 # ------------------------------------------------------------------ choosing tokens
 
 def test_argmax_rows(ops):
