@@ -338,6 +338,15 @@ def test_attention_generic_chunk_over_prefix(ops, nh, nkv, d, ps, dtype):
     close(got, want, dtype)
 
 
+@pytest.mark.parametrize("nh,nkv,d,prefix", [(2, 1, 6, 14), (2, 2, 68, 15), (3, 1, 132, 16), (4, 2, 250, 17), (2, 1, 4, 63), (2, 1, 12, 128)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_attention_generic_rows_of_odd_pieces(ops, nh, nkv, d, prefix, dtype):
+    """Key rows of whole pieces of 16 bytes and not, more of them than are loaded at once, and counts of keys around the
+    number of value rows in flight."""
+    got, want = paged_case(ops, dtype, nh, nkv, d, 16, prefix=prefix, new=2, window=None, seed=d + prefix)
+    close(got, want, dtype)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_attention_generic_decode_far_key_among_hundreds(ops, dtype):
     # 700 cached keys, one query; key 3 (on the first page) carries most of the weight
