@@ -8,86 +8,193 @@
 //                    (+ sigmoid(g_t) * s[t, :] when a shared expert's output s and its gate g are given)
 //   relu_squared     act over the first F columns of rows (the shared expert's inner rows)
 //
-// A wavefront computes one output at a time: its lanes walk the weight row together (contiguous loads), each lane
-// summing its columns in ascending order, then the lanes' sums are added in a fixed order; products and sums are
-// float32.  Only the chosen experts' weights are read, which is what a step of few tokens needs; steps of many tokens
-// go through the grouped products of moe_group.hip, which read an expert's weights once for all of its tokens.
+// A wavefront computes MOE_ROWS outputs: its lanes walk the weight rows together (contiguous loads), each lane summing its
+// columns in ascending order, then the lanes' sums are added in a fixed order; products and sums are float32.  What binds is
+// the expert's weights (32 pairs of 704 x 2048: 92 MB, 61 MB of them different), so the loads of all rows are in flight
+// before the first is used, and before the token's row, which comes through LDS, has arrived.  Blocks are numbered slice of
+// outputs first, in multiples of eight, and blocks go to the eight XCDs in turn: tokens that share an expert find a slice's
+// weights in one XCD's L2.  8 tokens, 4 of 32 experts each, 704 x 2048: up 15.9 us, down 17.0 (a wavefront an output at a time,
+// token first: 25.4 and 33.2; all blocks resident at once counts for more than more loads a wavefront: down with four visits in
+// flight, half of the blocks waiting, 28.3).  Only the chosen experts' weights are read, which is what a step of few tokens needs; steps of many
+// tokens go through the grouped products of moe_group.hip, which read an expert's weights once for all of its tokens.
 #include "common.h"
 
+#define MOE_WAVES 4
+#define MOE_ROWS 4
+#define MOE_SLICE (MOE_WAVES * MOE_ROWS)
+
+// MOE_ROWS rows of n weights (from `row` on, `stride` apart) in pieces of eight a lane, P pieces of 512 columns from column
+// j0 on; a piece beyond the row's end reads the row's beginning (and is not used).
+template <int P, typename TW>
+struct MoePieces {
+  float4 raw[MOE_ROWS][P][sizeof(TW) / 2];
+  __device__ __forceinline__ void load(const TW* __restrict__ row, const size_t* at, int j0, int n) {
+#pragma unroll
+    for (int r = 0; r < MOE_ROWS; ++r)
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        const int j = j0 + 512 * p < n ? j0 + 512 * p : 0;
+#pragma unroll
+        for (int q = 0; q < (int)sizeof(TW) / 2; ++q) raw[r][p][q] = *(reinterpret_cast<const float4*>(row + at[r] + j) + q);
+      }
+  }
+  __device__ __forceinline__ void add(float* s, const float* __restrict__ x, int j0, int n) const {
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const int j = j0 + 512 * p;
+      if (j < n) {
+        float xv[8];
+        load8f(x + j, xv);
+#pragma unroll
+        for (int r = 0; r < MOE_ROWS; ++r) {
+          float w8[8];
+          load8f(reinterpret_cast<const TW*>(&raw[r][p][0]), w8);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) s[r] = fmaf(w8[i], xv[i], s[r]);
+        }
+      }
+    }
+  }
+};
+
+// n numbers of a row as floats into LDS, by the whole block.
+template <typename T>
+__device__ __forceinline__ void moe_stage(const T* __restrict__ row, float* __restrict__ to, int n) {
+  if ((n & 7) == 0 && aligned16(row)) {
+    for (int j = 8 * threadIdx.x; j < n; j += 8 * MOE_WAVES * 64) {
+      float v[8];
+      load8f(row + j, v);
+      store8f(to + j, v);
+    }
+  } else {
+    for (int j = threadIdx.x; j < n; j += MOE_WAVES * 64) to[j] = to_f32(row[j]);
+  }
+}
+
 template <typename T, typename TW>
-__global__ void moe_table_up_kernel(const T* __restrict__ x, int ldx, const int* __restrict__ ids,
-                                    const int* __restrict__ table, int top, const TW* __restrict__ up, int F, int H,
-                                    T* __restrict__ a) {
-  extern __shared__ float xs[];      // H floats
-  const int t = blockIdx.x / top, k = blockIdx.x % top;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  for (int j = threadIdx.x; j < H; j += blockDim.x) xs[j] = to_f32(x[(size_t)t * ldx + j]);
-  __syncthreads();
+__global__ __launch_bounds__(MOE_WAVES * 64) void moe_table_up_kernel(const T* __restrict__ x, int ldx,
+                                                                      const int* __restrict__ ids,
+                                                                      const int* __restrict__ table, int top,
+                                                                      const TW* __restrict__ up, int F, int H,
+                                                                      T* __restrict__ a, int pairs) {
+  extern __shared__ float4 staged[];
+  float* xs = reinterpret_cast<float*>(staged);      // H floats
+  constexpr int P = 4 / (sizeof(TW) / 2);
+  const int pair = blockIdx.y + blockIdx.z * gridDim.y;
+  if (pair >= pairs) return;
+  const int t = pair / top, k = pair % top;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int f0 = blockIdx.x * MOE_SLICE + wave * MOE_ROWS;
   const int e = table[(size_t)ids[t] * top + k];
   const TW* w = up + (size_t)e * F * H;
   T* dst = a + ((size_t)t * top + k) * F;
   // rows of whole 16-byte pieces: eight weights a lane and load (the order of the sums depends on H alone)
   const bool vec = (H & 7) == 0 && aligned16(w);
-  for (int f = blockIdx.y * nw + wave; f < F; f += gridDim.y * nw) {
-    const TW* row = w + (size_t)f * H;
-    float s = 0.f;
-    if (vec) {
-      for (int j = lane * 8; j < H; j += 512) {
-        float w8[8];
-        load8f(row + j, w8);
+  size_t at[MOE_ROWS];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) s = fmaf(w8[i], xs[j + i], s);
-      }
-    } else {
-      for (int j = lane; j < H; j += 64) s = fmaf(to_f32(row[j]), xs[j], s);
+  for (int r = 0; r < MOE_ROWS; ++r) at[r] = (size_t)(f0 + r < F ? f0 + r : F - 1) * H;
+  MoePieces<P, TW> b;
+  if (vec) b.load(w, at, lane * 8, H);
+  moe_stage(x + (size_t)t * ldx, xs, H);
+  __syncthreads();
+  if (f0 >= F) return;
+  float s[MOE_ROWS];
+#pragma unroll
+  for (int r = 0; r < MOE_ROWS; ++r) s[r] = 0.f;
+  if (vec) {
+    for (int j = lane * 8; j - lane * 8 < H; j += 512 * P) {
+      b.add(s, xs, j, H);
+      if (j - lane * 8 + 512 * P < H) b.load(w, at, j + 512 * P, H);
     }
-    s = wave_sum(s);
-    if (lane == 0) {
+  } else {
+#pragma unroll
+    for (int r = 0; r < MOE_ROWS; ++r)
+      for (int j = lane; j < H; j += 64) s[r] = fmaf(to_f32(w[at[r] + j]), xs[j], s[r]);
+  }
+#pragma unroll
+  for (int r = 0; r < MOE_ROWS; ++r) {
+    const float v = wave_sum(s[r]);
+    if (lane == 0 && f0 + r < F) {
       // the product is stored in the activation type before the activation, as a product of its own would be
-      float z = to_f32(from_f32<T>(s));
+      float z = to_f32(from_f32<T>(v));
       z = z > 0.f ? z : 0.f;
-      dst[f] = from_f32<T>(z * z);
+      dst[f0 + r] = from_f32<T>(z * z);
     }
   }
 }
 
 template <typename T, typename TW>
-__global__ void moe_table_down_kernel(const T* __restrict__ a, const int* __restrict__ ids,
-                                      const int* __restrict__ table, int top, const TW* __restrict__ down, int F, int H,
-                                      const T* __restrict__ shared, const T* __restrict__ gate, int ldg,
-                                      T* __restrict__ y) {
-  extern __shared__ float as[];      // top * F floats
-  const int t = blockIdx.x;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  for (int j = threadIdx.x; j < top * F; j += blockDim.x) as[j] = to_f32(a[(size_t)t * top * F + j]);
-  __syncthreads();
+__global__ __launch_bounds__(MOE_WAVES * 64) void moe_table_down_kernel(const T* __restrict__ a, const int* __restrict__ ids,
+                                                                        const int* __restrict__ table, int top,
+                                                                        const TW* __restrict__ down, int F, int H,
+                                                                        const T* __restrict__ shared,
+                                                                        const T* __restrict__ gate, int ldg,
+                                                                        T* __restrict__ y, int ntok) {
+  extern __shared__ float4 staged[];
+  float* as = reinterpret_cast<float*>(staged);      // top * F floats
+  constexpr int P = 2 / (sizeof(TW) / 2);            // pieces a visit: a row of up to 1024 is one visit
+  constexpr int D = 2;                               // visits in flight (4: 173 registers, half of the blocks wait for the others)
+  const int t = blockIdx.y + blockIdx.z * gridDim.y;
+  if (t >= ntok) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int i0 = blockIdx.x * MOE_SLICE + wave * MOE_ROWS;
   const float share = 1.0f / (float)top;
+  const int* mine = table + (size_t)ids[t] * top;
+  const bool vec = (F & 7) == 0 && aligned16(down);
+  size_t at[MOE_ROWS];
+#pragma unroll
+  for (int r = 0; r < MOE_ROWS; ++r) at[r] = (size_t)(i0 + r < H ? i0 + r : H - 1) * F;
+  const int per = (F + 512 * P - 1) / (512 * P), visits = top * per;      // visit v: piece group v % per of choice v / per
+  MoePieces<P, TW> b[D];
+  auto load = [&](MoePieces<P, TW>& p, int v) __attribute__((always_inline)) {
+    v = v < visits ? v : visits - 1;
+    p.load(down + (size_t)mine[v / per] * H * F, at, lane * 8 + v % per * 512 * P, F);
+  };
+  if (vec) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) load(b[d], d);
+  }
+  moe_stage(a + (size_t)t * top * F, as, top * F);
   float g = 0.f;
   if (shared) g = 1.f / (1.f + expf(-to_f32(gate[(size_t)t * ldg])));
-  const bool vec = (F & 7) == 0 && aligned16(down);
-  for (int i = blockIdx.y * nw + wave; i < H; i += gridDim.y * nw) {
-    float total = 0.f;
-    for (int k = 0; k < top; ++k) {
-      const int e = table[(size_t)ids[t] * top + k];
-      const TW* row = down + ((size_t)e * H + i) * F;
-      float s = 0.f;
-      if (vec) {
-        for (int j = lane * 8; j < F; j += 512) {
-          float w8[8];
-          load8f(row + j, w8);
+  __syncthreads();
+  if (i0 >= H) return;
+  float s[MOE_ROWS], total[MOE_ROWS];
 #pragma unroll
-          for (int u = 0; u < 8; ++u) s = fmaf(w8[u], as[k * F + j + u], s);
-        }
-      } else {
-        for (int j = lane; j < F; j += 64) s = fmaf(to_f32(row[j]), as[k * F + j], s);
-      }
-      total += wave_sum(s) * share;
+  for (int r = 0; r < MOE_ROWS; ++r) s[r] = total[r] = 0.f;
+  auto finish = [&]() __attribute__((always_inline)) {                    // a choice's sums are complete
+#pragma unroll
+    for (int r = 0; r < MOE_ROWS; ++r) {
+      total[r] += wave_sum(s[r]) * share;
+      s[r] = 0.f;
     }
-    if (lane == 0) {
-      if (shared) total += g * to_f32(shared[(size_t)t * H + i]);
-      y[(size_t)t * H + i] = from_f32<T>(total);
+  };
+  if (vec) {
+    for (int v0 = 0; v0 < visits; v0 += D)
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        const int v = v0 + d;
+        if (v < visits) {
+          b[d].add(s, as + (size_t)(v / per) * F, lane * 8 + v % per * 512 * P, F);
+          if (v0 + D < visits) load(b[d], v + D);
+          if (v % per == per - 1) finish();
+        }
+      }
+  } else {
+    for (int k = 0; k < top; ++k) {
+      const TW* w = down + (size_t)mine[k] * H * F;
+#pragma unroll
+      for (int r = 0; r < MOE_ROWS; ++r)
+        for (int j = lane; j < F; j += 64) s[r] = fmaf(to_f32(w[at[r] + j]), as[k * F + j], s[r]);
+      finish();
     }
   }
+#pragma unroll
+  for (int r = 0; r < MOE_ROWS; ++r)
+    if (lane == 0 && i0 + r < H) {
+      if (shared) total[r] += g * to_f32(shared[(size_t)t * H + i0 + r]);
+      y[(size_t)t * H + i0 + r] = from_f32<T>(total[r]);
+    }
 }
 
 template <typename T>
@@ -101,12 +208,10 @@ __global__ void relu_squared_kernel(const T* __restrict__ x, int ldx, T* __restr
   out[i] = from_f32<T>(z * z);
 }
 
-static int moe_blocks_y(int outputs, int tokens) {
-  // enough blocks to fill the chip when tokens are few, one block a token when they are many
-  int y = gs_ceil_div(outputs, 4);
-  int cap = 2048 / (tokens > 0 ? tokens : 1);
-  if (cap < 1) cap = 1;
-  return y < cap ? y : cap;
+// Slices of outputs, in a multiple of the eight XCDs that blocks go to in turn, by what they are of (a launch takes 65535 in y).
+static dim3 moe_grid(int outputs, long of) {
+  const int y = of < 65535 ? (int)of : 65535;
+  return dim3(gs_ceil_div(gs_ceil_div(outputs, MOE_SLICE), 8) * 8, y, gs_ceil_div(of, y));
 }
 
 extern "C" int gs_moe_table_up(const void* x, int dtype, int ldx, const int* ids, const int* table, int top,
@@ -114,17 +219,17 @@ extern "C" int gs_moe_table_up(const void* x, int dtype, int ldx, const int* ids
   GS_REQUIRE(ntok >= 0 && top > 0 && F > 0 && H > 0 && ldx >= H, "moe_table_up: bad sizes T=%d top=%d F=%d H=%d", ntok, top, F, H);
   GS_REQUIRE(H * sizeof(float) <= 65536, "moe_table_up: rows of %d are wider than the kernel's staging", H);
   if (ntok == 0) return 0;
-  dim3 grid(ntok * top, moe_blocks_y(F, ntok * top));
+  const dim3 grid = moe_grid(F, (long)ntok * top);
   const size_t lds = H * sizeof(float);
   if (dtype == GS_F32 && w_dtype == GS_F32)
     moe_table_up_kernel<float, float><<<grid, 256, lds, stream>>>((const float*)x, ldx, ids, table, top, (const float*)up,
-                                                                  F, H, (float*)a);
+                                                                  F, H, (float*)a, ntok * top);
   else if (dtype == GS_BF16 && w_dtype == GS_BF16)
     moe_table_up_kernel<bf16, bf16><<<grid, 256, lds, stream>>>((const bf16*)x, ldx, ids, table, top, (const bf16*)up, F,
-                                                                H, (bf16*)a);
+                                                                H, (bf16*)a, ntok * top);
   else if (dtype == GS_BF16 && w_dtype == GS_F32)
     moe_table_up_kernel<bf16, float><<<grid, 256, lds, stream>>>((const bf16*)x, ldx, ids, table, top, (const float*)up,
-                                                                 F, H, (bf16*)a);
+                                                                 F, H, (bf16*)a, ntok * top);
   else
     GS_REQUIRE(false, "moe_table_up: unsupported types %d %d", dtype, w_dtype);
   GS_LAUNCH_CHECK("moe_table_up");
@@ -138,20 +243,20 @@ extern "C" int gs_moe_table_down(const void* a, int dtype, const int* ids, const
   GS_REQUIRE((long)top * F * sizeof(float) <= 65536, "moe_table_down: %d x %d inner values are more than the kernel stages", top, F);
   GS_REQUIRE((shared == nullptr) == (gate == nullptr), "moe_table_down: a shared expert's rows come with their gate");
   if (ntok == 0) return 0;
-  dim3 grid(ntok, moe_blocks_y(H, ntok));
+  const dim3 grid = moe_grid(H, ntok);
   const size_t lds = (size_t)top * F * sizeof(float);
   if (dtype == GS_F32 && w_dtype == GS_F32)
     moe_table_down_kernel<float, float><<<grid, 256, lds, stream>>>((const float*)a, ids, table, top, (const float*)down,
                                                                     F, H, (const float*)shared, (const float*)gate, ldg,
-                                                                    (float*)y);
+                                                                    (float*)y, ntok);
   else if (dtype == GS_BF16 && w_dtype == GS_BF16)
     moe_table_down_kernel<bf16, bf16><<<grid, 256, lds, stream>>>((const bf16*)a, ids, table, top, (const bf16*)down, F,
                                                                   H, (const bf16*)shared, (const bf16*)gate, ldg,
-                                                                  (bf16*)y);
+                                                                  (bf16*)y, ntok);
   else if (dtype == GS_BF16 && w_dtype == GS_F32)
     moe_table_down_kernel<bf16, float><<<grid, 256, lds, stream>>>((const bf16*)a, ids, table, top, (const float*)down,
                                                                    F, H, (const bf16*)shared, (const bf16*)gate, ldg,
-                                                                   (bf16*)y);
+                                                                   (bf16*)y, ntok);
   else
     GS_REQUIRE(false, "moe_table_down: unsupported types %d %d", dtype, w_dtype);
   GS_LAUNCH_CHECK("moe_table_down");

@@ -45,7 +45,7 @@ def folders(tmp_path_factory):
 # ------------------------------------------------------------------ kernels alone
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("H", [100, 256, 1030])
+@pytest.mark.parametrize("H", [8, 100, 256, 1030, 2056, 4096, 4104])
 def test_norm_scaled_add(ops, dtype, H):
     res = torch.randn(5, H, generator=gen(0))
     y = (torch.randn(5, H, generator=gen(1)) * 3).to(dtype)
@@ -238,6 +238,24 @@ class Tokens:
     def __init__(self, ids):
         self.token_ids = torch.tensor(ids, dtype=torch.int32, device=DEV)
         self.T = len(ids)
+
+
+@pytest.mark.parametrize("xd,wd", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("T,E,top,F,H", [(1, 3, 1, 8, 8), (2, 4, 3, 520, 520), (5, 2, 2, 1032, 2056), (3, 5, 5, 15, 17), (4, 3, 2, 17, 4104), (2, 2, 1, 2056, 16)])
+def test_table_routed_kernels_token_by_token_at_the_edges_of_their_pieces(ops, xd, wd, T, E, top, F, H):
+    """Outputs that fill no slice, rows of less than a wavefront's piece and of several, and of no whole pieces at all."""
+    g = gen(T + E + top + F + H)
+    x, up, down = torch.randn(T, H, generator=g).to(xd), (torch.randn(E, F, H, generator=g) / H ** 0.5).to(wd), torch.randn(E, H, F, generator=g).to(wd)
+    table = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(9)]).to(torch.int32)
+    ids = torch.randint(0, 9, (T,), generator=g).to(torch.int32)
+    shared, gate = torch.randn(T, H, generator=g).to(xd), torch.randn(T, 3, generator=g).to(xd)
+    got = ops.moe_table(x.to(DEV), ids.to(DEV), table.to(DEV), up.to(DEV), down.to(DEV), shared.to(DEV), gate.to(DEV))
+    want = torch.sigmoid(gate[:, :1].double()) * shared.double()
+    for t in range(T):
+        for e in table[ids[t]].tolist():
+            z = (up[e].double() @ x[t].double()).to(xd).double().clamp(min=0)      # stored in the rows' type, as the kernel does
+            want[t] += down[e].double() @ (z * z).to(xd).double() / top
+    assert float((got.cpu().double() - want).abs().max()) <= tol(xd, want)
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
