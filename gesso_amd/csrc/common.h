@@ -124,20 +124,17 @@ __device__ __forceinline__ float wave_sum_dpp(float x) {
   return group4_sum(x);
 }
 
-// Sum over a block of up to 1024 threads; every thread gets the result.  `red` holds 17 floats.
+// Sum over a block of up to 1024 threads; every thread gets the result.  `red` holds 17 floats.  (Every thread adds the
+// wavefronts' sums itself: one barrier less than handing one thread's sum out.)
 __device__ __forceinline__ float block_sum(float v, float* red) {
   int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
   v = wave_sum(v);
   __syncthreads();
   if (lane == 0) red[wave] = v;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    float s = 0.f;
-    for (int i = 0; i < nw; ++i) s += red[i];
-    red[16] = s;
-  }
-  __syncthreads();
-  return red[16];
+  float s = 0.f;
+  for (int i = 0; i < nw; ++i) s += red[i];
+  return s;
 }
 
 // Eight consecutive values as float, from float32 or bfloat16 storage (16-byte aligned), and back.
