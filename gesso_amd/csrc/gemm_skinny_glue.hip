@@ -6,6 +6,7 @@ void gs_skinny_plain_rows(const SkinnyCall& c);
 void gs_skinny_residual_rows(const SkinnyCall& c);
 void gs_skinny_conv_rows(const SkinnyCall& c);
 void gs_skinny_plain_tiles(const SkinnyCall& c);
+void gs_skinny_plain_half_tiles(const SkinnyCall& c);
 void gs_skinny_residual_tiles(const SkinnyCall& c);
 void gs_skinny_residual_half_tiles(const SkinnyCall& c);
 void gs_skinny_conv_tiles(const SkinnyCall& c);
@@ -26,17 +27,19 @@ static void lazy(SkinnyCall& c, const float* res, const float* ssq, int nb, cons
   c.ex.res = res; c.ex.ssq = ssq; c.ex.nb = nb; c.ex.norm_w = norm_w; c.ex.eps = eps;
 }
 
+// A weight of few rows is shared out in half tiles, so that twice as many blocks stream it.
+bool gs_skinny_halves(int N) { return N % 16 == 0 && N / 16 <= 160; }
+
 void gs_skinny_run_plain(const void* X, int ldx, int x_tiled, const float* res, const float* ssq, int nb, const float* norm_w,
                          float eps, const void* W, const void* Wt, void* Y, int y_dtype, int ldy, int M, int N, int K,
                          int epilogue, int y_tiled, hipStream_t stream) {
   SkinnyCall c = base(X, ldx, x_tiled, W, Wt, Y, y_dtype, ldy, M, N, K, epilogue, stream);
   c.ex.y_tiled = y_tiled;
   if (res || ssq) lazy(c, res, ssq, nb, norm_w, eps);
-  Wt ? gs_skinny_plain_tiles(c) : gs_skinny_plain_rows(c);
+  // (with more rows of X the blocks' reading of X outweighs the fuller chip)
+  if (Wt && epilogue == 0 && gs_skinny_halves(N) && M <= 32) gs_skinny_plain_half_tiles(c);
+  else Wt ? gs_skinny_plain_tiles(c) : gs_skinny_plain_rows(c);
 }
-
-// A weight of few rows is shared out in half tiles, so that twice as many blocks stream it.
-bool gs_skinny_halves(int N) { return N % 16 == 0 && N / 16 <= 160; }
 
 void gs_skinny_run_residual(const void* X, int ldx, int x_tiled, const void* W, const void* Wt, float* res, float* ssq_out,
                             const float* next_w, void* xs_out, int xs_tiled, int M, int N, int K, hipStream_t stream) {

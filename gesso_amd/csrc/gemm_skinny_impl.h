@@ -134,7 +134,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16* __r
 #pragma unroll
     for (int r = 0; r < R; ++r) rowbase[r] = n0 + r * 16;
   }
-  static_assert(SHUF != 2 || (R == 1 && EPI == 2) || EPI == 3, "half tiles are written for the residual and the convolution epilogues");
+  static_assert(SHUF != 2 || (R == 1 && (EPI == 0 || EPI == 2)) || EPI == 3, "half tiles are written for plain products and for the residual and the convolution epilogues");
   const bool wact = SHUF != 2 || r16 < 8;  // half tiles: the lanes of the other eight rows load nothing
   const bf16* wrow[R];
 #pragma unroll
@@ -547,7 +547,7 @@ _Pragma("unroll")                                                               
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         const int n = rowbase[r] + kg * 4;
-        if (N - n > 0) store4<TOut>(Yp + (size_t)m * ldy + n, acc[r][mt], N - n);
+        if (N - n > 0 && half_ok) store4<TOut>(Yp + (size_t)m * ldy + n, acc[r][mt], N - n);
       }
     } else if (EPI == 1) {
       if (!live) continue;
@@ -685,6 +685,23 @@ static void skinny_plain(const SkinnyCall& c) {
     if (pro) { if (f32) { GS_BY_MT4(2, 8, 8, 4, 4, 1, 0, float, blocks) } else { GS_BY_MT4(2, 8, 8, 4, 4, 1, 0, bf16, blocks) } }
     else     { if (f32) { GS_BY_MT4(2, 8, 8, 4, 4, 0, 0, float, blocks) } else { GS_BY_MT4(2, 8, 8, 4, 4, 0, 0, bf16, blocks) } }
   }
+}
+
+// A plain product of a weight of few rows, half a tile a block (up to 32 rows of X: two row tiles).
+static void skinny_plain_halves(const SkinnyCall& c) {
+  constexpr int SHUF = 2;
+  const int blocks = gs_ceil_div(c.N, 8);
+#define GS_HALF(MT, PRO, TOut) \
+  launch_skinny<1, MT, 8, PRO, 0, SHUF, TOut>(blocks, c.x, c.ldx, c.w, (TOut*)c.Y, c.ldy, c.M, c.N, c.K, c.ex, c.stream)
+#define GS_HALF_PRO(MT, TOut) \
+  if (c.ex.res) GS_HALF(MT, 1, TOut); else GS_HALF(MT, 0, TOut)
+  if (c.y_dtype == GS_F32) {
+    if (c.M <= 16) { GS_HALF_PRO(1, float); } else { GS_HALF_PRO(2, float); }
+  } else {
+    if (c.M <= 16) { GS_HALF_PRO(1, bf16); } else { GS_HALF_PRO(2, bf16); }
+  }
+#undef GS_HALF_PRO
+#undef GS_HALF
 }
 
 template <int SHUF>

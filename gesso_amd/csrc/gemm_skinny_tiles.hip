@@ -7,3 +7,4 @@ void gs_skinny_residual_half_tiles(const SkinnyCall& c) { skinny_residual<2>(c);
 void gs_skinny_conv_tiles(const SkinnyCall& c) { skinny_conv<1>(c); }
 void gs_skinny_conv_half_tiles(const SkinnyCall& c) { skinny_conv<2>(c); }
 void gs_skinny_parts_tiles(const SkinnyCall& c, int parts) { skinny_parts<1>(c, parts); }
+void gs_skinny_plain_half_tiles(const SkinnyCall& c) { skinny_plain_halves(c); }
