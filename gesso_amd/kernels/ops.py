@@ -654,6 +654,27 @@ def gemm_tiled(x: torch.Tensor, w: torch.Tensor, bias=None, out_dtype=None, out:
     return out
 
 
+def mid_ok(x, w: torch.Tensor, wt, swiglu: bool = False) -> bool:
+    """Whether the product of some hundred rows is the kernel's that reads the weight's tile-major copy ``wt``: bfloat16,
+    aligned rows, and sizes for which it is the faster one."""
+    return (wt is not None and isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 and x.dim() == 2 and x.stride(1) == 1
+            and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
+            and bool(lib().gs_gemm_mid_takes(x.shape[0], w.shape[0], w.shape[1], 1 if swiglu else 0)))
+
+
+def gemm_mid(x, w: torch.Tensor, wt, swiglu: bool = False, out: torch.Tensor = None) -> torch.Tensor:
+    """``x @ w.T`` in bfloat16, or ``silu(gate) * up`` of it, for products :func:`mid_ok` takes."""
+    M, K = x.shape
+    N = w.shape[0]
+    _need(w.shape == (N, K) and wt.shape == w.shape and wt.dtype == torch.bfloat16 and wt.is_cuda, "gemm_mid: a weight (N, K) and its tile-major copy")
+    cols = N // 2 if swiglu else N
+    if out is None:
+        out = torch.empty((M, cols), dtype=torch.bfloat16, device=x.device)
+    _need(out.shape == (M, cols) and out.dtype == torch.bfloat16 and out.stride(1) == 1, "gemm_mid: out has the wrong shape or type")
+    _check(lib().gs_gemm_mid(_p(x), x.stride(0), _p(wt), _p(out), out.stride(0), M, N, K, 1 if swiglu else 0, _stream()))
+    return out
+
+
 def mfma_ok(x, w: torch.Tensor) -> bool:
     """Whether the matrix-core product for many rows takes these operands (bfloat16, K a multiple of 8, aligned)."""
     return (isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2

@@ -202,6 +202,10 @@ class Runtime:
             if ops.skinny_ok(x, w):
                 return ops.gemm_skinny(x, w, out_dtype=out_dtype, out=out, wt=self.tiles_of(w))
             library = out_dtype == torch.bfloat16 and not self.no_library and self.many_rows != "own"
+            if library and self.many_rows == "auto" and (out is None or (out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0)):
+                wt = self.tiles_of(w)
+                if ops.mid_ok(x, w, wt):
+                    return ops.gemm_mid(x, w, wt, out=out)
             if library:
                 return self._library_product(x, w, out)
             if self.many_rows != "library" and ops.mfma_ok(x, w) and (out is None or out.is_contiguous()):
@@ -249,6 +253,8 @@ class Runtime:
         if ((self.many_rows == "own" or (self.no_library and self.many_rows != "library"))
                 and self.dtype == torch.bfloat16 and ops.mfma_ok(x, w13) and w13.shape[0] % 2 == 0):
             return ops.gemm_mfma(x, w13, swiglu=True)          # gate|up never goes to memory
+        if self.many_rows == "auto" and not self.no_library and ops.mid_ok(x, w13, self.tiles_of(w13), swiglu=True):
+            return ops.gemm_mid(x, w13, self.tiles_of(w13), swiglu=True)
         return ops.swiglu(self.linear(x, w13))
 
     def project(self, x: torch.Tensor, w: torch.Tensor, bias=None):

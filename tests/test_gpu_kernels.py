@@ -436,6 +436,34 @@ def test_float32_product_on_the_matrix_cores_adds_in_the_tiled_kernels_order(ops
     assert torch.equal(room[1:M + 1], want) and bool((room[0] == 7).all() and (room[M + 1] == 7).all())
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 32, 32), (96, 64, 96), (97, 1024, 1024), (192, 3072, 64), (193, 160, 992), (333, 9216, 96), (512, 1056, 2048),
+                                   (1000, 96, 2016), (130, 16384, 160), (2000, 32, 128)])
+def test_product_of_some_hundred_rows_from_the_tile_major_weight(ops, M, N, K):
+    """Rows that fill no tile, weights of a few tiles and of many, K that ends within a step, plain and with SwiGLU; what the
+    choice by sizes does not take is refused."""
+    g = gen(M + N + K)
+    x = torch.randn(M + 1, K + 8, generator=g).bfloat16().to(DEV)[:M, :K]              # rows of a wider buffer
+    w = (torch.randn(N, K, generator=g) / math.sqrt(K)).bfloat16().to(DEV)
+    wt = ops.tile_major(w)
+    want = x.double().cpu() @ w.double().cpu().T
+    gate, up = want[:, :N // 2].bfloat16().double(), want[:, N // 2:].bfloat16().double()
+    room = torch.full((M + 2, N), 7.0, dtype=torch.bfloat16, device=DEV)
+    assert ops.mid_ok(x, w, wt) and ops.mid_ok(x, w, wt, swiglu=True)
+    ops.gemm_mid(x, w, wt, out=room[1:M + 1])
+    close(room[1:M + 1], want, torch.bfloat16)
+    assert bool((room[0] == 7).all() and (room[M + 1] == 7).all())
+    close(ops.gemm_mid(x, w, wt, swiglu=True), gate * torch.sigmoid(gate) * up, torch.bfloat16, scale=2)
+
+
+def test_product_of_some_hundred_rows_leaves_the_others_alone(ops):
+    from gesso_amd.errors import KernelError
+    for M, N, K in ((64, 1024, 1024), (192, 1024, 4608), (2048, 16384, 2048)):
+        assert not ops.lib().gs_gemm_mid_takes(M, N, K, 0)
+        x, w = torch.zeros(M, K, dtype=torch.bfloat16, device=DEV), torch.zeros(N, K, dtype=torch.bfloat16, device=DEV)
+        with pytest.raises(KernelError):
+            ops.gemm_mid(x, w, w)
+
+
 # ------------------------------------------------------------------ choosing tokens
 
 def test_argmax_rows(ops):
