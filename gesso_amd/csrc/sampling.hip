@@ -138,18 +138,25 @@ struct Crossing {
 // 0x3F: a weight is at most 1), then 256 for the second byte under each first byte from 0x3C on; after these
 // NUC_GHIST sums the counts, in the same order.  Where the first byte's crossing falls below 2^-63 the passes start
 // again and read the row themselves.
+// Above its low NUC_COUNT bits a count holds a bit for each span of NUC_SPAN ids that has a weight in that bucket (rows of
+// up to NUC_SPANS spans; longer ones: none), so that the ids of a bucket are looked for where there are any.
 #define NUC_G0 8
 #define NUC_GHIST (NUC_G0 + 4 * 256)
+#define NUC_COUNT 24
+#define NUC_SPAN 4096
+#define NUC_SPANS 40
 __device__ Crossing radix_descend(const double* __restrict__ w, int V, double target, int strict,
                                   unsigned long long* hmass, int* hcount, Crossing* shared_out, int* clist,
                                   unsigned long long* lbits, const unsigned long long* __restrict__ ghist = nullptr) {
   __shared__ int cn, picked;
+  __shared__ unsigned long long in_spans;       // the spans that hold the second byte's bucket; 0: not known
   __shared__ unsigned long long cbits[NUC_DIRECT], cmass[NUC_DIRECT];
   unsigned long long prefix = 0;
   double above = 0.0;
   int lv = 1;                                   // V <= 2^lv
   while ((1 << lv) < V && lv < 30) ++lv;
   int nlist = -1;                               // ids in the list, or -1: no list yet
+  const unsigned long long counts = V < 1 << NUC_COUNT ? (1ull << NUC_COUNT) - 1ull : ~0ull;   // (longer rows: no marks)
   for (int pass = 0; pass < 8; ++pass) {
     int shift = 56 - 8 * pass;
     for (int b = threadIdx.x; b < 256; b += blockDim.x) {
@@ -170,13 +177,13 @@ __device__ Crossing radix_descend(const double* __restrict__ w, int V, double ta
     if (ready && pass == 0) {
       for (int b = threadIdx.x; b < 5; b += blockDim.x) {
         hmass[0x3B + b] = ghist[b];
-        hcount[0x3B + b] = (int)ghist[NUC_GHIST + b];
+        hcount[0x3B + b] = (int)(ghist[NUC_GHIST + b] & counts);
       }
     } else if (ready) {
       const int under = (int)(prefix >> 56) - 0x3C;
       for (int b = threadIdx.x; b < 256; b += blockDim.x) {
         hmass[b] = ghist[NUC_G0 + under * 256 + b];
-        hcount[b] = (int)ghist[NUC_GHIST + NUC_G0 + under * 256 + b];
+        hcount[b] = (int)(ghist[NUC_GHIST + NUC_G0 + under * 256 + b] & counts);
       }
     }
     const int n = ready ? 0 : (nlist >= 0 ? nlist : V);
@@ -245,6 +252,8 @@ __device__ Crossing radix_descend(const double* __restrict__ w, int V, double ta
         shared_out->above = above + (double)(before + run[i] - m[i]) * unscale;
         picked = c[i];
         cn = 0;
+        if (pass == 0) in_spans = 0ull;
+        if (pass == 1 && ready) in_spans = ghist[NUC_GHIST + NUC_G0 + ((int)(prefix >> 56) - 0x3C) * 256 + pick] >> NUC_COUNT;
       }
     }
     __syncthreads();
@@ -266,17 +275,32 @@ __device__ Crossing radix_descend(const double* __restrict__ w, int V, double ta
       // a thread are asked for before the first is looked at (a turn of the loop is otherwise a round trip to memory,
       // 64 of them a row; loads of two weights, and sixteen in flight, need more registers than 1,024 threads leave
       // a lane and came out slower: 72 to 80 us against 64 for the step's three kernels on peaked rows).
-      constexpr int GATHER = 8;
-      for (int j0 = 0; j0 < V; j0 += GATHER * blockDim.x) {   // every thread makes every turn: the wavefront votes
+      // Two spans a turn, and only those that hold the bucket (a peaked row's nucleus ends in a bucket of a few ids: one turn
+      // instead of eight; a step's pick over 12 rows that draw 43 us without, 31 with).
+      constexpr int GATHER = 8, HALF = GATHER / 2;
+      static_assert(HALF * SAMP_THREADS == NUC_SPAN, "a span is what a block loads in half a turn");
+      const int nspan = (V + NUC_SPAN - 1) / NUC_SPAN;
+      unsigned long long held = in_spans;
+      const bool known = held != 0ull;
+      for (int turn = 0; known ? held != 0ull : 2 * turn < nspan; ++turn) {   // every thread makes every turn: the wavefront votes
+        int at[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          at[q] = 2 * turn + q;
+          if (known) {
+            at[q] = held ? __ffsll((long long)held) - 1 : nspan;              // (past the row: nothing)
+            held &= held - 1ull;
+          }
+        }
         unsigned long long got[GATHER];
 #pragma unroll
         for (int g = 0; g < GATHER; ++g) {
-          const int j = j0 + g * blockDim.x + threadIdx.x;
+          const int j = at[g / HALF] * NUC_SPAN + (g % HALF) * SAMP_THREADS + threadIdx.x;
           got[g] = j < V ? (unsigned long long)__double_as_longlong(w[j]) : 0ull;
         }
 #pragma unroll
         for (int g = 0; g < GATHER; ++g) {
-          const int j = j0 + g * blockDim.x + threadIdx.x;
+          const int j = at[g / HALF] * NUC_SPAN + (g % HALF) * SAMP_THREADS + threadIdx.x;
           const bool take = j < V && (got[g] & sofar) == prefix;
           const unsigned long long votes = __ballot(take);
           if (votes) {
@@ -511,6 +535,7 @@ extern "C" int gs_decode_choose(const float* logits, int rows, int V, int* count
 // from the same weights.  part: rows x nparts float64, nparts = gs_choice_parts(V).
 #define WIDE_CH 4
 #define WIDE_SPAN (SAMP_THREADS * WIDE_CH)
+static_assert(WIDE_SPAN == NUC_SPAN, "a block of choose_weights_kernel weighs a span");
 
 extern "C" int gs_choice_parts(int V) { return ((V + WIDE_SPAN - 1) / WIDE_SPAN) * SAMP_THREADS; }
 
@@ -564,27 +589,51 @@ __global__ __launch_bounds__(SAMP_THREADS) void choose_weights_kernel(
       int lv = 1;
       while ((1 << lv) < V && lv < 30) ++lv;
       const double scale0 = exp2((double)(62 - lv));
+      // The first byte has five sums, and nearly all of a wavefront's weights share two of them: an atomic add a weight would
+      // queue up on one address (150 rows of 65,536 drawing: 83 us a step; like this 56; 12 rows: 16 and 11).  So a wavefront adds up
+      // its weights of each first byte that it holds (integers: the order does not matter) and one lane adds the sum.
+      unsigned long long m0[WIDE_CH];
+      int i0[WIDE_CH];
 #pragma unroll
       for (int k = 0; k < WIDE_CH; ++k) {
-        if (j0 + k >= V) continue;
-        const unsigned long long bits = (unsigned long long)__double_as_longlong(w[k]);
-        const int b0 = (int)(bits >> 56);
-        const int i0 = b0 < 0x3C ? 0 : b0 - 0x3B;
-        atomicAdd(&lm[i0], (unsigned long long)__double2ll_rn(w[k] * scale0));
-        atomicAdd(&lc[i0], 1);
-        if (b0 >= 0x3C) {
-          const double wmax = __longlong_as_double((long long)(((unsigned long long)b0 << 56) | ((1ull << 56) - 1ull)));
-          const int i1 = NUC_G0 + (b0 - 0x3C) * 256 + (int)((bits >> 48) & 0xff);
-          atomicAdd(&lm[i1], (unsigned long long)__double2ll_rn(w[k] * (scale0 / wmax)));
-          atomicAdd(&lc[i1], 1);
+        const int b0 = (int)((unsigned long long)__double_as_longlong(w[k]) >> 56);
+        i0[k] = j0 + k < V ? (b0 < 0x3C ? 0 : b0 - 0x3B) : -1;
+        m0[k] = (unsigned long long)__double2ll_rn(w[k] * scale0);
+      }
+      for (int f = 0; f < 5; ++f) {
+        int held = 0;
+        unsigned long long m = 0ull;
+#pragma unroll
+        for (int k = 0; k < WIDE_CH; ++k) {
+          held += __popcll(__ballot(i0[k] == f));
+          m += i0[k] == f ? m0[k] : 0ull;
         }
+        if (held == 0) continue;                             // (the same for the whole wavefront)
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) m += __shfl_xor(m, o, 64);
+        if ((threadIdx.x & 63) == 0) {
+          atomicAdd(&lm[f], m);
+          atomicAdd(&lc[f], held);
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < WIDE_CH; ++k) {
+        if (i0[k] < 1) continue;
+        const unsigned long long bits = (unsigned long long)__double_as_longlong(w[k]);
+        const int b0 = i0[k] + 0x3B;
+        const double wmax = __longlong_as_double((long long)(((unsigned long long)b0 << 56) | ((1ull << 56) - 1ull)));
+        const int i1 = NUC_G0 + (b0 - 0x3C) * 256 + (int)((bits >> 48) & 0xff);
+        atomicAdd(&lm[i1], (unsigned long long)__double2ll_rn(w[k] * (scale0 / wmax)));
+        atomicAdd(&lc[i1], 1);
       }
       __syncthreads();
       unsigned long long* g = ghist + (size_t)row * 2 * NUC_GHIST;
+      const bool marks = gridDim.x <= NUC_SPANS && V < 1 << NUC_COUNT;
       for (int i = threadIdx.x; i < NUC_GHIST; i += blockDim.x)
         if (lc[i]) {
           atomicAdd(&g[i], lm[i]);
-          atomicAdd(&g[NUC_GHIST + i], (unsigned long long)lc[i]);
+          // (a block is a span: its bit is added once)
+          atomicAdd(&g[NUC_GHIST + i], (unsigned long long)lc[i] + (marks ? 1ull << (NUC_COUNT + blockIdx.x) : 0ull));
         }
     }
   }

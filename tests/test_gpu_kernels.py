@@ -569,6 +569,27 @@ def test_sample_top_p_gives_the_same_id_every_time_and_at_the_models_vocabulary(
         assert first[r].item() == P.sample_id(logits[r].tolist(), 0.9, 0.73, 40 + r)[0], r
 
 
+@pytest.mark.parametrize("V", [4096, 8193, 163840, 163841])
+def test_the_choices_nucleus_is_looked_for_in_the_spans_that_hold_it(ops, V):
+    """Rows of one span of 4,096 ids, of a few and of the most that have a mark each, and of one more (none have): nuclei that
+    end among a few heavy ids in the first, a middle and the last span, and among thousands everywhere."""
+    rows = 6
+    logits = torch.randn(rows, V, generator=gen(V)) * 0.5
+    for r, ids in enumerate(([3], [V - 1], [V // 2, 1, V - 2], [V // 3, V // 3 + 1, V - 1, 0], [])):
+        for i, at in enumerate(ids):
+            logits[r, at] = 14.0 - 0.3 * i
+    temp, top_p = [1.0] * rows, [0.5, 0.9, 0.9, 0.99, 0.8, 0.3]
+    u = torch.tensor([[P.splitmix64_unit(60 + r)[1] for r in range(rows)]], dtype=torch.float64)
+    i32 = lambda *a: torch.tensor(*a, dtype=torch.int32, device=DEV)
+    ring, bad = i32([[-1] * rows]), i32([[-1] * rows])
+    scratch = (torch.empty(rows * ops.choice_parts(V), dtype=torch.float64, device=DEV), i32([7] * rows), i32([7] * rows),
+               torch.full((rows * ops.choice_hist(),), 12345, dtype=torch.int64, device=DEV))
+    ops.decode_choose(logits.to(DEV), torch.tensor(temp, dtype=torch.float64).to(DEV), u.to(DEV), i32([0] * rows), i32([0] * rows), ring, bad,
+                      i32([0] * rows), i32([1] * rows), i32([1] * rows), scratch, top_p=torch.tensor(top_p, dtype=torch.float64).to(DEV),
+                      wbuf=torch.empty(rows * V, dtype=torch.float64, device=DEV))
+    assert not bad.any() and ring[0].tolist() == [P.sample_id(logits[r].tolist(), 1.0, top_p[r], 60 + r)[0] for r in range(rows)]
+
+
 @pytest.mark.parametrize("V", [777, 9000, 65536])
 def test_the_decode_loops_choice_draws_greedy_plain_and_nucleus_rows_side_by_side(ops, V):
     """What the recorded decode step ends with when rows draw (three kernels, the weights by many blocks): rows that are
