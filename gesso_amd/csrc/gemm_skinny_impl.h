@@ -52,6 +52,14 @@ typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
 __device__ __forceinline__ bf16x8_t load8(const bf16* p) { return *reinterpret_cast<const bf16x8_t*>(p); }
 
+// A piece of weight.  Of the tile-major copy it is loaded non-temporally: whole lines, each read by one compute unit and not
+// again in the step (a step at LFM2-1.2B sizes: 3.5 to 5 % shorter at 1 and 8 rows, 1.8 % at 64; the decode attention's keys,
+// whose lines two loads share, loaded like that: 2 to 3 % longer).  As rows of K a line is read in pieces, by several loads.
+template <int SHUF>
+__device__ __forceinline__ bf16x8_t load8w(const bf16* p) {
+  return SHUF ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(p)) : load8(p);
+}
+
 __device__ __forceinline__ bf16x8_t zero8() {
   bf16x8_t z;
 #pragma unroll
@@ -365,7 +373,7 @@ _Pragma("unroll")                                                               
 #pragma unroll
         for (int u = 0; u < U; ++u) {
 #pragma unroll
-          for (int r = 0; r < R; ++r) a[u][r] = wact ? load8(wrow[r] + (size_t)(s + u) * WSTEP) : zero8();
+          for (int r = 0; r < R; ++r) a[u][r] = wact ? load8w<SHUF>(wrow[r] + (size_t)(s + u) * WSTEP) : zero8();
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt) b[u][mt] = xok[mt] ? load_x(mt, s + u) : zero8();
         }
@@ -386,7 +394,7 @@ _Pragma("unroll")                                                               
 #pragma unroll
         for (int u = 0; u < U; ++u) {
 #pragma unroll
-          for (int r = 0; r < R; ++r) a[u][r] = wact ? load8(wrow[r] + (size_t)(s + u) * WSTEP) : zero8();
+          for (int r = 0; r < R; ++r) a[u][r] = wact ? load8w<SHUF>(wrow[r] + (size_t)(s + u) * WSTEP) : zero8();
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt) b[u][mt] = xok[mt] ? load_x(mt, s + u) : zero8();
         }
@@ -412,7 +420,7 @@ _Pragma("unroll")                                                               
       for (int r = 0; r < R; ++r) {
         // every lane loads (its address is a valid one): a load under a lane mask would hide from the
         // compiler how many loads are in flight, and it would wait for all of them
-        const bf16x8_t v = load8(wrow[r] + (size_t)step * WSTEP);
+        const bf16x8_t v = load8w<SHUF>(wrow[r] + (size_t)step * WSTEP);
         a[u][r] = (SHUF != 2 || wact) ? v : zero8();
       }
       // rows past M read row 0 or the padding of the last tile; their columns of the result are never stored
@@ -449,7 +457,7 @@ _Pragma("unroll")                                                               
     for (int mt = 0; mt < MT; ++mt) b[mt] = (kin && xok[mt]) ? load_x(mt, s) : zero8();
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      bf16x8_t a = ((kin || SHUF) && wact) ? load8(wrow[r] + (size_t)s * WSTEP) : zero8();
+      bf16x8_t a = ((kin || SHUF) && wact) ? load8w<SHUF>(wrow[r] + (size_t)s * WSTEP) : zero8();
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) acc[r][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[mt], acc[r][mt], 0, 0, 0);
     }
