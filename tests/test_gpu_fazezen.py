@@ -50,7 +50,7 @@ def folders(tmp_path_factory):
 # ------------------------------------------------------------------ kernels alone
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("H", [100, 256, 1030])
+@pytest.mark.parametrize("H", [100, 256, 1030, 2040, 2056])
 def test_two_adds_and_two_norms_of_one_row(ops, dtype, H):
     res = torch.randn(5, H, generator=gen(0))
     d1, d2 = (torch.randn(5, H, generator=gen(1)) * 2).to(dtype), torch.randn(5, H, generator=gen(2)).to(dtype)
@@ -258,6 +258,21 @@ def test_norm_and_gate_of_the_heads(ops, dtype, joint, gate):
     y = P.rms(od, 1e-5) * w.double() if joint else P.rms(od.reshape(T, H, m), 1e-5).reshape(T, H * m)
     want = y * (torch.sigmoid(z) if gate == "sigmoid" else P.silu(z))
     assert float((got - want).abs().max()) <= tol(dtype, want)
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,m,joint", [(16, 128, True), (17, 128, True), (3, 1000, True), (33, 160, True), (9, 256, False), (5, 258, False), (16, 128, False)])
+def test_norm_and_gate_of_rows_held_in_pieces(ops, dtype, H, m, joint):
+    """Joint rows of one, two and more pieces of eight values a thread; heads of up to four values a lane and of more."""
+    T = 3
+    o = torch.randn(T, H * m, generator=gen(22)) * 4
+    rows = torch.randn(T, 8 + H * m, generator=gen(23)).to(dtype)
+    w = 1 + 0.3 * torch.randn(H * m, generator=gen(24)) if joint else None
+    got = ops.gated_outnorm(o.to(DEV), rows.to(DEV), 8, w.to(DEV) if joint else None, 1e-5, H, m, joint, "silu", dtype).cpu().double()
+    od, z = o.double(), rows.double()[:, 8:]
+    want = (P.rms(od, 1e-5) * w.double() if joint else P.rms(od.reshape(T, H, m), 1e-5).reshape(T, H * m)) * z * torch.sigmoid(z)
+    # float32: a few roundings of each factor; bfloat16: one rounding of the result, 2^-9 of it
+    assert float(((got - want).abs() / want.abs().clamp_min(1e-3)).max()) <= (2.0 ** -8 if dtype == torch.bfloat16 else 2e-5)
+
 
 
 def tables(dims, base, P_max, freqs=None):

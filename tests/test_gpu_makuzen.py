@@ -74,7 +74,7 @@ def paged(rows, page_size, num_pages, seed, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("qr,c,r", [(40, 48, 8), (28, 36, 6), (64, 128, 32), (20, 40, 0)])
+@pytest.mark.parametrize("qr,c,r", [(40, 48, 8), (28, 36, 6), (64, 128, 32), (20, 40, 0), (1024, 512, 64), (768, 1030, 8)])
 def test_latent_prep_norms_rotates_and_writes_the_cache_row(ops, dtype, qr, c, r):
     T, ps, extra = 21, 8, 5
     down = (torch.randn(T, qr + c + r + extra, generator=gen(3)) * 2).to(dtype)
