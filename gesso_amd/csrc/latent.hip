@@ -247,12 +247,12 @@ __global__ void heads_product_kernel(const TX* __restrict__ X, int ldx, int hx, 
 // The same product on the matrix cores (bfloat16 rows and weights, float32 sums): v_mfma_f32_16x16x32_bf16 with both
 // operands loaded straight from memory in operand order (lane l: row or weight row l % 16, eight consecutive k at
 // 8 (l / 16)); a head's weight is small and stays in the caches, so nothing is staged.  A wavefront owns 16 MTW rows x
-// 16 NTW columns of one head; the four wavefronts of a block own four such pieces, and no barrier is needed.
+// 16 NTW columns of one head; the wavefronts of a block own such pieces of their own, and no barrier is needed.
 typedef __attribute__((ext_vector_type(8))) __bf16 hp_bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float hp_f32x4_t;
 typedef __attribute__((ext_vector_type(4))) unsigned hp_u32x4_t;
 
-template <int NTW, int MTW>
+template <int NTW, int MTW, int DEPTH>
 __global__ __launch_bounds__(256) void heads_product_mfma_kernel(const bf16* __restrict__ X, int ldx, int hx,
                                                                  const bf16* __restrict__ W, bf16* __restrict__ Y,
                                                                  int ldy, int hy, const bf16* __restrict__ G, int ldg,
@@ -260,7 +260,7 @@ __global__ __launch_bounds__(256) void heads_product_mfma_kernel(const bf16* __r
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, g = lane >> 4;
   const int h = blockIdx.y;
   const int mtiles = (M + 16 * MTW - 1) / (16 * MTW), ngroups = (N + 16 * NTW - 1) / (16 * NTW);
-  const int item = blockIdx.x * 4 + wave;
+  const int item = blockIdx.x * (blockDim.x >> 6) + wave;
   if (item >= mtiles * ngroups) return;
   const int m0 = (item % mtiles) * 16 * MTW, n0 = (item / mtiles) * 16 * NTW;
   const bf16* xp[MTW];
@@ -280,28 +280,30 @@ __global__ __launch_bounds__(256) void heads_product_mfma_kernel(const bf16* __r
   for (int i = 0; i < MTW; ++i)
 #pragma unroll
     for (int j = 0; j < NTW; ++j) acc[i][j] = hp_f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-  for (int k0 = 0; k0 < K; k0 += 32) {
-    const bool in = k0 + 8 * g < K;                      // K in whole pieces of 8: a piece is inside or outside
-    const int kk = in ? k0 : -8 * g;
-    hp_u32x4_t a[MTW];
+  // the loads of DEPTH steps of 32 k are issued before the first is multiplied (a piece beyond K is read from the row's start
+  // and counts as zeros: that is put in behind the loads, where a test between them would wait for each)
+  for (int k0 = 0; k0 < K; k0 += 32 * DEPTH) {
+    hp_u32x4_t a[DEPTH][MTW], b[DEPTH][NTW];
 #pragma unroll
-    for (int i = 0; i < MTW; ++i) {
-      a[i] = *reinterpret_cast<const hp_u32x4_t*>(xp[i] + kk);
-      a[i] = in ? a[i] : hp_u32x4_t{0u, 0u, 0u, 0u};
+    for (int d = 0; d < DEPTH; ++d) {
+      const int k = k0 + 32 * d, kk = k + 8 * g < K ? k : -8 * g;      // K in whole pieces of 8: a piece is inside or outside
+#pragma unroll
+      for (int i = 0; i < MTW; ++i) a[d][i] = *reinterpret_cast<const hp_u32x4_t*>(xp[i] + kk);
+#pragma unroll
+      for (int j = 0; j < NTW; ++j) b[d][j] = *reinterpret_cast<const hp_u32x4_t*>(wp[j] + kk);
     }
-    hp_u32x4_t b[NTW];
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int j = 0; j < NTW; ++j) {
-      b[j] = *reinterpret_cast<const hp_u32x4_t*>(wp[j] + kk);
-      b[j] = in ? b[j] : hp_u32x4_t{0u, 0u, 0u, 0u};
+    for (int d = 0; d < DEPTH; ++d) {
+      const bool in = k0 + 32 * d + 8 * g < K;
+#pragma unroll
+      for (int i = 0; i < MTW; ++i)
+#pragma unroll
+        for (int j = 0; j < NTW; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(hp_bf16x8_t, in ? a[d][i] : hp_u32x4_t{0u, 0u, 0u, 0u}),
+              __builtin_bit_cast(hp_bf16x8_t, in ? b[d][j] : hp_u32x4_t{0u, 0u, 0u, 0u}), acc[i][j], 0, 0, 0);
     }
-#pragma unroll
-    for (int i = 0; i < MTW; ++i)
-#pragma unroll
-      for (int j = 0; j < NTW; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(hp_bf16x8_t, a[i]),
-                                                            __builtin_bit_cast(hp_bf16x8_t, b[j]), acc[i][j], 0, 0, 0);
   }
 #pragma unroll
   for (int i = 0; i < MTW; ++i)
@@ -336,13 +338,23 @@ extern "C" int gs_heads_product(const void* X, int x_dtype, int ldx, int hx, con
     const int ntw = M <= 64 ? 1 : 4, mtw = M <= 64 ? 1 : 2;
     const int mtiles = gs_ceil_div(M, 16 * mtw);
     const long items = (long)mtiles * gs_ceil_div(N, 16 * ntw);
-    GS_REQUIRE(items / 4 + 1 < (1L << 31), "heads_product: too many tiles");
-    dim3 grid((unsigned)gs_ceil_div(items, 4), H);
-    if (ntw == 1)
-      heads_product_mfma_kernel<1, 1><<<grid, 256, 0, stream>>>((const bf16*)X, ldx, hx, (const bf16*)W, (bf16*)Y, ldy, hy,
-                                                            (const bf16*)G, ldg, gate_each, M, N, K);
+    GS_REQUIRE(items + 1 < (1L << 31), "heads_product: too many tiles");
+    // (few pieces: a wavefront a block, so that they spread over as many compute units)
+    const int waves = ntw == 1 && items * H < 1024 ? 1 : 4;
+    dim3 grid((unsigned)gs_ceil_div(items, waves), H);
+    // (few rows: all of K in flight up to 512, little loaded for nothing where it is short; 8 rows, 16 heads of 512 x 128 and
+    // 128 x 512 in a step: 4.7 us each in the mean, with four steps at a time, each waiting for its own, in blocks of four 7.3)
+    if (ntw == 1 && K <= 64)
+      heads_product_mfma_kernel<1, 1, 2><<<grid, 64 * waves, 0, stream>>>((const bf16*)X, ldx, hx, (const bf16*)W, (bf16*)Y, ldy, hy,
+                                                                          (const bf16*)G, ldg, gate_each, M, N, K);
+    else if (ntw == 1 && K <= 128)
+      heads_product_mfma_kernel<1, 1, 4><<<grid, 64 * waves, 0, stream>>>((const bf16*)X, ldx, hx, (const bf16*)W, (bf16*)Y, ldy, hy,
+                                                               (const bf16*)G, ldg, gate_each, M, N, K);
+    else if (ntw == 1)
+      heads_product_mfma_kernel<1, 1, 16><<<grid, 64 * waves, 0, stream>>>((const bf16*)X, ldx, hx, (const bf16*)W, (bf16*)Y, ldy, hy,
+                                                                (const bf16*)G, ldg, gate_each, M, N, K);
     else
-      heads_product_mfma_kernel<4, 2><<<grid, 256, 0, stream>>>((const bf16*)X, ldx, hx, (const bf16*)W, (bf16*)Y, ldy, hy,
+      heads_product_mfma_kernel<4, 2, 2><<<grid, 64 * waves, 0, stream>>>((const bf16*)X, ldx, hx, (const bf16*)W, (bf16*)Y, ldy, hy,
                                                             (const bf16*)G, ldg, gate_each, M, N, K);
     GS_LAUNCH_CHECK("heads_product_mfma");
     return 0;

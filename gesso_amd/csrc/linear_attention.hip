@@ -10,9 +10,10 @@
 // host), and k may be scaled, all in float32: what enters the state is never rounded to the activation type again.
 //
 // linear_attention_scan: one block per (sequence, head, tile of 64 value columns); the columns of S are independent
-// of each other, so wide values share out over blocks.  Thread (rg, jl) = (tid & 3, tid >> 2) holds the state's rows
-// rg, rg + 4, ... of column jl in registers; the four partial sums of a column's output are neighbours in a
-// wavefront.  A step's tokens come through LDS eight at a time.  The sums run in one fixed order per output, whatever
+// of each other, so wide values share out over blocks.  Lane l of wavefront w holds the state's rows rg, rg + 4, ...
+// (rg = l / 16) of column 16 w + l % 16 in registers, so that sixteen lanes move 64 contiguous bytes of a row (8 rows, 16
+// heads of 128 x 128: 10.9 us; neighbouring lanes in neighbouring rows 11.4); the four partial sums of a column's output lie
+// sixteen lanes apart.  A step's tokens come through LDS eight at a time.  The sums run in one fixed order per output, whatever
 // the step's cut: a sequence fed whole, in portions or token by token leaves the same state and outputs, bit for bit.
 // A step of single tokens is the same kernel with one token a block.  With `below` > 0 only the sequences that bring
 // fewer tokens than that are taken: the longer ones go to the kernel on the matrix cores (linear_attention_mfma.hip).
@@ -39,7 +40,7 @@ linear_attention_scan_kernel(const TI* __restrict__ x, int ld, int oq, int ok, i
   __shared__ float ks[LA_TB][NMAX];
   __shared__ float vs[LA_TB][LA_COLS];
   const int seq = blockIdx.x, h = blockIdx.y, j0 = blockIdx.z * LA_COLS;
-  const int tid = threadIdx.x, rg = tid & 3, jl = tid >> 2, j = j0 + jl;
+  const int tid = threadIdx.x, rg = (tid >> 4) & 3, jl = (tid >> 6) * 16 + (tid & 15), j = j0 + jl;
   const int t0 = q_start[seq], t1 = q_start[seq + 1];
   if (t1 <= t0 || (below > 0 && t1 - t0 >= below)) return;      // (longer sequences are another kernel's)
   const float d = decay[h];
@@ -89,8 +90,8 @@ linear_attention_scan_kernel(const TI* __restrict__ x, int ld, int oq, int ok, i
           part = fmaf(s[r], qs[tt][i], part);
         }
       }
-      part += __shfl_xor(part, 1, 64);
-      part += __shfl_xor(part, 2, 64);
+      part += __shfl_xor(part, 16, 64);
+      part += __shfl_xor(part, 32, 64);
       if (rg == 0 && j < m) out[((size_t)(tb + tt) * H + h) * m + j] = part;
     }
   }
