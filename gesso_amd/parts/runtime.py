@@ -2,11 +2,12 @@
 
 ``Runtime.linear`` is the one place where a matrix product is chosen:
 
-* float32 anywhere (activations, weight or wanted output) -> the tiled FMA kernel, which is the
-  true 32-bit product and also takes mixed storage (a weight stored in 32-bit stays so);
+* float32 anywhere (activations, weight or wanted output) -> ``gemm_tiled``, the true 32-bit product: the tiled
+  FMA kernel, which also takes mixed storage (a weight stored in 32-bit stays so), or for aligned float32 rows
+  the matrix cores in the same order of sums;
 * bfloat16 x bfloat16: the hand-written weight-streaming kernel for up to 64 rows; for more rows the
-  hand-written matrix-core kernel (``gemm_mfma``) or the vendor library through ``torch``, whichever
-  ``RuntimeOptions.many_rows`` says (the reference hands every matrix product to the vendor library,
+  hand-written matrix-core kernels (``gemm_mid`` for some hundred, ``gemm_mfma``) or the vendor library through
+  ``torch``, whichever ``RuntimeOptions.many_rows`` says (the reference hands every matrix product to the vendor library,
   ``ext/amdgpu_ops.jl:453-465``).
 
 What a mixer or a feed-forward does between its products is its own business (its file chooses its kernels);
@@ -28,8 +29,9 @@ class RuntimeOptions:
     """How kernels are chosen where more than one can do the work; given to the engine's constructor.
 
     ``many_rows``: products of more than 64 rows in bfloat16: ``"own"`` = the hand-written matrix-core kernel
-    everywhere (gate|up with SwiGLU in one kernel), ``"library"`` = the vendor's wherever it can go, ``"auto"`` = the
-    vendor's for bfloat16 results (measured on random data at 2,048 rows: 109 us against our 161 for gate|up, 124
+    everywhere (gate|up with SwiGLU in one kernel), ``"library"`` = the vendor's wherever it can go, ``"auto"`` = for
+    bfloat16 results of some hundred rows the hand-written kernel that reads the tile-major weight where it takes the
+    product (333 rows of 9216 x 1024 with SwiGLU: 16 us against 21), for other bfloat16 results the vendor's (measured on random data at 2,048 rows: 109 us against our 161 for gate|up, 124
     against 162 with the SwiGLU pass counted in; 50 against 75 for 6144 x 2048), ours where the result is float32 and
     inside the recording of the fused decode loop.
     ``tune_library``: where the vendor library computes a product of 128, 256, 512, 1024, ... rows (whole prompt portions, the decode loop for many rows),
