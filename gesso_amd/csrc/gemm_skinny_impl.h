@@ -9,7 +9,8 @@
 // output columns n for one token.
 //
 // A block of WAVES wavefronts owns R tiles of 16 rows of W; its wavefronts split K among themselves and
-// add their partial tiles through LDS in wavefront order.  Rows beyond N, tokens beyond M and k beyond K
+// add their partial tiles through LDS in wavefront order, each row tile's by a wavefront of its own, which
+// runs that row tile's epilogue.  Rows beyond N, tokens beyond M and k beyond K
 // are masked (K must be a multiple of 8 so that every 16-byte load is aligned).
 //
 // The weight is read either as it is stored, rows of K (SHUF = 0), or from a tile-major copy
@@ -29,7 +30,7 @@
 //   1  X is the RMSNorm of the float32 residual stream: x = res * inv_rms(row) * norm_weight, rounded to
 //      bfloat16 as the norm kernel would store it; the row's sum of squares comes as partial sums
 //      (row, nb), added in a fixed order.
-//   0 with partial sums given: X holds rows already multiplied by the norm's weight (res * norm_weight,
+//   2  X holds rows already multiplied by the norm's weight (res * norm_weight,
 //      written by the product that last added to the stream, EPI 2); the row's inverse root mean square,
 //      which no single block of that product knew, multiplies this product's result instead:
 //      (x inv) W^T = inv (x W^T).  The norm costs no kernel and no pass of its own.
@@ -123,8 +124,11 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16* __r
                                                                   TOut* __restrict__ Y, int ldy, int M, int N,
                                                                   int K, SkinnyExtra ex) {
   constexpr int SHUF = LAYOUT & ~SKINNY_ONCE;
-  extern __shared__ float red[];  // (WAVES - 1) x R x MT x 64 x 4 floats
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  extern __shared__ float red[];  // WAVES (one row tile: WAVES - 1) x R x MT x 64 x 4 floats
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  static_assert(WAVES >= MT, "a wavefront for each row tile's epilogue");
+  // wavefront w adds up and finishes row tile w
+  const int emt = MT > 1 ? wave : 0;
   const int r16 = lane & 15, kg = lane >> 4;
   const int half = N >> 1;
   // rows of W this block owns
@@ -176,10 +180,12 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16* __r
     xrow[mt] = nullptr;
     rrow[mt] = nullptr;
     inv[mt] = 0.f;
-    if (PRO == 0) {
-      xrow[mt] = ex.x_tiled ? X + (size_t)(mt * 64 + lane) * 8 : X + (size_t)(xok[mt] ? m : 0) * ldx + kg * 8;
+    if (PRO != 1) {
+      // (a row past M: the last, whose line a neighbour asks for anyway; its column of the result is never stored)
+      const int mc = m < M ? m : M - 1;
+      xrow[mt] = ex.x_tiled ? X + (size_t)((mc >> 4) * 64 + kg * 16 + (mc & 15)) * 8 : X + (size_t)mc * ldx + kg * 8;
     } else {
-      rrow[mt] = ex.res + (size_t)(xok[mt] ? m : 0) * K;
+      rrow[mt] = ex.res + (size_t)(xok[mt] ? m : M - 1) * K;
     }
     if (PRO == 1) {
       // the row's sum of squares: this lane group adds every fourth partial, then the four groups are added
@@ -196,28 +202,32 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16* __r
   // the rows; a lane adds every 64th partial sum and the wavefront adds its lanes (an order that depends on
   // nothing but the number of partials).  The first row's loads start here, under the product's own.
   __shared__ float inv_s[64];
-  const bool scaled = PRO == 0 && ex.ssq != nullptr;
-  float pre[4] = {0.f, 0.f, 0.f, 0.f};
+  constexpr bool scaled = PRO == 2;
+  // With two row tiles all of a wavefront's rows are asked for here: after the loop they were a round trip of their own
+  // (20 rows of 9216 x 1024 9.3 against 8.7 us).
+  constexpr int RPW = (MT * 16 + WAVES - 1) / WAVES;      // rows a wavefront
+  constexpr int EARLY = MT == 2 ? RPW : 1;
+  float pre[EARLY][4];
   if (scaled && wave < M) {
+    // (a row or a partial sum that does not exist is read from one that does and not counted: no load sits behind a branch)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (lane + 64 * j < ex.nb) pre[j] = ex.ssq[(size_t)wave * ex.nb + lane + 64 * j];
+    for (int i = 0; i < EARLY; ++i) {
+      const int m = wave + i * WAVES;
+      const float* row = ex.ssq + (size_t)(m < M ? m : M - 1) * ex.nb;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) pre[i][j] = row[lane + 64 * j < ex.nb ? lane + 64 * j : 0];
+    }
   }
 
   // The convolution's slots, by scalar loads (the row number is the same for every lane), each lane then picking its
   // row's: the history's addresses wait for them, and scalar loads return on a counter of their own.
-  int cslot[EPI == 3 ? MT : 1];
+  int cslot = 0;
   if (EPI == 3) {
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      int mine = 0;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int row = mt * 16 + i;
-        const int sv = ex.slots[row < M ? row : 0];
-        mine = r16 == i ? sv : mine;
-      }
-      cslot[mt] = mine;
+    for (int i = 0; i < 16; ++i) {
+      const int row = emt * 16 + i;
+      const int sv = ex.slots[row < M ? row : 0];
+      cslot = r16 == i ? sv : cslot;
     }
   }
 
@@ -230,10 +240,11 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16* __r
   // the first weight was asked for (measured on cold weights of 6144 x 2048, 8 rows: 10.6 against 9.6 us a kernel).
   constexpr int PRE_TAPS = 4;                       // convolutions of up to this width are held in registers
   const bool half_ok = SHUF != 2 || kg < 2;
-  f32x4_t rold[EPI == 2 ? R : 1][EPI == 2 ? MT : 1], nextw[EPI == 2 ? R : 1];
-  float chist[EPI == 3 ? MT : 1][4][PRE_TAPS - 1], ctap[4][PRE_TAPS], cbias[4];
+  f32x4_t rold[EPI == 2 ? R : 1], nextw[EPI == 2 ? R : 1];
+  float chist[4][PRE_TAPS - 1], ctap[4][PRE_TAPS], cbias[4];
   const bool vec4 = (N & 3) == 0;
-  if (EPI == 2 && wave == 0) {
+  const int em = emt * 16 + r16;                    // the epilogue's row
+  if (EPI == 2 && wave < MT) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int n = rowbase[r] + kg * 4;
@@ -245,16 +256,13 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16* __r
           for (int i = 0; i < 4; ++i)
             if (n + i < N) nextw[r][i] = ex.next_w[n + i];
       }
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        rold[r][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        if (ok && xok[mt]) {
-          const float* p = ex.res_out + (size_t)(mt * 16 + r16) * N + n;
-          if (vec4) rold[r][mt] = *reinterpret_cast<const f32x4_t*>(p);
-          else
-            for (int i = 0; i < 4; ++i)
-              if (n + i < N) rold[r][mt][i] = p[i];
-        }
+      rold[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      if (ok && em < M) {
+        const float* p = ex.res_out + (size_t)em * N + n;
+        if (vec4) rold[r] = *reinterpret_cast<const f32x4_t*>(p);
+        else
+          for (int i = 0; i < 4; ++i)
+            if (n + i < N) rold[r][i] = p[i];
       }
     }
   }
@@ -277,17 +285,14 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16* __r
     _Pragma("unroll") for (int q = 0; q < WD; ++q) tq[q] = *reinterpret_cast<const f32x4_t*>(ex.taps + (size_t)cc0_ * WD + 4 * q); \
     _Pragma("unroll") for (int i = 0; i < 4; ++i)                                                                       \
       _Pragma("unroll") for (int p = 0; p < WD; ++p) ctap[i][p] = tq[(i * WD + p) / 4][(i * WD + p) % 4];               \
-    _Pragma("unroll") for (int mt = 0; mt < MT; ++mt) {                                                                 \
-      f32x4_t hq[WD - 1];                                                                                               \
-      const float* hp = ex.state + ((size_t)cslot[mt] * H_ + cc0_) * (WD - 1);                                          \
-      _Pragma("unroll") for (int q = 0; q < WD - 1; ++q) hq[q] = *reinterpret_cast<const f32x4_t*>(hp + 4 * q);         \
-      _Pragma("unroll") for (int i = 0; i < 4; ++i)                                                                     \
-        _Pragma("unroll") for (int p = 0; p < WD - 1; ++p)                                                              \
-          chist[mt][i][p] = hq[(i * (WD - 1) + p) / 4][(i * (WD - 1) + p) % 4];                                         \
-    }                                                                                                                   \
+    f32x4_t hq[WD - 1];                                                                                                 \
+    const float* hp = ex.state + ((size_t)cslot * H_ + cc0_) * (WD - 1);                                                \
+    _Pragma("unroll") for (int q = 0; q < WD - 1; ++q) hq[q] = *reinterpret_cast<const f32x4_t*>(hp + 4 * q);           \
+    _Pragma("unroll") for (int i = 0; i < 4; ++i)                                                                       \
+      _Pragma("unroll") for (int p = 0; p < WD - 1; ++p) chist[i][p] = hq[(i * (WD - 1) + p) / 4][(i * (WD - 1) + p) % 4]; \
   }
 #define GS_PRELOAD_CONV()                                                                                              \
-  if (EPI == 3 && wave == 0 && pre_conv) {                                                                              \
+  if (EPI == 3 && wave < MT && pre_conv) {                                                                              \
     const int H_ = N / 3;                                                                                               \
     const int c0_ = blockIdx.x * (SHUF == 2 ? 8 : 16) + kg * 4;                                                         \
     const int cc0_ = c0_ + 3 < H_ ? c0_ : H_ - 4;                                                                       \
@@ -300,25 +305,25 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16* __r
           f32x4_t out, nh[WD - 1];                                                                                     \
 _Pragma("unroll")                                                                                                      \
           for (int i = 0; i < 4; ++i) {                                                                                \
-            const float Bv = to_f32(f32_to_bf16(acc[0][mt][i])), Cv = to_f32(f32_to_bf16(acc[R > 1 ? 1 : 0][mt][i])),  \
-                        Xv = to_f32(f32_to_bf16(acc[R > 2 ? 2 : 0][mt][i]));                                           \
+            const float Bv = to_f32(f32_to_bf16(sum[0][i])), Cv = to_f32(f32_to_bf16(sum[R > 1 ? 1 : 0][i])),          \
+                        Xv = to_f32(f32_to_bf16(sum[R > 2 ? 2 : 0][i]));                                               \
             const float u = Bv * Xv;                                                                                   \
             float y = 0.f;                                                                                             \
 _Pragma("unroll")                                                                                                      \
-            for (int p = 0; p < WD - 1; ++p) y += ctap[i][p] * chist[mt][i][p];                                        \
+            for (int p = 0; p < WD - 1; ++p) y += ctap[i][p] * chist[i][p];                                            \
             y += ctap[i][WD - 1] * u;                                                                                  \
             if (ex.conv_bias) y += cbias[i];                                                                           \
             out[i] = Cv * y;                                                                                           \
 _Pragma("unroll")                                                                                                      \
             for (int p = 0; p < WD - 1; ++p)                                                                           \
-              nh[(i * (WD - 1) + p) / 4][(i * (WD - 1) + p) % 4] = p < WD - 2 ? chist[mt][i][p + 1] : u;               \
+              nh[(i * (WD - 1) + p) / 4][(i * (WD - 1) + p) % 4] = p < WD - 2 ? chist[i][p + 1] : u;                   \
           }                                                                                                            \
-          store4<TOut>(Y + (ex.y_tiled ? tiled_index(m, c0, MT) : (size_t)m * ldy + c0), out, 4);                      \
-          float* hp = ex.state + ((size_t)slot * H + c0) * (WD - 1);                                                   \
+          store4<TOut>(Y + (ex.y_tiled ? tiled_index(em, c0, MT) : (size_t)em * ldy + c0), out, 4);                    \
+          float* hp = ex.state + ((size_t)cslot * H + c0) * (WD - 1);                                                  \
 _Pragma("unroll")                                                                                                      \
           for (int q = 0; q < WD - 1; ++q) *reinterpret_cast<f32x4_t*>(hp + 4 * q) = nh[q];                            \
         }
-  if (EPI == 3 && MT >= 3) GS_PRELOAD_CONV()   // the loop of many row tiles keeps its order
+  if (EPI == 3 && MT >= 2) GS_PRELOAD_CONV()   // the loop of many row tiles keeps its order
   f32x4_t acc[R][MT];
 #pragma unroll
   for (int r = 0; r < R; ++r)
@@ -327,7 +332,7 @@ _Pragma("unroll")                                                               
 
   const int xstep = ex.x_tiled ? MT * 512 : 32;   // elements between a row tile's consecutive k steps
   auto load_x = [&](int mt, int s) -> bf16x8_t {
-    if (PRO == 0) {
+    if (PRO != 1) {
       return load8(xrow[mt] + (size_t)s * xstep);
     } else {
       const int k = (s << 5) + kg * 8;
@@ -367,66 +372,47 @@ _Pragma("unroll")                                                               
   constexpr int UQ = (WAVES >= 16 ? 12 : 24) / (R + MT);   // sixteen wavefronts leave a lane 128 registers
   constexpr int U = UQ >= 8 ? 8 : (UQ >= 4 ? 4 : (UQ >= 2 ? 2 : 1));
   constexpr int WSTEP = SHUF ? 512 : 32;  // elements between a row tile's consecutive k steps
-  if (MT < 3) {
+  const bool whole = SHUF || (K & 31) == 0;
+  // C steps, their loads issued together, then multiplied.  (One row tile: the lanes without a row load nothing.  A macro, as above.)
+#define GS_BATCH(C, BETWEEN)                                                                                           \
+  {                                                                                                                     \
+    bf16x8_t a[C][R], b[C][MT];                                                                                         \
+    _Pragma("unroll") for (int u = 0; u < C; ++u) {                                                                     \
+      _Pragma("unroll") for (int r = 0; r < R; ++r)                                                                     \
+        a[u][r] = MT > 1 || wact ? load8w<LAYOUT>(wrow[r] + (size_t)(s + u) * WSTEP) : zero8();                         \
+      _Pragma("unroll") for (int mt = 0; mt < MT; ++mt) b[u][mt] = MT > 1 || xok[mt] ? load_x(mt, s + u) : zero8();     \
+    }                                                                                                                   \
+    BETWEEN                                                                                                             \
+    _Pragma("unroll") for (int u = 0; u < C; ++u)                                                                       \
+      _Pragma("unroll") for (int r = 0; r < R; ++r)                                                                     \
+        _Pragma("unroll") for (int mt = 0; mt < MT; ++mt)                                                               \
+          acc[r][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][r], b[u][mt], acc[r][mt], 0, 0, 0);                 \
+    s += C;                                                                                                             \
+  }
+  if (MT == 1) {
     // few rows: the steps' loads are issued U at a time, then multiplied (the ring below costs registers, and with
     // them a resident wavefront per SIMD, which these shapes need more)
-    if ((K & 31) == 0 || SHUF) {
-      if (EPI == 3 && s + U <= s1) {
-        bf16x8_t a[U][R], b[U][MT];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-#pragma unroll
-          for (int r = 0; r < R; ++r) a[u][r] = wact ? load8w<LAYOUT>(wrow[r] + (size_t)(s + u) * WSTEP) : zero8();
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt) b[u][mt] = xok[mt] ? load_x(mt, s + u) : zero8();
-        }
-        GS_PRELOAD_CONV()
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-          for (int r = 0; r < R; ++r)
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-              acc[r][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][r], b[u][mt], acc[r][mt], 0, 0, 0);
-        s += U;
-      } else if (EPI == 3) {
-        GS_PRELOAD_CONV()
-      }
-      for (; s + U <= s1; s += U) {
-        bf16x8_t a[U][R], b[U][MT];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-#pragma unroll
-          for (int r = 0; r < R; ++r) a[u][r] = wact ? load8w<LAYOUT>(wrow[r] + (size_t)(s + u) * WSTEP) : zero8();
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt) b[u][mt] = xok[mt] ? load_x(mt, s + u) : zero8();
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-          for (int r = 0; r < R; ++r)
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-              acc[r][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][r], b[u][mt], acc[r][mt], 0, 0, 0);
-      }
-    } else if (EPI == 3) {
-      GS_PRELOAD_CONV()
+    if (EPI == 3) {
+      if (whole && s + U <= s1) GS_BATCH(U, GS_PRELOAD_CONV())
+      else GS_PRELOAD_CONV()
     }
-  } else if (((K & 31) == 0 || SHUF) && s1 - s0 >= U) {
+    if (whole)
+      while (s + U <= s1) GS_BATCH(U, )
+  } else if (whole && s1 - s0 >= U) {
     // many rows: a ring of U steps in registers: a step is multiplied as soon as it has arrived and its place is
     // asked for again at once, U steps ahead, so that loads are in flight the whole time (loads return in order).
     // Measured against issuing U steps at a time, both builds run in turn on one GPU, six repeats each, gate|up of
-    // 16384 x 2048: 18.6-18.7 against 19.3-19.4 us at 64 rows, 16.8-16.9 against 17.2-17.3 us at 48 rows.
+    // 16384 x 2048: 18.6-18.7 against 19.3-19.4 us at 64 rows, 16.8-16.9 against 17.2-17.3 us at 48 rows; two row tiles: the
+    // convolution's input product of 6144 x 2048 10.5 against 11.5 us at 32 rows, 2048 x 8192 13.9 against 14.8.
     bf16x8_t a[U][R], b[U][MT];
     auto fetch = [&](int u, int step) {
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         // every lane loads (its address is a valid one): a load under a lane mask would hide from the
-        // compiler how many loads are in flight, and it would wait for all of them
-        const bf16x8_t v = load8w<LAYOUT>(wrow[r] + (size_t)step * WSTEP);
-        a[u][r] = (SHUF != 2 || wact) ? v : zero8();
+        // compiler how many loads are in flight, and it would wait for all of them (half tiles: the lanes of
+        // the other eight rows load the first eight's again; those rows are never stored)
+        a[u][r] = load8w<LAYOUT>(wrow[r] + (size_t)step * WSTEP);
       }
-      // rows past M read row 0 or the padding of the last tile; their columns of the result are never stored
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) b[u][mt] = load_x(mt, step);
     };
@@ -452,12 +438,19 @@ _Pragma("unroll")                                                               
     for (int u = 0; u < U; ++u) multiply(u);
     s = s0 + groups * U;
   }
+  // What is left of a wavefront's share: four and two steps together where U is more.  K = 1024 is four steps a wavefront, and
+  // one by one each was a round trip of its own (8 rows, microseconds one by one and together: 1024 x 1024 4.35 and 3.6, 2048 x
+  // 1024 4.4 and 3.5, gate and up of 9216 x 1024 8.2 and 7.1; 1024 x 4608, eighteen steps, 7.2 and 6.7).
+  if (whole) {
+    if (U > 4 && s + 4 <= s1) GS_BATCH(4, )
+    if (U > 2 && EPI != 3 && s + 2 <= s1) GS_BATCH(2, )
+  }
   for (; s < s1; ++s) {
     const int k = (s << 5) + kg * 8;
     const bool kin = k < K;
     bf16x8_t b[MT];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) b[mt] = (kin && xok[mt]) ? load_x(mt, s) : zero8();
+    for (int mt = 0; mt < MT; ++mt) b[mt] = kin ? load_x(mt, s) : zero8();
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       bf16x8_t a = ((kin || SHUF) && wact) ? load8w<LAYOUT>(wrow[r] + (size_t)s * WSTEP) : zero8();
@@ -470,13 +463,18 @@ _Pragma("unroll")                                                               
     // a wavefront's first row was asked for at the start; its further rows (row wave + WAVES, ...) are asked for here
     // in batches, every load of a batch in flight before the first is added, at addresses that always exist (a row
     // or a partial sum that does not is read from the first and counted as zero): no load sits behind a branch
-    constexpr int RPW = (MT * 16 + WAVES - 1) / WAVES;
     constexpr int BATCH = RPW - 1 < 8 ? (RPW > 1 ? RPW - 1 : 1) : 8;
-    if (wave < M) {
-      float ssum = (pre[0] + pre[1]) + (pre[2] + pre[3]);
-      for (int b = 256 + lane; b < ex.nb; b += 64) ssum += ex.ssq[(size_t)wave * ex.nb + b];
-      ssum = wave_sum_dpp(ssum);
-      if (lane == 0) inv_s[wave] = norm_inverse(ssum, (float)K, ex.eps);
+#pragma unroll
+    for (int i = 0; i < EARLY; ++i) {
+      const int m = wave + i * WAVES;
+      if (m < M) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) pre[i][j] = lane + 64 * j < ex.nb ? pre[i][j] : 0.f;
+        float ssum = (pre[i][0] + pre[i][1]) + (pre[i][2] + pre[i][3]);
+        for (int b = 256 + lane; b < ex.nb; b += 64) ssum += ex.ssq[(size_t)m * ex.nb + b];
+        ssum = wave_sum_dpp(ssum);
+        if (lane == 0) inv_s[m] = norm_inverse(ssum, (float)K, ex.eps);
+      }
     }
     if (MT == 1) {   // at most one further row: the plain loop is the smallest code, and the step of few rows feels it
       for (int m = wave + WAVES; m < M; m += WAVES) {
@@ -487,7 +485,7 @@ _Pragma("unroll")                                                               
       }
     }
 #pragma unroll
-    for (int i0 = 1; MT > 1 && i0 < RPW; i0 += BATCH) {
+    for (int i0 = 1; MT > 2 && i0 < RPW; i0 += BATCH) {
       if (wave + i0 * WAVES < M) {
         float q[BATCH][4];
 #pragma unroll
@@ -513,116 +511,128 @@ _Pragma("unroll")                                                               
     if (WAVES == 1) __syncthreads();
   }
 
-  // add the wavefronts' partial tiles: wave 0 keeps its own, the others pass theirs through LDS
-  if (WAVES > 1) {
+  // Add the wavefronts' partial tiles, in wavefront order: wavefront w takes row tile w, its own part of it from registers and
+  // the others' from LDS.  (With one wavefront for all of them: gate and up of 16384 x 2048 at 64 rows 19.1 against 17.9 us, the
+  // convolution's input product of 6144 x 2048 15.0 against 13.0.)
+  f32x4_t sum[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) sum[r] = acc[r][0];
+  if (MT == 1 && WAVES > 1) {
     if (wave > 0) {
-      float* dst = red + ((size_t)(wave - 1) * R * MT) * 256;
 #pragma unroll
-      for (int r = 0; r < R; ++r)
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-          *reinterpret_cast<f32x4_t*>(dst + ((r * MT + mt) * 64 + lane) * 4) = acc[r][mt];
+      for (int r = 0; r < R; ++r) *reinterpret_cast<f32x4_t*>(red + (((wave - 1) * R + r) * 64 + lane) * 4) = acc[r][0];
     }
     __syncthreads();
     if (wave > 0) return;
-    for (int w = 0; w < WAVES - 1; ++w) {
-      const float* src = red + ((size_t)w * R * MT) * 256;
+    for (int w = 0; w < WAVES - 1; ++w)
 #pragma unroll
-      for (int r = 0; r < R; ++r)
+      for (int r = 0; r < R; ++r) sum[r] += *reinterpret_cast<const f32x4_t*>(red + ((w * R + r) * 64 + lane) * 4);
+  } else if (WAVES > 1) {
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          f32x4_t v = *reinterpret_cast<const f32x4_t*>(src + ((r * MT + mt) * 64 + lane) * 4);
-          acc[r][mt] += v;
-        }
-    }
+    for (int mt = 0; mt < MT; ++mt)
+      if (wave != mt) {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          *reinterpret_cast<f32x4_t*>(red + (((wave * R + r) * MT + mt) * 64 + lane) * 4) = acc[r][mt];
+      }
+    __syncthreads();
+    if (wave >= MT) return;
+    f32x4_t own[R];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+      if (wave == mt) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) own[r] = acc[r][mt];
+      }
+    const float* src = red + (emt * 64 + lane) * 4;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w)
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        f32x4_t v = own[r];
+        if (w >= MT || w != wave) v = *reinterpret_cast<const f32x4_t*>(src + (size_t)(w * R + r) * MT * 256);
+        if (w == 0) sum[r] = v; else sum[r] += v;
+      }
   }
 
   // rows that came pre-weighted get their inverse root mean square now
   if (scaled) {
+    const float iv = inv_s[em < M ? em : 0];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const float iv = inv_s[(mt * 16 + r16 < M) ? mt * 16 + r16 : 0];
-#pragma unroll
-      for (int r = 0; r < R; ++r) acc[r][mt] *= iv;
-    }
+    for (int r = 0; r < R; ++r) sum[r] *= iv;
   }
 
-  // lane l holds, for token mt*16 + l%16, columns rowbase + 4*(l/16) + 0..3 of every tile
+  // lane l holds, for token 16 wave + l%16, columns rowbase + 4*(l/16) + 0..3 of every tile
+  const bool live = em < M;
+  if (EPI == 0 || EPI == 5) {
+    if (!live) return;
+    TOut* Yp = EPI == 5 ? Y + (size_t)blockIdx.x * M * ldy : Y;   // partial sums: one (M, N) sheet per part of K
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    const int m = mt * 16 + r16;
-    const bool live = m < M;
-    if (EPI == 0 || EPI == 5) {
-      if (!live) continue;
-      TOut* Yp = EPI == 5 ? Y + (size_t)blockIdx.x * M * ldy : Y;   // partial sums: one (M, N) sheet per part of K
+    for (int r = 0; r < R; ++r) {
+      const int n = rowbase[r] + kg * 4;
+      if (N - n > 0 && half_ok) store4<TOut>(Yp + (size_t)em * ldy + n, sum[r], N - n);
+    }
+  } else if (EPI == 1) {
+    if (!live) return;
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const int n = rowbase[r] + kg * 4;
-        if (N - n > 0 && half_ok) store4<TOut>(Yp + (size_t)m * ldy + n, acc[r][mt], N - n);
-      }
-    } else if (EPI == 1) {
-      if (!live) continue;
+    for (int r = 0; r < R; r += 2) {
+      const int n = rowbase[r] + kg * 4;  // output column in [0, N/2)
+      f32x4_t g = sum[r], u = sum[r + 1], o;
 #pragma unroll
-      for (int r = 0; r < R; r += 2) {
-        const int n = rowbase[r] + kg * 4;  // output column in [0, N/2)
-        f32x4_t g = acc[r][mt], u = acc[r + 1][mt], o;
+      for (int i = 0; i < 4; ++i) o[i] = g[i] / (1.0f + expf(-g[i])) * u[i];
+      if (half - n > 0) store4<TOut>(Y + (ex.y_tiled ? tiled_index(em, n, MT) : (size_t)em * ldy + n), o, half - n);
+    }
+  } else if (EPI == 2) {
+    // every lane takes part in the shuffles, live or not
+    float ss = 0.f;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = g[i] / (1.0f + expf(-g[i])) * u[i];
-        if (half - n > 0) store4<TOut>(Y + (ex.y_tiled ? tiled_index(m, n, MT) : (size_t)m * ldy + n), o, half - n);
-      }
-    } else if (EPI == 2) {
-      // every lane takes part in the shuffles, live or not
-      float ss = 0.f;
+    for (int r = 0; r < R; ++r) {
+      const int n = rowbase[r] + kg * 4;
+      if (live && n < N && half_ok) {
+        float* p = ex.res_out + (size_t)em * N + n;
+        f32x4_t nv, xv;
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const int n = rowbase[r] + kg * 4;
-        if (live && n < N && half_ok) {
-          float* p = ex.res_out + (size_t)m * N + n;
-          f32x4_t nv, xv;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            // the product is rounded to bfloat16 first, as the unfused path stores it before the add
-            nv[i] = rold[r][mt][i] + to_f32(f32_to_bf16(acc[r][mt][i]));
-            if (n + i < N) ss += nv[i] * nv[i];
-            xv[i] = nv[i] * nextw[r][i];
-          }
-          if (vec4) *reinterpret_cast<f32x4_t*>(p) = nv;
-          else
-            for (int i = 0; i < 4; ++i)
-              if (n + i < N) p[i] = nv[i];
-          if (ex.xs_out) store4<bf16>(ex.xs_out + (ex.y_tiled ? tiled_index(m, n, MT) : (size_t)m * N + n), xv, N - n);
+        for (int i = 0; i < 4; ++i) {
+          // the product is rounded to bfloat16 first, as the unfused path stores it before the add
+          nv[i] = rold[r][i] + to_f32(f32_to_bf16(sum[r][i]));
+          if (n + i < N) ss += nv[i] * nv[i];
+          xv[i] = nv[i] * nextw[r][i];
         }
+        if (vec4) *reinterpret_cast<f32x4_t*>(p) = nv;
+        else
+          for (int i = 0; i < 4; ++i)
+            if (n + i < N) p[i] = nv[i];
+        if (ex.xs_out) store4<bf16>(ex.xs_out + (ex.y_tiled ? tiled_index(em, n, MT) : (size_t)em * N + n), xv, N - n);
       }
-      ss += __shfl_xor(ss, 16, 64);
-      ss += __shfl_xor(ss, 32, 64);
-      if (live && kg == 0) ex.ssq_out[(size_t)m * gridDim.x + blockIdx.x] = ss;
-    } else if (EPI == 3) {
-      if (!live) continue;
-      const int H = N / 3, Wd = ex.conv_w;
-      const int slot = cslot[mt];
-      const int c0 = blockIdx.x * (SHUF == 2 ? 8 : 16) + kg * 4;
-      if (pre_conv) {
-        if (c0 >= H || !half_ok) continue;
-        GS_CONV_WIDTH(GS_CONV_EPI_BODY)
-        continue;
-      }
+    }
+    ss += __shfl_xor(ss, 16, 64);
+    ss += __shfl_xor(ss, 32, 64);
+    if (live && kg == 0) ex.ssq_out[(size_t)em * gridDim.x + blockIdx.x] = ss;
+  } else if (EPI == 3) {
+    if (!live) return;
+    const int H = N / 3, Wd = ex.conv_w;
+    const int c0 = blockIdx.x * (SHUF == 2 ? 8 : 16) + kg * 4;
+    if (pre_conv) {
+      if (c0 >= H || !half_ok) return;
+      GS_CONV_WIDTH(GS_CONV_EPI_BODY)
+      return;
+    }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int c = c0 + i;
-        if (c >= H || !half_ok) break;
-        const float Bv = to_f32(f32_to_bf16(acc[0][mt][i])), Cv = to_f32(f32_to_bf16(acc[R > 1 ? 1 : 0][mt][i])),
-                    Xv = to_f32(f32_to_bf16(acc[R > 2 ? 2 : 0][mt][i]));
-        const float u = Bv * Xv;
-        float* hist = ex.state + ((size_t)slot * H + c) * (Wd - 1);
-        const float* wt = ex.taps + (size_t)c * Wd;
-        float y = 0.f;
-        for (int p = 0; p < Wd - 1; ++p) y += wt[p] * hist[p];
-        y += wt[Wd - 1] * u;
-        if (ex.conv_bias) y += ex.conv_bias[c];
-        Y[ex.y_tiled ? tiled_index(m, c, MT) : (size_t)m * ldy + c] = from_f32<TOut>(Cv * y);
-        for (int p = 0; p < Wd - 2; ++p) hist[p] = hist[p + 1];
-        hist[Wd - 2] = u;
-      }
+    for (int i = 0; i < 4; ++i) {
+      const int c = c0 + i;
+      if (c >= H || !half_ok) break;
+      const float Bv = to_f32(f32_to_bf16(sum[0][i])), Cv = to_f32(f32_to_bf16(sum[R > 1 ? 1 : 0][i])),
+                  Xv = to_f32(f32_to_bf16(sum[R > 2 ? 2 : 0][i]));
+      const float u = Bv * Xv;
+      float* hist = ex.state + ((size_t)cslot * H + c) * (Wd - 1);
+      const float* wt = ex.taps + (size_t)c * Wd;
+      float y = 0.f;
+      for (int p = 0; p < Wd - 1; ++p) y += wt[p] * hist[p];
+      y += wt[Wd - 1] * u;
+      if (ex.conv_bias) y += ex.conv_bias[c];
+      Y[ex.y_tiled ? tiled_index(em, c, MT) : (size_t)em * ldy + c] = from_f32<TOut>(Cv * y);
+      for (int p = 0; p < Wd - 2; ++p) hist[p] = hist[p + 1];
+      hist[Wd - 2] = u;
     }
   }
 }
@@ -630,7 +640,7 @@ _Pragma("unroll")                                                               
 template <int R, int MT, int WAVES, int PRO, int EPI, int LAYOUT, typename TOut>
 static void launch_skinny(int blocks, const bf16* X, int ldx, const bf16* W, TOut* Y, int ldy, int M, int N, int K,
                           const SkinnyExtra& ex, hipStream_t stream) {
-  const size_t lds = (size_t)(WAVES - 1) * R * MT * 256 * sizeof(float);
+  const size_t lds = (size_t)(MT > 1 ? WAVES : WAVES - 1) * R * MT * 256 * sizeof(float);
   if (lds > 64 * 1024) {
     // more than the default limit of dynamic LDS: asked for once per kernel
     static const hipError_t asked = hipFuncSetAttribute(
@@ -645,13 +655,13 @@ static void launch_skinny(int blocks, const bf16* X, int ldx, const bf16* W, TOu
 template <int R, int MT, int WAVES, int LAYOUT>
 static void launch_skinny_parts(int blocks, int parts, const bf16* X, int ldx, const bf16* W, float* Y, int M, int N,
                                 int K, const SkinnyExtra& ex, hipStream_t stream) {
-  const size_t lds = (size_t)(WAVES - 1) * R * MT * 256 * sizeof(float);
+  const size_t lds = (size_t)(MT > 1 ? WAVES : WAVES - 1) * R * MT * 256 * sizeof(float);
   gemm_skinny_kernel<R, MT, WAVES, 0, 5, LAYOUT, float>
       <<<dim3(parts, blocks), WAVES * 64, lds, stream>>>(X, ldx, W, Y, N, M, N, K, ex);
 }
 
 // MT from M; the wavefronts per block are given per MT so that the LDS for the partial tiles,
-// (WAVES - 1) * R * MT KB, stays within 64 KB
+// WAVES * R * MT KB, leaves a compute unit room
 #define GS_BY_MT4(R, W1, W2, W3, W4, PRO, EPI, TOut, blocks)                                                            \
   switch ((M + 15) / 16) {                                                                                              \
     case 1: launch_skinny<R, 1, W1, PRO, EPI, LAYOUT, TOut>(blocks, x, ldx, w, (TOut*)Y, ldy, M, N, K, ex, stream); break;  \
@@ -680,30 +690,34 @@ struct SkinnyCall {
   hipStream_t stream;
 };
 
-template <int LAYOUT>
-static void skinny_plain(const SkinnyCall& c) {
+template <int LAYOUT, int PRO>
+static void skinny_plain_pro(const SkinnyCall& c) {
   const bf16 *x = c.x, *w = c.w;
   void* Y = c.Y;
   const int ldx = c.ldx, ldy = c.ldy, M = c.M, N = c.N, K = c.K;
   const SkinnyExtra& ex = c.ex;
   hipStream_t stream = c.stream;
-  const bool pro = ex.res != nullptr, f32 = c.y_dtype == GS_F32;
+  const bool f32 = c.y_dtype == GS_F32;
   const int cols = c.epilogue == 1 ? N / 2 : N;
   const bool narrow = cols <= 8192;
   // few output columns: more wavefronts per block split K further, so that the whole chip streams
   if (c.epilogue == 1) {
     const int blocks = gs_ceil_div(cols, 16);
-    if (pro) { if (f32) { GS_BY_MT4(2, 8, 8, 4, 4, 1, 1, float, blocks) } else { GS_BY_MT4(2, 8, 8, 4, 4, 1, 1, bf16, blocks) } }
-    else     { if (f32) { GS_BY_MT4(2, 8, 8, 4, 4, 0, 1, float, blocks) } else { GS_BY_MT4(2, 8, 8, 4, 4, 0, 1, bf16, blocks) } }
+    if (f32) { GS_BY_MT4(2, 8, 8, 4, 4, PRO, 1, float, blocks) } else { GS_BY_MT4(2, 8, 8, 4, 4, PRO, 1, bf16, blocks) }
   } else if (narrow) {
     const int blocks = gs_ceil_div(cols, 16);
-    if (pro) { if (f32) { GS_BY_MT(1, 8, 1, 0, float, blocks) } else { GS_BY_MT(1, 8, 1, 0, bf16, blocks) } }
-    else     { if (f32) { GS_BY_MT(1, 8, 0, 0, float, blocks) } else { GS_BY_MT(1, 8, 0, 0, bf16, blocks) } }
+    if (f32) { GS_BY_MT(1, 8, PRO, 0, float, blocks) } else { GS_BY_MT(1, 8, PRO, 0, bf16, blocks) }
   } else {
     const int blocks = gs_ceil_div(cols, 32);
-    if (pro) { if (f32) { GS_BY_MT4(2, 8, 8, 4, 4, 1, 0, float, blocks) } else { GS_BY_MT4(2, 8, 8, 4, 4, 1, 0, bf16, blocks) } }
-    else     { if (f32) { GS_BY_MT4(2, 8, 8, 4, 4, 0, 0, float, blocks) } else { GS_BY_MT4(2, 8, 8, 4, 4, 0, 0, bf16, blocks) } }
+    if (f32) { GS_BY_MT4(2, 8, 8, 4, 4, PRO, 0, float, blocks) } else { GS_BY_MT4(2, 8, 8, 4, 4, PRO, 0, bf16, blocks) }
   }
+}
+
+template <int LAYOUT>
+static void skinny_plain(const SkinnyCall& c) {
+  if (c.ex.res) skinny_plain_pro<LAYOUT, 1>(c);
+  else if (c.ex.ssq) skinny_plain_pro<LAYOUT, 2>(c);
+  else skinny_plain_pro<LAYOUT, 0>(c);
 }
 
 // A plain product of a weight of few rows, half a tile a block (up to 32 rows of X: two row tiles).
@@ -713,7 +727,7 @@ static void skinny_plain_halves(const SkinnyCall& c) {
 #define GS_HALF(MT, PRO, TOut) \
   launch_skinny<1, MT, 8, PRO, 0, LAYOUT, TOut>(blocks, c.x, c.ldx, c.w, (TOut*)c.Y, c.ldy, c.M, c.N, c.K, c.ex, c.stream)
 #define GS_HALF_PRO(MT, TOut) \
-  if (c.ex.res) GS_HALF(MT, 1, TOut); else GS_HALF(MT, 0, TOut)
+  if (c.ex.res) GS_HALF(MT, 1, TOut); else if (c.ex.ssq) GS_HALF(MT, 2, TOut); else GS_HALF(MT, 0, TOut)
   if (c.y_dtype == GS_F32) {
     if (c.M <= 16) { GS_HALF_PRO(1, float); } else { GS_HALF_PRO(2, float); }
   } else {
@@ -755,5 +769,7 @@ static void skinny_conv(const SkinnyCall& c) {
   const SkinnyExtra& ex = c.ex;
   hipStream_t stream = c.stream;
   const int blocks = gs_ceil_div(N / 3, (LAYOUT & 3) == 2 ? 8 : 16);
-  if (ex.res) { GS_BY_MT4(3, 8, 8, 4, 4, 1, 3, bf16, blocks) } else { GS_BY_MT4(3, 8, 8, 8, 8, 0, 3, bf16, blocks) }
+  if (ex.res) { GS_BY_MT4(3, 8, 8, 4, 4, 1, 3, bf16, blocks) }
+  else if (ex.ssq) { GS_BY_MT4(3, 8, 8, 8, 8, 2, 3, bf16, blocks) }
+  else { GS_BY_MT4(3, 8, 8, 8, 8, 0, 3, bf16, blocks) }
 }

@@ -9,7 +9,7 @@ where the next step's embedding reads it, so ``n`` steps run back to back withou
 host reads the chosen tokens once per call.  The reference decodes one row per call with one
 host round trip per token (``src/Inference/Inference.jl:2547-2712``).
 
-Rows beyond the live batch (the capacity is the batch rounded up to a power of two, or to 48) point at the
+Rows beyond the live batch (the capacity is the batch rounded up to a power of two, or to 24 or 48) point at the
 scratch page and the scratch slot, so they compute and write garbage that nobody reads.
 
 Graph hygiene: nothing in the graph clears memory with a memset node; the step counters are reset by
@@ -29,13 +29,17 @@ from .batch import BatchContext
 
 
 def _capacity(n: int) -> int:
-    """The batch rounded up to a power of two, or to 48: the products take rows in tiles of 16, and a step of three
-    tiles is measurably shorter than one of four.  (The most requests a step takes is the engine's
-    ``DECODE_MAX_BATCH``, which it has from the runtime's product kernels.)"""
+    """The batch rounded up to a power of two, or to 24 or 48: the products take rows in tiles of 16, and a step of three
+    tiles is measurably shorter than one of four; half a tile less is eight rows of X that no block brings in (24 rows
+    against 32: gate and up of 16384 x 2048 15.2 and 16.3 us, 2048 x 8192 12.4 and 14.4).  (The most requests a step takes
+    is the engine's ``DECODE_MAX_BATCH``, which it has from the runtime's product kernels.)"""
+    for c in (24, 48):
+        if c * 2 // 3 < n <= c:
+            return c
     c = 1
     while c < n:
         c *= 2
-    return 48 if 32 < n <= 48 else c
+    return c
 
 
 class DecodeContext(BatchContext):
