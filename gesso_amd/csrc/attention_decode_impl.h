@@ -69,6 +69,45 @@ __device__ __forceinline__ void finish_maps(const float* o1, const float* o2, co
     if (lane + 64 * i < DV) dst[lane + 64 * i] = f32_to_bf16(o[i] * f);
 }
 
+// x of the lane whose number differs in bit O.
+template <int O>
+__device__ __forceinline__ float lane_xor(float x) {
+  if constexpr (O == 8) return dpp_move<0x128>(x);   // row_ror:8
+  else return __shfl_xor(x, O, 64);
+}
+
+// Sums over the lanes that differ in the bits from O up to 32, shared out: with each bit a lane keeps half of its N values, those
+// of the half that the bit names, and adds to them what the other lane had of them (N odd: all of them).  Returns where a lane's
+// values stand among the N; `left` of them.  The sums are those of adding the lanes' values bit by bit.  (Every lane with every
+// sum was 96 passes through the LDS crossbar for 32 values: one sequence of 530 keys 10.9 against 10.0 us with this and the
+// wavefronts' merge below, whose loads then waited for one another; 64 of 230 12.9 against 11.6, 160 of 100 23.4 against 20.2.)
+template <int N, int O>
+__device__ __forceinline__ int sum_shared_out(float* v, int lane, int at = 0) {
+  if constexpr (O >= 64) return at;
+  else if constexpr (N % 2 == 0) {
+    constexpr int H = N / 2;
+#pragma unroll
+    for (int i = 0; i < H; ++i) {
+      if constexpr (O == 32) {
+        auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[i]), __float_as_uint(v[i + H]), false, false);
+        v[i] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+      } else if constexpr (O == 16) {
+        auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[i]), __float_as_uint(v[i + H]), false, false);
+        v[i] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+      } else {
+        const float give = lane & O ? v[i] : v[i + H], keep = lane & O ? v[i + H] : v[i];
+        v[i] = keep + lane_xor<O>(give);
+      }
+    }
+    return sum_shared_out<H, O * 2>(v, lane, lane & O ? at + H : at);
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] += lane_xor<O>(v[i]);
+    return sum_shared_out<N, O * 2>(v, lane, at);
+  }
+}
+constexpr int sums_left(int n, int o) { return o >= 64 ? n : sums_left(n % 2 == 0 ? n / 2 : n, o * 2); }
+
 template <int D, int G, int W, int RAW, int DV = D, int MAPS = 1>
 __global__ __launch_bounds__(W * 64) void attention_decode_kernel(
     const bf16* __restrict__ q, int q_stride, bf16* kcache, bf16* vcache,
@@ -86,6 +125,7 @@ __global__ __launch_bounds__(W * 64) void attention_decode_kernel(
   // What the registers allow (256 a lane at eight wavefronts a block): the next tile's rows in flight while
   // this one is computed, for rows of up to 64.
   constexpr bool PIPE = D <= 64 && DV <= 64;
+  constexpr bool PAGES = RAW != 0 && W >= 8;
   __shared__ float ps[W][G][64];          // a tile's probabilities, then read per key in the value phase
   __shared__ float al[W][G];              // by how much a tile shrinks what was accumulated before it
   __shared__ float wm[W][G], wl[W][G];
@@ -127,15 +167,33 @@ __global__ __launch_bounds__(W * 64) void attention_decode_kernel(
   auto issue = [&](int t, bf16x8_t (*kreg)[KS], uint4* vreg) {
     const int base = lo + (t << 6);
     long ko[4], vo[NI];
+    // The tile's pages follow one another in the table (RAW: no kept first positions): lane i asks for the i-th of them, and
+    // every row's page comes from the lane that has it.  (A load a row was twelve, for whose 64 addresses each eight wavefronts
+    // queue up: 8 sequences of 530 keys 11.1 against 10.7 us, heads of 128 and 24 of 800 23.9 against 21.4.  Blocks of four
+    // wavefronts lose by the exchange: 64 of 230 11.6 against 11.8.)
+    int tile_page = 0, page0 = 0;
+    if constexpr (PAGES) {
+      page0 = (int)__umulhi((unsigned)base, page_magic);
+      const int last = (int)__umulhi((unsigned)pos, page_magic);
+      tile_page = bt[page0 + lane < last ? page0 + lane : last];
+    }
+    auto row_of = [&](int u) -> long {
+      if constexpr (PAGES) {
+        const int pg = (int)__umulhi((unsigned)u, page_magic);
+        // (rows are counted in 32 bits: 2^32 rows of 64 features are more than the card holds)
+        return (long)(((unsigned)__shfl(tile_page, pg - page0, 64) * (unsigned)nkc + (unsigned)kvc) * (unsigned)page_size + (unsigned)(u - pg * page_size));
+      } else
+        return row_off(u);
+    };
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt) {
       const int u = base + 4 * r16 + kt;
-      ko[kt] = row_off(u <= pos ? u : pos) * D + kg * 8;
+      ko[kt] = row_of(u <= pos ? u : pos) * D + kg * 8;
     }
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       const int uu = base + kq + i * KG;
-      vo[i] = row_off(uu <= pos ? uu : pos) * DV + dc * 8;
+      vo[i] = row_of(uu <= pos ? uu : pos) * DV + dc * 8;
     }
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt)
@@ -398,20 +456,13 @@ __global__ __launch_bounds__(W * 64) void attention_decode_kernel(
       compute(t, kn, vn);
     }
   }
-  // key groups of a wavefront hold partial sums over different keys for the same features: add them
+  // key groups of a wavefront hold partial sums over different keys for the same features: add them.  (Each lane ends with some of
+  // its chunk's sums; where a value count is odd, several lanes hold the same ones and write them alike.)
+  constexpr int LEFT = sums_left(G * 8, DL);
+  const int at = sum_shared_out<G * 8, DL>(&acc[0][0], lane);
+  if (dlive) {
 #pragma unroll
-  for (int g = 0; g < G; ++g)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      float v = acc[g][j];
-      for (int o = DL; o < 64; o <<= 1) v += __shfl_xor(v, o, 64);
-      acc[g][j] = v;
-    }
-  if (kq == 0 && dlive) {
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) wacc[wave][g][dc * 8 + j] = acc[g][j];
+    for (int i = 0; i < LEFT; ++i) wacc[wave][(at + i) >> 3][dc * 8 + ((at + i) & 7)] = (&acc[0][0])[i];
   }
   if (lane < G) {
     wm[wave][lane] = m;
@@ -423,16 +474,24 @@ __global__ __launch_bounds__(W * 64) void attention_decode_kernel(
   const size_t unit = ((size_t)seq * nkv + kvh) * nsplit + split;  // this block's partial
   for (int i = tid; i < G * DV; i += blockDim.x) {
     int g = i / DV, j = i - g * DV;
+    // (all asked for before the first is used; a wavefront without a key counts nothing)
+    float mw[W], lw[W], ow[W];
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      mw[w] = wm[w][g];
+      lw[w] = wl[w][g];
+      ow[w] = wacc[w][g][j];
+    }
     float M = -INFINITY;
-    for (int w = 0; w < W; ++w) M = fmaxf(M, wm[w][g]);
+#pragma unroll
+    for (int w = 0; w < W; ++w) M = fmaxf(M, mw[w]);
     float o = 0.f, L = 0.f;
-    if (M > -INFINITY)
-      for (int w = 0; w < W; ++w)
-        if (wm[w][g] > -INFINITY) {
-          float f = __builtin_amdgcn_exp2f(wm[w][g] - M);
-          o += wacc[w][g][j] * f;
-          L += wl[w][g] * f;
-        }
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      const float f = mw[w] > -INFINITY ? __builtin_amdgcn_exp2f(mw[w] - M) : 0.f;
+      o += ow[w] * f;
+      L += lw[w] * f;
+    }
     if (MAPS == 2 && nsplit == 1) {
       wacc[0][g][j] = o / L;                // (nobody else reads this place)
     } else if (nsplit == 1) {
