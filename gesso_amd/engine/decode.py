@@ -32,13 +32,13 @@ def _capacity(n: int) -> int:
     """The batch rounded up to a power of two, or to 24 or 48: the products take rows in tiles of 16, and a step of three
     tiles is measurably shorter than one of four; half a tile less is eight rows of X that no block brings in (24 rows
     against 32: gate and up of 16384 x 2048 15.2 and 16.3 us, 2048 x 8192 12.4 and 14.4).  (The most requests a step takes
-    is the engine's ``DECODE_MAX_BATCH``, which it has from the runtime's product kernels.)"""
-    for c in (24, 48):
-        if c * 2 // 3 < n <= c:
-            return c
+    is the engine's ``DECODE_MAX_BATCH`` and ``DECODE_WIDE_MAX``.)"""
     c = 1
     while c < n:
         c *= 2
+    for less in (c * 3 // 4,) if c in (32, 64) else ():
+        if n <= less:
+            return less
     return c
 
 
@@ -65,17 +65,18 @@ class DecodeRunner:
         i32 = dict(dtype=torch.int32, device=dev)
         self.max_blocks = -(-engine.max_context // engine.page_size)
         st = engine.storage
-        self.tok = torch.zeros(cap, **i32)
-        self.pos = torch.zeros(cap, **i32)
-        self.kv_len = torch.ones(cap, **i32)
-        self.slots = torch.full((cap,), st.scratch_slot, **i32)
-        self.live = torch.zeros(cap, **i32)
+        # the rows' facts lie side by side (each from a multiple of 64 bytes on), so that one copy brings them
+        self.row = -(-cap // 16) * 16
+        self.facts = torch.zeros((5, self.row), **i32)
+        self.tok, self.pos, self.kv_len, self.slots, self.live = (self.facts[i, :cap] for i in range(5))
+        self.kv_len.fill_(1)
+        self.slots.fill_(st.scratch_slot)
         self.seq_of_token = torch.arange(cap, **i32)
         self.q_start = torch.arange(cap + 1, **i32)
         self.block_tables = [torch.full((cap, self.max_blocks), n, **i32) for n in st.num_pages]
         self.temperature = torch.zeros(cap, dtype=torch.float64, device=dev)
         self.top_p = torch.ones(cap, dtype=torch.float64, device=dev)
-        self.weights, self.wide = engine.choice_scratch(max(cap, engine.DECODE_MAX_BATCH))      # shared by all capacities
+        self.weights = self.wide = None                 # the draws' scratch, asked for by the first step that draws
         self.u = torch.zeros((self.MAX_STEPS, cap), dtype=torch.float64, device=dev)
         self.counter = torch.zeros(cap, **i32)          # steps made since the host last looked, per row
         self.ring = torch.zeros((self.MAX_STEPS, cap), **i32)
@@ -84,10 +85,10 @@ class DecodeRunner:
         # one recording per bound on the context length (launch shapes, how attention splits its keys, depend on it)
         # and per kind of choice: all rows greedy (one kernel), or some rows draw (three, the weights by many blocks)
         self.graphs: Dict[Tuple[int, bool], torch.cuda.CUDAGraph] = {}
+        self.logits_of: Dict[Tuple[int, bool], torch.Tensor] = {}     # where each recording leaves its logits
         self.draws = False
 
-    def _body(self) -> None:
-        ops = self.engine.rt.ops
+    def _forward(self) -> torch.Tensor:
         rt = self.engine.rt
         # up to the weight-streaming products' limit of rows: their fused forms, no library call in the graph; beyond
         # it the kernels of prompt steps, the library's products among them (their plans are made by the eager run
@@ -96,12 +97,17 @@ class DecodeRunner:
         rt.no_library = streaming
         rt.fused = streaming and rt.dtype == torch.bfloat16
         try:
-            logits = self.engine.model.forward(self.ctx)
+            return self.engine.model.forward(self.ctx)
         finally:
             rt.no_library = rt.fused = False
-        self.logits = logits
+
+    def _body(self) -> None:
+        ops, rt = self.engine.rt.ops, self.engine.rt
+        self.logits = logits = self._forward()
         with rt.stage("sample"):
             if self.draws:
+                if self.wide is None:
+                    self.weights, self.wide = self.engine.choice_scratch(max(self.cap, self.engine.DECODE_MAX_BATCH))
                 ops.decode_choose(logits, self.temperature, self.u, self.counter, self.tok, self.ring, self.bad_ring,
                                   self.pos, self.kv_len, self.live, self.wide, top_p=self.top_p, wbuf=self.weights)
             else:
@@ -143,6 +149,7 @@ class DecodeRunner:
             if collecting:
                 gc.enable()
         self.graphs[(bound, draws)] = graph
+        self.logits_of[(bound, draws)] = self.logits
 
     def run(self, rids: Sequence[Hashable], tokens: Sequence[int], n: int, samplers=None
             ) -> Tuple[np.ndarray, np.ndarray]:
@@ -182,12 +189,12 @@ class DecodeRunner:
         eng.steps += n
         return ids, bad
 
-    def _run(self, rids, rcs, tokens, n, samplers, graph):
-        eng, cap, B = self.engine, self.cap, len(rids)
+    def _fill(self, rcs, tokens, n: int) -> None:
+        """What the step's kernels read of the rows that bring ``tokens``, with room for ``n`` more tokens each."""
+        eng, cap, B = self.engine, self.cap, len(rcs)
         st = eng.storage
-        eng.prepare_cache()
         # one int32 buffer for the per-row facts, one copy
-        host = np.zeros((5, cap), dtype=np.int32)
+        host = np.zeros((5, self.row), dtype=np.int32)
         host[0, :B] = tokens
         host[1, :B] = [rc.length for rc in rcs]
         host[2] = 1
@@ -195,9 +202,7 @@ class DecodeRunner:
         host[3] = st.scratch_slot
         host[3, :B] = [st.scratch_slot if rc.slot is None else rc.slot for rc in rcs]
         host[4, :B] = 1
-        dev = torch.from_numpy(host).pin_memory().to(eng.device, non_blocking=True)
-        self.tok.copy_(dev[0]); self.pos.copy_(dev[1]); self.kv_len.copy_(dev[2])
-        self.slots.copy_(dev[3]); self.live.copy_(dev[4])
+        self.facts.copy_(torch.from_numpy(host).pin_memory(), non_blocking=True)
         width = max(1, max(-(-(rc.length + n) // eng.page_size) for rc in rcs))
         for g, bt in enumerate(self.block_tables):
             tab = np.full((cap, width), st.num_pages[g], dtype=np.int32)
@@ -206,10 +211,31 @@ class DecodeRunner:
                 row[row < 0] = st.num_pages[g]
                 tab[i, :len(row)] = row
             bt[:, :width].copy_(torch.from_numpy(tab).pin_memory().to(eng.device, non_blocking=True))
-        temp = np.zeros((2, cap), dtype=np.float64)          # temperatures, then top_p (1: the whole row)
-        temp[1] = 1.0
+
+    def step(self, rids: Sequence[Hashable], tokens: Sequence[int]) -> torch.Tensor:
+        """One step whose caller chooses the next tokens: float32 logits ``(batch, vocab)``.  The rows' room is reserved and
+        the cache prepared.  The kernels are those of the loop's step, replayed where the loop has recorded one for such
+        contexts, else launched (the same bits): some seventy launches at LFM2-1.2B's layers, where a step of prompt
+        portions' kernels is some 140."""
+        rcs = [self.engine.manager.get(r) for r in rids]
+        self._fill(rcs, tokens, 1)
+        bound = self._bound(max(rc.length for rc in rcs) + 1)
+        graph = self.graphs.get((bound, False))
+        if graph is None:
+            self.ctx.max_kv_len = bound
+            return self._forward()[:len(rids)]
+        self.counter.zero_()                             # (the recording ends with the choice, which writes the counters' rows)
+        graph.replay()
+        return self.logits_of[(bound, False)][:len(rids)].clone()
+
+    def _run(self, rids, rcs, tokens, n, samplers, graph):
+        eng, cap, B = self.engine, self.cap, len(rids)
+        eng.prepare_cache()
+        self._fill(rcs, tokens, n)
         before = {}               # row -> the sampler's state before each of its draws
         if samplers is not None and any(s is not None for s in samplers):
+            temp = np.zeros((2, cap), dtype=np.float64)          # temperatures, then top_p (1: the whole row)
+            temp[1] = 1.0
             u = np.zeros((n, cap), dtype=np.float64)
             for i, s in enumerate(samplers):
                 if s is not None:
@@ -220,8 +246,8 @@ class DecodeRunner:
                         before[i].append(s.state)
                         u[k, i] = s.unit()
             self.u[:n].copy_(torch.from_numpy(u).pin_memory().to(eng.device, non_blocking=True))
-        tp = torch.from_numpy(temp).pin_memory().to(eng.device, non_blocking=True)
-        self.temperature.copy_(tp[0]); self.top_p.copy_(tp[1])
+            tp = torch.from_numpy(temp).pin_memory().to(eng.device, non_blocking=True)
+            self.temperature.copy_(tp[0]); self.top_p.copy_(tp[1])
         self.counter.zero_()
         profile = eng.rt.profile
         if profile is None:

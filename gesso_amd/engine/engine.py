@@ -182,7 +182,13 @@ class Engine:
         # from here on the cache is written: an error leaves the requests of this step without a usable state
         try:
             self.prepare_cache()
-            logits = self._step_recorded(entries, ids) if self.recorder is not None else False
+            logits = False
+            if (len(entries) <= self.DECODE_MAX_BATCH and self.model.graph_safe
+                    and all(len(e.tokens) == 1 and len(e.want) == 1 for e in entries)):
+                # every request brings one token and wants its logits: the decode loop's step, without its choice
+                logits = self._runner(len(entries)).step([e.rid for e in entries], ids)
+            elif self.recorder is not None:
+                logits = self._step_recorded(entries, ids)
             if logits is False:
                 ctx = StepContext(entries, self.manager, self.storage, self.spec.vocab, self.device, token_ids=ids)
                 logits = self.model.forward(ctx)
@@ -224,7 +230,6 @@ class Engine:
         (temperature, with or without a nucleus).  Returns ``(ids, bad)`` as ``(n, batch)`` arrays; a row of
         ``bad`` marks a step whose logits were not finite.  Raises :class:`~gesso_amd.errors.OutOfPages` before changing anything.
         """
-        from .decode import DecodeRunner, _capacity
         most = max(self.DECODE_MAX_BATCH, self.DECODE_WIDE_MAX)
         if not 1 <= len(rids) <= most:
             raise InvalidPlan(f"the recorded decode loop takes 1 to {most} requests, not {len(rids)}")
@@ -232,11 +237,15 @@ class Engine:
             raise InvalidPlan("one token per request, each request once")
         if not self.model.graph_safe:
             return self._decode_eager(rids, tokens, n, samplers)
-        cap = _capacity(len(rids))
+        return self._runner(len(rids)).run(rids, tokens, n, samplers)
+
+    def _runner(self, requests: int):
+        from .decode import DecodeRunner, _capacity
+        cap = _capacity(requests)
         runner = self._runners.get(cap)
         if runner is None:
             runner = self._runners[cap] = DecodeRunner(self, cap)
-        return runner.run(rids, tokens, n, samplers)
+        return runner
 
     def choice_scratch(self, rows: int):
         """What the recorded loop's choice needs when rows draw: float64 room for the weights of ``rows`` rows of logits

@@ -582,6 +582,47 @@ def test_recorded_decode_loop_equals_single_steps(folders, name, dtype):
     assert [eng2.length(i) for i in range(3)] == [len(p) + 21 for p in prompts]
 
 
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+@pytest.mark.parametrize("nreq", [1, 3, 17, 40])
+def test_a_step_of_single_tokens_is_the_recorded_loops_step(folders, dtype, nreq):
+    """``Engine.step`` with one token a request: launched where nothing is recorded yet, replayed after a run of the loop, the
+    same bits; each result is the caller's own.  A step in which one request wants no logits runs as any other step does, and
+    what follows it sees the same cache."""
+    from gesso_amd import Engine, StepEntry
+    d = write_tiny(folders, "A", torch.bfloat16 if dtype == "bfloat16" else torch.float32)
+    cfg = P.read_config(d)
+    prompts = [random_ids(3 + (7 * i) % 19, cfg["V"], 900 + i) for i in range(nreq)]
+    engines = [Engine.from_folder(d, dtype=dtype, page_size=8, max_tokens=128 * nreq + 256, num_slots=2 * nreq + 1,
+                                 poison=True) for _ in range(2)]
+    kept = []
+    for which, eng in enumerate(engines):
+        for i, p in enumerate(prompts):
+            eng.add_request(i)
+            eng.step([StepEntry(i, p, [])])
+        if which:                                # other requests' run through the loop records its step
+            others = [("other", i) for i in range(nreq)]
+            for rid, p in zip(others, prompts):
+                eng.add_request(rid)
+                eng.step([StepEntry(rid, p, [])])
+            eng.decode(others, [1] * nreq, 2)
+            for rid in others:
+                eng.finish_request(rid)
+            assert eng._runner(nreq).graphs
+        rows = []
+        for turn in range(4):
+            toks = [(7 * turn + 3 * i + 1) % cfg["V"] for i in range(nreq)]
+            want = [[0]] * nreq if turn != 2 else [[0]] * (nreq - 1) + [[]]
+            rows.append(eng.step([StepEntry(i, [t], w) for i, (t, w) in enumerate(zip(toks, want))]))
+            if rows[-1] is not None:
+                assert torch.isfinite(rows[-1]).all()
+        kept.append([None if r is None else r.clone() for r in rows])
+        torch.cuda.synchronize()
+        for a, b in zip(rows, kept[-1]):
+            assert (a is None and b is None) or torch.equal(a, b)
+    for a, b in zip(*kept):
+        assert (a is None) == (b is None) and (a is None or torch.equal(a, b))
+
+
 @pytest.mark.parametrize("name", ["A", "B", "C", "D"])
 @pytest.mark.parametrize("nreq,steps", [(3, 20), (20, 4), (40, 4), (70, 3), (130, 2)])
 def test_recorded_decode_logits_follow_the_plain_model(folders, name, nreq, steps):
