@@ -31,12 +31,13 @@ from .batch import BatchContext
 def _capacity(n: int) -> int:
     """The batch rounded up to a power of two, or to 24 or 48: the products take rows in tiles of 16, and a step of three
     tiles is measurably shorter than one of four; half a tile less is eight rows of X that no block brings in (24 rows
-    against 32: gate and up of 16384 x 2048 15.2 and 16.3 us, 2048 x 8192 12.4 and 14.4).  (The most requests a step takes
+    against 32: gate and up of 16384 x 2048 15.2 and 16.3 us, 2048 x 8192 12.4 and 14.4).  From 128 on, where the products
+    take as long as their rows, to five and six quarters of a power of two as well (150 rows of LFM2-350M's sizes in 160 and in 256: a case of 33 steps 51.1 and 53.9 ms).  (The most requests a step takes
     is the engine's ``DECODE_MAX_BATCH`` and ``DECODE_WIDE_MAX``.)"""
     c = 1
     while c < n:
         c *= 2
-    for less in (c * 3 // 4,) if c in (32, 64) else ():
+    for less in (c * 3 // 4,) if c in (32, 64) else (c * 5 // 8, c * 3 // 4) if c >= 256 else ():
         if n <= less:
             return less
     return c
