@@ -124,11 +124,11 @@ __device__ __forceinline__ float wave_sum_dpp(float x) {
   return group4_sum(x);
 }
 
-// Sum over a block of up to 1024 threads; every thread gets the result.  `red` holds 17 floats.  (Every thread adds the
+// Sum over a block of up to 1024 threads, whole wavefronts; every thread gets the result.  `red` holds 17 floats.  (Every thread adds the
 // wavefronts' sums itself: one barrier less than handing one thread's sum out.)
 __device__ __forceinline__ float block_sum(float v, float* red) {
   int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
-  v = wave_sum(v);
+  v = wave_sum_dpp(v);
   __syncthreads();
   if (lane == 0) red[wave] = v;
   __syncthreads();

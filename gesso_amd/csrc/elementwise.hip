@@ -346,14 +346,56 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ res, const TD* __restrict
   }
 }
 
+// The same for rows that their block's threads hold, eight neighbours each (H a multiple of eight, everything 16-byte aligned):
+// stream, output and weight are asked for together, behind no branch, before the first is used; no wavefront is without a
+// share; the row's sum costs one barrier, and none where one wavefront holds the row.  (bfloat16, microseconds with a loop over the
+// row and loads behind tests, and so: 8 rows of 2048 3.1 and 2.55, 160 of 1024 3.2 and 2.55, 512 of 1024 4.4 and 3.55, 2,048 of
+// 2048 13.0 and 11.9.)
+template <bool HAS, typename TD, typename TO>
+__global__ __launch_bounds__(1024) void add_rmsnorm_held_kernel(float* __restrict__ res, const TD* __restrict__ delta,
+                                                                const float* __restrict__ w, float eps, TO* __restrict__ out,
+                                                                const int* __restrict__ rows, int H) {
+  __shared__ float red[16];
+  const int r = blockIdx.x, s = rows ? rows[r] : r;
+  const int j = threadIdx.x * 8, at = j < H ? j : 0;
+  float* x = res + (size_t)s * H;
+  float v[8], d[8], wv[8];
+  load8f(x + at, v);
+  if (HAS) load8f(delta + (size_t)s * H + at, d);
+  load8f(w + at, wv);
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    if (HAS) v[i] += d[i];
+    ss += v[i] * v[i];
+  }
+  if (HAS && !rows && j < H) store8f(x + j, v);
+  ss = wave_sum_dpp(j < H ? ss : 0.f);
+  if (blockDim.x > 64) {
+    const int nw = blockDim.x >> 6;
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    ss = 0.f;
+    for (int i = 0; i < nw; ++i) ss += red[i];
+  }
+  if (j >= H) return;
+  const float inv = norm_inverse(ss, (float)H, eps);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = v[i] * inv * wv[i];
+  store8f(out + (size_t)r * H + j, v);
+}
+
 extern "C" int gs_add_rmsnorm(float* res, const void* delta, int delta_dtype, const float* w, float eps, void* out,
                               int out_dtype, const int* rows, int n_out, int H, hipStream_t stream) {
   GS_REQUIRE(n_out >= 0 && H > 0, "add_rmsnorm: bad sizes rows=%d H=%d", n_out, H);
   GS_REQUIRE(eps > 0.f, "add_rmsnorm: eps must be positive");
   if (n_out == 0) return 0;
-  int threads = H >= 1024 ? 256 : (H >= 256 ? 128 : 64);
+  const bool held = H % 8 == 0 && H <= 8192 && (((uintptr_t)res | (uintptr_t)delta | (uintptr_t)w | (uintptr_t)out) & 15) == 0;
+  const int threads = held ? gs_ceil_div(H, 512) * 64 : H >= 1024 ? 256 : (H >= 256 ? 128 : 64);
 #define GS_RUN(TD, TO)                                                                                          \
-  add_rmsnorm_kernel<TD, TO><<<n_out, threads, 0, stream>>>(res, (const TD*)delta, w, eps, (TO*)out, rows, H)
+  if (held && delta) add_rmsnorm_held_kernel<true, TD, TO><<<n_out, threads, 0, stream>>>(res, (const TD*)delta, w, eps, (TO*)out, rows, H); \
+  else if (held) add_rmsnorm_held_kernel<false, TD, TO><<<n_out, threads, 0, stream>>>(res, nullptr, w, eps, (TO*)out, rows, H); \
+  else add_rmsnorm_kernel<TD, TO><<<n_out, threads, 0, stream>>>(res, (const TD*)delta, w, eps, (TO*)out, rows, H)
   if (delta_dtype == GS_F32 && out_dtype == GS_F32)
     GS_RUN(float, float);
   else if (delta_dtype == GS_BF16 && out_dtype == GS_BF16)
@@ -572,21 +614,39 @@ extern "C" int gs_add_bias(const float* y, const float* bias, void* out, int out
 
 // ------------------------------------------------------------------ SwiGLU
 
+// Eight or four consecutive values, aligned to 16 bytes or to four values.
+template <int N, typename T>
+__device__ __forceinline__ void load_n(const T* p, float* v) {
+  if constexpr (N == 8) load8f(p, v);
+  else if constexpr (sizeof(T) == 4) {
+    const float4 a = *reinterpret_cast<const float4*>(p);
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+  } else {
+    const uint2 a = *reinterpret_cast<const uint2*>(p);
+    v[0] = __uint_as_float(a.x << 16); v[1] = __uint_as_float(a.x & 0xffff0000u);
+    v[2] = __uint_as_float(a.y << 16); v[3] = __uint_as_float(a.y & 0xffff0000u);
+  }
+}
+template <int N, typename T>
+__device__ __forceinline__ void store_n(T* p, const float* v) {
+  if constexpr (N == 8) store8f(p, v);
+  else store4f(p, v);
+}
+
 // in (T, 2F): gate in columns [0, F), up in [F, 2F).  out[t, j] = silu(gate) * up, silu(g) = g / (1 + exp(-g)).
-// Eight outputs per thread with 16-byte loads and stores; F a multiple of 8, rows 16-byte aligned.
-template <typename T>
-__global__ void swiglu8_kernel(const T* __restrict__ in, T* __restrict__ out, int F, long n8) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n8) return;
-  const int f8 = F / 8;
-  long t = i / f8;
-  int j = (int)(i - t * f8) * 8;
-  float g[8], u[8];
-  load8f(in + t * 2 * F + j, g);
-  load8f(in + t * 2 * F + F + j, u);
+// N outputs per thread (eight: 16-byte loads and stores); F a multiple of 8, rows 16-byte aligned, fewer than 2^32 outputs.
+template <int N, typename T>
+__global__ void swiglu8_kernel(const T* __restrict__ in, T* __restrict__ out, unsigned F, unsigned n) {
+  const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const unsigned f = F / N, t = i / f, j = (i - t * f) * N;
+  const T* row = in + (size_t)t * 2 * F + j;
+  float g[N], u[N];
+  load_n<N>(row, g);
+  load_n<N>(row + F, u);
 #pragma unroll
-  for (int k = 0; k < 8; ++k) g[k] = g[k] / (1.0f + expf(-g[k])) * u[k];
-  store8f(out + t * F + j, g);
+  for (int k = 0; k < N; ++k) g[k] = g[k] / (1.0f + expf(-g[k])) * u[k];
+  store_n<N>(out + (size_t)t * F + j, g);
 }
 
 template <typename T>
@@ -604,12 +664,17 @@ extern "C" int gs_swiglu(const void* in, void* out, int dtype, int T, int F, hip
   GS_REQUIRE(T >= 0 && F > 0, "swiglu: bad sizes T=%d F=%d", T, F);
   long n = (long)T * F;
   if (n == 0) return 0;
-  if (F % 8 == 0 && ((uintptr_t)in & 15) == 0 && ((uintptr_t)out & 15) == 0 && (dtype == GS_F32 || dtype == GS_BF16)) {
-    long n8 = n / 8;
-    if (dtype == GS_F32)
-      swiglu8_kernel<float><<<gs_ceil_div(n8, 256), 256, 0, stream>>>((const float*)in, (float*)out, F, n8);
-    else
-      swiglu8_kernel<bf16><<<gs_ceil_div(n8, 256), 256, 0, stream>>>((const bf16*)in, (bf16*)out, F, n8);
+  if (F % 8 == 0 && n < (1L << 32) && ((uintptr_t)in & 15) == 0 && ((uintptr_t)out & 15) == 0 && (dtype == GS_F32 || dtype == GS_BF16)) {
+    // (few rows: a thread's eight exponentials one after the other are longer than the loads: 6 x 8192 in float32 2.5 and 2.35 us)
+    const bool few = n <= (1L << 19);
+    const int blocks8 = gs_ceil_div(few ? n / 4 : n / 8, 256);
+    if (dtype == GS_F32) {
+      if (few) swiglu8_kernel<4, float><<<blocks8, 256, 0, stream>>>((const float*)in, (float*)out, F, (unsigned)(n / 4));
+      else swiglu8_kernel<8, float><<<blocks8, 256, 0, stream>>>((const float*)in, (float*)out, F, (unsigned)(n / 8));
+    } else {
+      if (few) swiglu8_kernel<4, bf16><<<blocks8, 256, 0, stream>>>((const bf16*)in, (bf16*)out, F, (unsigned)(n / 4));
+      else swiglu8_kernel<8, bf16><<<blocks8, 256, 0, stream>>>((const bf16*)in, (bf16*)out, F, (unsigned)(n / 8));
+    }
     GS_LAUNCH_CHECK("swiglu");
     return 0;
   }
@@ -919,31 +984,31 @@ __global__ void gated_act_kernel(const TI* __restrict__ in, const float* __restr
   out[i] = from_f32<TO>(gated_act(g, act) * u);
 }
 
-// The same, eight columns a thread with 16-byte accesses (F a multiple of eight, everything aligned).
-template <typename TI, typename TO>
-__global__ void gated_act8_kernel(const TI* __restrict__ in, const float* __restrict__ bias, TO* __restrict__ out, int F,
-                                  long n8, int act) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n8) return;
-  const int f8 = F >> 3;
-  const long t = i / f8;
-  const int j = (int)(i - t * f8) * 8;
-  float g[8], u[8], o[8];
-  load8f(in + t * 2 * F + j, g);
-  load8f(in + t * 2 * F + F + j, u);
+// The same, N columns a thread with 16-byte accesses (8-byte ones where four bfloat16 are a thread's share; F a multiple of eight,
+// everything aligned).
+template <int N, typename TI, typename TO>
+__global__ void gated_act8_kernel(const TI* __restrict__ in, const float* __restrict__ bias, TO* __restrict__ out, unsigned F,
+                                  unsigned n, int act) {
+  const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const unsigned f = F / N, t = i / f, j = (i - t * f) * N;
+  const TI* row = in + (size_t)t * 2 * F + j;
+  float g[N], u[N], o[N];
+  load_n<N>(row, g);
+  load_n<N>(row + F, u);
   if (bias) {
-    float bg[8], bu[8];
-    load8f(bias + j, bg);
-    load8f(bias + F + j, bu);
+    float bg[N], bu[N];
+    load_n<N>(bias + j, bg);
+    load_n<N>(bias + F + j, bu);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
+    for (int e = 0; e < N; ++e) {
       g[e] += bg[e];
       u[e] += bu[e];
     }
   }
 #pragma unroll
-  for (int e = 0; e < 8; ++e) o[e] = gated_act(g[e], act) * u[e];
-  store8f(out + t * F + j, o);
+  for (int e = 0; e < N; ++e) o[e] = gated_act(g[e], act) * u[e];
+  store_n<N>(out + (size_t)t * F + j, o);
 }
 
 extern "C" int gs_gated_act(const void* in, int in_dtype, const float* bias, void* out, int out_dtype, int T, int F,
@@ -952,11 +1017,15 @@ extern "C" int gs_gated_act(const void* in, int in_dtype, const float* bias, voi
   GS_REQUIRE(act >= 0 && act <= 3, "gated_act: unknown activation %d", act);
   const long n = (long)T * F;
   if (n == 0) return 0;
-  const bool v8 = F % 8 == 0 && ((uintptr_t)in & 15) == 0 && ((uintptr_t)out & 15) == 0 && ((uintptr_t)bias & 15) == 0;
-  const int blocks = gs_ceil_div(v8 ? n / 8 : n, 256);
+  const bool v8 = F % 8 == 0 && n < (1L << 32) && ((uintptr_t)in & 15) == 0 && ((uintptr_t)out & 15) == 0 && ((uintptr_t)bias & 15) == 0;
+  // Few rows: four columns a thread, for a thread's eight tanh in a row are longer than the loads (8 x 8192 in bfloat16
+  // 3.65 and 2.8 us, with the division of 64-bit numbers that stood here before); at 160 x 4608 the two take the same.
+  const bool v4 = v8 && n <= (1L << 19);
+  const int blocks = gs_ceil_div(v4 ? n / 4 : v8 ? n / 8 : n, 256);
 #define GS_RUN(TI, TO)                                                                                            \
   do {                                                                                                            \
-    if (v8) gated_act8_kernel<TI, TO><<<blocks, 256, 0, stream>>>((const TI*)in, bias, (TO*)out, F, n / 8, act);   \
+    if (v4) gated_act8_kernel<4, TI, TO><<<blocks, 256, 0, stream>>>((const TI*)in, bias, (TO*)out, F, (unsigned)(n / 4), act); \
+    else if (v8) gated_act8_kernel<8, TI, TO><<<blocks, 256, 0, stream>>>((const TI*)in, bias, (TO*)out, F, (unsigned)(n / 8), act); \
     else gated_act_kernel<TI, TO><<<blocks, 256, 0, stream>>>((const TI*)in, bias, (TO*)out, F, n, act);           \
   } while (0)
   if (in_dtype == GS_F32 && out_dtype == GS_F32)
