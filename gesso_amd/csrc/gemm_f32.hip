@@ -327,13 +327,23 @@ extern "C" int gs_gemm_f32_takes(int M, int N, int K, int ldx, const void* X, co
 template <int WR, int XR, int D, typename TO>
 static void run_rows(const float* X, int ldx, const float* W, const float* bias, TO* Y, int ldy, int M, int N, int K,
                      hipStream_t stream) {
-  constexpr int out = (XR > 16 ? XR : 16) * WR, most = 7168 / out;         // 28 KB of LDS for the sums, beside 34 KB
-  const int blocks = gs_ceil_div(N, WR), chunks = gs_ceil_div(K, GS_SUM_CHUNK), room = chunks < most ? chunks : most;
+  // LDS for the chunk sums, beside 34 KB: 32 KB, which leaves a compute unit room for two blocks, or 64 KB where there is no more than
+  // one a unit.  A pass that ends before K does drains every load in flight and adds up before it asks for the next
+  // (28 KB for all: 6 rows of 16384 x 2048, 28 of 32 chunks, 33.3 against 27.5 us; of 2048 x 8192 21.4 against 20.5; 40 rows of it
+  // 70 against 57, of 2048 x 2048 18.4 against 14.6).
+  constexpr int out = (XR > 16 ? XR : 16) * WR;
+  const int blocks = gs_ceil_div(N, WR), chunks = gs_ceil_div(K, GS_SUM_CHUNK), most = (blocks <= 256 ? 16384 : 8192) / out;
+  const int room = chunks < most ? chunks : most;
   const size_t lds = (size_t)room * out * sizeof(float);
-  if (K % GS_SUM_CHUNK == 0)
-    gemm_f32_rows_kernel<WR, XR, D, false, TO><<<blocks, GF_WAVES * 64, lds, stream>>>(X, ldx, W, bias, Y, ldy, M, N, K, room);
-  else
-    gemm_f32_rows_kernel<WR, XR, D, true, TO><<<blocks, GF_WAVES * 64, lds, stream>>>(X, ldx, W, bias, Y, ldy, M, N, K, room);
+  auto kernel = K % GS_SUM_CHUNK == 0 ? &gemm_f32_rows_kernel<WR, XR, D, false, TO> : &gemm_f32_rows_kernel<WR, XR, D, true, TO>;
+  if (lds + sizeof(float) * GF_WAVES * 16 * (GS_SUM_CHUNK + 4) > 64 * 1024) {
+    // more than the default limit of LDS: asked for once per kernel
+    static const hipError_t asked[2] = {
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_rows_kernel<WR, XR, D, false, TO>), hipFuncAttributeMaxDynamicSharedMemorySize, 65536),
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_rows_kernel<WR, XR, D, true, TO>), hipFuncAttributeMaxDynamicSharedMemorySize, 65536)};
+    (void)asked;
+  }
+  kernel<<<blocks, GF_WAVES * 64, lds, stream>>>(X, ldx, W, bias, Y, ldy, M, N, K, room);
 }
 
 template <int MB, typename TO>
