@@ -113,7 +113,7 @@ __global__ __launch_bounds__(MOE_WAVES * 64) void moe_table_up_kernel(const T* _
   }
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) {
-    const float v = wave_sum(s[r]);
+    const float v = wave_sum_dpp(s[r]);
     if (lane == 0 && f0 + r < F) {
       // the product is stored in the activation type before the activation, as a product of its own would be
       float z = to_f32(from_f32<T>(v));
@@ -165,7 +165,7 @@ __global__ __launch_bounds__(MOE_WAVES * 64) void moe_table_down_kernel(const T*
   auto finish = [&]() __attribute__((always_inline)) {                    // a choice's sums are complete
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) {
-      total[r] += wave_sum(s[r]) * share;
+      total[r] += wave_sum_dpp(s[r]) * share;
       s[r] = 0.f;
     }
   };
