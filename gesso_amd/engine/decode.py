@@ -31,16 +31,19 @@ from .batch import BatchContext
 def _capacity(n: int) -> int:
     """The batch rounded up to a power of two, or to 24 or 48: the products take rows in tiles of 16, and a step of three
     tiles is measurably shorter than one of four; half a tile less is eight rows of X that no block brings in (24 rows
-    against 32: gate and up of 16384 x 2048 15.2 and 16.3 us, 2048 x 8192 12.4 and 14.4).  From 128 on, where the products
-    take as long as their rows, to five and six quarters of a power of two as well (150 rows of LFM2-350M's sizes in 160 and in 256: a case of 33 steps 51.1 and 53.9 ms).  (The most requests a step takes
+    against 32: gate and up of 16384 x 2048 15.2 and 16.3 us, 2048 x 8192 12.4 and 14.4).  (The most requests a step takes
     is the engine's ``DECODE_MAX_BATCH`` and ``DECODE_WIDE_MAX``.)"""
     c = 1
     while c < n:
         c *= 2
-    for less in (c * 3 // 4,) if c in (32, 64) else (c * 5 // 8, c * 3 // 4) if c >= 256 else ():
-        if n <= less:
-            return less
-    return c
+    return c * 3 // 4 if c in (32, 64) and n <= c * 3 // 4 else c
+
+
+def _rows(cap: int, n: int) -> int:
+    """The rows a step of ``n`` requests is recorded with in a capacity of ``cap``: all of them, or five or six eighths from
+    256 on, where the products take as long as their rows (150 requests at LFM2-350M's sizes as 160 and as 256 rows: a case
+    of 33 steps 51.1 and 53.9 ms)."""
+    return next((r for r in (cap * 5 // 8, cap * 3 // 4) if n <= r), cap) if cap >= 256 else cap
 
 
 class DecodeContext(BatchContext):
@@ -60,8 +63,10 @@ class DecodeRunner:
 
     MAX_STEPS = 32
 
-    def __init__(self, engine, cap: int):
+    def __init__(self, engine, cap: int, whole: "DecodeRunner" = None):
         self.engine, self.cap = engine, cap
+        self.whole = whole or self                      # the runner of the whole capacity, where this one has fewer rows
+        self.fewer: Dict[int, DecodeRunner] = {}
         dev = engine.device
         i32 = dict(dtype=torch.int32, device=dev)
         self.max_blocks = -(-engine.max_context // engine.page_size)
@@ -89,6 +94,15 @@ class DecodeRunner:
         self.logits_of: Dict[Tuple[int, bool], torch.Tensor] = {}     # where each recording leaves its logits
         self.draws = False
 
+    def fit(self, n: int) -> "DecodeRunner":
+        """The runner of as many rows as ``n`` requests are recorded with (:func:`_rows`)."""
+        rows = _rows(self.cap, n)
+        if rows == self.cap:
+            return self
+        if rows not in self.fewer:
+            self.fewer[rows] = DecodeRunner(self.engine, rows, self)
+        return self.fewer[rows]
+
     def _forward(self) -> torch.Tensor:
         rt = self.engine.rt
         # up to the weight-streaming products' limit of rows: their fused forms, no library call in the graph; beyond
@@ -104,7 +118,7 @@ class DecodeRunner:
 
     def _body(self) -> None:
         ops, rt = self.engine.rt.ops, self.engine.rt
-        self.logits = logits = self._forward()
+        self.logits = self.whole.logits = logits = self._forward()
         with rt.stage("sample"):
             if self.draws:
                 if self.wide is None:

@@ -245,7 +245,7 @@ class Engine:
         runner = self._runners.get(cap)
         if runner is None:
             runner = self._runners[cap] = DecodeRunner(self, cap)
-        return runner
+        return runner.fit(requests)
 
     def choice_scratch(self, rows: int):
         """What the recorded loop's choice needs when rows draw: float64 room for the weights of ``rows`` rows of logits
