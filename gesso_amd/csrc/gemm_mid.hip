@@ -14,6 +14,9 @@
 // last and never stored; K is a multiple of 32, and what a step or a group holds beyond it is loaded but not multiplied (an
 // infinite weight times a zero put in its place would be no zero).
 //
+// EPI 2 (a K too long for one block's chain: a feed-forward's last product): K is shared out over blocks as well, and each stores its
+// float32 sums as its part's sheet (parts, M, N); the pass that adds the product to the stream adds the sheets.
+//
 // EPI 1 (SwiGLU): W holds gate rows [0, N/2), then up rows, N / 2 a multiple of 16; a wavefront owns NT / 2 tiles of gate rows
 // and the up rows of the same columns.  silu(gate) * up is taken of the values as they would have been stored.
 #include "common.h"
@@ -26,10 +29,10 @@ constexpr int GD_BK = 64, GD_LDR = GD_BK + 8, GD_AHEAD = 4;
 
 template <int BM, int NT, int KG, int EPI>
 __global__ __launch_bounds__(KG * 256) void gemm_mid_kernel(const bf16* __restrict__ X, int ldx, const bf16* __restrict__ Wt,
-                                                            bf16* __restrict__ Y, int ldy, int M, int N, int K) {
+                                                            bf16* __restrict__ Y, int ldy, int M, int N, int K, int part_steps) {
   constexpr int TM = BM / 16, LA = BM / 32, STAGE = BM * GD_LDR;           // 16-byte loads of X a thread and step
   constexpr int COLS = 64 * (EPI == 1 ? NT / 2 : NT);                      // columns of Y a block
-  static_assert(EPI == 0 || NT % 2 == 0, "SwiGLU pairs gate tiles with up tiles");
+  static_assert(EPI != 1 || NT % 2 == 0, "SwiGLU pairs gate tiles with up tiles");
   extern __shared__ __align__(16) uint16_t gd_lds[];
   const int tid = threadIdx.x & 255, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), kg = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
@@ -37,12 +40,17 @@ __global__ __launch_bounds__(KG * 256) void gemm_mid_kernel(const bf16* __restri
   // Blocks go to the eight XCDs in turn, each with an L2 of its own: a run of consecutive tile numbers goes to one XCD, row
   // tiles fastest, so that the tiles that read the same weights read them from one L2.
   const int tiles_m = (M + BM - 1) / BM;
-  int bm, bn;
+  int bm, bn, part = 0;
   {
     const int nb = (int)gridDim.x, per = nb / 8, rem = nb % 8, xcd = (int)blockIdx.x % 8;
     const int t = xcd * per + (xcd < rem ? xcd : rem) + (int)blockIdx.x / 8;
     bm = t % tiles_m;
     bn = t / tiles_m;
+    if (EPI == 2) {
+      const int tiles_n = (N + COLS - 1) / COLS;
+      part = bn / tiles_n;
+      bn %= tiles_n;
+    }
   }
   const int m0 = bm * BM, n0 = bn * COLS + wave * (COLS / 4);               // the wavefront's first column
   const int r0 = tid >> 3, c = tid & 7;                                     // this thread's loads: row r0 + 32 i, piece c of eight k
@@ -62,7 +70,8 @@ __global__ __launch_bounds__(KG * 256) void gemm_mid_kernel(const bf16* __restri
     wp[j] = Wt + (size_t)(n >> 4) * ksteps * 512 + lane * 8;
   }
   // the groups' steps: a run each; as many for every group (what lies beyond K is not multiplied)
-  const int steps = (K + GD_BK - 1) / GD_BK, per = (steps + KG - 1) / KG, first = kg * per;
+  const int steps = EPI == 2 ? part_steps : (K + GD_BK - 1) / GD_BK, per = (steps + KG - 1) / KG, first = part * part_steps + kg * per;
+  const int kend = EPI == 2 && 2 * (part + 1) * part_steps < ksteps ? 2 * (part + 1) * part_steps : ksteps;
   struct Step {
     gd_u32x4_t a[LA];
     gd_bf16x8_t w[2][NT];
@@ -91,7 +100,7 @@ __global__ __launch_bounds__(KG * 256) void gemm_mid_kernel(const bf16* __restri
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[i][j] = gd_f32x4_t{0.f, 0.f, 0.f, 0.f};
   auto multiply = [&](const Step& s, int buf, int step) __attribute__((always_inline)) {
-    const int left = ksteps - 2 * (first + step);          // runs of 32 k from here on (the same for the whole wavefront)
+    const int left = kend - 2 * (first + step);          // runs of 32 k from here on (the same for the whole wavefront)
     const uint16_t* a = mine + buf * STAGE + r16 * GD_LDR + g * 8;
     gd_bf16x8_t x[2][TM];                                  // all asked for before the first is used
 #pragma unroll
@@ -160,6 +169,10 @@ __global__ __launch_bounds__(KG * 256) void gemm_mid_kernel(const bf16* __restri
     for (int j = 0; j < (EPI == 1 ? NT / 2 : NT); ++j) {
       const int n = n0 + 16 * j + 4 * g;
       if (n >= width) continue;                            // (whole tiles: the width is a multiple of 16)
+      if (EPI == 2) {
+        *reinterpret_cast<gd_f32x4_t*>(reinterpret_cast<float*>(Y) + ((size_t)part * M + m) * N + n) = acc[i][j];
+        continue;
+      }
       float v[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -178,20 +191,20 @@ __global__ __launch_bounds__(KG * 256) void gemm_mid_kernel(const bf16* __restri
 }
 
 template <int BM, int NT, int KG, int EPI>
-static void run_mid(const bf16* X, int ldx, const bf16* Wt, bf16* Y, int ldy, int M, int N, int K, hipStream_t stream) {
+static void run_mid(const bf16* X, int ldx, const bf16* Wt, bf16* Y, int ldy, int M, int N, int K, hipStream_t stream, int parts = 1) {
   const int cols = 64 * (EPI == 1 ? NT / 2 : NT), width = EPI == 1 ? N / 2 : N;
-  const long tiles = (long)gs_ceil_div(M, BM) * gs_ceil_div(width, cols);
+  const long tiles = (long)gs_ceil_div(M, BM) * gs_ceil_div(width, cols) * parts;
   const size_t held = (size_t)KG * 2 * BM * GD_LDR * sizeof(uint16_t), sums = (size_t)(KG - 1) * BM * 64 * NT * sizeof(float);
   const size_t lds = held > sums ? held : sums;
   static const hipError_t asked = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_mid_kernel<BM, NT, KG, EPI>),
                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   (void)asked;
-  gemm_mid_kernel<BM, NT, KG, EPI><<<(unsigned)tiles, KG * 256, lds, stream>>>(X, ldx, Wt, Y, ldy, M, N, K);
+  gemm_mid_kernel<BM, NT, KG, EPI><<<(unsigned)tiles, KG * 256, lds, stream>>>(X, ldx, Wt, Y, ldy, M, N, K, gs_ceil_div(gs_ceil_div(K, GD_BK), parts));
 }
 
 // Which tile, and whether this kernel at all.  What a compute unit brings in (some 55 bytes a nanosecond, however the tile is
 // cut) is what a product takes beyond 3 to 4 us: the rows of X and W of a block times K, times the rounds in which a unit works
-// off its blocks.  So the tile with the least of that is taken.  None for K beyond 2048, where the vendor shares K out over
+// off its blocks.  So the tile with the least of that is taken.  None for K beyond 2048, where the vendor and the products in parts below share K out over
 // blocks (192 rows of 1024 x 4608: 17.1 us here, 13.5 there), and none where the vendor's larger tiles, which read less, win.
 // Microseconds here / there (gate and up: with the SwiGLU pass), weights that lie in no cache:
 // - plain, one round, up to 2^18 rows times k a unit: 192 rows of 3072 x 1024 8.7 / 13.5, 1024 x 1024 7.1 / 11.0, 2048 x 2048
@@ -257,5 +270,60 @@ extern "C" int gs_gemm_mid(const void* X, int ldx, const void* Wt, void* Y, int 
   }
 #undef GD_RUN
   GS_LAUNCH_CHECK("gemm_mid");
+  return 0;
+}
+
+// The product in parts of K: which tile and how many parts.  As above, a unit's rows of X and W times k bind, and a sheet is written
+// and read once more (counted as the rows times k that take as long; at a quarter of that, 160 rows of 1024 x 4608 took 15 parts and 15.8
+// us); none beyond what one round of blocks holds.  Microseconds with the pass that adds and norms, the vendor's product and the
+// plain pass / here, weights that lie in no cache: 1024 x 4608, 65 rows 12.3 / 10.2, 160 13.7 / 12.1, 333 17.6 / 15.8, 768 23.1 /
+// 22.4; 2048 x 8192, 65 rows 24.2 / 15.8, 192 29.8 / 22.0, 512 37.8 / 36.2, 768 48.7 / 46.6; 2048 x 4096, 128 rows 15.7 / 13.8, 768 29.6
+// / 29.5; 512 x 4096, 256 rows 11.6 / 10.7; 4096 x 4096, 128 rows 28.3 / 19.1, 256 26.8 / 25.2, 333 29.7 / 30.8; 1,024 rows of 1024 x
+// 3072 18.5 / 19.0.
+struct MidParts {
+  int tile, parts;
+};
+static MidParts mid_parts_choice(int M, int N, int K) {
+  MidParts best = {-1, 0};
+  if (M <= 64 || K <= 2048 || N > 4096 || M > (N <= 2048 ? 768 : 256)) return best;
+  const int steps = gs_ceil_div(K, GD_BK);
+  long least = 0;
+  for (int i = 0; i < 5; ++i) {
+    const long tiles = (long)gs_ceil_div(M, mid_plain[i].bm) * gs_ceil_div(N, 64 * mid_plain[i].nt);
+    for (int parts = 2; parts <= 16 && parts * tiles <= 256; ++parts) {
+      const int each = gs_ceil_div(steps, parts);
+      if (each < 4 || (long)(parts - 1) * each >= steps) continue;      // (no part without a step)
+      const long cost = (long)(mid_plain[i].bm + 64 * mid_plain[i].nt) * each * GD_BK + (long)parts * M * N / 16;
+      if (best.parts == 0 || cost < least) {
+        least = cost;
+        best = {i, parts};
+      }
+    }
+  }
+  return best;
+}
+
+// Into how many parts of K the product of M rows with a tile-major weight (N, K) is shared out; 0: it is not this kernel's.
+extern "C" int gs_gemm_mid_parts_takes(int M, int N, int K) {
+  return K > 0 && K % 32 == 0 && N > 0 && N % 16 == 0 ? mid_parts_choice(M, N, K).parts : 0;
+}
+
+// part (parts, M, N) float32 = partial sums of X W^T over gs_gemm_mid_parts_takes parts of K; gs_residual_from_parts adds them up.
+extern "C" int gs_gemm_mid_parts(const void* X, int ldx, const void* Wt, float* part, int parts, int M, int N, int K, hipStream_t stream) {
+  GS_REQUIRE(parts > 0 && gs_gemm_mid_parts_takes(M, N, K) == parts, "gemm_mid_parts: not a product of this kernel in %d parts (M=%d N=%d K=%d)", parts, M, N, K);
+  GS_REQUIRE(ldx >= K && ldx % 8 == 0 && (((uintptr_t)X | (uintptr_t)Wt | (uintptr_t)part) & 15) == 0,
+             "gemm_mid_parts: X, W and the sheets must be 16-byte aligned, the row stride of X a multiple of 8");
+  const bf16 *x = (const bf16*)X, *w = (const bf16*)Wt;
+  bf16* y = (bf16*)part;
+#define GD_RUN(BM, NT, KG) run_mid<BM, NT, KG, 2>(x, ldx, w, y, N, M, N, K, stream, parts)
+  switch (mid_parts_choice(M, N, K).tile) {
+    case 0: GD_RUN(32, 1, 4); break;
+    case 1: GD_RUN(64, 1, 2); break;
+    case 2: GD_RUN(96, 1, 2); break;
+    case 3: GD_RUN(64, 2, 2); break;
+    default: GD_RUN(96, 2, 1); break;
+  }
+#undef GD_RUN
+  GS_LAUNCH_CHECK("gemm_mid_parts");
   return 0;
 }

@@ -681,6 +681,35 @@ def gemm_mid(x, w: torch.Tensor, wt, swiglu: bool = False, out: torch.Tensor = N
     return out
 
 
+def mid_parts(x, w: torch.Tensor, wt) -> int:
+    """Into how many parts of K :func:`gemm_mid_residual_parts` shares this product out; 0: it is not for it.  Operands as for
+    :func:`mid_ok`."""
+    if not (wt is not None and isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 and x.dim() == 2 and x.is_cuda
+            and x.shape[1] == w.shape[1] and x.stride(1) == 1 and x.stride(0) >= x.shape[1] and x.stride(0) % 8 == 0
+            and x.data_ptr() % 16 == 0 and wt.shape == w.shape and w.is_contiguous()):
+        return 0
+    return lib().gs_gemm_mid_parts_takes(x.shape[0], w.shape[0], w.shape[1])
+
+
+def gemm_mid_residual_parts(x, w: torch.Tensor, wt, res: torch.Tensor, next_weight=None, eps: float = 0.0):
+    """``res += x @ w.T`` for some hundred rows and a long K in two kernels: partial sums over parts of K, then one pass that adds
+    them to the stream.  Returns the rows normed with ``next_weight`` and ``eps`` for the norm that reads the stream next, or None."""
+    M, K = x.shape
+    N = w.shape[0]
+    parts = mid_parts(x, w, wt)
+    _need(parts > 0, f"gemm_mid_residual_parts: not a product of this kernel, M={M} N={N} K={K}")
+    _need(wt.dtype == torch.bfloat16 and wt.is_cuda and wt.is_contiguous(), "gemm_mid_residual_parts: the weight's tile-major copy is bfloat16 on the GPU")
+    _need(res.shape == (M, N) and res.dtype == torch.float32 and res.is_contiguous(), "gemm_mid_residual_parts: shapes")
+    _need(next_weight is None or (next_weight.dtype == torch.float32 and next_weight.shape == (N,)), "next_weight must be float32 (N,)")
+    _dev(res, next_weight)
+    part = torch.empty((parts, M, N), dtype=torch.float32, device=res.device)
+    _check(lib().gs_gemm_mid_parts(_p(x), x.stride(0), _p(wt), _p(part), parts, M, N, K, _stream()))
+    ssq = torch.empty((M, 1), dtype=torch.float32, device=res.device)
+    normed = None if next_weight is None else torch.empty((M, N), dtype=torch.bfloat16, device=res.device)
+    _check(lib().gs_residual_from_parts(_p(part), parts, _p(res), _p(ssq), _p(next_weight), eps, _p(normed), 1, 0, M, N, _stream()))
+    return normed
+
+
 def mfma_ok(x, w: torch.Tensor) -> bool:
     """Whether the matrix-core product for many rows takes these operands (bfloat16, K a multiple of 8, aligned)."""
     return (isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2

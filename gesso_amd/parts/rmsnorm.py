@@ -42,7 +42,16 @@ class ResidualStream:
         from .runtime import DeferredLinear
         self.flush(rt)
         self.xs = self.xs_for = self.normed = self.rows = None
-        if isinstance(out, DeferredLinear) and self.res.shape[0] > rt.weighted_rows_max:
+        if isinstance(out, DeferredLinear) and self.res.shape[0] > rt.streaming_rows_max:
+            # some hundred rows: the same in two kernels, the rows normed by the second
+            w = getattr(next_norm, "row_weight", None)
+            eps = getattr(getattr(next_norm, "spec", None), "eps", None)
+            if w is not None and (w.shape != (self.res.shape[1],) or eps is None):
+                w = None
+            self.normed = rt.ops.gemm_mid_residual_parts(out.x, out.w, rt.tiles_of(out.w), self.res, next_weight=w,
+                                                         eps=0.0 if w is None else eps)
+            self.ssq, self.xs_for = None, next_norm if w is not None else None
+        elif isinstance(out, DeferredLinear) and self.res.shape[0] > rt.weighted_rows_max:
             # many rows: K is shared out over many blocks, and the pass that adds their partial sums to the stream
             # norms the rows for the next norm on its way (it sees whole rows)
             w = getattr(next_norm, "row_weight", None)
@@ -123,6 +132,9 @@ class RMSNorm(Part):
             mine = stream.xs_for is self
             return self.rt.ops.LazyNorm(stream.res, stream.ssq, self.weight, self.spec.eps, self.rt.dtype,
                                         xs=stream.xs if mine else None, ready=stream.normed if mine else None)
+        if (not self.rt.fused and rows is None and out is None and stream.pending is None and stream.normed is not None
+                and stream.xs_for is self and stream.normed.dtype == (out_dtype or self.rt.dtype)):
+            return stream.normed             # (the pass that added the last product has normed the rows)
         y = self.rt.ops.add_rmsnorm(stream.res, stream.pending, self.weight, self.spec.eps, out_dtype or self.rt.dtype,
                                     rows=rows, out=out)
         if rows is None:

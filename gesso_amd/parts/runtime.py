@@ -182,6 +182,8 @@ class Runtime:
 
     def dense(self, x):
         """``x`` as an ordinary tensor, whatever handle it came as."""
+        if isinstance(x, DeferredLinear):
+            return self.linear(x.x, x.w)
         if isinstance(x, self.ops.LazyNorm):
             x = x.materialize()
         return x.rows() if isinstance(x, self.ops.TiledRows) else x
@@ -262,9 +264,11 @@ class Runtime:
         return ops.swiglu(self.linear(x, w13))
 
     def project(self, x: torch.Tensor, w: torch.Tensor, bias=None):
-        """A sub-layer's last product.  While fused kernels are on it is deferred, so that the block can
-        compute it straight into the residual stream; else it is computed here."""
-        if self.fused and bias is None and self.ops.skinny_ok(x, w):
+        """A sub-layer's last product.  It is deferred while fused kernels are on, and for some hundred rows with a K so long
+        that it comes in parts, so that the block can compute it straight into the residual stream (:meth:`dense` computes it
+        for a block that does not); else it is computed here."""
+        if bias is None and (self.ops.skinny_ok(x, w) if self.fused else
+                             self.many_rows == "auto" and not self.no_library and self.ops.mid_parts(x, w, self.tiles_of(w)) > 0):
             return DeferredLinear(x, w)
         return self.linear(x, w, bias)
 
