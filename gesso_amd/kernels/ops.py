@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes
 from ctypes import c_float, c_int, c_long
+from functools import lru_cache
 
 import torch
 
@@ -654,14 +655,30 @@ def gemm_tiled(x: torch.Tensor, w: torch.Tensor, bias=None, out_dtype=None, out:
     return out
 
 
+@lru_cache(maxsize=4096)
+def _mid_takes(M: int, N: int, K: int, swiglu: bool) -> bool:
+    return bool(lib().gs_gemm_mid_takes(M, N, K, 1 if swiglu else 0))
+
+
+@lru_cache(maxsize=4096)
+def _mid_parts(M: int, N: int, K: int) -> int:
+    return lib().gs_gemm_mid_parts_takes(M, N, K)
+
+
+def _mid_operands(x, w: torch.Tensor, wt) -> bool:
+    """bfloat16 rows on the GPU, aligned, that do not overlap, and the whole weight ``wt`` was made of as it lies there (a part
+    or a transposed view of it can share its address)."""
+    if wt is None or not isinstance(x, torch.Tensor) or x.dtype is not torch.bfloat16 or not x.is_cuda or x.dim() != 2:
+        return False
+    K, (s0, s1) = x.shape[1], x.stride()
+    return (s1 == 1 and s0 >= K and s0 % 8 == 0 and x.data_ptr() % 16 == 0 and K == w.shape[1] and wt.shape == w.shape
+            and w.is_contiguous())
+
+
 def mid_ok(x, w: torch.Tensor, wt, swiglu: bool = False, out: torch.Tensor = None) -> bool:
-    """Whether the product of some hundred rows is the kernel's that reads the weight's tile-major copy ``wt``: bfloat16 rows
-    on the GPU, aligned, that do not overlap, the whole weight ``wt`` was made of as it lies there (a part or a transposed view
-    of it can share its address), an ``out`` the kernel can write, and sizes for which it is the faster one."""
-    return (wt is not None and isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 and x.dim() == 2 and x.is_cuda
-            and x.shape[1] == w.shape[1] and x.stride(1) == 1 and x.stride(0) >= x.shape[1] and x.stride(0) % 8 == 0
-            and x.data_ptr() % 16 == 0 and wt.shape == w.shape and w.is_contiguous()
-            and bool(lib().gs_gemm_mid_takes(x.shape[0], w.shape[0], w.shape[1], 1 if swiglu else 0))
+    """Whether the product of some hundred rows is the kernel's that reads the weight's tile-major copy ``wt``: operands as
+    :func:`_mid_operands` has them, an ``out`` the kernel can write, and sizes for which it is the faster one."""
+    return (_mid_operands(x, w, wt) and _mid_takes(x.shape[0], w.shape[0], w.shape[1], swiglu)
             and (out is None or (out.is_cuda and out.dtype == torch.bfloat16
                                  and out.shape == (x.shape[0], w.shape[0] // 2 if swiglu else w.shape[0])
                                  and out.stride(1) == 1 and out.stride(0) >= out.shape[1] and out.stride(0) % 4 == 0
@@ -673,8 +690,10 @@ def gemm_mid(x, w: torch.Tensor, wt, swiglu: bool = False, out: torch.Tensor = N
     asked it about these operands."""
     M, K = x.shape
     N = w.shape[0]
-    _need(checked or mid_ok(x, w, wt, swiglu, out), f"gemm_mid: not a product of this kernel, M={M} N={N} K={K}")
-    _need(wt.dtype == torch.bfloat16 and wt.is_cuda and wt.is_contiguous(), "gemm_mid: the weight's tile-major copy is bfloat16 on the GPU")
+    if not (checked or mid_ok(x, w, wt, swiglu, out)):
+        raise KernelError(f"gemm_mid: not a product of this kernel, M={M} N={N} K={K}")
+    if not (wt.dtype is torch.bfloat16 and wt.is_cuda and wt.is_contiguous()):
+        raise KernelError("gemm_mid: the weight's tile-major copy is bfloat16 on the GPU")
     if out is None:
         out = torch.empty((M, N // 2 if swiglu else N), dtype=torch.bfloat16, device=x.device)
     _check(lib().gs_gemm_mid(_p(x), x.stride(0), _p(wt), _p(out), out.stride(0), M, N, K, 1 if swiglu else 0, _stream()))
@@ -684,29 +703,31 @@ def gemm_mid(x, w: torch.Tensor, wt, swiglu: bool = False, out: torch.Tensor = N
 def mid_parts(x, w: torch.Tensor, wt) -> int:
     """Into how many parts of K :func:`gemm_mid_residual_parts` shares this product out; 0: it is not for it.  Operands as for
     :func:`mid_ok`."""
-    if not (wt is not None and isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 and x.dim() == 2 and x.is_cuda
-            and x.shape[1] == w.shape[1] and x.stride(1) == 1 and x.stride(0) >= x.shape[1] and x.stride(0) % 8 == 0
-            and x.data_ptr() % 16 == 0 and wt.shape == w.shape and w.is_contiguous()):
-        return 0
-    return lib().gs_gemm_mid_parts_takes(x.shape[0], w.shape[0], w.shape[1])
+    return _mid_parts(x.shape[0], w.shape[0], w.shape[1]) if w.shape[1] > 2048 and _mid_operands(x, w, wt) else 0
 
 
-def gemm_mid_residual_parts(x, w: torch.Tensor, wt, res: torch.Tensor, next_weight=None, eps: float = 0.0):
+def gemm_mid_residual_parts(x, w: torch.Tensor, wt, res: torch.Tensor, next_weight=None, eps: float = 0.0, parts: int = None):
     """``res += x @ w.T`` for some hundred rows and a long K in two kernels: partial sums over parts of K, then one pass that adds
-    them to the stream.  Returns the rows normed with ``next_weight`` and ``eps`` for the norm that reads the stream next, or None."""
+    them to the stream.  Returns the rows normed with ``next_weight`` and ``eps`` for the norm that reads the stream next, or None.
+    ``parts``: what :func:`mid_parts` has told the caller about these operands."""
     M, K = x.shape
     N = w.shape[0]
-    parts = mid_parts(x, w, wt)
-    _need(parts > 0, f"gemm_mid_residual_parts: not a product of this kernel, M={M} N={N} K={K}")
-    _need(wt.dtype == torch.bfloat16 and wt.is_cuda and wt.is_contiguous(), "gemm_mid_residual_parts: the weight's tile-major copy is bfloat16 on the GPU")
-    _need(res.shape == (M, N) and res.dtype == torch.float32 and res.is_contiguous(), "gemm_mid_residual_parts: shapes")
-    _need(next_weight is None or (next_weight.dtype == torch.float32 and next_weight.shape == (N,)), "next_weight must be float32 (N,)")
-    _dev(res, next_weight)
-    part = torch.empty((parts, M, N), dtype=torch.float32, device=res.device)
-    _check(lib().gs_gemm_mid_parts(_p(x), x.stride(0), _p(wt), _p(part), parts, M, N, K, _stream()))
-    ssq = torch.empty((M, 1), dtype=torch.float32, device=res.device)
+    parts = mid_parts(x, w, wt) if parts is None else parts
+    if parts <= 0:
+        raise KernelError(f"gemm_mid_residual_parts: not a product of this kernel, M={M} N={N} K={K}")
+    if not (wt.dtype is torch.bfloat16 and wt.is_cuda and wt.is_contiguous()):
+        raise KernelError("gemm_mid_residual_parts: the weight's tile-major copy is bfloat16 on the GPU")
+    if not (res.shape == (M, N) and res.dtype is torch.float32 and res.is_cuda and res.is_contiguous()):
+        raise KernelError("gemm_mid_residual_parts: shapes")
+    if next_weight is not None and not (next_weight.dtype is torch.float32 and next_weight.shape == (N,) and next_weight.is_cuda
+                                        and next_weight.is_contiguous()):
+        raise KernelError("next_weight must be float32 (N,)")
+    sheets = torch.empty(parts * M * N + M, dtype=torch.float32, device=res.device)      # and the new rows' sums of squares
+    at, stream = sheets.data_ptr(), _stream()
+    _check(lib().gs_gemm_mid_parts(x.data_ptr(), x.stride(0), wt.data_ptr(), at, parts, M, N, K, stream))
     normed = None if next_weight is None else torch.empty((M, N), dtype=torch.bfloat16, device=res.device)
-    _check(lib().gs_residual_from_parts(_p(part), parts, _p(res), _p(ssq), _p(next_weight), eps, _p(normed), 1, 0, M, N, _stream()))
+    _check(lib().gs_residual_from_parts(at, parts, res.data_ptr(), at + 4 * parts * M * N, _p(next_weight), eps, _p(normed), 1, 0,
+                                        M, N, stream))
     return normed
 
 
@@ -842,7 +863,7 @@ def skinny_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     if isinstance(x, TiledRows):
         return (w.dtype == torch.bfloat16 and x.shape[0] <= SKINNY_MAX_ROWS and w.is_contiguous()
                 and w.data_ptr() % 16 == 0)
-    return (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2 and x.shape[0] <= SKINNY_MAX_ROWS
+    return (x.dim() == 2 and x.shape[0] <= SKINNY_MAX_ROWS and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
             and x.shape[1] % 8 == 0 and x.stride(1) == 1 and (x.shape[0] <= 1 or x.stride(0) % 8 == 0)
             and x.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0)
 

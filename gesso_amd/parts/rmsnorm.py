@@ -42,14 +42,14 @@ class ResidualStream:
         from .runtime import DeferredLinear
         self.flush(rt)
         self.xs = self.xs_for = self.normed = self.rows = None
-        if isinstance(out, DeferredLinear) and self.res.shape[0] > rt.streaming_rows_max:
+        if isinstance(out, DeferredLinear) and out.parts:
             # some hundred rows: the same in two kernels, the rows normed by the second
             w = getattr(next_norm, "row_weight", None)
             eps = getattr(getattr(next_norm, "spec", None), "eps", None)
             if w is not None and (w.shape != (self.res.shape[1],) or eps is None):
                 w = None
             self.normed = rt.ops.gemm_mid_residual_parts(out.x, out.w, rt.tiles_of(out.w), self.res, next_weight=w,
-                                                         eps=0.0 if w is None else eps)
+                                                         eps=0.0 if w is None else eps, parts=out.parts)
             self.ssq, self.xs_for = None, next_norm if w is not None else None
         elif isinstance(out, DeferredLinear) and self.res.shape[0] > rt.weighted_rows_max:
             # many rows: K is shared out over many blocks, and the pass that adds their partial sums to the stream

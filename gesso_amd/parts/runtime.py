@@ -105,10 +105,11 @@ _NO_STAGE = _NoStage()
 class DeferredLinear:
     """A sub-layer's last product, not yet computed: ``x @ w.T`` to be added to the residual stream."""
 
-    __slots__ = ("x", "w")
+    __slots__ = ("x", "w", "parts")
 
-    def __init__(self, x, w):
+    def __init__(self, x, w, parts: int = 0):
         self.x, self.w = x, w
+        self.parts = parts            # into how many parts of K the product of some hundred rows is shared out
 
 
 class Runtime:
@@ -267,9 +268,14 @@ class Runtime:
         """A sub-layer's last product.  It is deferred while fused kernels are on, and for some hundred rows with a K so long
         that it comes in parts, so that the block can compute it straight into the residual stream (:meth:`dense` computes it
         for a block that does not); else it is computed here."""
-        if bias is None and (self.ops.skinny_ok(x, w) if self.fused else
-                             self.many_rows == "auto" and not self.no_library and self.ops.mid_parts(x, w, self.tiles_of(w)) > 0):
-            return DeferredLinear(x, w)
+        if bias is None:
+            if self.fused:
+                if self.ops.skinny_ok(x, w):
+                    return DeferredLinear(x, w)
+            elif self.many_rows == "auto" and not self.no_library:
+                parts = self.ops.mid_parts(x, w, self.tiles_of(w))
+                if parts:
+                    return DeferredLinear(x, w, parts)
         return self.linear(x, w, bias)
 
     # ------------------------------------------------------------------ handles between fused kernels
