@@ -137,6 +137,19 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
   return s;
 }
 
+// The activations of gated feed-forwards.  act 0: silu, z / (1 + exp(-z)); act 1: the tanh form of gelu, 0.5 z (1 + tanh(sqrt(2/pi) (z +
+// 0.044715 z^3))); act 2: gelu's error-function form; act 3: the square of relu.
+__device__ __forceinline__ float gated_act(float z, int act) {
+  if (act == 0) return z / (1.0f + expf(-z));
+  if (act == 2) return 0.5f * z * (1.0f + erff(z * 0.7071067811865476f));
+  if (act == 3) {
+    const float u = z < 0.f ? 0.f : z;               // (NaN stays NaN)
+    return u * u;
+  }
+  const float u = 0.7978845608028654f * (z + 0.044715f * z * z * z);
+  return 0.5f * z * (1.0f + tanhf(u));
+}
+
 // Eight consecutive values as float, from float32 or bfloat16 storage (16-byte aligned), and back.
 __device__ __forceinline__ void load8f(const float* p, float* v) {
   const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4);

@@ -956,19 +956,6 @@ extern "C" int gs_add_rmsnorm_pair(float* res, const void* d1, const void* d2, i
 
 // in (T, 2F) = gate | up (a product's float32 sums or rounded rows), bias (2F) float32 or absent:
 //   out[t, j] = act(gate[t, j] + bias[j]) * (up[t, j] + bias[F + j])
-// act 0: silu, z / (1 + exp(-z)); act 1: the tanh form of gelu, 0.5 z (1 + tanh(sqrt(2/pi) (z + 0.044715 z^3))); act 2: gelu's
-// error-function form; act 3: the square of relu.
-__device__ __forceinline__ float gated_act(float z, int act) {
-  if (act == 0) return z / (1.0f + expf(-z));
-  if (act == 2) return 0.5f * z * (1.0f + erff(z * 0.7071067811865476f));
-  if (act == 3) {
-    const float u = z < 0.f ? 0.f : z;               // (NaN stays NaN)
-    return u * u;
-  }
-  const float u = 0.7978845608028654f * (z + 0.044715f * z * z * z);
-  return 0.5f * z * (1.0f + tanhf(u));
-}
-
 template <typename TI, typename TO>
 __global__ void gated_act_kernel(const TI* __restrict__ in, const float* __restrict__ bias, TO* __restrict__ out, int F,
                                  long n, int act) {

@@ -75,6 +75,19 @@ extern "C" int gs_gemm_skinny(const void* X, int ldx, int x_tiled, const float* 
   return 0;
 }
 
+// Y (M, N / 2) = act(X Wg^T + bg) * (X Wu^T + bu): Wt the tile-major copy of the gate rows, then the up rows; bias (N) float32 in the
+// same order, or null; act as gated_act numbers them.
+extern "C" int gs_gemm_skinny_gated(const void* X, int ldx, int x_tiled, const void* Wt, const float* bias, int act, void* Y, int y_tiled,
+                                    int M, int N, int K, hipStream_t stream) {
+  GS_REQUIRE(Wt && N % 32 == 0 && act >= 0 && act <= 3, "gemm_skinny_gated: needs the tile-major weight, whole tiles of gate and of up rows (N=%d) and a known activation (%d)", N, act);
+  if (check_common(Wt, M, N, K) || check_tiles(Wt, N, K, N / 2) || check_rows(X, ldx, x_tiled, K) || check_tiled_out(y_tiled, GS_BF16, N / 2)) return -1;
+  GS_REQUIRE(Y && (((uintptr_t)Y | (uintptr_t)bias) & 15) == 0, "gemm_skinny_gated: the result and the bias must be 16-byte aligned");
+  if (M == 0) return 0;
+  gs_skinny_run_gated(X, ldx, x_tiled, Wt, bias, act, Y, y_tiled, M, N, K, stream);
+  GS_LAUNCH_CHECK("gemm_skinny_gated");
+  return 0;
+}
+
 // Partial sums per row that gs_gemm_skinny_residual writes for N columns.
 extern "C" int gs_gemm_skinny_residual_blocks(int N, int tile_major) {
   return gs_ceil_div(N, tile_major && gs_skinny_halves(N) ? 8 : 16);

@@ -7,6 +7,7 @@ void gs_skinny_residual_rows(const SkinnyCall& c);
 void gs_skinny_conv_rows(const SkinnyCall& c);
 void gs_skinny_plain_tiles(const SkinnyCall& c);
 void gs_skinny_plain_half_tiles(const SkinnyCall& c);
+void gs_skinny_gated_tiles(const SkinnyCall& c);
 void gs_skinny_residual_tiles(const SkinnyCall& c);
 void gs_skinny_residual_half_tiles(const SkinnyCall& c);
 void gs_skinny_conv_tiles(const SkinnyCall& c);
@@ -44,6 +45,15 @@ void gs_skinny_run_plain(const void* X, int ldx, int x_tiled, const float* res, 
   // 2304 x 4608 26.8 and 16.9).
   if (Wt && epilogue == 0 && N % 16 == 0 && N <= 2048 && K >= 2048 && M >= 4 && M <= 32) gs_skinny_plain_half_tiles(c);
   else Wt ? gs_skinny_plain_tiles(c) : gs_skinny_plain_rows(c);
+}
+
+void gs_skinny_run_gated(const void* X, int ldx, int x_tiled, const void* Wt, const float* bias, int act, void* Y, int y_tiled, int M,
+                         int N, int K, hipStream_t stream) {
+  SkinnyCall c = base(X, ldx, x_tiled, Wt, Wt, Y, GS_BF16, N / 2, M, N, K, 4, stream);
+  c.ex.y_tiled = y_tiled;
+  c.ex.act_bias = bias;
+  c.ex.act = act;
+  gs_skinny_gated_tiles(c);
 }
 
 void gs_skinny_run_residual(const void* X, int ldx, int x_tiled, const void* W, const void* Wt, float* res, float* ssq_out,

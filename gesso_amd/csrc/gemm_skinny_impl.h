@@ -42,6 +42,8 @@
 //      weight rows and the more of K a block takes, the more X traffic; sharing K over blocks caps it.
 //   2  added to the residual stream in place (float32), and the sums of squares of the new rows over this
 //      block's columns stored as partial sums for the next norm.
+//   4  gated activation: as 1, but the two products are rounded as they would be stored, then biased (float32, or none), and the
+//      activation is the one asked for: the feed-forwards whose gate is no silu.
 //   3  gated short convolution of a decode step: tiles are the B, C, X rows of 16 channels; u = B X,
 //      y = taps . (history, u) + bias, out = C y, history shifted; one token per sequence.
 #pragma once
@@ -115,7 +117,10 @@ struct SkinnyExtra {
                          // and history in registers and moves them sixteen bytes at a time
   // layouts
   int x_tiled;           // X comes as tiled rows (PRO 0 only; K a multiple of 32)
-  int y_tiled;           // EPI 1, 3: Y, EPI 2: xs_out are written as tiled rows (their width a multiple of 32)
+  // EPI 4
+  const float* act_bias; // (N): the gate rows', then the up rows'; or null
+  int act;
+  int y_tiled;           // EPI 1, 3, 4: Y, EPI 2: xs_out are written as tiled rows (their width a multiple of 32)
 };
 
 template <int R, int MT, int WAVES, int PRO, int EPI, int LAYOUT, typename TOut>
@@ -124,6 +129,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16* __r
                                                                   TOut* __restrict__ Y, int ldy, int M, int N,
                                                                   int K, SkinnyExtra ex) {
   constexpr int SHUF = LAYOUT & ~SKINNY_ONCE;
+  constexpr bool GLU = EPI == 1 || EPI == 4;
   extern __shared__ float red[];  // WAVES (one row tile: WAVES - 1) x R x MT x 64 x 4 floats
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   static_assert(WAVES >= MT, "a wavefront for each row tile's epilogue");
@@ -133,7 +139,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16* __r
   const int half = N >> 1;
   // rows of W this block owns
   int rowbase[R];
-  if (EPI == 1) {
+  if (GLU) {
     const int n0 = blockIdx.x * 16 * (R / 2);
 #pragma unroll
     for (int r = 0; r < R; ++r) rowbase[r] = n0 + (r >> 1) * 16 + ((r & 1) ? half : 0);
@@ -155,7 +161,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16* __r
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     int n = rowbase[r] + r16;
-    if (EPI == 1 && !(r & 1) && n >= half) n = half - 1;  // gate rows end at N/2
+    if (GLU && !(r & 1) && n >= half) n = half - 1;  // gate rows end at N/2
     if (EPI == 3 && n >= (r + 1) * (N / 3)) n = (r + 1) * (N / 3) - 1;
     if (n >= N) n = N - 1;                                // clamped: loaded, never stored
     if (SHUF == 2)
@@ -264,6 +270,15 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16* __r
           for (int i = 0; i < 4; ++i)
             if (n + i < N) rold[r][i] = p[i];
       }
+    }
+  }
+  f32x4_t gbias[EPI == 4 ? R : 1];
+  if (EPI == 4 && wave < MT) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int n = rowbase[r] + kg * 4;               // (whole tiles: N / 2 is a multiple of 16; a tile past the last reads the last)
+      const int end = r & 1 ? N : half;
+      gbias[r] = ex.act_bias ? *reinterpret_cast<const f32x4_t*>(ex.act_bias + (n < end ? n : end - 4)) : f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
   }
   const bool pre_conv = EPI == 3 && ex.conv_vec != 0;
@@ -572,6 +587,17 @@ _Pragma("unroll")                                                               
       const int n = rowbase[r] + kg * 4;
       if (N - n > 0 && half_ok) store4<TOut>(Yp + (size_t)em * ldy + n, sum[r], N - n);
     }
+  } else if (EPI == 4) {
+    if (!live) return;
+#pragma unroll
+    for (int r = 0; r < R; r += 2) {
+      const int n = rowbase[r] + kg * 4;
+      f32x4_t o;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        o[i] = gated_act(to_f32(f32_to_bf16(sum[r][i])) + gbias[r][i], ex.act) * (to_f32(f32_to_bf16(sum[r + 1][i])) + gbias[EPI == 4 ? r + 1 : 0][i]);
+      if (half - n > 0) store4<TOut>(Y + (ex.y_tiled ? tiled_index(em, n, MT) : (size_t)em * ldy + n), o, half - n);
+    }
   } else if (EPI == 1) {
     if (!live) return;
 #pragma unroll
@@ -741,6 +767,18 @@ static void skinny_plain_halves(const SkinnyCall& c) {
   }
 #undef GS_HALF_PRO
 #undef GS_HALF
+}
+
+// Gate and up with biases and an activation of choice (EPI 4): bfloat16 rows in and out, the tile-major weight.
+template <int LAYOUT>
+static void skinny_gated(const SkinnyCall& c) {
+  const bf16 *x = c.x, *w = c.w;
+  void* Y = c.Y;
+  const int ldx = c.ldx, ldy = c.ldy, M = c.M, N = c.N, K = c.K;
+  const SkinnyExtra& ex = c.ex;
+  hipStream_t stream = c.stream;
+  const int blocks = gs_ceil_div(N / 2, 16);
+  GS_BY_MT4(2, 8, 8, 4, 4, 0, 4, bf16, blocks)
 }
 
 template <int LAYOUT>

@@ -2,6 +2,7 @@
 #include "gemm_skinny_impl.h"
 
 void gs_skinny_plain_tiles_once(const SkinnyCall& c) { skinny_plain<1 | SKINNY_ONCE>(c); }
+void gs_skinny_gated_tiles_once(const SkinnyCall& c) { skinny_gated<1 | SKINNY_ONCE>(c); }
 void gs_skinny_plain_half_tiles_once(const SkinnyCall& c) { skinny_plain_halves<2 | SKINNY_ONCE>(c); }
 void gs_skinny_residual_tiles_once(const SkinnyCall& c) { skinny_residual<1 | SKINNY_ONCE>(c); }
 void gs_skinny_residual_half_tiles_once(const SkinnyCall& c) { skinny_residual<2 | SKINNY_ONCE>(c); }

@@ -956,6 +956,22 @@ def gemm_skinny(x, w: torch.Tensor, out_dtype=None, out=None, swiglu: bool = Fal
     return out
 
 
+def gemm_skinny_gated(x, w: torch.Tensor, wt, bias, activation: str, tiled: bool = False):
+    """``act(x @ wg.T + bg) * (x @ wu.T + bu)`` in bfloat16 for at most 64 rows: ``w`` holds gate rows, then up rows, ``wt`` its
+    tile-major copy, ``bias`` float32 in the same order or None.  The two products are rounded before the biases, as
+    :func:`gated_act` reads them.  ``tiled``: the result as :class:`TiledRows`."""
+    _dev(w, wt, bias)
+    M, K = x.shape
+    N = w.shape[0]
+    _need(skinny_ok(x, w) and wt is not None and wt.shape == w.shape == (N, K) and wt.dtype == torch.bfloat16 and N % 32 == 0,
+          "gemm_skinny_gated: operands must be bfloat16, at most 64 rows, with the weight's tile-major copy")
+    _need(bias is None or (bias.dtype == torch.float32 and bias.shape == (N,)), "gemm_skinny_gated: bias must be float32 (2F,)")
+    _need(activation in GATED_ACTS, f"gemm_skinny_gated: the activation is one of {sorted(GATED_ACTS)}, not {activation!r}")
+    out, buf, otiled = _rows_out(bool(tiled), M, N // 2, w.device)
+    _check(lib().gs_gemm_skinny_gated(*_x_args(x), _p(wt), _p(bias), GATED_ACTS[activation], _p(buf), otiled, M, N, K, _stream()))
+    return out
+
+
 def gemm_skinny_residual(x: torch.Tensor, w: torch.Tensor, res: torch.Tensor, wt=None, next_weight=None,
                          xs: torch.Tensor = None) -> torch.Tensor:
     """``res += x @ w.T`` in place (float32); returns the new rows' sums of squares as partial sums ``(M, nb)``.

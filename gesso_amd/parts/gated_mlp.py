@@ -49,8 +49,13 @@ class GatedMLP(Part):
         bias where it adds the product."""
         rt = self.rt
         with rt.stage("ffn_gateup"):
-            gu = rt.linear(rt.dense(x), self.w_gu)
-            a = rt.ops.gated_act(gu, self.b_gu, self.spec.activation, rt.dtype)
+            x, wt = rt.dense(x), rt.tiles_of(self.w_gu)
+            if rt.dtype == torch.bfloat16 and wt is not None and self.w_gu.shape[0] % 32 == 0 and rt.ops.skinny_ok(x, self.w_gu):
+                # few rows: biases, activation and the halves' product in the product's own epilogue
+                tiled = (defer_bias or self.b_down is None) and rt.rows_tiled(self.w_gu.shape[0] // 2)
+                a = rt.ops.gemm_skinny_gated(x, self.w_gu, wt, self.b_gu, self.spec.activation, tiled=tiled)
+            else:
+                a = rt.ops.gated_act(rt.linear(x, self.w_gu), self.b_gu, self.spec.activation, rt.dtype)
         if defer_bias:
             return rt.linear(a, self.w_down), self.b_down
         return rt.linear(a, self.w_down, self.b_down)
