@@ -30,7 +30,10 @@ typedef __attribute__((ext_vector_type(2))) unsigned u32x2_t;
 #define LM_ROWS 64     // query rows a block
 
 // CT: the most tiles of 16 value columns (c <= 16 CT); the score product takes up to CT / 2 + 2 steps of 32 columns.
-template <int CT, int KSTEP>
+// SHARE: a block has at most 16 query rows (a single token of up to 16 heads): every wavefront holds the same rows and computes the
+// same scores, and takes a quarter of the value columns, whose sums alone it holds (rows of 512 + 64, with the merge: 8 sequences of 290
+// rows 15.4 and 14.6 us with a test on each of all columns' sums and so, 32 sequences 21.7 and 21.0).
+template <int CT, int KSTEP, bool SHARE>
 __global__ __launch_bounds__(256) void attention_latent_mfma_kernel(
     const bf16* __restrict__ qa, const bf16* __restrict__ cache, const int* __restrict__ positions,
     const int* __restrict__ tile_seq, const int* __restrict__ tile_row, const int* __restrict__ tile_n,
@@ -56,9 +59,8 @@ __global__ __launch_bounds__(256) void attention_latent_mfma_kernel(
   const int nrows = nt * hb;
   const int pos0 = positions[row0];                  // a tile's tokens stand at consecutive positions
   const int* bt = block_table + (size_t)seq * max_blocks;
-  // A block with at most 16 query rows (a single token of up to 16 heads): every wavefront holds the same rows and
-  // computes the same scores, and takes a quarter of the value columns.
-  const bool share = nrows <= 16;
+  const bool share = SHARE || nrows <= 16;        // (a block of a list may have as few rows: the same, with room for all columns)
+  constexpr int LG = SHARE ? (CT / 4 + 3) / 4 : CT / 4;       // groups of four value tiles a wavefront has room for
   const int wrow = share ? 0 : wave * 16;
   const int m = wrow + r16;
   const bool valid = m < nrows;
@@ -77,9 +79,9 @@ __global__ __launch_bounds__(256) void attention_latent_mfma_kernel(
     if (valid && f < D) v = *reinterpret_cast<const u32x4_t*>(qa + qrow * D + f);
     qf[kk] = __builtin_bit_cast(bf16x8_t, v);
   }
-  f32x4_t acc[CT];
+  f32x4_t acc[4 * LG];
 #pragma unroll
-  for (int dt = 0; dt < CT; ++dt) acc[dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int dt = 0; dt < 4 * LG; ++dt) acc[dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float mrun = -INFINITY, lrun = 0.f;
   if (sinks && blockIdx.z == 0) {                    // the sink's own term, counted by the first of the blocks that share a row's keys
     mrun = sinks[head] * LM_LOG2E;
@@ -95,6 +97,7 @@ __global__ __launch_bounds__(256) void attention_latent_mfma_kernel(
   const int g_lo = share ? wave * gq : 0;
   const int g_hi = share ? ((wave + 1) * gq < ngr ? (wave + 1) * gq : ngr) : ngr;
   const int dt_lo = 4 * g_lo, dt_hi = 4 * g_hi < ct ? 4 * g_hi : ct;
+  const int dt_0 = SHARE ? dt_lo : 0;                // the tile that acc[0] is
   // with the rows shared out over nsplit blocks (blockIdx.z), each takes a run of whole steps
   const int nsteps = (kmax - kmin) / KSTEP + 1;
   const int per = (nsteps + nsplit - 1) / nsplit;
@@ -204,12 +207,13 @@ __global__ __launch_bounds__(256) void attention_latent_mfma_kernel(
     // value columns in groups of four tiles: eight independent products side by side (four tiles, each with the
     // weights' first and second term)
 #pragma unroll
-    for (int g4 = 0; g4 < CT / 4; ++g4)
+    for (int lg = 0; lg < LG; ++lg) {
+      const int g4 = SHARE ? g_lo + lg : lg;
       if (g4 >= g_lo && g4 < g_hi) {
 #pragma unroll
         for (int u = 0; u < 4; ++u)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) acc[4 * g4 + u][e] *= alpha;
+          for (int e = 0; e < 4; ++e) acc[4 * lg + u][e] *= alpha;
 #pragma unroll
         for (int ch = 0; ch < NC; ++ch) {
           bf16x8_t a[4];
@@ -222,12 +226,13 @@ __global__ __launch_bounds__(256) void attention_latent_mfma_kernel(
           }
 #pragma unroll
           for (int u = 0; u < 4; ++u)
-            acc[4 * g4 + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], phi[ch], acc[4 * g4 + u], 0, 0, 0);
+            acc[4 * lg + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], phi[ch], acc[4 * lg + u], 0, 0, 0);
 #pragma unroll
           for (int u = 0; u < 4; ++u)
-            acc[4 * g4 + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], plo[ch], acc[4 * g4 + u], 0, 0, 0);
+            acc[4 * lg + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], plo[ch], acc[4 * lg + u], 0, 0, 0);
         }
       }
+    }
   }
   if (!valid) return;
   if (nsplit > 1) {
@@ -238,28 +243,41 @@ __global__ __launch_bounds__(256) void attention_latent_mfma_kernel(
       part_ml[prow * 2 + 1] = lrun;
     }
 #pragma unroll
-    for (int dt = 0; dt < CT; ++dt)
-      if (dt >= dt_lo && dt < dt_hi)
-        *reinterpret_cast<f32x4_t*>(part_o + prow * c + 16 * dt + 4 * g) = acc[dt];
+    for (int i = 0; i < 4 * LG; ++i) {
+      const int dt = dt_0 + i;
+      if (dt >= dt_lo && dt < dt_hi) *reinterpret_cast<f32x4_t*>(part_o + prow * c + 16 * dt + 4 * g) = acc[i];
+    }
     return;
   }
   const float inv = 1.0f / lrun;
 #pragma unroll
-  for (int dt = 0; dt < CT; ++dt)
+  for (int i = 0; i < 4 * LG; ++i) {
+    const int dt = dt_0 + i;
     if (dt >= dt_lo && dt < dt_hi) {
       u32x2_t w;
-      w.x = (unsigned)f32_to_bf16(acc[dt][0] * inv).x | ((unsigned)f32_to_bf16(acc[dt][1] * inv).x << 16);
-      w.y = (unsigned)f32_to_bf16(acc[dt][2] * inv).x | ((unsigned)f32_to_bf16(acc[dt][3] * inv).x << 16);
+      w.x = (unsigned)f32_to_bf16(acc[i][0] * inv).x | ((unsigned)f32_to_bf16(acc[i][1] * inv).x << 16);
+      w.y = (unsigned)f32_to_bf16(acc[i][2] * inv).x | ((unsigned)f32_to_bf16(acc[i][3] * inv).x << 16);
       *reinterpret_cast<u32x2_t*>(out + qrow * c + 16 * dt + 4 * g) = w;
     }
+  }
 }
 
 // out[row, :] = sum_z part_o[z, row, :] 2^(m_z - M) / sum_z l_z 2^(m_z - M), M = max_z m_z: the shares of the blocks
-// that walked a row's keys in parts, added in the order of the parts.
-__global__ void attention_latent_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
+// that walked a row's keys in parts, added in the order of the parts.  The loads of eight parts are asked for together, the first
+// eight before the weights are known (8 sequences of 290 rows, both kernels: 16.7 us with one load after the other, so 15.4).
+__global__ __launch_bounds__(512) void attention_latent_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                               int nsplit, int rows_total, int c, bf16* __restrict__ out) {
   __shared__ float wz[64];           // the parts' weights 2^(m_z - M) / L (at most 64 parts)
   const int row = blockIdx.x, lane = threadIdx.x & 63;
+  const size_t sheet = (size_t)rows_total * c;
+  const float* src = part_o + (size_t)row * c;
+  // (a part or a column that does not exist is read from the last and not counted)
+  auto ask = [&](float* v, int z0, int j) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = src[(size_t)(z0 + q < nsplit ? z0 + q : nsplit - 1) * sheet + (j < c ? j : c - 1)];
+  };
+  float v[8];
+  ask(v, 0, threadIdx.x);
   // every wavefront of the block finds the weights itself: lane z holds part z
   float m = -INFINITY, l = 0.f;
   if (lane < nsplit) {
@@ -267,14 +285,19 @@ __global__ void attention_latent_merge_kernel(const float* __restrict__ part_o, 
     m = ml[0];
     l = ml[1];
   }
-  const float M = wave_max(m);
+  const float M = wave_max_dpp(m);
   const float w = lane < nsplit ? __builtin_amdgcn_exp2f(m - M) : 0.f;
-  const float L = wave_sum(l * w);
+  const float L = wave_sum_dpp(l * w);
   if (threadIdx.x < 64) wz[lane] = w / L;
   __syncthreads();
   for (int j = threadIdx.x; j < c; j += blockDim.x) {
     float a = 0.f;
-    for (int z = 0; z < nsplit; ++z) a += part_o[((size_t)z * rows_total + row) * c + j] * wz[z];
+    for (int z0 = 0; z0 < nsplit; z0 += 8) {
+      if (z0 > 0 || j != (int)threadIdx.x) ask(v, z0, j);
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        if (z0 + q < nsplit) a += v[q] * wz[z0 + q];
+    }
     out[(size_t)row * c + j] = f32_to_bf16(a);
   }
 }
@@ -311,42 +334,32 @@ extern "C" int gs_attention_latent_mfma(const void* qa, const void* cache, const
   const int hgroups = gs_ceil_div(H, HB);
   GS_REQUIRE(hgroups <= 65535, "attention_latent_mfma: too many heads");
   dim3 grid(ntiles, hgroups, nsplit);
+  // (a step of single tokens without a list, of up to 16 heads: its blocks have no more rows than that)
+  const bool few = tile_seq == nullptr && HB <= 16;
+#define LM_RUN(CT, KSTEP, FEW)                                                                                         \
+  do {                                                                                                                  \
+    const size_t lds = (size_t)KSTEP * (Dp + 8) * 2 + (size_t)((c + 63) & ~63) * (KSTEP + 4) * 2;                       \
+    /* more than the default limit of dynamic LDS: asked for once per kernel */                                         \
+    static const hipError_t asked = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_latent_mfma_kernel<CT, KSTEP, FEW>), \
+                                                        hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);         \
+    GS_REQUIRE(asked == hipSuccess, "attention_latent_mfma: cannot raise the LDS limit: %s", hipGetErrorString(asked)); \
+    GS_REQUIRE(lds <= 96 * 1024, "attention_latent_mfma: %zu bytes of LDS", lds);                                       \
+    attention_latent_mfma_kernel<CT, KSTEP, FEW><<<grid, 256, lds, stream>>>(                                           \
+        (const bf16*)qa, (const bf16*)cache, positions, tile_seq, tile_row, tile_n, block_table, max_blocks, page_size, \
+        window, scale, (bf16*)out, part_o, part_ml, nsplit, rows_total, H, HB, c, D, sinks);                            \
+  } while (0)
   if (c <= 128 && D <= 32 * (8 / 2 + 2)) {
-    const size_t lds = (size_t)64 * (Dp + 8) * 2 + (size_t)((c + 63) & ~63) * (64 + 4) * 2;
-    attention_latent_mfma_kernel<8, 64><<<grid, 256, lds, stream>>>(
-        (const bf16*)qa, (const bf16*)cache, positions, tile_seq, tile_row, tile_n, block_table, max_blocks, page_size,
-        window, scale, (bf16*)out, part_o, part_ml, nsplit, rows_total, H, HB, c, D, sinks);
+    if (few) LM_RUN(8, 64, true); else LM_RUN(8, 64, false);
   } else if (c <= 256 && D <= 32 * (16 / 2 + 2)) {
     // latents up to 256: half the accumulators of the widest form, so steps of 64 rows fit
-    const size_t lds = (size_t)64 * (Dp + 8) * 2 + (size_t)((c + 63) & ~63) * (64 + 4) * 2;
-    static bool raised_mid = false;
-    if (!raised_mid) {
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_latent_mfma_kernel<16, 64>),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
-      GS_REQUIRE(e == hipSuccess, "attention_latent_mfma: cannot raise the LDS limit: %s", hipGetErrorString(e));
-      raised_mid = true;
-    }
-    GS_REQUIRE(lds <= 96 * 1024, "attention_latent_mfma: %zu bytes of LDS", lds);
-    attention_latent_mfma_kernel<16, 64><<<grid, 256, lds, stream>>>(
-        (const bf16*)qa, (const bf16*)cache, positions, tile_seq, tile_row, tile_n, block_table, max_blocks, page_size,
-        window, scale, (bf16*)out, part_o, part_ml, nsplit, rows_total, H, HB, c, D, sinks);
+    if (few) LM_RUN(16, 64, true); else LM_RUN(16, 64, false);
   } else {
-    const size_t lds = (size_t)32 * (Dp + 8) * 2 + (size_t)((c + 63) & ~63) * (32 + 4) * 2;
-    static bool raised = false;
-    if (!raised) {
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_latent_mfma_kernel<32, 32>),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
-      GS_REQUIRE(e == hipSuccess, "attention_latent_mfma: cannot raise the LDS limit: %s", hipGetErrorString(e));
-      raised = true;
-    }
-    GS_REQUIRE(lds <= 96 * 1024, "attention_latent_mfma: %zu bytes of LDS", lds);
-    attention_latent_mfma_kernel<32, 32><<<grid, 256, lds, stream>>>(
-        (const bf16*)qa, (const bf16*)cache, positions, tile_seq, tile_row, tile_n, block_table, max_blocks, page_size,
-        window, scale, (bf16*)out, part_o, part_ml, nsplit, rows_total, H, HB, c, D, sinks);
+    if (few) LM_RUN(32, 32, true); else LM_RUN(32, 32, false);
   }
+#undef LM_RUN
   GS_LAUNCH_CHECK("attention_latent_mfma");
   if (nsplit > 1) {
-    attention_latent_merge_kernel<<<rows_total, c >= 256 ? 256 : 64, 0, stream>>>(part_o, part_ml, nsplit, rows_total, c, (bf16*)out);
+    attention_latent_merge_kernel<<<rows_total, gs_ceil_div(c, 64) * 64, 0, stream>>>(part_o, part_ml, nsplit, rows_total, c, (bf16*)out);
     GS_LAUNCH_CHECK("attention_latent_merge");
   }
   return 0;

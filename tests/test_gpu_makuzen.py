@@ -224,6 +224,34 @@ def test_attention_over_latent_rows_on_the_matrix_cores_at_other_sizes(ops, H, n
     assert float((got[0] - want[-1]).abs().max()) <= tol(dtype, want, 1e-5, 2e-2)
 
 
+@pytest.mark.parametrize("H,c,r", [(1, 16, 8), (16, 128, 32), (5, 144, 8), (16, 256, 32), (16, 512, 64), (7, 272, 16)])
+@pytest.mark.parametrize("nsplit", [1, 3, 9, 20])
+@pytest.mark.parametrize("sink", [False, True])
+def test_single_tokens_over_latent_rows_in_all_parts_are_those_of_a_list_of_tiles(ops, H, c, r, nsplit, sink):
+    """A step of single tokens of up to 16 heads runs the form whose wavefronts hold a quarter of the value columns' sums; the same
+    tokens as a list of tiles of one run the other: the same bits, with one part, with fewer and with more parts than the merge
+    asks for at once (some without a row), and against the general kernel."""
+    g = gen(H + c + nsplit)
+    lens, ps = [1, 40, 333], 16
+    pages = [-(-n // ps) for n in lens]
+    pool = torch.randn(sum(pages), 1, ps, c + r, generator=g).bfloat16().to(DEV)
+    table = torch.zeros(3, max(pages), dtype=torch.int32)
+    order = torch.randperm(sum(pages), generator=g).tolist()
+    for i, n in enumerate(pages):
+        table[i, :n] = torch.tensor([order.pop() for _ in range(n)], dtype=torch.int32)
+    table = table.to(DEV)
+    qa = (torch.randn(3, H * (c + r), generator=g) * 0.3).bfloat16().to(DEV)
+    positions = torch.tensor([n - 1 for n in lens], dtype=torch.int32, device=DEV)
+    sinks = torch.randn(H, generator=g).to(DEV) if sink else None
+    tiles = torch.tensor([[0, 1, 2], [0, 1, 2], [1, 1, 1]], dtype=torch.int32, device=DEV)
+    run = lambda t: ops.attention_latent_mfma(qa, pool, positions, t, table, ps, None, 0.2, H, c, r, 3, nsplit=nsplit, sinks=sinks)
+    got = run(None)
+    assert bool(torch.isfinite(got.float()).all()) and torch.equal(got, run(tiles))
+    if not sink:
+        want = ops.attention_latent(qa, pool, positions, torch.arange(3, dtype=torch.int32, device=DEV), table, ps, None, 0.2, H, c, r, 3)
+        assert float((got.float() - want.float()).abs().max()) <= 2e-2 * max(1.0, float(want.float().abs().max()))
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("window,ps", [(24, 8), (21, 8), (33, 16), (None, 16)])
 def test_a_row_that_stands_out_is_found_far_back_at_page_borders_and_just_inside_the_window(ops, dtype, window, ps):
