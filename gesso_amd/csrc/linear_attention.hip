@@ -45,17 +45,46 @@ linear_attention_scan_kernel(const TI* __restrict__ x, int ld, int oq, int ok, i
   if (t1 <= t0 || (below > 0 && t1 - t0 >= below)) return;      // (longer sequences are another kernel's)
   const float d = decay[h];
   float* S = state + (((size_t)slots[seq] * H + h) * n) * m;
+  // The first token's values are asked for before the state (loads return in order: behind it they would come last, and the
+  // conversion and the barrier after all of it).  A thread's feature, its partner of the rotation and its value column; what it has
+  // none of is read from the first.  (8 rows, 16 heads of 128 x 128 10.35 and 8.15 us, one row 9.05 and 6.65, turned heads of 64 x 128 6.9 and
+  // 5.85.)
+  const int half = rd >> 1;
+  const bool ahead = n <= 256;
+  const int mine = tid < n ? tid : 0, pair = mine < half ? mine + half : mine < rd ? mine - half : mine;
+  const TI* first = x + (size_t)t0 * ld;
+  const TI q1 = first[oq + h * n + mine], k1 = first[ok + h * n + mine], q2 = first[oq + h * n + pair], k2 = first[ok + h * n + pair];
+  const TI v1 = first[ov + h * m + (tid < LA_COLS && j0 + tid < m ? j0 + tid : 0)];
+  float c1 = 1.f, s1 = 0.f;
+  if (rd > 0) {
+    const size_t at = (size_t)positions[t0] * half + (mine < half ? mine : mine < rd ? mine - half : 0);
+    c1 = cos_t[at];
+    s1 = sin_t[at];
+  }
   float s[RMAX];
 #pragma unroll
   for (int r = 0; r < RMAX; ++r) {
     const int i = rg + 4 * r;
     s[r] = (i < n && j < m) ? S[(size_t)i * m + j] : 0.f;
   }
-  const int half = rd >> 1;
   for (int tb = t0; tb < t1; tb += LA_TB) {
     const int nb = t1 - tb < LA_TB ? t1 - tb : LA_TB;
     __syncthreads();                                   // the batch before has been read
-    for (int idx = tid; idx < nb * n; idx += 256) {
+    const int done = ahead && tb == t0 ? 1 : 0;        // tokens of this batch whose values are at hand
+    if (done) {
+      float qv = la_act(to_f32(q1), act), kv = la_act(to_f32(k1), act);
+      if (mine < rd) {
+        const float qo = la_act(to_f32(q2), act), ko = la_act(to_f32(k2), act);
+        qv = mine < half ? qv * c1 - qo * s1 : qv * c1 + qo * s1;
+        kv = mine < half ? kv * c1 - ko * s1 : kv * c1 + ko * s1;
+      }
+      if (tid < n) {
+        qs[0][tid] = qv;
+        ks[0][tid] = kv * key_scale;
+      }
+      if (tid < LA_COLS) vs[0][tid] = j0 + tid < m ? la_act(to_f32(v1), act) : 0.f;
+    }
+    for (int idx = tid + done * n; idx < nb * n; idx += 256) {
       const int tt = idx / n, i = idx - tt * n;
       const TI* row = x + (size_t)(tb + tt) * ld;
       float qv = la_act(to_f32(row[oq + h * n + i]), act);
@@ -74,7 +103,7 @@ linear_attention_scan_kernel(const TI* __restrict__ x, int ld, int oq, int ok, i
       qs[tt][i] = qv;
       ks[tt][i] = kv * key_scale;
     }
-    for (int idx = tid; idx < nb * LA_COLS; idx += 256) {
+    for (int idx = tid + done * LA_COLS; idx < nb * LA_COLS; idx += 256) {
       const int tt = idx / LA_COLS, c = idx - tt * LA_COLS;
       vs[tt][c] = j0 + c < m ? la_act(to_f32(x[(size_t)(tb + tt) * ld + ov + h * m + j0 + c]), act) : 0.f;
     }
