@@ -12,7 +12,7 @@
 // linear_attention_scan: one block per (sequence, head, tile of 64 value columns); the columns of S are independent
 // of each other, so wide values share out over blocks.  Lane l of wavefront w holds the state's rows rg, rg + 4, ...
 // (rg = l / 16) of column 16 w + l % 16 in registers, so that sixteen lanes move 64 contiguous bytes of a row (8 rows, 16
-// heads of 128 x 128: 10.9 us; neighbouring lanes in neighbouring rows 11.4); the four partial sums of a column's output lie
+// heads of 128 x 128: 8.15 us; neighbouring lanes in neighbouring rows were 0.5 us slower); the four partial sums of a column's output lie
 // sixteen lanes apart.  A step's tokens come through LDS eight at a time.  The sums run in one fixed order per output, whatever
 // the step's cut: a sequence fed whole, in portions or token by token leaves the same state and outputs, bit for bit.
 // A step of single tokens is the same kernel with one token a block.  With `below` > 0 only the sequences that bring
