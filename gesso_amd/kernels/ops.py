@@ -1450,16 +1450,18 @@ def attention_latent_mfma_tokens(H: int) -> int:
     return int(lib().gs_attention_latent_mfma_tokens(H))
 
 
-_latent_parts = {}
+_latent_parts = {}        # per device: the buffers made so far, the largest last
 
 
 def _latent_workspace(device, rows: int, c: int, nsplit: int):
-    """Room for the shares of blocks that walk a row's keys in parts: kept per device and made anew when more is asked."""
+    """Room for the shares of blocks that walk a row's keys in parts, kept per device.  A recorded step writes to the buffer
+    it was recorded with for as long as it is replayed, so where more is asked a larger one comes beside the smaller ones,
+    each at least twice the one before it (all the smaller ones together are no more than the largest)."""
     need = nsplit * rows * (c + 2)
-    held = _latent_parts.get(device)
-    if held is None or held.numel() < need:
-        held = _latent_parts[device] = torch.empty(need, dtype=torch.float32, device=device)
-    return held[:nsplit * rows * c], held[nsplit * rows * c:need]
+    held = _latent_parts.setdefault(device, [])
+    if not held or held[-1].numel() < need:
+        held.append(torch.empty(max(need, 2 * held[-1].numel() if held else 0), dtype=torch.float32, device=device))
+    return held[-1][:nsplit * rows * c], held[-1][nsplit * rows * c:need]
 
 
 def attention_latent_mfma(qa, cache, positions, tiles, block_table, page_size, window, scale, H, c, r, ntok,
