@@ -11,6 +11,7 @@ before it has changed anything; the scheduler decides what to do then.
 """
 from __future__ import annotations
 
+import threading
 from typing import Hashable, Optional, Sequence
 
 import torch
@@ -34,6 +35,41 @@ def parse_dtype(dtype) -> torch.dtype:
         return _DTYPES[dtype]
     except KeyError:
         raise InvalidPlan(f"dtype must be bfloat16 or float32, got {dtype!r}") from None
+
+
+class _Turn:
+    """An engine's calls one at a time, whichever threads and streams they come from.  Steps share the buffers of the decode
+    loop's recordings, the kernels' workspaces and the runtime's switches: a second thread waits until the first one's call
+    has returned, and a call on another stream than the one before runs behind it on the device (a step returns while its
+    kernels still run)."""
+
+    def __init__(self, device):
+        self.device, self.lock = device, threading.RLock()
+        self.depth, self.last, self.done = 0, None, None
+
+    def __enter__(self):
+        self.lock.acquire()
+        try:
+            if self.depth == 0 and self.last is not None:
+                stream = torch.cuda.current_stream(self.device)
+                if stream.cuda_stream != self.last and not torch.cuda.is_current_stream_capturing():
+                    stream.wait_event(self.done)
+        except BaseException:
+            self.lock.release()
+            raise
+        self.depth += 1
+
+    def __exit__(self, *exc):
+        self.depth -= 1
+        try:
+            if self.depth == 0 and not torch.cuda.is_current_stream_capturing():
+                stream = torch.cuda.current_stream(self.device)
+                self.done = self.done or torch.cuda.Event()
+                self.done.record(stream)
+                self.last = stream.cuda_stream
+        finally:
+            self.lock.release()
+        return False
 
 
 class Engine:
@@ -74,6 +110,7 @@ class Engine:
             self.storage.poison_all()
         self.steps = 0
         self._runners = {}
+        self._turn = _Turn(self.device)
         # steps of prompt portions whose kind recurs are recorded and replayed, where the options ask for it and every
         # part can be (bfloat16: the 32-bit path has no such parts' kernels)
         self.recorder = None
@@ -177,6 +214,10 @@ class Engine:
         entries = [e if isinstance(e, StepEntry) else StepEntry(*e) for e in entries]
         if not entries:
             return None
+        with self._turn:
+            return self._step(entries)
+
+    def _step(self, entries) -> Optional[torch.Tensor]:
         ids = check_entries(entries, self.manager, self.spec.vocab)
         self.manager.reserve_many([(e.rid, len(e.tokens)) for e in entries])
         # from here on the cache is written: an error leaves the requests of this step without a usable state
@@ -235,9 +276,10 @@ class Engine:
             raise InvalidPlan(f"the recorded decode loop takes 1 to {most} requests, not {len(rids)}")
         if len(set(rids)) != len(rids) or len(tokens) != len(rids):
             raise InvalidPlan("one token per request, each request once")
-        if not self.model.graph_safe:
-            return self._decode_eager(rids, tokens, n, samplers)
-        return self._runner(len(rids)).run(rids, tokens, n, samplers)
+        with self._turn:
+            if not self.model.graph_safe:
+                return self._decode_eager(rids, tokens, n, samplers)
+            return self._runner(len(rids)).run(rids, tokens, n, samplers)
 
     def _runner(self, requests: int):
         from .decode import DecodeRunner, _capacity

@@ -1,0 +1,181 @@
+"""An engine's calls from several threads and on several streams run one after another: steps share the decode loop's
+buffers, the kernels' workspaces and the runtime's switches.  On stand-ins for streams and kernels, then on the GPU."""
+import threading
+import time
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from gesso_amd.engine import engine as engine_module
+from gesso_amd.engine.batch import StepEntry
+from gesso_amd.engine.engine import Engine
+
+
+class Streams:
+    """Stands for ``torch.cuda``'s streams and events: ``log`` has what was enqueued, in the order the host enqueued it."""
+
+    def __init__(self):
+        self.log, self.now = [], 1
+        outer = self
+
+        class Event:
+            def record(self, stream=None):
+                self.at = outer.now if stream is None else stream.cuda_stream
+                outer.log.append(("record", self.at))
+
+        self.Event = Event
+
+    def current_stream(self, device=None):
+        return SimpleNamespace(cuda_stream=self.now, wait_event=lambda e, s=self.now: self.log.append(("wait", s, e.at)))
+
+
+def stand_in(monkeypatch, work):
+    """An engine whose loop step calls ``work()`` and whose cache takes everything."""
+    streams = Streams()
+    for name in ("current_stream", "Event"):
+        monkeypatch.setattr(torch.cuda, name, getattr(streams, name))
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(engine_module, "Runtime", lambda *a: SimpleNamespace(
+        streaming_rows_max=64, profile=None, ops=None, options=SimpleNamespace(record_portions=False)))
+    monkeypatch.setattr(engine_module, "Model", lambda spec, rt: SimpleNamespace(
+        graph_safe=True, bind=lambda t: None, cache_needs=lambda: []))
+    monkeypatch.setattr(engine_module, "CacheStorage", lambda *a: SimpleNamespace(num_pages=[]))
+    spec = SimpleNamespace(max_position=512, schedule=[], vocab=100)
+    eng = Engine(spec, {}, "bfloat16", device="cuda:0", page_size=16, num_pages=8, num_slots=4)
+    eng._runner = lambda n: SimpleNamespace(step=lambda rids, ids: work(streams, rids), run=lambda rids, *a: work(streams, rids))
+    for rid in "ab":
+        eng.add_request(rid)
+    return eng, streams
+
+
+def test_a_call_on_another_stream_waits_for_the_one_before(monkeypatch):
+    eng, streams = stand_in(monkeypatch, lambda st, rids: st.log.append(("work", st.now, rids[0])))
+    for stream, rid in ((1, "a"), (1, "b"), (2, "a"), (1, "b")):
+        streams.now = stream
+        eng.step([StepEntry(rid, [3], [0])])
+    streams.now = 2
+    eng.decode(["a"], [3], 1)
+    work = [(i, e[1]) for i, e in enumerate(streams.log) if e[0] == "work"]
+    for (i, before), (k, at) in zip(work, work[1:]):
+        between = streams.log[i + 1:k]
+        assert before == at or between == [("record", before), ("wait", at, before)], streams.log
+    assert [e for e in streams.log if e[0] == "wait"] == [("wait", 2, 1), ("wait", 1, 2), ("wait", 2, 1)]
+
+
+def test_a_second_thread_waits_until_the_first_ones_call_has_returned(monkeypatch):
+    inside, most = [], []
+
+    def work(st, rids):
+        inside.append(rids[0])
+        most.append(len(inside))
+        time.sleep(0.02)
+        inside.remove(rids[0])
+
+    eng, _ = stand_in(monkeypatch, work)
+
+    def calls(rid, decode):
+        for _ in range(5):
+            eng.decode([rid], [3], 1) if decode else eng.step([StepEntry(rid, [3], [0])])
+
+    threads = [threading.Thread(target=calls, args=(rid, rid == "b")) for rid in "ab"]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(most) == 10 and max(most) == 1
+
+
+def test_a_call_that_fails_lets_the_next_one_in(monkeypatch):
+    def work(st, rids):
+        raise RuntimeError("no")
+
+    eng, _ = stand_in(monkeypatch, work)
+    for rid in "ab":
+        with pytest.raises(Exception, match="no"):
+            eng.step([StepEntry(rid, [3], [0])])
+    assert eng._turn.depth == 0 and eng._turn.lock.acquire(blocking=False)
+    eng._turn.lock.release()
+
+
+def tiny_engine(tmp_path, **kw):
+    from gesso_amd.weights import write_model_folder
+    from tiny import STD, TINY_B
+    d = write_model_folder(str(tmp_path / "b"), TINY_B, 31, torch.bfloat16, std=STD)
+    return Engine.from_folder(d, dtype="bfloat16", page_size=8, max_tokens=1024, num_slots=8, **kw)
+
+
+def tokens_of(eng, rid, n):
+    return [(17 * i + 5 * len(str(rid)) + sum(map(ord, str(rid)))) % eng.spec.vocab for i in range(n)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("recorded", [False, True])
+def test_steps_of_two_streams_leave_each_others_requests_alone(tmp_path, recorded):
+    """Two requests stepped in turn on two streams, nothing waited for in between: the logits of each alone."""
+    def trace(rids, streams):
+        eng = tiny_engine(tmp_path)
+        if recorded:
+            eng.add_request("other")
+            eng.step([StepEntry("other", [1, 2, 3], [])])
+            eng.decode(["other"], [4], 2)
+        for r in rids:
+            eng.add_request(r)
+        torch.cuda.synchronize()
+        rows = {r: [] for r in rids}
+        for i in range(24):
+            for r, s in zip(rids, streams):
+                with torch.cuda.stream(s):
+                    rows[r].append(eng.step([StepEntry(r, [tokens_of(eng, r, 24)[i]], [0])]))
+        torch.cuda.synchronize()
+        return {r: torch.cat(rows[r]).cpu() for r in rids}
+
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    both = trace(["x", "y"], [a, b])
+    for r in "xy":
+        assert torch.equal(both[r], trace([r], [torch.cuda.current_stream()])[r])
+
+
+@pytest.mark.gpu
+def test_a_thread_that_decodes_beside_one_that_steps(tmp_path):
+    """One thread runs the recorded loop, the other steps single tokens and prompts of the same engine; each gets what it gets
+    alone."""
+    def decoded(eng, out):
+        eng.add_request("d")
+        tok = int(eng.step([StepEntry("d", tokens_of(eng, "d", 9), [8])]).argmax())
+        for _ in range(6):
+            ids, bad = eng.decode(["d"], [tok], 8)
+            assert not bad.any()
+            out += ids[:, 0].tolist()
+            tok = out[-1]
+
+    def stepped(eng, out):
+        for k in range(4):
+            rid = ("s", k)
+            eng.add_request(rid)
+            out.append(eng.step([StepEntry(rid, tokens_of(eng, rid, 30), list(range(30)))]).cpu())
+            for t in tokens_of(eng, rid, 12):
+                out.append(eng.step([StepEntry(rid, [t], [0])]).cpu())
+            eng.finish_request(rid)
+
+    alone = []
+    for f in (decoded, stepped):
+        out = []
+        f(tiny_engine(tmp_path), out)
+        alone.append(out)
+    eng, both, failed = tiny_engine(tmp_path), [[], []], []
+
+    def guarded(f, out):
+        try:
+            f(eng, out)
+        except BaseException as err:
+            failed.append(err)
+
+    threads = [threading.Thread(target=guarded, args=(f, o)) for f, o in zip((decoded, stepped), both)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed, failed
+    assert both[0] == alone[0]
+    assert len(both[1]) == len(alone[1]) and all(torch.equal(x, y) for x, y in zip(both[1], alone[1]))
