@@ -207,25 +207,30 @@ class DecodeRunner:
     def _fill(self, rcs, tokens, n: int) -> None:
         """What the step's kernels read of the rows that bring ``tokens``, with room for ``n`` more tokens each."""
         eng, cap, B = self.engine, self.cap, len(rcs)
-        st = eng.storage
-        # one int32 buffer for the per-row facts, one copy
-        host = np.zeros((5, self.row), dtype=np.int32)
-        host[0, :B] = tokens
-        host[1, :B] = [rc.length for rc in rcs]
-        host[2] = 1
-        host[2, :B] = [rc.length + 1 for rc in rcs]
-        host[3] = st.scratch_slot
-        host[3, :B] = [st.scratch_slot if rc.slot is None else rc.slot for rc in rcs]
-        host[4, :B] = 1
-        self.facts.copy_(torch.from_numpy(host).pin_memory(), non_blocking=True)
+        st, groups = eng.storage, len(self.block_tables)
         width = max(1, max(-(-(rc.length + n) // eng.page_size) for rc in rcs))
-        for g, bt in enumerate(self.block_tables):
-            tab = np.full((cap, width), st.num_pages[g], dtype=np.int32)
+        # one int32 buffer, one copy: the per-row facts, then the tables as wide as the longest row's
+        host = np.zeros(5 * self.row + groups * cap * width, dtype=np.int32)
+        facts, tables = host[:5 * self.row].reshape(5, self.row), host[5 * self.row:].reshape(groups, cap, width)
+        facts[0, :B] = tokens
+        facts[1, :B] = [rc.length for rc in rcs]
+        facts[2] = 1
+        facts[2, :B] = facts[1, :B] + 1
+        facts[3] = st.scratch_slot
+        facts[3, :B] = [st.scratch_slot if rc.slot is None else rc.slot for rc in rcs]
+        facts[4, :B] = 1
+        for g in range(groups):
+            tab = tables[g]
+            tab[:] = st.num_pages[g]
             for i, rc in enumerate(rcs):
-                row = np.asarray(rc.tables[g][:width], dtype=np.int32)
-                row[row < 0] = st.num_pages[g]
-                tab[i, :len(row)] = row
-            bt[:, :width].copy_(torch.from_numpy(tab).pin_memory().to(eng.device, non_blocking=True))
+                held = rc.tables[g]
+                m = min(len(held), width)
+                tab[i, :m] = held[:m]
+            tab[tab < 0] = st.num_pages[g]
+        dev = torch.from_numpy(host).pin_memory().to(eng.device, non_blocking=True)
+        self.facts.copy_(dev[:5 * self.row].view(5, self.row))
+        for bt, tab in zip(self.block_tables, dev[5 * self.row:].view(groups, cap, width)):
+            bt[:, :width].copy_(tab)
 
     def step(self, rids: Sequence[Hashable], tokens: Sequence[int]) -> torch.Tensor:
         """One step whose caller chooses the next tokens: float32 logits ``(batch, vocab)``.  The rows' room is reserved and

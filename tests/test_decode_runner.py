@@ -1,0 +1,53 @@
+"""The decode loop's runner on the CPU: what it hands the kernels of a step, on stand-ins for the engine and its kernels."""
+from types import SimpleNamespace
+
+import numpy as np
+import pytest
+import torch
+
+from gesso_amd.engine.decode import DecodeRunner
+
+
+def stand_in(pages=(40, 30), page_size=8, max_context=256, vocab=50):
+    """As much of an engine as a runner asks of it; ``pages``: the page groups' sizes."""
+    storage = SimpleNamespace(scratch_slot=9, num_pages=list(pages))
+    return SimpleNamespace(device=torch.device("cpu"), max_context=max_context, page_size=page_size, storage=storage, dtype=torch.bfloat16,
+                           DECODE_MAX_BATCH=64, spec=SimpleNamespace(vocab=vocab))
+
+
+@pytest.fixture
+def pinned(monkeypatch):
+    """Pinned buffers asked for (there is no pinned memory without a GPU: the tensor itself)."""
+    made = []
+    monkeypatch.setattr(torch.Tensor, "pin_memory", lambda t: made.append(t.numel()) or t)
+    return made
+
+
+@pytest.mark.parametrize("groups", [0, 1, 2])
+@pytest.mark.parametrize("B,cap", [(1, 1), (3, 4), (5, 8), (16, 16)])
+def test_a_steps_facts_and_tables_come_by_one_copy(pinned, groups, B, cap):
+    """What the rows' kernels read, against the same looked up row by row: pages that a window has given back and columns
+    beyond a row's pages name the scratch page, rows beyond the batch the scratch page and slot."""
+    eng = stand_in(pages=(40, 30)[:groups])
+    runner = DecodeRunner(eng, cap)
+    rng = np.random.default_rng(B)
+    for turn in range(2):                          # (what the first filled in must not show in the second)
+        lengths = [int(x) for x in rng.integers(1, 100 - 60 * turn, B)]
+        tables = [[[-1 if rng.random() < 0.2 else int(rng.integers(0, 30)) for _ in range(-(-(n + 3) // 8) + int(rng.integers(0, 2)))]
+                   for n in lengths] for _ in range(groups)]
+        rcs = [SimpleNamespace(length=n, slot=None if i == 1 else i, tables=[t[i] for t in tables]) for i, n in enumerate(lengths)]
+        tokens = rng.integers(0, 50, B)
+        pinned.clear()
+        runner._fill(rcs, tokens, 3)
+        assert len(pinned) == 1
+        assert runner.tok.tolist() == list(tokens) + [0] * (cap - B)
+        assert runner.pos.tolist() == lengths + [0] * (cap - B)
+        assert runner.kv_len.tolist() == [n + 1 for n in lengths] + [1] * (cap - B)
+        assert runner.slots.tolist() == [9 if i == 1 else i for i in range(B)] + [9] * (cap - B)
+        assert runner.live.tolist() == [1] * B + [0] * (cap - B)
+        for g in range(groups):
+            scratch = eng.storage.num_pages[g]
+            for i in range(cap):
+                reach = -(-(lengths[i] + 3) // 8) if i < B else max(-(-(n + 3) // 8) for n in lengths)
+                want = [tables[g][i][c] if i < B and tables[g][i][c] >= 0 else scratch for c in range(reach)]
+                assert runner.block_tables[g][i, :reach].tolist() == want
