@@ -25,6 +25,7 @@ from ..models.model import Model, tensor_table, tied_aliases
 from ..parts.runtime import Runtime, RuntimeOptions
 from ..weights.loader import load_tensors, random_tensors
 from .batch import StepContext, StepEntry, check_entries
+from .decode import DecodeRunner, _capacity
 
 _DTYPES = {"bfloat16": torch.bfloat16, "bf16": torch.bfloat16, "float32": torch.float32, "fp32": torch.float32,
            torch.bfloat16: torch.bfloat16, torch.float32: torch.float32}
@@ -73,6 +74,8 @@ class _Turn:
 
 
 class Engine:
+    LOOP_STEP_MAX_F32 = 16       # the most requests of a float32 step that runs as the decode loop's
+
     def __init__(self, spec: ModelSpec, tensors, dtype, device="cuda:0", page_size: int = 16,
                  num_pages: Optional[int] = None, max_tokens: Optional[int] = None, num_slots: int = 8,
                  max_context: Optional[int] = None, options: Optional[RuntimeOptions] = None, poison: bool = False,
@@ -120,6 +123,7 @@ class Engine:
         # the most requests one recorded decode step takes: as many rows as the runtime's weight-streaming products do
         # (the limit is the product kernels', asked of the runtime, not a number of the engine's own)
         self.DECODE_MAX_BATCH = self.rt.streaming_rows_max
+        self._loop_steps, self._padding_free = self.model.graph_safe, self.model.padding_free
         # More requests than that decode through a recording of the same loop in which the many-row products (the
         # vendor's, each weight read once for all rows) and the kernels of prompt steps stand for the fused
         # weight-streaming ones: up to this many at once (bfloat16; 0: no such loop).
@@ -224,9 +228,7 @@ class Engine:
         try:
             self.prepare_cache()
             logits = False
-            if (len(entries) <= self.DECODE_MAX_BATCH and self.model.graph_safe
-                    and all(len(e.tokens) == 1 and len(e.want) == 1 for e in entries)):
-                # every request brings one token and wants its logits: the decode loop's step, without its choice
+            if self._is_loop_step(entries):
                 logits = self._runner(len(entries)).step([e.rid for e in entries], ids)
             elif self.recorder is not None:
                 logits = self._step_recorded(entries, ids)
@@ -239,6 +241,20 @@ class Engine:
             self.manager.commit(e.rid, len(e.tokens))
         self.steps += 1
         return logits
+
+    def _is_loop_step(self, entries) -> bool:
+        """Whether a step is the decode loop's, without its choice: every request brings one token and wants its logits.  (The
+        answer is one by the number of requests alone, whether the loop has recorded that step or not: the two ways would
+        round differently.)  Left to the ordinary step: numbers that the loop's capacities fill up with rows of padding where
+        those cost as much as live ones (experts by a table, 9 to 12 requests in 16 rows: 1,480 us launched as it is and
+        1,720 in the loop's rows; 24 requests in 24 rows 1,700 and 1,750, with the recording 810), and in float32 more than
+        16, where the device is what takes the time (33 requests in 48 rows: 1,410 us, 1,500 launched, 1,540 with the
+        recording; 9 requests in 16 rows 1,463, 1,437 and 862)."""
+        n = len(entries)
+        return (n <= self.DECODE_MAX_BATCH and self._loop_steps
+                and (self.dtype == torch.bfloat16 or n <= self.LOOP_STEP_MAX_F32)
+                and (self._padding_free or n == _capacity(n))
+                and all(len(e.tokens) == 1 and len(e.want) == 1 for e in entries))
 
     def _step_recorded(self, entries, ids):
         """The step through a recording of its kind (:mod:`gesso_amd.engine.planned`), or False where there is none."""
@@ -282,7 +298,6 @@ class Engine:
             return self._runner(len(rids)).run(rids, tokens, n, samplers)
 
     def _runner(self, requests: int):
-        from .decode import DecodeRunner, _capacity
         cap = _capacity(requests)
         runner = self._runners.get(cap)
         if runner is None:

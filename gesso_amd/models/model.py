@@ -110,6 +110,11 @@ class Model:
         norms = [self.final_norm] + ([self.embed_norm] if self.embed_norm is not None else [])
         return all(getattr(b, "graph_safe", False) for b in self.blocks) and all(getattr(n, "graph_safe", False) for n in norms)
 
+    @property
+    def padding_free(self) -> bool:
+        """Whether a few rows of padding cost a step next to nothing (no part says that each of them costs what a live one does)."""
+        return not any(getattr(p, "padding_costs", False) for b in self.blocks for p in vars(b).values())
+
     def forward(self, ctx) -> Optional[torch.Tensor]:
         """Run the tokens of ``ctx`` through every scheduled block; float32 logits at ``ctx.want_rows``."""
         stream = self.run_blocks(ctx)

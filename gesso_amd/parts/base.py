@@ -119,6 +119,7 @@ class Part:
     """Base of parts: keeps spec and runtime; subclasses fill the rest."""
 
     graph_safe = False      # True: forward makes no host round trip, so a decode step through it may be recorded
+    padding_costs = False   # True: a row of padding in a step costs what a live one does (experts it brings in)
     row_weight = None       # norms: see the module's text
     first_norm = None       # blocks: see the module's text
 

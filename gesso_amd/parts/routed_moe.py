@@ -23,6 +23,7 @@ from .registry import register
 
 class RoutedMoE(Part):
     graph_safe = True
+    padding_costs = True
     stage, out_stage = "moe_ffn", "ffn_down"
 
     @staticmethod

@@ -20,6 +20,7 @@ from .registry import register
 
 class TableMoE(Part):
     graph_safe = True
+    padding_costs = True
     stage, out_stage = "moe_ffn", "ffn_down"
 
     @staticmethod

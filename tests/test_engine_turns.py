@@ -30,8 +30,8 @@ class Streams:
         return SimpleNamespace(cuda_stream=self.now, wait_event=lambda e, s=self.now: self.log.append(("wait", s, e.at)))
 
 
-def stand_in(monkeypatch, work):
-    """An engine whose loop step calls ``work()`` and whose cache takes everything."""
+def stand_in(monkeypatch, work, dtype="bfloat16", padding_free=True):
+    """An engine whose steps call ``work()``, an ordinary one with ``["ordinary"]``, the loop's with the requests."""
     streams = Streams()
     for name in ("current_stream", "Event"):
         monkeypatch.setattr(torch.cuda, name, getattr(streams, name))
@@ -39,10 +39,12 @@ def stand_in(monkeypatch, work):
     monkeypatch.setattr(engine_module, "Runtime", lambda *a: SimpleNamespace(
         streaming_rows_max=64, profile=None, ops=None, options=SimpleNamespace(record_portions=False)))
     monkeypatch.setattr(engine_module, "Model", lambda spec, rt: SimpleNamespace(
-        graph_safe=True, bind=lambda t: None, cache_needs=lambda: []))
+        graph_safe=True, padding_free=padding_free, bind=lambda t: None, cache_needs=lambda: [],
+        forward=lambda ctx: work(streams, ["ordinary"])))
+    monkeypatch.setattr(engine_module, "StepContext", lambda *a, **kw: None)
     monkeypatch.setattr(engine_module, "CacheStorage", lambda *a: SimpleNamespace(num_pages=[]))
     spec = SimpleNamespace(max_position=512, schedule=[], vocab=100)
-    eng = Engine(spec, {}, "bfloat16", device="cuda:0", page_size=16, num_pages=8, num_slots=4)
+    eng = Engine(spec, {}, dtype, device="cuda:0", page_size=16, num_pages=64, num_slots=65)
     eng._runner = lambda n: SimpleNamespace(step=lambda rids, ids: work(streams, rids), run=lambda rids, *a: work(streams, rids))
     for rid in "ab":
         eng.add_request(rid)
@@ -96,6 +98,25 @@ def test_a_call_that_fails_lets_the_next_one_in(monkeypatch):
             eng.step([StepEntry(rid, [3], [0])])
     assert eng._turn.depth == 0 and eng._turn.lock.acquire(blocking=False)
     eng._turn.lock.release()
+
+
+@pytest.mark.parametrize("dtype,padding_free,loop", [
+    ("bfloat16", True, range(1, 65)), ("bfloat16", False, (1, 2, 4, 8, 16, 24, 32, 48, 64)),
+    ("float32", True, range(1, 17)), ("float32", False, (1, 2, 4, 8, 16))])
+def test_which_steps_of_single_tokens_are_the_loops(monkeypatch, dtype, padding_free, loop):
+    """By the number of requests alone: rows of padding that cost what live ones do are not added to a step that has none, nor
+    any to a float32 step that keeps the device busy."""
+    ran = []
+    eng, _ = stand_in(monkeypatch, lambda st, rids: ran.append(rids[0] != "ordinary"), dtype, padding_free)
+    for i in range(65):
+        eng.add_request(i)
+    for n in range(1, 66):
+        eng.step([StepEntry(i, [3], [0]) for i in range(n)])
+    assert [n for n, through in enumerate(ran, 1) if through] == list(loop)
+    ran.clear()
+    eng.step([StepEntry(0, [3], [0]), StepEntry(1, [3], [])])          # a request that wants no logits
+    eng.step([StepEntry(0, [3, 4], [1])])                              # a portion of two tokens
+    assert ran == [False, False]
 
 
 def tiny_engine(tmp_path, **kw):
