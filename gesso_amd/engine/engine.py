@@ -123,7 +123,11 @@ class Engine:
         # the most requests one recorded decode step takes: as many rows as the runtime's weight-streaming products do
         # (the limit is the product kernels', asked of the runtime, not a number of the engine's own)
         self.DECODE_MAX_BATCH = self.rt.streaming_rows_max
-        self._loop_steps, self._padding_free = self.model.graph_safe, self.model.padding_free
+        # (the loop's page tables are as wide as a whole context.  Pages so large that the attention kernels' division of a
+        # position does not reach its end leave the loop's step out; an ordinary step's tables are as wide as its requests')
+        self._loop_steps = (self.model.graph_safe
+                            and -(-self.max_context // self.page_size) * self.page_size ** 2 < 1 << 32)
+        self._padding_free = self.model.padding_free
         # More requests than that decode through a recording of the same loop in which the many-row products (the
         # vendor's, each weight read once for all rows) and the kernels of prompt steps stand for the fused
         # weight-streaming ones: up to this many at once (bfloat16; 0: no such loop).

@@ -30,7 +30,7 @@ class Streams:
         return SimpleNamespace(cuda_stream=self.now, wait_event=lambda e, s=self.now: self.log.append(("wait", s, e.at)))
 
 
-def stand_in(monkeypatch, work, dtype="bfloat16", padding_free=True):
+def stand_in(monkeypatch, work, dtype="bfloat16", padding_free=True, page_size=16, context=512):
     """An engine whose steps call ``work()``, an ordinary one with ``["ordinary"]``, the loop's with the requests."""
     streams = Streams()
     for name in ("current_stream", "Event"):
@@ -43,8 +43,8 @@ def stand_in(monkeypatch, work, dtype="bfloat16", padding_free=True):
         forward=lambda ctx: work(streams, ["ordinary"])))
     monkeypatch.setattr(engine_module, "StepContext", lambda *a, **kw: None)
     monkeypatch.setattr(engine_module, "CacheStorage", lambda *a: SimpleNamespace(num_pages=[]))
-    spec = SimpleNamespace(max_position=512, schedule=[], vocab=100)
-    eng = Engine(spec, {}, dtype, device="cuda:0", page_size=16, num_pages=64, num_slots=65)
+    spec = SimpleNamespace(max_position=context, schedule=[], vocab=100)
+    eng = Engine(spec, {}, dtype, device="cuda:0", page_size=page_size, num_pages=64, num_slots=65)
     eng._runner = lambda n: SimpleNamespace(step=lambda rids, ids: work(streams, rids), run=lambda rids, *a: work(streams, rids))
     for rid in "ab":
         eng.add_request(rid)
@@ -119,11 +119,21 @@ def test_which_steps_of_single_tokens_are_the_loops(monkeypatch, dtype, padding_
     assert ran == [False, False]
 
 
-def tiny_engine(tmp_path, **kw):
+@pytest.mark.parametrize("page_size,through", [(16, True), (20000, True), (32768, False), (40000, False)])
+def test_pages_too_large_for_a_whole_contexts_table_leave_the_loop_out(monkeypatch, page_size, through):
+    """A table of a whole context of 131,072 positions, and what the kernels divide positions by: 2^32 at most."""
+    ran = []
+    eng, _ = stand_in(monkeypatch, lambda st, rids: ran.append(rids[0] != "ordinary"), page_size=page_size, context=131072)
+    eng.step([StepEntry("a", [3], [0])])
+    assert ran == [through]
+
+
+def tiny_engine(tmp_path, page_size=8, max_tokens=1024, **fields):
+    import dataclasses
     from gesso_amd.weights import write_model_folder
     from tiny import STD, TINY_B
-    d = write_model_folder(str(tmp_path / "b"), TINY_B, 31, torch.bfloat16, std=STD)
-    return Engine.from_folder(d, dtype="bfloat16", page_size=8, max_tokens=1024, num_slots=8, **kw)
+    d = write_model_folder(str(tmp_path / "b"), dataclasses.replace(TINY_B, **fields), 31, torch.bfloat16, std=STD)
+    return Engine.from_folder(d, dtype="bfloat16", page_size=page_size, max_tokens=max_tokens, num_slots=8)
 
 
 def tokens_of(eng, rid, n):
@@ -200,3 +210,22 @@ def test_a_thread_that_decodes_beside_one_that_steps(tmp_path):
     assert not failed, failed
     assert both[0] == alone[0]
     assert len(both[1]) == len(alone[1]) and all(torch.equal(x, y) for x, y in zip(both[1], alone[1]))
+
+
+@pytest.mark.gpu
+def test_single_tokens_in_pages_that_hold_a_third_of_a_context(tmp_path):
+    """Pages of 40,000 tokens with a context of 120,000: single tokens follow a prompt, as they do with small pages."""
+    import plain_lfm2 as P
+    from noise import NoiseBound
+    eng = tiny_engine(tmp_path, 40000, 80000, max_position_embeddings=120000)
+    d = str(tmp_path / "b")
+    cfg, w = P.read_config(d), P.read_weights(d)
+    eng.add_request("r")
+    seq = tokens_of(eng, "r", 30)
+    got = [eng.step([StepEntry("r", seq[:21], [20])])] + [eng.step([StepEntry("r", [t], [0])]) for t in seq[21:]]
+    ref, rounded = P.forward(cfg, w, seq), P.forward(cfg, w, seq, store=P.to_bfloat16)
+    bound = NoiseBound()
+    for i, row in enumerate(got):
+        bound.add(row[0].double().cpu(), ref[20 + i], rounded[20 + i], i)
+    bound.check("single tokens in large pages,")
+    assert eng.length("r") == 30
