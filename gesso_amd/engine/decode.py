@@ -91,7 +91,7 @@ class DecodeRunner:
         # one recording per bound on the context length (launch shapes, how attention splits its keys, depend on it)
         # and per kind of choice: all rows greedy (one kernel), or some rows draw (three, the weights by many blocks)
         self.graphs: Dict[Tuple[int, bool], torch.cuda.CUDAGraph] = {}
-        self.logits_of: Dict[Tuple[int, bool], torch.Tensor] = {}     # where each recording leaves its logits
+        self.logits_of: Dict[Tuple[int, bool], torch.Tensor] = {}     # where the recordings that ``step`` replays leave their logits
         self.draws = False
 
     def fit(self, n: int) -> "DecodeRunner":
@@ -122,7 +122,8 @@ class DecodeRunner:
         with rt.stage("sample"):
             if self.draws:
                 if self.wide is None:
-                    self.weights, self.wide = self.engine.choice_scratch(max(self.cap, self.engine.DECODE_MAX_BATCH))
+                    # (as much as the whole capacity's rows need: the runners of fewer rows share one set with it)
+                    self.weights, self.wide = self.engine.choice_scratch(max(self.whole.cap, self.engine.DECODE_MAX_BATCH))
                 ops.decode_choose(logits, self.temperature, self.u, self.counter, self.tok, self.ring, self.bad_ring,
                                   self.pos, self.kv_len, self.live, self.wide, top_p=self.top_p, wbuf=self.weights)
             else:
@@ -164,7 +165,8 @@ class DecodeRunner:
             if collecting:
                 gc.enable()
         self.graphs[(bound, draws)] = graph
-        self.logits_of[(bound, draws)] = self.logits
+        if not draws and self.cap <= self.engine.DECODE_MAX_BATCH:
+            self.logits_of[(bound, draws)] = self.logits            # (a recording that ``step`` may replay)
 
     def run(self, rids: Sequence[Hashable], tokens: Sequence[int], n: int, samplers=None
             ) -> Tuple[np.ndarray, np.ndarray]:

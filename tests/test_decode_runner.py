@@ -1,4 +1,5 @@
 """The decode loop's runner on the CPU: what it hands the kernels of a step, on stand-ins for the engine and its kernels."""
+import contextlib
 from types import SimpleNamespace
 
 import numpy as np
@@ -51,3 +52,24 @@ def test_a_steps_facts_and_tables_come_by_one_copy(pinned, groups, B, cap):
                 reach = -(-(lengths[i] + 3) // 8) if i < B else max(-(-(n + 3) // 8) for n in lengths)
                 want = [tables[g][i][c] if i < B and tables[g][i][c] >= 0 else scratch for c in range(reach)]
                 assert runner.block_tables[g][i, :reach].tolist() == want
+
+
+def test_the_runners_of_a_capacity_share_one_set_of_the_draws_scratch(monkeypatch):
+    """A batch of drawing requests that grows from 129 to 512 passes runners of 160, 192, 256, 320, 384 and 512 rows; what
+    their draws write to is one set a capacity, not one a runner."""
+    from gesso_amd.engine.decode import _capacity
+    from gesso_amd.engine.engine import Engine
+    eng = stand_in(pages=())
+    eng.rt = SimpleNamespace(ops=SimpleNamespace(choice_parts=lambda V: 3, choice_hist=lambda: 5, decode_choose=lambda *a, **kw: None),
+                             stage=lambda name: contextlib.nullcontext())
+    eng.choice_scratch = lambda rows: Engine.choice_scratch(eng, rows)
+    monkeypatch.setattr(DecodeRunner, "_forward", lambda self: None)
+    runners, sets = {}, {}
+    for n in (129, 170, 200, 260, 330, 500, 150):
+        cap = _capacity(n)
+        runner = runners.setdefault(cap, DecodeRunner(eng, cap)).fit(n)
+        runner.draws = True
+        runner._body()
+        assert runner.weights.numel() >= n * eng.spec.vocab
+        sets.setdefault(cap, set()).add(runner.weights.data_ptr())
+    assert {cap: len(s) for cap, s in sets.items()} == {256: 1, 512: 1}
