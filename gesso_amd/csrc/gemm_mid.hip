@@ -275,11 +275,7 @@ extern "C" int gs_gemm_mid(const void* X, int ldx, const void* Wt, void* Y, int 
 
 // The product in parts of K: which tile and how many parts.  As above, a unit's rows of X and W times k bind, and a sheet is written
 // and read once more (counted as the rows times k that take as long; at a quarter of that, 160 rows of 1024 x 4608 took 15 parts and 15.8
-// us); none beyond what one round of blocks holds.  Microseconds with the pass that adds and norms, the vendor's product and the
-// plain pass / here, weights that lie in no cache: 1024 x 4608, 65 rows 12.3 / 10.2, 160 13.7 / 12.1, 333 17.6 / 15.8, 768 23.1 /
-// 22.4; 2048 x 8192, 65 rows 24.2 / 15.8, 192 29.8 / 22.0, 512 37.8 / 36.2, 768 48.7 / 46.6; 2048 x 4096, 128 rows 15.7 / 13.8, 768 29.6
-// / 29.5; 512 x 4096, 256 rows 11.6 / 10.7; 4096 x 4096, 128 rows 28.3 / 19.1, 256 26.8 / 25.2, 333 29.7 / 30.8; 1,024 rows of 1024 x
-// 3072 18.5 / 19.0.
+// us); none beyond what one round of blocks holds.
 struct MidParts {
   int tile, parts;
 };
@@ -307,6 +303,29 @@ static MidParts mid_parts_choice(int M, int N, int K) {
 extern "C" int gs_gemm_mid_parts_takes(int M, int N, int K) {
   return K > 0 && K % 32 == 0 && N > 0 && N % 16 == 0 ? mid_parts_choice(M, N, K).parts : 0;
 }
+
+// Whether that is faster than the vendor's product and the plain pass, by measurement of both with the pass that adds and norms:
+// 1,242 products of 65 to 768 rows, 14 widths of W from 256 to 4,096 and K from 2,304 to 14,336, weights that lie in no cache (700 MB of
+// them in turn; where some 200 MB stay in the last-level cache the vendor's gain more).  Of the 877 taken here 5 are slower,
+// by 2 % at most; together they take 0.75 of the vendor's time, the others would take 1.02.  The vendor's time over this one's:
+// - up to 1,024 rows of W: 1.02 and more, at any K (1024 x 4608: 65 rows 1.49, 160 1.31, 768 1.18);
+// - 2,048 and 4,096 rows: the more rows of X the longer K has to be (2048 x 8192, 65 rows 1.46, 512 1.04; 2048 x 2304, 320 rows 1.05,
+//   448 0.93; 2048 x 3072, 512 rows 1.02, 768 0.96; 4096 x 2304, 160 rows 1.23, 256 0.93);
+// - others up to 2,048 rows, whose tiles suit the vendor: from a K of 6,144 on, for up to 96 rows of X of 10,240 (1280 x 4608,
+//   65 rows 0.95, 320 0.95; 1280 x 7168, 128 rows 1.23; 1280 x 8192, 65 rows 0.85; 1536 x 6144, 512 rows 1.00, 768 0.97);
+// - others beyond: the vendor's step from 96 to 128 rows of X is large (2560 x 3072, 96 rows 0.80, 128 1.38; 3584 x 3072, 160 rows 1.25,
+//   200 0.90); else from a K of 4,608, 6,144 or 10,240 on (2304 x 4608, 65 rows 0.97, 2304 x 6144 1.10; 3072 x 3072, 256 rows 0.90, 3072 x
+//   11008 1.15).
+static bool mid_parts_pay(int M, int N, int K) {
+  if (N <= 1024) return true;
+  if ((N & (N - 1)) == 0) return M <= (N > 2048 ? 160 : 320) || (M <= 512 && K >= 3072) || K >= 4096;
+  if (N < 2048) return (M > 96 && M <= 384 && K >= 6144) || (M <= 640 && K >= 10240);
+  if (M > 96 && M <= (N < 3328 ? 128 : 160)) return true;
+  return N < 2816 ? K >= 6144 : (M <= 128 && K >= 4608) || (M <= 160 && K >= 6144) || K >= 10240;
+}
+
+// The same, 0 also where the vendor's product is the faster one.
+extern "C" int gs_gemm_mid_parts_pay(int M, int N, int K) { return mid_parts_pay(M, N, K) ? gs_gemm_mid_parts_takes(M, N, K) : 0; }
 
 // part (parts, M, N) float32 = partial sums of X W^T over gs_gemm_mid_parts_takes parts of K; gs_residual_from_parts adds them up.
 extern "C" int gs_gemm_mid_parts(const void* X, int ldx, const void* Wt, float* part, int parts, int M, int N, int K, hipStream_t stream) {

@@ -665,6 +665,11 @@ def _mid_parts(M: int, N: int, K: int) -> int:
     return lib().gs_gemm_mid_parts_takes(M, N, K)
 
 
+@lru_cache(maxsize=4096)
+def _mid_parts_pay(M: int, N: int, K: int) -> int:
+    return lib().gs_gemm_mid_parts_pay(M, N, K)
+
+
 def _mid_operands(x, w: torch.Tensor, wt) -> bool:
     """bfloat16 rows on the GPU, aligned, that do not overlap, and the whole weight ``wt`` was made of as it lies there (a part
     or a transposed view of it can share its address)."""
@@ -704,6 +709,11 @@ def mid_parts(x, w: torch.Tensor, wt) -> int:
     """Into how many parts of K :func:`gemm_mid_residual_parts` shares this product out; 0: it is not for it.  Operands as for
     :func:`mid_ok`."""
     return _mid_parts(x.shape[0], w.shape[0], w.shape[1]) if w.shape[1] > 2048 and _mid_operands(x, w, wt) else 0
+
+
+def mid_parts_pay(x, w: torch.Tensor, wt) -> int:
+    """:func:`mid_parts`, and 0 also where the vendor's product and the plain pass are the faster way."""
+    return _mid_parts_pay(x.shape[0], w.shape[0], w.shape[1]) if w.shape[1] > 2048 and _mid_operands(x, w, wt) else 0
 
 
 def gemm_mid_residual_parts(x, w: torch.Tensor, wt, res: torch.Tensor, next_weight=None, eps: float = 0.0, parts: int = None):

@@ -273,7 +273,7 @@ class Runtime:
                 if self.ops.skinny_ok(x, w):
                     return DeferredLinear(x, w)
             elif self.many_rows == "auto" and not self.no_library:
-                parts = self.ops.mid_parts(x, w, self.tiles_of(w))
+                parts = self.ops.mid_parts_pay(x, w, self.tiles_of(w))
                 if parts:
                     return DeferredLinear(x, w, parts)
         return self.linear(x, w, bias)
