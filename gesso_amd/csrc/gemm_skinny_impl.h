@@ -55,6 +55,8 @@ typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
 // A kernel's LAYOUT is SHUF, with SKINNY_ONCE added where the weight's pieces are loaded non-temporally.
 #define SKINNY_ONCE 4
+// And SKINNY_PAIRED for two row tiles whose blocks come two to a compute unit: a lane then has 128 registers.
+#define SKINNY_PAIRED 8
 
 __device__ __forceinline__ bf16x8_t load8(const bf16* p) { return *reinterpret_cast<const bf16x8_t*>(p); }
 
@@ -124,11 +126,12 @@ struct SkinnyExtra {
 };
 
 template <int R, int MT, int WAVES, int PRO, int EPI, int LAYOUT, typename TOut>
-__global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16* __restrict__ X, int ldx,
+__global__ __launch_bounds__(WAVES * 64, LAYOUT & SKINNY_PAIRED ? WAVES / 2 : 1) void gemm_skinny_kernel(const bf16* __restrict__ X, int ldx,
                                                                   const bf16* __restrict__ W,
                                                                   TOut* __restrict__ Y, int ldy, int M, int N,
                                                                   int K, SkinnyExtra ex) {
-  constexpr int SHUF = LAYOUT & ~SKINNY_ONCE;
+  constexpr int SHUF = LAYOUT & 3;
+  constexpr bool RING = MT > 1 && !(LAYOUT & SKINNY_PAIRED);     // see the loop
   constexpr bool GLU = EPI == 1 || EPI == 4;
   extern __shared__ float red[];  // WAVES (one row tile: WAVES - 1) x R x MT x 64 x 4 floats
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -209,10 +212,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16* __r
   // nothing but the number of partials).  The first row's loads start here, under the product's own.
   __shared__ float inv_s[64];
   constexpr bool scaled = PRO == 2;
-  // With two row tiles all of a wavefront's rows are asked for here: after the loop they were a round trip of their own
+  // With two row tiles all of a wavefront's rows are asked for here (where the registers allow): after the loop they were a round trip of their own
   // (20 rows of 9216 x 1024 9.3 against 8.7 us).
   constexpr int RPW = (MT * 16 + WAVES - 1) / WAVES;      // rows a wavefront
-  constexpr int EARLY = MT == 2 ? RPW : 1;
+  constexpr int EARLY = MT == 2 && RING ? RPW : 1;
   float pre[EARLY][4];
   if (scaled && wave < M) {
     // (a row or a partial sum that does not exist is read from one that does and not counted: no load sits behind a branch)
@@ -404,15 +407,16 @@ _Pragma("unroll")                                                               
           acc[r][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][r], b[u][mt], acc[r][mt], 0, 0, 0);                 \
     s += C;                                                                                                             \
   }
-  if (MT == 1) {
+  if (!RING) {
     // few rows: the steps' loads are issued U at a time, then multiplied (the ring below costs registers, and with
-    // them a resident wavefront per SIMD, which these shapes need more)
+    // them a resident wavefront per SIMD, which these shapes need more; two row tiles: all loads before the first product, which
+    // the compiler would else move up between them to save registers)
     if (EPI == 3) {
       if (whole && s + U <= s1) GS_BATCH(U, GS_PRELOAD_CONV())
       else GS_PRELOAD_CONV()
     }
     if (whole)
-      while (s + U <= s1) GS_BATCH(U, )
+      while (s + U <= s1) GS_BATCH(U, if (MT > 1) __builtin_amdgcn_sched_barrier(0);)
   } else if (whole && s1 - s0 >= U) {
     // many rows: a ring of U steps in registers: a step is multiplied as soon as it has arrived and its place is
     // asked for again at once, U steps ahead, so that loads are in flight the whole time (loads return in order).
@@ -500,7 +504,7 @@ _Pragma("unroll")                                                               
       }
     }
 #pragma unroll
-    for (int i0 = 1; MT > 2 && i0 < RPW; i0 += BATCH) {
+    for (int i0 = 1; MT > 1 && EARLY == 1 && i0 < RPW; i0 += BATCH) {
       if (wave + i0 * WAVES < M) {
         float q[BATCH][4];
 #pragma unroll
@@ -742,7 +746,16 @@ static void skinny_plain_pro(const SkinnyCall& c) {
     } else if (f32) { GS_BY_MT4(2, 8, 8, 4, 4, PRO, 1, float, blocks) } else { GS_BY_MT4(2, 8, 8, 4, 4, PRO, 1, bf16, blocks) }
   } else if (narrow) {
     const int blocks = gs_ceil_div(cols, 16);
-    if (f32) { GS_BY_MT(1, 8, PRO, 0, float, blocks) } else { GS_BY_MT(1, 8, PRO, 0, bf16, blocks) }
+    // Two row tiles and more blocks than compute units: the ring's registers would leave a unit one block, so that a few blocks
+    // more are a round more (rows weighted before, 20 rows, microseconds with the ring and with batches: 6144 x 4096 19.4 and 17.6,
+    // 5120 x 1024 9.2 and 7.5; plain rows 8192 x 1024 7.7 and 6.6).  Plain rows of up to 24 and a K from 4,096 on: the ring (17
+    // rows of 6144 x 8192 27.4 and 28.0).
+    const bool paired = PRO != 1 && M > 16 && M <= 32 && blocks > 256 && (PRO == 2 || M > 24 || K < 4096);
+    if (paired) {
+      constexpr int PAIRED = LAYOUT | (PRO != 1 ? SKINNY_PAIRED : 0);
+      if (f32) launch_skinny<1, 2, 8, PRO, 0, PAIRED, float>(blocks, x, ldx, w, (float*)Y, ldy, M, N, K, ex, stream);
+      else launch_skinny<1, 2, 8, PRO, 0, PAIRED, bf16>(blocks, x, ldx, w, (bf16*)Y, ldy, M, N, K, ex, stream);
+    } else if (f32) { GS_BY_MT(1, 8, PRO, 0, float, blocks) } else { GS_BY_MT(1, 8, PRO, 0, bf16, blocks) }
   } else {
     const int blocks = gs_ceil_div(cols, 32);
     if (f32) { GS_BY_MT4(2, 8, 8, 4, 4, PRO, 0, float, blocks) } else { GS_BY_MT4(2, 8, 8, 4, 4, PRO, 0, bf16, blocks) }
