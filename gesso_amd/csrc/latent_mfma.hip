@@ -263,8 +263,11 @@ __global__ __launch_bounds__(256) void attention_latent_mfma_kernel(
 }
 
 // out[row, :] = sum_z part_o[z, row, :] 2^(m_z - M) / sum_z l_z 2^(m_z - M), M = max_z m_z: the shares of the blocks
-// that walked a row's keys in parts, added in the order of the parts.  The loads of eight parts are asked for together, the first
-// eight before the weights are known (8 sequences of 290 rows, both kernels: 16.7 us with one load after the other, so 15.4).
+// that walked a row's keys in parts, added in the order of the parts.  The loads of P parts are asked for together, the first
+// P before the weights are known (8 sequences of 290 rows, both kernels: 16.7 us with one load after the other, so 15.4).  P is four
+// where there are no more parts: the loads of parts that do not exist cost as much as others (64 sequences of 32 heads in 4 parts,
+// both kernels: 21.7 us with eight and 21.1 with four; of 16 heads 17.0 and 16.4).
+template <int P>
 __global__ __launch_bounds__(512) void attention_latent_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                               int nsplit, int rows_total, int c, bf16* __restrict__ out) {
   __shared__ float wz[64];           // the parts' weights 2^(m_z - M) / L (at most 64 parts)
@@ -274,9 +277,9 @@ __global__ __launch_bounds__(512) void attention_latent_merge_kernel(const float
   // (a part or a column that does not exist is read from the last and not counted)
   auto ask = [&](float* v, int z0, int j) __attribute__((always_inline)) {
 #pragma unroll
-    for (int q = 0; q < 8; ++q) v[q] = src[(size_t)(z0 + q < nsplit ? z0 + q : nsplit - 1) * sheet + (j < c ? j : c - 1)];
+    for (int q = 0; q < P; ++q) v[q] = src[(size_t)(z0 + q < nsplit ? z0 + q : nsplit - 1) * sheet + (j < c ? j : c - 1)];
   };
-  float v[8];
+  float v[P];
   ask(v, 0, threadIdx.x);
   // every wavefront of the block finds the weights itself: lane z holds part z
   float m = -INFINITY, l = 0.f;
@@ -292,10 +295,10 @@ __global__ __launch_bounds__(512) void attention_latent_merge_kernel(const float
   __syncthreads();
   for (int j = threadIdx.x; j < c; j += blockDim.x) {
     float a = 0.f;
-    for (int z0 = 0; z0 < nsplit; z0 += 8) {
+    for (int z0 = 0; z0 < nsplit; z0 += P) {
       if (z0 > 0 || j != (int)threadIdx.x) ask(v, z0, j);
 #pragma unroll
-      for (int q = 0; q < 8; ++q)
+      for (int q = 0; q < P; ++q)
         if (z0 + q < nsplit) a += v[q] * wz[z0 + q];
     }
     out[(size_t)row * c + j] = f32_to_bf16(a);
@@ -359,7 +362,8 @@ extern "C" int gs_attention_latent_mfma(const void* qa, const void* cache, const
 #undef LM_RUN
   GS_LAUNCH_CHECK("attention_latent_mfma");
   if (nsplit > 1) {
-    attention_latent_merge_kernel<<<rows_total, gs_ceil_div(c, 64) * 64, 0, stream>>>(part_o, part_ml, nsplit, rows_total, c, (bf16*)out);
+    auto merge = nsplit <= 4 ? &attention_latent_merge_kernel<4> : &attention_latent_merge_kernel<8>;
+    merge<<<rows_total, gs_ceil_div(c, 64) * 64, 0, stream>>>(part_o, part_ml, nsplit, rows_total, c, (bf16*)out);
     GS_LAUNCH_CHECK("attention_latent_merge");
   }
   return 0;

@@ -225,7 +225,7 @@ def test_attention_over_latent_rows_on_the_matrix_cores_at_other_sizes(ops, H, n
 
 
 @pytest.mark.parametrize("H,c,r", [(1, 16, 8), (16, 128, 32), (5, 144, 8), (16, 256, 32), (16, 512, 64), (7, 272, 16)])
-@pytest.mark.parametrize("nsplit", [1, 3, 9, 20])
+@pytest.mark.parametrize("nsplit", [1, 3, 4, 5, 9, 20])
 @pytest.mark.parametrize("sink", [False, True])
 def test_single_tokens_over_latent_rows_in_all_parts_are_those_of_a_list_of_tiles(ops, H, c, r, nsplit, sink):
     """A step of single tokens of up to 16 heads runs the form whose wavefronts hold a quarter of the value columns' sums; the same
