@@ -183,6 +183,8 @@ class Runtime:
 
     def dense(self, x):
         """``x`` as an ordinary tensor, whatever handle it came as."""
+        if isinstance(x, torch.Tensor):
+            return x
         if isinstance(x, DeferredLinear):
             return self.linear(x.x, x.w)
         if isinstance(x, self.ops.LazyNorm):
@@ -272,7 +274,7 @@ class Runtime:
             if self.fused:
                 if self.ops.skinny_ok(x, w):
                     return DeferredLinear(x, w)
-            elif self.many_rows == "auto" and not self.no_library:
+            elif x.shape[0] > self.streaming_rows_max and self.many_rows == "auto" and not self.no_library:
                 parts = self.ops.mid_parts_pay(x, w, self.tiles_of(w))
                 if parts:
                     return DeferredLinear(x, w, parts)

@@ -73,3 +73,20 @@ def test_the_runners_of_a_capacity_share_one_set_of_the_draws_scratch(monkeypatc
         assert runner.weights.numel() >= n * eng.spec.vocab
         sets.setdefault(cap, set()).add(runner.weights.data_ptr())
     assert {cap: len(s) for cap, s in sets.items()} == {256: 1, 512: 1}
+
+
+def test_a_last_product_of_few_rows_asks_nothing_about_parts():
+    """A prompt of some rows has thirty last products, each a host call of some microseconds: up to 64 rows, which never come in
+    parts, cost no check of the operands for that."""
+    from gesso_amd.parts.runtime import DeferredLinear, Runtime
+    asked = []
+    rt = object.__new__(Runtime)
+    rt.ops = SimpleNamespace(mid_parts_pay=lambda x, w, wt: asked.append(x.shape[0]) or 3)
+    rt.fused, rt.no_library, rt.many_rows, rt.streaming_rows_max, rt._tiles = False, False, "auto", 64, {}
+    rt.linear = lambda x, w, bias=None: "computed"
+    w = torch.zeros(16, 4096)
+    for rows in (1, 13, 64):
+        assert rt.project(torch.zeros(rows, 4096), w) == "computed"
+    assert asked == []
+    out = rt.project(torch.zeros(65, 4096), w)
+    assert isinstance(out, DeferredLinear) and out.parts == 3 and asked == [65]
