@@ -21,6 +21,7 @@ from ..cache.storage import CacheStorage
 from ..config.registry import load_config
 from ..config.spec import ModelSpec
 from ..errors import InvalidPlan, StepFailed
+from ..kernels import ops
 from ..models.model import Model, tensor_table, tied_aliases
 from ..parts.runtime import Runtime, RuntimeOptions
 from ..weights.loader import load_tensors, random_tensors
@@ -51,10 +52,8 @@ class _Turn:
     def __enter__(self):
         self.lock.acquire()
         try:
-            if self.depth == 0 and self.last is not None:
-                stream = torch.cuda.current_stream(self.device)
-                if stream.cuda_stream != self.last and not torch.cuda.is_current_stream_capturing():
-                    stream.wait_event(self.done)
+            if self.depth == 0 and self.last is not None and ops._stream() != self.last and not torch.cuda.is_current_stream_capturing():
+                torch.cuda.current_stream(self.device).wait_event(self.done)
         except BaseException:
             self.lock.release()
             raise
@@ -64,10 +63,9 @@ class _Turn:
         self.depth -= 1
         try:
             if self.depth == 0 and not torch.cuda.is_current_stream_capturing():
-                stream = torch.cuda.current_stream(self.device)
                 self.done = self.done or torch.cuda.Event()
-                self.done.record(stream)
-                self.last = stream.cuda_stream
+                self.done.record()
+                self.last = ops._stream()
         finally:
             self.lock.release()
         return False

@@ -36,6 +36,7 @@ def stand_in(monkeypatch, work, dtype="bfloat16", padding_free=True, page_size=1
     for name in ("current_stream", "Event"):
         monkeypatch.setattr(torch.cuda, name, getattr(streams, name))
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(engine_module.ops, "_stream", lambda: streams.now)
     monkeypatch.setattr(engine_module, "Runtime", lambda *a: SimpleNamespace(
         streaming_rows_max=64, profile=None, ops=None, options=SimpleNamespace(record_portions=False)))
     monkeypatch.setattr(engine_module, "Model", lambda spec, rt: SimpleNamespace(
