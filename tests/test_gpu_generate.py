@@ -99,7 +99,7 @@ def test_seventy_requests_at_once_decode_through_the_recorded_loop_in_groups(pla
 @pytest.mark.parametrize("record", [False, True])
 def test_a_hundred_and_fifty_requests_at_once_decode_through_the_loop_for_many_rows(folders, record):
     """In bfloat16 more requests than the weight-streaming products take rows (64) decode through a recording of the
-    loop with the many-row products (a capacity of 256 here, then 128 and the fused loop as requests end); steps that
+    loop with the many-row products (160 rows of a capacity of 256 here, then 128 and the fused loop as requests end); steps that
     hold prompt portions beside their tokens are launched, or with ``record_portions`` replayed.  The tokens are ones the
     plain logits support, requests end at different lengths and their pages and slots come back."""
     from gesso_amd import Session
@@ -530,7 +530,8 @@ def test_random_weights_session_and_cli(tmp_path):
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("name", ["A", "B"])
 def test_recorded_decode_loop_equals_single_steps(folders, name, dtype):
-    """Replays of the recorded step, several runs with other work between them, against step-by-step decoding."""
+    """Replays of the recorded step, several runs with other work between them, against step-by-step decoding by ordinary steps
+    (whose kernels, rows and tables are not the loop's)."""
     from gesso_amd import Engine, Sampler, StepEntry
     d = write_tiny(folders, name, torch.float32 if dtype == "float32" else torch.bfloat16)
     cfg, _ = CONFIGS[name]
@@ -546,8 +547,9 @@ def test_recorded_decode_loop_equals_single_steps(folders, name, dtype):
             firsts.append(int(eng.step([StepEntry(i, p, [len(p) - 1])]).argmax()))
         return firsts
 
-    # step by step through the plain step function
+    # step by step, each step of single tokens an ordinary one
     eng = Engine.from_folder(d, dtype=dtype, page_size=8, max_tokens=512)
+    eng._loop_steps = False
     toks, sm, ref = prefill(eng), samplers(), []
     from gesso_amd.sampling import choose
     for _ in range(21):
@@ -567,18 +569,20 @@ def test_recorded_decode_loop_equals_single_steps(folders, name, dtype):
         eng2.step([StepEntry("other", prompts[0], [0])])
         eng2.finish_request("other")
         torch.cuda.synchronize()
+    assert not eng._runners and eng2._runners
     if dtype == "float32":
         assert got == ref
     else:
-        # bfloat16: the recorded loop's fused kernels round elsewhere than the step-by-step ones, so a near-tie may fall
-        # the other way; every token it chose must be the plain model's best, or as good within the logits' tolerance
+        # bfloat16: the recorded loop's fused kernels round elsewhere than the ordinary step's, so a near-tie may fall
+        # the other way; every token that either chose must be the plain model's best, or as good within the logits' tolerance
         cfgp, w = P.read_config(d), P.read_weights(d)
-        for i, p in enumerate(prompts):
-            seq = list(p) + [first[i]] + [row[i] for row in got]
-            plain_rows = P.forward(cfgp, w, seq[:-1])
-            slack = 2 * WORST * float((P.forward(cfgp, w, seq[:-1], store=P.to_bfloat16) - plain_rows).abs().max())
-            for at in range(len(p) + 1, len(seq)):
-                assert supported(plain_rows[at - 1], seq[at], slack), (i, at, slack)
+        for rows in (got, ref):
+            for i, p in enumerate(prompts):
+                seq = list(p) + [first[i]] + [row[i] for row in rows]
+                plain_rows = P.forward(cfgp, w, seq[:-1])
+                slack = 2 * WORST * float((P.forward(cfgp, w, seq[:-1], store=P.to_bfloat16) - plain_rows).abs().max())
+                for at in range(len(p) + 1, len(seq)):
+                    assert supported(plain_rows[at - 1], seq[at], slack), (i, at, slack)
     assert [eng2.length(i) for i in range(3)] == [len(p) + 21 for p in prompts]
 
 
@@ -586,15 +590,17 @@ def test_recorded_decode_loop_equals_single_steps(folders, name, dtype):
 @pytest.mark.parametrize("nreq", [1, 3, 17, 40])
 def test_a_step_of_single_tokens_is_the_recorded_loops_step(folders, dtype, nreq):
     """``Engine.step`` with one token a request: launched where nothing is recorded yet, replayed after a run of the loop, the
-    same bits; each result is the caller's own.  A step in which one request wants no logits runs as any other step does, and
-    what follows it sees the same cache."""
+    same bits (float32 beyond 16 requests: an ordinary step either way); each result is the caller's own, and every row is the
+    plain model's.  A step in which one request wants no logits runs as any other step does, and what follows it sees the same
+    cache."""
     from gesso_amd import Engine, StepEntry
     d = write_tiny(folders, "A", torch.bfloat16 if dtype == "bfloat16" else torch.float32)
-    cfg = P.read_config(d)
+    cfg, w = P.read_config(d), P.read_weights(d)
     prompts = [random_ids(3 + (7 * i) % 19, cfg["V"], 900 + i) for i in range(nreq)]
     engines = [Engine.from_folder(d, dtype=dtype, page_size=8, max_tokens=128 * nreq + 256, num_slots=2 * nreq + 1,
                                  poison=True) for _ in range(2)]
-    kept = []
+    through = dtype == "bfloat16" or nreq <= Engine.LOOP_STEP_MAX_F32
+    kept, seqs = [], [list(p) for p in prompts]
     for which, eng in enumerate(engines):
         for i, p in enumerate(prompts):
             eng.add_request(i)
@@ -612,15 +618,33 @@ def test_a_step_of_single_tokens_is_the_recorded_loops_step(folders, dtype, nreq
         for turn in range(4):
             toks = [(7 * turn + 3 * i + 1) % cfg["V"] for i in range(nreq)]
             want = [[0]] * nreq if turn != 2 else [[0]] * (nreq - 1) + [[]]
-            rows.append(eng.step([StepEntry(i, [t], w) for i, (t, w) in enumerate(zip(toks, want))]))
+            rows.append(eng.step([StepEntry(i, [t], wanted) for i, (t, wanted) in enumerate(zip(toks, want))]))
             if rows[-1] is not None:
                 assert torch.isfinite(rows[-1]).all()
+            if which == 0:
+                for s, t in zip(seqs, toks):
+                    s.append(t)
+        assert bool(eng._runners) == (through or which == 1)
         kept.append([None if r is None else r.clone() for r in rows])
         torch.cuda.synchronize()
         for a, b in zip(rows, kept[-1]):
             assert (a is None and b is None) or torch.equal(a, b)
     for a, b in zip(*kept):
         assert (a is None) == (b is None) and (a is None or torch.equal(a, b))
+    bound = NoiseBound()
+    for i, s in enumerate(seqs):
+        ref = P.forward(cfg, w, s)
+        rounded = P.forward(cfg, w, s, store=P.to_bfloat16) if dtype == "bfloat16" else None
+        for turn in range(4):
+            if turn == 2 and i == nreq - 1:
+                continue
+            got, at = kept[0][turn][i].double().cpu(), len(s) - 4 + turn
+            if dtype == "bfloat16":
+                bound.add(got, ref[at], rounded[at], (turn, i))
+            else:
+                assert float((got - ref[at].double()).abs().max()) <= 1e-4 * max(1.0, float(ref[at].abs().max()))
+    if dtype == "bfloat16":
+        bound.check(f"single tokens of {nreq} requests,")
 
 
 @pytest.mark.parametrize("name", ["A", "B", "C", "D"])
@@ -628,7 +652,7 @@ def test_a_step_of_single_tokens_is_the_recorded_loops_step(folders, dtype, nreq
 def test_recorded_decode_logits_follow_the_plain_model(folders, name, nreq, steps):
     """The fused kernels of the recorded step, row by row against the plain implementation (bfloat16): few rows
     (rows pre-weighted for the next norm), more than sixteen, and more than thirty-two (products in parts of K); and
-    more than sixty-four, in capacities of 128 and 256: the loop with the many-row products."""
+    more than sixty-four, in 128 rows and in 160 of a capacity of 256: the loop with the many-row products."""
     from gesso_amd import Engine, StepEntry
     from gesso_amd.engine.decode import _capacity
     d = write_tiny(folders, name, torch.bfloat16)

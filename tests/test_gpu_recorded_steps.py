@@ -2,6 +2,7 @@
 kernel by kernel, bit for bit: the same kernels run with the same arguments.  Two engines over one model folder take the
 same steps, one with ``record_portions``; the steps keep their token count while the sequences in them come, grow
 and go, and pages and slots are used again (poisoned in between)."""
+import dataclasses
 import random
 
 import pytest
@@ -23,6 +24,8 @@ WIDE_E = Lfm2Config(
     vocab_size=333, hidden_size=256, num_hidden_layers=4, num_attention_heads=4, num_key_value_heads=1,
     layer_types=("conv", "full_attention", "conv", "full_attention"), conv_L_cache=4, conv_bias=True,
     intermediate_size=344, norm_eps=1e-6, rope_theta=1e6, tie_word_embeddings=False, max_position_embeddings=8192)
+# a feed-forward so wide that its last product comes in parts of K, the stream normed by the pass that adds them
+WIDE_F = dataclasses.replace(WIDE_E, intermediate_size=2304)
 
 
 def engines(folder, **kw):
@@ -131,6 +134,25 @@ def test_recorded_steps_of_portions_equal_the_launched_ones(tmp_path, name, T):
     run_both(plain, recorded, work, 60, kinds)
     rec = recorded.recorder
     assert rec.replays == replays_expected(kinds, rec) and rec.replays >= 20, (rec.replays, kinds)
+
+
+@pytest.mark.parametrize("T", [72, 160, 700])
+def test_recorded_steps_whose_last_products_come_in_parts_of_k(tmp_path, T):
+    """The sheets of the parts lie in the recording's memory and the norm after each of them takes the rows that the adding pass
+    normed: the launched steps' logits, bit for bit."""
+    folder = str(tmp_path / "F")
+    write_model_folder(folder, WIDE_F, 17, torch.bfloat16, std=STD)
+    plain, recorded = engines(folder, page_size=16, max_tokens=6 * 1300, num_slots=7)
+    for eng in (plain, recorded):
+        w = eng.model.blocks[0].ffn.w2
+        x = torch.empty(T, w.shape[1], dtype=torch.bfloat16, device=eng.device)
+        assert w.shape == (256, 2304) and eng.rt.ops.mid_parts_pay(x, w, eng.rt.tiles_of(w)) >= 2
+    rng = random.Random(T)
+    work = Workload(WIDE_F.vocab_size, T, seed=T, prompt_lens=[rng.randint(20, 400 if T < 700 else 1200) for _ in range(40)])
+    kinds = {}
+    run_both(plain, recorded, work, 40, kinds)
+    rec = recorded.recorder
+    assert rec.replays == replays_expected(kinds, rec) and rec.replays >= 10, (rec.replays, kinds)
 
 
 def test_recorded_steps_with_thousands_of_keys_walk_them_whole(tmp_path):

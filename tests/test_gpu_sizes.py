@@ -216,13 +216,13 @@ def test_recorded_decode_at_the_real_layer_sizes(balanced, others, size, nreq, s
     and 64 rows (capacities 1, 8 and 64 of the recording: one row tile, and four with the register ring), at the layer
     sizes of LFM2-1.2B; at 8 and 64 rows with LFM2-350M's (groups of two in decode attention, products over 4,608), at
     40 with LFM2-2.6B's (over 7,168).  And the loop for more than 64 rows, whose products are the library's: 100 rows
-    (a capacity of 128) at LFM2-1.2B's sizes, 130 (of 256) at LFM2-350M's."""
+    (a capacity of 128) at LFM2-1.2B's sizes, 130 (160 rows of a capacity of 256) at LFM2-350M's."""
     from gesso_amd import Engine, StepEntry
     from gesso_amd.engine.decode import _capacity
     m = balanced if size == "1.2B" else others(size)
     prompts = [random_ids(n, 65536, 7000 + 13 * i + n) for i, n in enumerate(([3, 18, 33] + [4 + (5 * i) % 17 for i in range(nreq)])[:nreq])]
     # poisoned: free pages, the scratch page and the scratch slot hold NaN, so the rows beyond the live batch (the
-    # capacity is 4, 32 and 48) compute NaN throughout, and nothing of it may reach a live row
+    # capacity is 4, 24 and 48) compute NaN throughout, and nothing of it may reach a live row
     eng = Engine.from_folder(m.dir, dtype="bfloat16", page_size=16, max_tokens=64 * nreq + 256, num_slots=nreq + 1,
                              poison=True)
     seqs, toks = [list(p) for p in prompts], []
