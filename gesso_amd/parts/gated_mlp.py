@@ -2,7 +2,8 @@
 ``W_down (act(W_gate x + b_gate) * (W_up x + b_up)) + b_down``; ``act`` is silu or the tanh form of gelu.
 
 W_gate and W_up are laid side by side at load so that one product feeds both (as :mod:`gesso_amd.parts.swiglu` does);
-biases, activation and the product of the two halves are one pass in float32 over the product's rows.
+biases, activation and the product of the two halves are float32 arithmetic on the product's rows, in the product's own
+epilogue for few bfloat16 rows, else one pass over them.
 """
 from __future__ import annotations
 
