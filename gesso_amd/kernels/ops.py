@@ -462,25 +462,27 @@ def attention_decode_maps_blocks(nh: int, nkv: int) -> int:
     return int(lib().gs_attention_decode_maps_blocks(nh, nkv))
 
 
-_maps_ws = {}
+# Device memory that kernels share their keys' sums through, for calls that bring none of their own: by sizes, never given back.
+# (Two callers whose kernels may run at one time bring a dict each: an engine's parts bring their runtime's.)
+_workspaces = {}
 
 
 def attention_decode_maps(rows, kcache, vcache, positions, block_table, page_size, window, scale, lam: float, eps: float,
                           out_scale: float, gate_col: int, nh, nkv, d, vd, nseq: int, nsplit: int,
-                          out: torch.Tensor = None) -> torch.Tensor:
+                          out: torch.Tensor = None, workspaces: dict = None) -> torch.Tensor:
     """:func:`attention_maps` for one query per sequence (bfloat16): sequence ``i`` is row ``i``, its keys split over
-    ``nsplit`` blocks."""
+    ``nsplit`` blocks, whose sums go through memory kept in ``workspaces``."""
     _maps_operands(rows, kcache, vcache, positions, block_table, page_size, gate_col, nh, nkv, d, vd, "attention_decode_maps")
     _need(rows.dtype == torch.bfloat16 and rows.shape[0] >= nseq, "attention_decode_maps takes bfloat16, a row a sequence")
     _i32(positions, nseq, "positions")
     _need(block_table.shape[0] >= nseq, "block_table must be int32 (nseq, max_blocks)")
     ws = None
     if nsplit > 1:
-        key = (rows.device, nseq, nh, vd, nsplit)
-        ws = _maps_ws.get(key)
+        held, key = _workspaces if workspaces is None else workspaces, (rows.device, nseq, nh, vd, nsplit)
+        ws = held.get(key)
         if ws is None:
             floats = int(lib().gs_attention_decode_maps_workspace(nseq, nh, vd, nsplit))
-            ws = _maps_ws[key] = torch.empty(max(1, floats), dtype=torch.float32, device=rows.device)
+            ws = held[key] = torch.empty(max(1, floats), dtype=torch.float32, device=rows.device)
     if out is None:
         out = torch.empty((nseq, nh * vd), dtype=rows.dtype, device=rows.device)
     _need(out.shape == (nseq, nh * vd) and out.dtype == rows.dtype and out.is_contiguous(), "attention_decode_maps: out has the wrong shape or type")
@@ -1116,24 +1118,22 @@ def attention_decode_supports(nh: int, nkv: int, d: int) -> bool:
     return bool(lib().gs_attention_decode_supports(c_int(nh), c_int(nkv), c_int(d)))
 
 
-_decode_ws = {}
-
-
-def _decode_workspace(device, nseq, nh, nkv, d, nsplit):
-    key = (device, nseq, nh, nkv, d, nsplit)
-    ws = _decode_ws.get(key)
+def _decode_workspace(held, device, nseq, nh, nkv, d, nsplit):
+    held, key = _workspaces if held is None else held, (device, nseq, nh, nkv, d, nsplit)
+    ws = held.get(key)
     if ws is None:
         n = lib().gs_attention_decode_workspace
         n.restype = c_long
         floats = n(c_int(nseq), c_int(nh), c_int(nkv), c_int(d), c_int(nsplit))
-        ws = _decode_ws[key] = torch.empty(max(1, floats), dtype=torch.float32, device=device)
+        ws = held[key] = torch.empty(max(1, floats), dtype=torch.float32, device=device)
     return ws
 
 
 def attention_decode(q, q_stride, kcache, vcache, positions, block_table, page_size, window, scale, nh, nkv, d, nseq,
                      nsplit: int, out=None, chunk: int = None, sink: bool = False, softcap: float = None,
-                     keep_first: int = 0, sinks=None):
-    """One query per sequence over its paged keys (bfloat16), keys split over ``nsplit`` blocks per key head.
+                     keep_first: int = 0, sinks=None, workspaces: dict = None):
+    """One query per sequence over its paged keys (bfloat16), keys split over ``nsplit`` blocks per key head, whose sums go
+    through memory kept in ``workspaces``.
     ``out``: a tensor, or True / a :class:`TiledRows` for tiled rows.  ``chunk``: the query sees only the keys of its
     own run of ``chunk`` positions; ``sink``: one more term ``exp(0)`` in the softmax's denominator; ``softcap``: scores
     become ``softcap tanh(score / softcap)``; ``keep_first``: with a window, the sequence's first positions that stay
@@ -1148,7 +1148,7 @@ def attention_decode(q, q_stride, kcache, vcache, positions, block_table, page_s
     _i32(positions, nseq, "positions")
     _need(block_table.dtype == torch.int32 and block_table.dim() == 2 and block_table.shape[0] >= nseq,
           "block_table must be int32 (nseq, max_blocks)")
-    ws = _decode_workspace(q.device, nseq, nh, nkv, d, nsplit)
+    ws = _decode_workspace(workspaces, q.device, nseq, nh, nkv, d, nsplit)
     out, buf, tiled = _rows_out(out, nseq, nh * d, q.device, q.dtype)
     _need(tuple(out.shape) == (nseq, nh * d) and out.dtype == q.dtype, "attention_decode: out has the wrong shape or type")
     if softcap or keep_first or sinks is not None:
@@ -1179,7 +1179,7 @@ def attention_decode_raw_supports(nh: int, nkv: int, d: int, rotary_dim: int) ->
 
 def attention_decode_raw(qkv, q_stride, kcache, vcache, positions, block_table, page_size, window, scale, q_weight,
                          k_weight, head_eps, cos, sin, nh, nkv, d, nseq, nsplit: int, write_kv: bool = True,
-                         out=None):
+                         out=None, workspaces: dict = None):
     """Decode attention straight from the rows of q|k|v as their product left them: the kernel norms and rotates
     the queries and the new key, writes the new key and value into their pages, and attends."""
     _dev(qkv, kcache, vcache, positions, block_table, q_weight, k_weight, cos, sin,
@@ -1196,7 +1196,7 @@ def attention_decode_raw(qkv, q_stride, kcache, vcache, positions, block_table, 
     _i32(positions, nseq, "positions")
     _need(block_table.dtype == torch.int32 and block_table.dim() == 2 and block_table.shape[0] >= nseq,
           "block_table must be int32 (nseq, max_blocks)")
-    ws = _decode_workspace(qkv.device, nseq, nh, nkv, d, nsplit)
+    ws = _decode_workspace(workspaces, qkv.device, nseq, nh, nkv, d, nsplit)
     out, buf, tiled = _rows_out(out, nseq, nh * d, qkv.device, qkv.dtype)
     _need(tuple(out.shape) == (nseq, nh * d) and out.dtype == qkv.dtype, "attention_decode_raw: out has the wrong shape or type")
     _check(lib().gs_attention_decode_raw(_p(qkv), c_int(q_stride), _p(kcache), _p(vcache), _p(positions), _p(block_table),
@@ -1460,26 +1460,23 @@ def attention_latent_mfma_tokens(H: int) -> int:
     return int(lib().gs_attention_latent_mfma_tokens(H))
 
 
-_latent_parts = {}        # per device: the buffers made so far, the largest last
-
-
-def _latent_workspace(device, rows: int, c: int, nsplit: int):
-    """Room for the shares of blocks that walk a row's keys in parts, kept per device.  A recorded step writes to the buffer
-    it was recorded with for as long as it is replayed, so where more is asked a larger one comes beside the smaller ones,
-    each at least twice the one before it (all the smaller ones together are no more than the largest)."""
+def _latent_workspace(held: dict, device, rows: int, c: int, nsplit: int):
+    """Room for the shares of blocks that walk a row's keys in parts, kept in ``held`` per device.  A recorded step writes to
+    the buffer it was recorded with for as long as it is replayed, so where more is asked a larger one comes beside the smaller
+    ones, each at least twice the one before it (all the smaller ones together are no more than the largest)."""
     need = nsplit * rows * (c + 2)
-    held = _latent_parts.setdefault(device, [])
-    if not held or held[-1].numel() < need:
-        held.append(torch.empty(max(need, 2 * held[-1].numel() if held else 0), dtype=torch.float32, device=device))
-    return held[-1][:nsplit * rows * c], held[-1][nsplit * rows * c:need]
+    made = (_workspaces if held is None else held).setdefault(device, [])
+    if not made or made[-1].numel() < need:
+        made.append(torch.empty(max(need, 2 * made[-1].numel() if made else 0), dtype=torch.float32, device=device))
+    return made[-1][:nsplit * rows * c], made[-1][nsplit * rows * c:need]
 
 
 def attention_latent_mfma(qa, cache, positions, tiles, block_table, page_size, window, scale, H, c, r, ntok,
-                          out: torch.Tensor = None, nsplit: int = 1, sinks=None) -> torch.Tensor:
+                          out: torch.Tensor = None, nsplit: int = 1, sinks=None, workspaces: dict = None) -> torch.Tensor:
     """:func:`attention_latent` on the matrix cores (bfloat16).  ``tiles``: int32 ``(3, n)``, the sequence, first row
     and token count (at most :func:`attention_latent_mfma_tokens`) of every tile of consecutive tokens of one
     sequence; None: sequence ``i`` brings the single token ``i``.  ``nsplit`` > 1: as many blocks share a tile's keys out
-    between them in runs of whole steps, and a second kernel adds their shares."""
+    between them in runs of whole steps, and a second kernel adds their shares, which lie in memory kept in ``workspaces``."""
     _dev(qa, cache, positions, block_table, out, tiles, sinks)
     _need(sinks is None or (sinks.dtype == torch.float32 and sinks.shape == (H,)), "attention_latent_mfma: sinks must be float32 (H,)")
     _need(1 <= nsplit <= 64, "attention_latent_mfma: 1 to 64 parts")
@@ -1499,7 +1496,7 @@ def attention_latent_mfma(qa, cache, positions, tiles, block_table, page_size, w
         out = torch.empty((ntok, H * c), dtype=qa.dtype, device=qa.device)
     _need(out.shape == (ntok, H * c) and out.dtype == qa.dtype and out.data_ptr() % 16 == 0,
           "attention_latent_mfma: out has the wrong shape or type")
-    part_o, part_ml = _latent_workspace(qa.device, ntok * H, c, nsplit) if nsplit > 1 else (None, None)
+    part_o, part_ml = _latent_workspace(workspaces, qa.device, ntok * H, c, nsplit) if nsplit > 1 else (None, None)
     _check(lib().gs_attention_latent_mfma(_p(qa), _p(cache), _p(positions), _p(rows[0]), _p(rows[1]), _p(rows[2]), n,
                                           _p(block_table), block_table.shape[1], page_size, window or 0, float(scale),
                                           _p(out), H, c, r, nsplit, _p(part_o), _p(part_ml), ntok, _p(sinks), _stream()))

@@ -193,9 +193,10 @@ class Attention(Part):
             return ops.attention_decode_raw(q.qkv, q_stride, cache.k, cache.v, ctx.positions, cache.block_table,
                                             cache.page_size, window, self.scale, q.q_norm, q.k_norm, q.eps,
                                             q.position.cos, q.position.sin, nh, nkv, d, nseq, nsplit,
-                                            write_kv=cache.write, out=out)
+                                            write_kv=cache.write, out=out, workspaces=self.rt.workspaces)
         return ops.attention_decode(q, q_stride, cache.k, cache.v, ctx.positions, cache.block_table,
-                                    cache.page_size, window, self.scale, nh, nkv, d, nseq, nsplit, out=out)
+                                    cache.page_size, window, self.scale, nh, nkv, d, nseq, nsplit, out=out,
+                                    workspaces=self.rt.workspaces)
 
     def prompt_walk(self, q_lens, max_kv_len):
         """How the kernel for long portions takes sequences that bring ``q_lens`` tokens: ``(sub-tiles a block, key
@@ -282,7 +283,8 @@ class Attention(Part):
                 nsplit = max(1, min(tiles // 16, 64, 256 // max(1, ctx.nseq * nkv)))
                 return ops.attention_decode(q, q_stride, cache.k, cache.v, ctx.positions, cache.block_table, cache.page_size,
                                             s.window, self.scale, nh, nkv, d, ctx.nseq, nsplit, chunk=self.chunk, sink=self.sink,
-                                            softcap=self.softcap, keep_first=self.keep_first, sinks=self.sinks)
+                                            softcap=self.softcap, keep_first=self.keep_first, sinks=self.sinks,
+                                            workspaces=rt.workspaces)
             if (q.dtype == torch.bfloat16 and not ctx.all_single and self.value_dim == d and cache.page_size >= 2
                     and q_stride % 8 == 0 and ops.attention_prefill_supports(nh, nkv, d) and ctx.recording is None
                     and vp is None and not (self.keep_first and self.chunk)):
@@ -309,7 +311,8 @@ class Attention(Part):
             tiles = max(1, -(-longest // 64))
             nsplit = max(1, min(tiles // 16, 64, 256 // max(1, ctx.nseq * nkv)))
             out = ops.attention_decode(q, q_stride, cache.k, cache.v, ctx.positions, cache.block_table, cache.page_size,
-                                       s.window, self.scale, nh, nkv, d, ctx.nseq, nsplit, chunk=self.chunk, sink=self.sink)
+                                       s.window, self.scale, nh, nkv, d, ctx.nseq, nsplit, chunk=self.chunk, sink=self.sink,
+                                       workspaces=rt.workspaces)
             if vp is not None:
                 ops.turn_heads(out, vp.cos, vp.sin, ctx.positions, nh, d, sign=-1.0, layout=layout)
             return out

@@ -143,7 +143,7 @@ class LatentAttention(Part):
                 nsplit = max(1, min(longest // 64, 64, self.rt.compute_units // max(1, blocks)))
             return ops.attention_latent_mfma(qa, cache.k, ctx.positions, tiles, cache.block_table, cache.page_size,
                                              s.window, s.scale, s.n_heads, s.kv_rank, s.rot_dim, ctx.T, nsplit=nsplit,
-                                             sinks=self.sinks)
+                                             sinks=self.sinks, workspaces=self.rt.workspaces)
         return ops.attention_latent(qa, cache.k, ctx.positions, ctx.seq_of_token, cache.block_table, cache.page_size,
                                     s.window, s.scale, s.n_heads, s.kv_rank, s.rot_dim, ctx.T, sinks=self.sinks)
 

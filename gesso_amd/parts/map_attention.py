@@ -81,7 +81,7 @@ class MapAttention(Part):
         blocks = ops.attention_decode_maps_blocks(s.n_heads, s.n_kv_heads)
         nsplit = max(1, min(-(-longest // 64) // 16, 64, 256 // max(1, nseq * blocks)))
         return ops.attention_decode_maps(rows, cache.k, cache.v, ctx.positions, cache.block_table, cache.page_size, *self._rule(),
-                                         nseq, nsplit, out=out)
+                                         nseq, nsplit, out=out, workspaces=self.rt.workspaces)
 
     def _rule(self):
         """Window, scale, share, norm, gate and sizes, in the order in which the kernels' faces take them."""

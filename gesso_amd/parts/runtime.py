@@ -125,6 +125,7 @@ class Runtime:
         self.dtype = dtype
         self.options = options = options or RuntimeOptions()
         self._shared = {}
+        self.workspaces = {}           # what kernels share their keys' sums through, by sizes (two engines may run at one time)
         self.no_library = False        # set while a HIP graph is recorded: only our own kernels go into it
         self.fused = False             # set while a decode step is recorded: norms, adds and small ops fold into products
         self.tile_weights = dtype == torch.bfloat16 and options.tile_weights

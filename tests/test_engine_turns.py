@@ -230,3 +230,33 @@ def test_single_tokens_in_pages_that_hold_a_third_of_a_context(tmp_path):
         bound.add(row[0].double().cpu(), ref[20 + i], rounded[20 + i], i)
     bound.check("single tokens in large pages,")
     assert eng.length("r") == 30
+
+
+@pytest.mark.gpu
+def test_two_engines_share_no_memory_that_their_kernels_write(tmp_path):
+    """Two engines of one model, each on a stream of its own, nothing waited for in between: what the steps' kernels share keys'
+    sums through is the engine's own, and the logits are those of each alone."""
+    from tiny_makuzen import write_tiny
+    d = write_tiny(str(tmp_path), "C", torch.bfloat16)
+
+    def made():
+        eng = Engine.from_folder(d, dtype="bfloat16", page_size=16, max_tokens=512, num_slots=2)
+        eng.add_request("r")
+        eng.step([StepEntry("r", tokens_of(eng, "r", 40), [])])
+        torch.cuda.synchronize()
+        return eng
+
+    engines, streams = [made(), made()], [torch.cuda.Stream(), torch.cuda.Stream()]
+    toks = [[(5 * i + 11 * k) % 97 for i in range(20)] for k in range(2)]
+    rows = [[], []]
+    for i in range(20):
+        for k in range(2):
+            with torch.cuda.stream(streams[k]):
+                rows[k].append(engines[k].step([StepEntry("r", [toks[k][i]], [0])]))
+    torch.cuda.synchronize()
+    held = [{t.data_ptr() for v in e.rt.workspaces.values() for t in (v if isinstance(v, list) else [v])} for e in engines]
+    assert held[0] and held[1] and not held[0] & held[1]
+    for k in range(2):
+        alone = made()
+        want = [alone.step([StepEntry("r", [t], [0])]) for t in toks[k]]
+        assert torch.equal(torch.cat(rows[k]), torch.cat(want))

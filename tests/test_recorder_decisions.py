@@ -126,26 +126,25 @@ def test_the_tally_of_kinds_starts_over_when_it_is_full(recorder):
     assert list(recorder.seen) == [(105, 4096, (2,), 64)]
 
 
-def test_room_that_a_recorded_step_writes_to_is_never_given_back(monkeypatch):
+def test_room_that_a_recorded_step_writes_to_is_never_given_back():
     """Single tokens over cached latent rows leave their parts' sums in a buffer that all steps share.  A step that asks for
     more gets a larger one; the one before, whose address a recorded step holds, must not go back to the allocator (the
     replay would write into whatever lies there by then)."""
     import weakref
     import torch
     from gesso_amd.kernels import ops
-    monkeypatch.setattr(ops, "_latent_parts", {})
-    cpu = torch.device("cpu")
-    recorded, sums = ops._latent_workspace(cpu, 32, 64, 4)
+    cpu, held = torch.device("cpu"), {}
+    recorded, sums = ops._latent_workspace(held, cpu, 32, 64, 4)
     address = recorded.data_ptr()
     bases = [weakref.ref(recorded._base)]
     del recorded, sums
     for rows, parts in ((64, 4), (65, 4), (16, 2), (512, 16), (511, 16)):
-        o, ml = ops._latent_workspace(cpu, rows, 64, parts)
+        o, ml = ops._latent_workspace(held, cpu, rows, 64, parts)
         assert o.numel() == parts * rows * 64 and ml.numel() == parts * rows * 2
         assert ml.data_ptr() == o.data_ptr() + 4 * o.numel() and o.data_ptr() != address
         bases.append(weakref.ref(o._base))
         del o, ml
-    held = [b() for b in bases]
-    assert all(b is not None for b in held)
-    sizes = sorted({b.data_ptr(): b.numel() for b in held}.values())
+    kept = [b() for b in bases]
+    assert all(b is not None for b in kept)
+    sizes = sorted({b.data_ptr(): b.numel() for b in kept}.values())
     assert sum(sizes[:-1]) <= sizes[-1]                  # what is kept is bounded by what was asked for
