@@ -19,6 +19,16 @@
 //
 // EPI 1 (SwiGLU): W holds gate rows [0, N/2), then up rows, N / 2 a multiple of 16; a wavefront owns NT / 2 tiles of gate rows
 // and the up rows of the same columns.  silu(gate) * up is taken of the values as they would have been stored.
+//
+// EPI 3 (a sub-layer's last product): the sums are added to the float32 stream where they arise, and the new rows go out
+// weighted for the norm that reads them next, each wavefront's sum of their squares beside them; SCALED: such rows come in, the
+// partial sums of squares are asked for before the first weights and added while those travel, and the results are multiplied
+// by the rows' inverse root mean squares.  Between the two stands no pass: a layer's output projection, gate and up, and down product
+// (1024 wide, 4608 inside; weights in turn, a graph) take 160 rows 32.4 us with the norm's pass and 31.4 without, 72 rows 29.0 and
+// 27.5, 333 rows 41.3 and 40.1; 2048 wide and 8192 inside, 72 rows 47.4 and 45.9, 160 rows 56.3 and 55.6.
+//
+// The groups' sums (KG > 1) are added by two groups, half of the block's rows each: the wavefronts that add, and their loads from
+// LDS, are twice as many as with one.
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 gd_bf16x8_t;
@@ -27,11 +37,34 @@ typedef __attribute__((ext_vector_type(4))) unsigned gd_u32x4_t;
 
 constexpr int GD_BK = 64, GD_LDR = GD_BK + 8, GD_AHEAD = 4;
 
-template <int BM, int NT, int KG, int EPI>
+// Bytes of LDS: two steps' rows of X a group, and in their place at the end the groups' sums.
+constexpr size_t mid_lds(int BM, int NT, int KG) {
+  const size_t held = (size_t)KG * 2 * BM * GD_LDR * sizeof(uint16_t), sums = KG > 1 ? (size_t)KG * BM * 64 * NT * sizeof(float) : 0;
+  return held > sums ? held : sums;
+}
+
+constexpr int GD_SSQ_MAX = 128;         // partial sums of squares a row that a SCALED product takes
+
+// What EPI 3 writes (the stream, the next norm's weight, the rows weighted with it, their partial sums of squares; the last three
+// together or not at all) and what SCALED reads (partial sums of squares, eps).
+struct MidNorm {
+  float* res;
+  const float* weight;
+  bf16* rows;
+  float* ssq_out;
+  const float* ssq;
+  int nssq;
+  float eps;
+};
+
+template <int BM, int NT, int KG, int EPI, bool SCALED>
 __global__ __launch_bounds__(KG * 256) void gemm_mid_kernel(const bf16* __restrict__ X, int ldx, const bf16* __restrict__ Wt,
-                                                            bf16* __restrict__ Y, int ldy, int M, int N, int K, int part_steps) {
+                                                            bf16* __restrict__ Y, int ldy, int M, int N, int K, int part_steps,
+                                                            MidNorm norm) {
   constexpr int TM = BM / 16, LA = BM / 32, STAGE = BM * GD_LDR;           // 16-byte loads of X a thread and step
   constexpr int COLS = 64 * (EPI == 1 ? NT / 2 : NT);                      // columns of Y a block
+  constexpr int UM = KG > 1 ? TM / 2 : TM;                                 // row tiles that a group finishes
+  constexpr size_t AFTER = mid_lds(BM, NT, KG);                            // bytes of LDS before the rows' inverses
   static_assert(EPI != 1 || NT % 2 == 0, "SwiGLU pairs gate tiles with up tiles");
   extern __shared__ __align__(16) uint16_t gd_lds[];
   const int tid = threadIdx.x & 255, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
@@ -53,6 +86,7 @@ __global__ __launch_bounds__(KG * 256) void gemm_mid_kernel(const bf16* __restri
     }
   }
   const int m0 = bm * BM, n0 = bn * COLS + wave * (COLS / 4);               // the wavefront's first column
+  const int mu = KG > 1 ? m0 + (kg & 1) * (BM / 2) : m0;                    // the first of the rows its group finishes
   const int r0 = tid >> 3, c = tid & 7;                                     // this thread's loads: row r0 + 32 i, piece c of eight k
   const bf16* ap[LA];
 #pragma unroll
@@ -117,9 +151,70 @@ __global__ __launch_bounds__(KG * 256) void gemm_mid_kernel(const bf16* __restri
         for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(s.w[ks][j], x[ks][i], acc[i][j], 0, 0, 0);
     }
   };
+  // EPI 3: the stream's values and the next norm's weights, asked for first: they are there when the sums are
+  gd_f32x4_t held[EPI == 3 ? UM : 1][EPI == 3 ? NT : 1], nw[EPI == 3 ? NT : 1];
+  constexpr bool ROOM = KG == 1 || NT == 1;               // (else the weights come when the groups' sums are added)
+  auto next_weights = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const int n = n0 + 16 * j + 4 * g < N ? n0 + 16 * j + 4 * g : N - 4;
+      nw[j] = *reinterpret_cast<const gd_f32x4_t*>((norm.rows ? norm.weight : norm.res) + n);
+    }
+  };
+  if constexpr (EPI == 3) {
+    if constexpr (ROOM) next_weights();
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const int n = n0 + 16 * j + 4 * g < N ? n0 + 16 * j + 4 * g : N - 4;
+#pragma unroll
+      for (int i = 0; i < UM; ++i) {
+        const int m = mu + 16 * i + r16 < M ? mu + 16 * i + r16 : M - 1;
+        held[i][j] = *reinterpret_cast<const gd_f32x4_t*>(norm.res + (size_t)m * N + n);
+      }
+    }
+  }
+  // SCALED: four threads a row, a quarter of its partial sums each (what lies beyond them is loaded from the first and not added;
+  // the second half only where there are more than half as many as there may be)
+  constexpr int NTH = KG * 256, SR = SCALED ? (BM * 4 + NTH - 1) / NTH : 1, SP = GD_SSQ_MAX / 16;
+  gd_f32x4_t sq[SR][SP];
+  auto squares_of = [&](int half) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < SR; ++i) {
+      const int at = (int)threadIdx.x + i * NTH, m = m0 + (at >> 2) < M ? m0 + (at >> 2) : M - 1;
+#pragma unroll
+      for (int q = half * SP / 2; q < (half + 1) * SP / 2; ++q) {
+        const int p = 4 * ((at & 3) + 4 * q);
+        sq[i][q] = *reinterpret_cast<const gd_f32x4_t*>(norm.ssq + (size_t)m * norm.nssq + (p < norm.nssq ? p : 0));
+      }
+    }
+  };
+  if constexpr (SCALED) {
+#pragma unroll
+    for (int i = 0; i < SR; ++i)
+#pragma unroll
+      for (int q = SP / 2; q < SP; ++q) sq[i][q] = gd_f32x4_t{0.f, 0.f, 0.f, 0.f};
+    squares_of(0);
+    if (norm.nssq > GD_SSQ_MAX / 2) squares_of(1);
+  }
   Step s[GD_AHEAD];
 #pragma unroll
   for (int d = 0; d < GD_AHEAD; ++d) load(s[d], d);
+  float* inverse = reinterpret_cast<float*>(reinterpret_cast<char*>(gd_lds) + AFTER);       // (SCALED: BM floats)
+  if constexpr (SCALED) {
+#pragma unroll
+    for (int i = 0; i < SR; ++i) {
+      const int at = (int)threadIdx.x + i * NTH;
+      float sum = 0.f;
+#pragma unroll
+      for (int q = 0; q < SP; ++q) {
+        const float four = (sq[i][q][0] + sq[i][q][1]) + (sq[i][q][2] + sq[i][q][3]);
+        sum += 4 * ((at & 3) + 4 * q) < norm.nssq ? four : 0.f;
+      }
+      sum += dpp_move<0xB1>(sum);
+      sum += dpp_move<0x4E>(sum);
+      if ((at & 3) == 0 && at < BM * 4) inverse[at >> 2] = norm_inverse(sum, (float)K, norm.eps);
+    }
+  }
   put(s[0], 0);
   __syncthreads();
   int it = 0;
@@ -141,44 +236,87 @@ __global__ __launch_bounds__(KG * 256) void gemm_mid_kernel(const bf16* __restri
       put(s[d + 1], (d + 1) & 1);
       __syncthreads();
     }
-  if (KG > 1) {
-    // the other groups' sums, tile after tile, in group order
+  if constexpr (EPI == 3 && !ROOM) next_weights();
+  gd_f32x4_t out[UM][NT];
+  if constexpr (KG > 1) {
+    // the groups' sums, in group order: two groups finish half of the block's rows each
     float* sums = reinterpret_cast<float*>(gd_lds);
-    if (kg > 0) {
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j)
-          *reinterpret_cast<gd_f32x4_t*>(sums + (((kg - 1) * TM * NT + i * NT + j) * 256 + tid) * 4) = acc[i][j];
-    }
+      for (int j = 0; j < NT; ++j) *reinterpret_cast<gd_f32x4_t*>(sums + ((kg * TM * NT + i * NT + j) * 256 + tid) * 4) = acc[i][j];
     __syncthreads();
-    if (kg > 0) return;
-    for (int q = 0; q < KG - 1; ++q)
+    if (kg > 1) return;
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < UM; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j)
-          acc[i][j] += *reinterpret_cast<const gd_f32x4_t*>(sums + ((q * TM * NT + i * NT + j) * 256 + tid) * 4);
+      for (int j = 0; j < NT; ++j) {
+        const float* at = sums + (((kg * UM + i) * NT + j) * 256 + tid) * 4;
+        gd_f32x4_t each[KG];
+#pragma unroll
+        for (int q = 0; q < KG; ++q) each[q] = *reinterpret_cast<const gd_f32x4_t*>(at + q * TM * NT * 1024);
+        out[i][j] = each[0];
+#pragma unroll
+        for (int q = 1; q < KG; ++q) out[i][j] += each[q];
+      }
+  } else {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) out[i][j] = acc[i][j];
   }
   // element e of lane l: row 4 (l / 16) + e of W, row l % 16 of X
+  if constexpr (EPI == 3) {
+    const int tiles_n = (N + COLS - 1) / COLS;
 #pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int m = m0 + 16 * i + r16;
+    for (int i = 0; i < UM; ++i) {
+      const int m = mu + 16 * i + r16;
+      float squares = 0.f;
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const int n = n0 + 16 * j + 4 * g;
+        const gd_f32x4_t v = held[i][j] + out[i][j];
+        if (m >= M || n >= N) continue;
+        *reinterpret_cast<gd_f32x4_t*>(norm.res + (size_t)m * N + n) = v;
+        if (norm.rows) {
+          squares += (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
+          uint2 o;
+          o.x = (uint32_t)f32_to_bf16(v[0] * nw[j][0]).x | ((uint32_t)f32_to_bf16(v[1] * nw[j][1]).x << 16);
+          o.y = (uint32_t)f32_to_bf16(v[2] * nw[j][2]).x | ((uint32_t)f32_to_bf16(v[3] * nw[j][3]).x << 16);
+          *reinterpret_cast<uint2*>(norm.rows + (size_t)m * N + n) = o;
+        }
+      }
+      if (norm.rows) {
+        squares = group4_sum(squares);                     // (a row's columns lie in four lanes; a tile past the last adds zero)
+        if (g == 0 && m < M) norm.ssq_out[(size_t)m * (4 * tiles_n) + bn * 4 + wave] = squares;
+      }
+    }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < UM; ++i) {
+    const int m = mu + 16 * i + r16;
     if (m >= M) continue;
+    const float inv = SCALED ? inverse[mu - m0 + 16 * i + r16] : 1.0f;
 #pragma unroll
     for (int j = 0; j < (EPI == 1 ? NT / 2 : NT); ++j) {
       const int n = n0 + 16 * j + 4 * g;
       if (n >= width) continue;                            // (whole tiles: the width is a multiple of 16)
       if (EPI == 2) {
-        *reinterpret_cast<gd_f32x4_t*>(reinterpret_cast<float*>(Y) + ((size_t)part * M + m) * N + n) = acc[i][j];
+        *reinterpret_cast<gd_f32x4_t*>(reinterpret_cast<float*>(Y) + ((size_t)part * M + m) * N + n) = out[i][j];
         continue;
       }
       float v[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        v[e] = acc[i][j][e];
+        v[e] = out[i][j][e];
         if (EPI == 1) {
-          const float gv = to_f32(f32_to_bf16(v[e])), u = to_f32(f32_to_bf16(acc[i][j + (EPI == 1 ? NT / 2 : 0)][e]));
+          float uv = out[i][j + (EPI == 1 ? NT / 2 : 0)][e];
+          if (SCALED) {
+            v[e] *= inv;
+            uv *= inv;
+          }
+          const float gv = to_f32(f32_to_bf16(v[e])), u = to_f32(f32_to_bf16(uv));
           v[e] = gv / (1.0f + expf(-gv)) * u;
         }
       }
@@ -190,16 +328,17 @@ __global__ __launch_bounds__(KG * 256) void gemm_mid_kernel(const bf16* __restri
   }
 }
 
-template <int BM, int NT, int KG, int EPI>
-static void run_mid(const bf16* X, int ldx, const bf16* Wt, bf16* Y, int ldy, int M, int N, int K, hipStream_t stream, int parts = 1) {
+template <int BM, int NT, int KG, int EPI, bool SCALED = false>
+static void run_mid(const bf16* X, int ldx, const bf16* Wt, bf16* Y, int ldy, int M, int N, int K, hipStream_t stream, int parts = 1,
+                    MidNorm norm = MidNorm()) {
   const int cols = 64 * (EPI == 1 ? NT / 2 : NT), width = EPI == 1 ? N / 2 : N;
   const long tiles = (long)gs_ceil_div(M, BM) * gs_ceil_div(width, cols) * parts;
-  const size_t held = (size_t)KG * 2 * BM * GD_LDR * sizeof(uint16_t), sums = (size_t)(KG - 1) * BM * 64 * NT * sizeof(float);
-  const size_t lds = held > sums ? held : sums;
-  static const hipError_t asked = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_mid_kernel<BM, NT, KG, EPI>),
+  const size_t lds = mid_lds(BM, NT, KG) + (SCALED ? BM * sizeof(float) : 0);
+  static const hipError_t asked = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_mid_kernel<BM, NT, KG, EPI, SCALED>),
                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   (void)asked;
-  gemm_mid_kernel<BM, NT, KG, EPI><<<(unsigned)tiles, KG * 256, lds, stream>>>(X, ldx, Wt, Y, ldy, M, N, K, gs_ceil_div(gs_ceil_div(K, GD_BK), parts));
+  gemm_mid_kernel<BM, NT, KG, EPI, SCALED><<<(unsigned)tiles, KG * 256, lds, stream>>>(X, ldx, Wt, Y, ldy, M, N, K,
+                                                                                       gs_ceil_div(gs_ceil_div(K, GD_BK), parts), norm);
 }
 
 // Which tile, and whether this kernel at all.  What a compute unit brings in (some 55 bytes a nanosecond, however the tile is
@@ -270,6 +409,65 @@ extern "C" int gs_gemm_mid(const void* X, int ldx, const void* Wt, void* Y, int 
   }
 #undef GD_RUN
   GS_LAUNCH_CHECK("gemm_mid");
+  return 0;
+}
+
+// Y (M, N / 2) = silu(X Wg^T) * (X Wu^T) of rows that are weighted for a norm but not yet scaled: ssq (M, nssq) holds partial sums of
+// the rows' squares, nssq a multiple of four up to 128.  The products of gs_gemm_mid's epilogue 1.
+extern "C" int gs_gemm_mid_swiglu_scaled(const void* X, int ldx, const float* ssq, int nssq, float eps, const void* Wt, void* Y, int ldy,
+                                         int M, int N, int K, hipStream_t stream) {
+  GS_REQUIRE(gs_gemm_mid_takes(M, N, K, 1), "gemm_mid_swiglu_scaled: not a product of this kernel (M=%d N=%d K=%d)", M, N, K);
+  GS_REQUIRE(ldx >= K && ldx % 8 == 0 && (((uintptr_t)X | (uintptr_t)Wt | (uintptr_t)ssq) & 15) == 0,
+             "gemm_mid_swiglu_scaled: X, W and the sums must be 16-byte aligned, the row stride of X a multiple of 8");
+  GS_REQUIRE(ssq && nssq > 0 && nssq % 4 == 0 && nssq <= GD_SSQ_MAX && eps > 0.f, "gemm_mid_swiglu_scaled: %d partial sums a row, eps %g", nssq, eps);
+  GS_REQUIRE(ldy >= N / 2 && ldy % 4 == 0 && ((uintptr_t)Y & 7) == 0, "gemm_mid_swiglu_scaled: rows of Y too short or not aligned (stride %d)", ldy);
+  const bf16 *x = (const bf16*)X, *w = (const bf16*)Wt;
+  bf16* y = (bf16*)Y;
+  MidNorm norm = {};
+  norm.ssq = ssq;
+  norm.nssq = nssq;
+  norm.eps = eps;
+#define GD_RUN(BM, NT, KG) run_mid<BM, NT, KG, 1, true>(x, ldx, w, y, ldy, M, N, K, stream, 1, norm)
+  const int i = mid_choice(M, N, K, 1);
+  if (i == 0) GD_RUN(32, 2, 2); else if (i == 1) GD_RUN(64, 2, 1); else if (i == 2) GD_RUN(96, 2, 1); else GD_RUN(64, 4, 1);
+#undef GD_RUN
+  GS_LAUNCH_CHECK("gemm_mid_swiglu_scaled");
+  return 0;
+}
+
+// How many partial sums of squares a row gs_gemm_mid_residual leaves; 0: the product is not its, or they are more than the product that
+// reads them takes.
+extern "C" int gs_gemm_mid_residual_sums(int M, int N, int K) {
+  if (!gs_gemm_mid_takes(M, N, K, 0)) return 0;
+  const int sums = 4 * gs_ceil_div(N, 64 * mid_plain[mid_choice(M, N, K, 0)].nt);
+  return sums <= GD_SSQ_MAX ? sums : 0;
+}
+
+// res (M, N) += X W^T in float32; with next_weight also rows (M, N) = res * next_weight in bfloat16 and ssq
+// (M, gs_gemm_mid_residual_sums) partial sums of the new rows' squares.
+extern "C" int gs_gemm_mid_residual(const void* X, int ldx, const void* Wt, float* res, const float* next_weight, void* rows, float* ssq,
+                                    int M, int N, int K, hipStream_t stream) {
+  GS_REQUIRE(gs_gemm_mid_residual_sums(M, N, K) > 0, "gemm_mid_residual: not a product of this kernel (M=%d N=%d K=%d)", M, N, K);
+  GS_REQUIRE(ldx >= K && ldx % 8 == 0 && (((uintptr_t)X | (uintptr_t)Wt | (uintptr_t)res | (uintptr_t)next_weight) & 15) == 0 && ((uintptr_t)rows & 7) == 0,
+             "gemm_mid_residual: X, W, the stream and the weight must be 16-byte aligned, the row stride of X a multiple of 8");
+  GS_REQUIRE(res && (next_weight != nullptr) == (rows != nullptr) && (rows != nullptr) == (ssq != nullptr),
+             "gemm_mid_residual: the next norm's weight, its rows and their sums come together");
+  const bf16 *x = (const bf16*)X, *w = (const bf16*)Wt;
+  MidNorm norm = {};
+  norm.res = res;
+  norm.weight = next_weight;
+  norm.rows = (bf16*)rows;
+  norm.ssq_out = ssq;
+#define GD_RUN(BM, NT, KG) run_mid<BM, NT, KG, 3>(x, ldx, w, nullptr, 0, M, N, K, stream, 1, norm)
+  switch (mid_choice(M, N, K, 0)) {
+    case 0: GD_RUN(32, 1, 4); break;
+    case 1: GD_RUN(64, 1, 2); break;
+    case 2: GD_RUN(96, 1, 2); break;
+    case 3: GD_RUN(64, 2, 2); break;
+    default: GD_RUN(96, 2, 1); break;
+  }
+#undef GD_RUN
+  GS_LAUNCH_CHECK("gemm_mid_residual");
   return 0;
 }
 

@@ -707,6 +707,61 @@ def gemm_mid(x, w: torch.Tensor, wt, swiglu: bool = False, out: torch.Tensor = N
     return out
 
 
+@lru_cache(maxsize=4096)
+def _mid_residual_sums(M: int, N: int, K: int) -> int:
+    return lib().gs_gemm_mid_residual_sums(M, N, K)
+
+
+def mid_residual_ok(x, w: torch.Tensor, wt) -> bool:
+    """Whether :func:`gemm_mid_residual` takes the product: those of :func:`mid_ok` whose rows' squares come in few partial sums."""
+    return _mid_operands(x, w, wt) and _mid_residual_sums(x.shape[0], w.shape[0], w.shape[1]) > 0
+
+
+def gemm_mid_residual(x, w: torch.Tensor, wt, res: torch.Tensor, next_weight: torch.Tensor):
+    """``res += x @ w.T`` in place (float32) for products :func:`mid_residual_ok` takes.  Returns the new rows times
+    ``next_weight`` in bfloat16 and partial sums of their squares ``(M, sums)``."""
+    M, K = x.shape
+    N = w.shape[0]
+    sums = _mid_residual_sums(M, N, K) if _mid_operands(x, w, wt) else 0
+    if sums <= 0:
+        raise KernelError(f"gemm_mid_residual: not a product of this kernel, M={M} N={N} K={K}")
+    if not (wt.dtype is torch.bfloat16 and wt.is_cuda and wt.is_contiguous()):
+        raise KernelError("gemm_mid_residual: the weight's tile-major copy is bfloat16 on the GPU")
+    if not (res.shape == (M, N) and res.dtype is torch.float32 and res.is_cuda and res.is_contiguous()):
+        raise KernelError("gemm_mid_residual: shapes")
+    if not (next_weight.dtype is torch.float32 and next_weight.shape == (N,) and next_weight.is_cuda and next_weight.is_contiguous()):
+        raise KernelError("next_weight must be float32 (N,)")
+    rows = torch.empty((M, N), dtype=torch.bfloat16, device=res.device)
+    ssq = torch.empty((M, sums), dtype=torch.float32, device=res.device)
+    rc = lib().gs_gemm_mid_residual(x.data_ptr(), x.stride(0), wt.data_ptr(), res.data_ptr(), next_weight.data_ptr(), rows.data_ptr(),
+                                    ssq.data_ptr(), M, N, K, _stream())
+    if rc != 0:
+        _check(rc)
+    return rows, ssq
+
+
+def mid_scaled_ok(x, w13: torch.Tensor, wt) -> bool:
+    """Whether :func:`gemm_mid_swiglu_scaled` takes a lazy norm's weighted rows against gate and up."""
+    return (isinstance(x.xs, torch.Tensor) and x.ssq.shape[1] <= 128 and x.ssq.shape[1] % 4 == 0 and x.ssq.is_contiguous()
+            and mid_ok(x.xs, w13, wt, swiglu=True))
+
+
+def gemm_mid_swiglu_scaled(x, w13: torch.Tensor, wt) -> torch.Tensor:
+    """``silu(gate) * up`` in bfloat16 of a lazy norm whose rows come weighted, for products :func:`mid_scaled_ok` takes."""
+    if not mid_scaled_ok(x, w13, wt):
+        raise KernelError(f"gemm_mid_swiglu_scaled: not a product of this kernel, M={x.shape[0]} N={w13.shape[0]} K={w13.shape[1]}")
+    if not (wt.dtype is torch.bfloat16 and wt.is_cuda and wt.is_contiguous()):
+        raise KernelError("gemm_mid_swiglu_scaled: the weight's tile-major copy is bfloat16 on the GPU")
+    xs, N = x.xs, w13.shape[0]
+    M, K = xs.shape
+    out = torch.empty((M, N // 2), dtype=torch.bfloat16, device=xs.device)
+    rc = lib().gs_gemm_mid_swiglu_scaled(xs.data_ptr(), xs.stride(0), x.ssq.data_ptr(), x.ssq.shape[1], x.eps, wt.data_ptr(),
+                                         out.data_ptr(), N // 2, M, N, K, _stream())
+    if rc != 0:
+        _check(rc)
+    return out
+
+
 def mid_parts(x, w: torch.Tensor, wt) -> int:
     """Into how many parts of K :func:`gemm_mid_residual_parts` shares this product out; 0: it is not for it.  Operands as for
     :func:`mid_ok`."""

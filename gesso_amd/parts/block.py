@@ -59,7 +59,8 @@ class PreNormBlock(Part):
         with rt.stage(getattr(self.mixer, "stage", "mixer")):
             out = self.mixer.forward(x, ctx, cache)
             with rt.stage(getattr(self.mixer, "out_stage", "mixer_out")):
-                stream.push(out, rt, next_norm=self.ffn_norm if self.ffn is not None else after)
+                stream.push(out, rt, next_norm=self.ffn_norm if self.ffn is not None else after,
+                            weighted=getattr(self.ffn, "takes_weighted", False))
         if self.ffn is not None:
             with rt.stage("norm"):
                 x = self.ffn_norm.add_norm(stream)

@@ -38,11 +38,21 @@ class ResidualStream:
         self.bias = None              # a float32 vector still to be added to every row (a last product's bias, left
                                       # for the pass that adds the product itself)
 
-    def push(self, out, rt, next_norm=None) -> None:
+    def push(self, out, rt, next_norm=None, weighted: bool = False) -> None:
+        """``weighted``: whoever reads ``next_norm``'s rows takes them weighted and not yet scaled, also for more rows than
+        the weight-streaming products take."""
         from .runtime import DeferredLinear
         self.flush(rt)
         self.xs = self.xs_for = self.normed = self.rows = None
-        if isinstance(out, DeferredLinear) and out.parts:
+        if isinstance(out, DeferredLinear) and out.parts == 1:
+            # some hundred rows: straight into the stream where the rows it leaves are taken as they are
+            w = getattr(next_norm, "row_weight", None) if weighted else None
+            if w is None or w.dtype != self.res.dtype or w.shape != (self.res.shape[1],):
+                self.pending, self.ssq = rt.linear(out.x, out.w), None
+            else:
+                self.xs, self.ssq = rt.ops.gemm_mid_residual(out.x, out.w, rt.tiles_of(out.w), self.res, w)
+                self.xs_for = next_norm
+        elif isinstance(out, DeferredLinear) and out.parts:
             # some hundred rows: the same in two kernels, the rows normed by the second
             w = getattr(next_norm, "row_weight", None)
             eps = getattr(getattr(next_norm, "spec", None), "eps", None)
@@ -117,7 +127,7 @@ class RMSNorm(Part):
 
         While a decode step is recorded with fused kernels, and the stream's sums of squares are at
         hand, the norm is not run: a :class:`~gesso_amd.kernels.ops.LazyNorm` goes to the product that
-        follows, which norms on the fly.
+        follows, which norms on the fly.  So it is where the last push has left rows weighted for this norm.
         """
         if isinstance(stream.pending, tuple) or stream.bias is not None:
             held = stream.pending if isinstance(stream.pending, tuple) else (stream.pending, None)
@@ -128,8 +138,9 @@ class RMSNorm(Part):
                 stream.pending = stream.ssq = stream.xs = stream.xs_for = stream.normed = stream.rows = stream.bias = None
                 return y
             stream.flush(self.rt)
-        if self.rt.fused and rows is None and stream.pending is None and stream.ssq is not None:
-            mine = stream.xs_for is self
+        mine = stream.xs_for is self
+        if ((self.rt.fused or (mine and stream.xs is not None and out is None and out_dtype is None)) and rows is None
+                and stream.pending is None and stream.ssq is not None):
             return self.rt.ops.LazyNorm(stream.res, stream.ssq, self.weight, self.spec.eps, self.rt.dtype,
                                         xs=stream.xs if mine else None, ready=stream.normed if mine else None)
         if (not self.rt.fused and rows is None and out is None and stream.pending is None and stream.normed is not None

@@ -109,7 +109,7 @@ class DeferredLinear:
 
     def __init__(self, x, w, parts: int = 0):
         self.x, self.w = x, w
-        self.parts = parts            # into how many parts of K the product of some hundred rows is shared out
+        self.parts = parts            # into how many parts of K the product of some hundred rows is shared out (1: whole)
 
 
 class Runtime:
@@ -252,6 +252,11 @@ class Runtime:
         ops = self.ops
         tiled = self.rows_tiled(w13.shape[0] // 2)
         if isinstance(x, ops.LazyNorm):
+            if not self.fused and x.xs is not None:
+                # some hundred rows, weighted by the product before
+                wt = self.tiles_of(w13)
+                if ops.mid_scaled_ok(x, w13, wt):
+                    return ops.gemm_mid_swiglu_scaled(x, w13, wt)
             if self.keep_lazy(x) and ops.lazy_ok(x, w13):
                 return ops.gemm_skinny(x, w13, swiglu=True, wt=self.tiles_of(w13), out=tiled)
             x = x.materialize()
@@ -269,16 +274,17 @@ class Runtime:
 
     def project(self, x: torch.Tensor, w: torch.Tensor, bias=None):
         """A sub-layer's last product.  It is deferred while fused kernels are on, and for some hundred rows with a K so long
-        that it comes in parts, so that the block can compute it straight into the residual stream (:meth:`dense` computes it
-        for a block that does not); else it is computed here."""
+        that it comes in parts or where one kernel can add it to the stream, so that the block can compute it straight into the
+        residual stream (:meth:`dense` computes it for a block that does not); else it is computed here."""
         if bias is None:
             if self.fused:
                 if self.ops.skinny_ok(x, w):
                     return DeferredLinear(x, w)
             elif x.shape[0] > self.streaming_rows_max and self.many_rows == "auto" and not self.no_library:
-                parts = self.ops.mid_parts_pay(x, w, self.tiles_of(w))
-                if parts:
-                    return DeferredLinear(x, w, parts)
+                wt = self.tiles_of(w)
+                parts = self.ops.mid_parts_pay(x, w, wt)
+                if parts or self.ops.mid_residual_ok(x, w, wt):
+                    return DeferredLinear(x, w, parts or 1)
         return self.linear(x, w, bias)
 
     # ------------------------------------------------------------------ handles between fused kernels

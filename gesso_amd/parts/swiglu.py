@@ -16,6 +16,7 @@ class SwiGLU(Part):
     graph_safe = True
     portions_recordable = True
     stage, out_stage = "dense_ffn", "ffn_down"        # the decode profiler's names
+    takes_weighted = True                             # a lazy norm goes straight to ``linear_swiglu``
 
     @staticmethod
     def tensor_specs(spec):
