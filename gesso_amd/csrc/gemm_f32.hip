@@ -18,9 +18,12 @@
 // FMAs, a lane a chunk.  With a K of a chunk or two most of a block of eight wavefronts has nothing to do, and there are many blocks
 // (1 row, 65536 x 64: 20 us, by lanes 6.6); with few weight rows and a long K there are too few blocks to hide the chain.
 //
-// Many rows: gemm_f32_tiles_kernel.  The matrix cores bind (157 TFLOP/s): a block owns 32 MT x 32 NT outputs, its four
-// wavefronts (two by two) MT x NT tiles of 16 x 16 each; the operands of the next 32 k are loaded under the products of
-// these.
+// Many rows: gemm_f32_tiles_kernel.  The matrix cores bind (157 TFLOP/s): a block's 2 x WN wavefronts own MT x NT tiles of 16 x 16
+// each.  A wavefront always has products to issue: rows are asked for two steps of 32 k ahead (or four), the next step's rows go to LDS half
+// way through a step, operands are read from LDS under the products of the k before, and the step's barrier stands before its last
+// products, with the next step's first operands asked for behind it.  (Written without fences between these, the compiler moved
+// the loads down to where their values are stored: 680 rows of 2048 x 8192 292 us, now 231.)  32 x 32 x 2 instructions give the same
+// chains and, alone, 3 % more; with their operands through LDS they were slower (2,048 rows of 16384 x 2048 1,130 us, these 1,050).
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(4))) float gf_f32x4_t;
@@ -208,81 +211,128 @@ __global__ __launch_bounds__(GF_LANES_WAVES * 64) void gemm_f32_lanes_kernel(con
   }
 }
 
-template <int MT, int NT, bool TAIL, typename TO>
-__global__ __launch_bounds__(256) void gemm_f32_tiles_kernel(const float* __restrict__ X, int ldx,
-                                                             const float* __restrict__ W,
-                                                             const float* __restrict__ bias, TO* __restrict__ Y, int ldy,
-                                                             int M, int N, int K) {
-  constexpr int KS = 32, LD = KS + 4, BM = 32 * MT, BN = 32 * NT;
-  __shared__ float xs[2][BM * LD], ws[2][BN * LD];
+// SHORT: a K of one chunk, whose rows are all asked for at once (333 rows of 2048 x 48 6.3 us as of a longer K, 5.2 here).
+template <int WN, int MT, int NT, bool TAIL, bool SHORT, typename TO>
+__global__ __launch_bounds__(WN * 128, WN == 2 ? 2 : 1) void gemm_f32_tiles_kernel(const float* __restrict__ X, int ldx,
+                                                                                   const float* __restrict__ W,
+                                                                                   const float* __restrict__ bias, TO* __restrict__ Y,
+                                                                                   int ldy, int M, int N, int K) {
+  constexpr int KS = 32, LD = KS + 4, BM = 32 * MT, BN = 16 * NT * WN, RPL = WN * 16;       // RPL: rows the block loads at a time
+  constexpr int LX = (BM + RPL - 1) / RPL, LW = (BN + RPL - 1) / RPL;
+  constexpr int G = MT * NT >= 4 ? 1 : MT * NT == 1 ? 4 : 2, NG = KS / 4 / G;               // fours of k read from LDS at a time
+  __shared__ __align__(16) float xs[2][BM * LD], ws[2][BN * LD];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, g = lane >> 4;
-  // (row tiles fastest, all in x: it takes as many tiles as there can be, y only 65,535)
+  // (row tiles fastest, all in x: it takes as many tiles as there can be, y only 65,535; the blocks of an XCD, every eighth, are
+  // neighbours, which share rows of W and X in its L2)
   const int tiles_m = (M + BM - 1) / BM;
-  const int mb = (int)(blockIdx.x % tiles_m) * BM, nb = (int)(blockIdx.x / tiles_m) * BN, mw = (wave & 1) * 16 * MT, nw = (wave >> 1) * 16 * NT;
-  // thread t loads the four k at 4 (t % 8) of row t / 8, 32 rows a load
+  const unsigned per = gridDim.x >> 3, rest = gridDim.x & 7, xcd = blockIdx.x & 7;
+  const unsigned tile = xcd * per + (xcd < rest ? xcd : rest) + (blockIdx.x >> 3);
+  const int mb = (int)(tile % tiles_m) * BM, nb = (int)(tile / tiles_m) * BN, mw = (wave & 1) * 16 * MT, nw = (wave >> 1) * 16 * NT;
+  // thread t loads the four k at 4 (t % 8) of row t / 8, RPL rows a load
   const int lr = threadIdx.x >> 3, lk = 4 * (threadIdx.x & 7);
-  const float* xp[MT];
-  const float* wp[NT];
+  const float* xp[LX];
+  const float* wp[LW];
 #pragma unroll
-  for (int i = 0; i < MT; ++i) xp[i] = X + (size_t)(mb + 32 * i + lr < M ? mb + 32 * i + lr : M - 1) * ldx;
+  for (int i = 0; i < LX; ++i) xp[i] = X + (size_t)(mb + RPL * i + lr < M ? mb + RPL * i + lr : M - 1) * ldx;
 #pragma unroll
-  for (int j = 0; j < NT; ++j) wp[j] = W + (size_t)(nb + 32 * j + lr < N ? nb + 32 * j + lr : N - 1) * K;
-  gf_f32x4_t xr[MT], wr[NT];
-  auto load = [&](int k) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < MT; ++i) xr[i] = gf_load<TAIL>(xp[i], k + lk, K);
-#pragma unroll
-    for (int j = 0; j < NT; ++j) wr[j] = gf_load<TAIL>(wp[j], k + lk, K);
+  for (int j = 0; j < LW; ++j) wp[j] = W + (size_t)(nb + RPL * j + lr < N ? nb + RPL * j + lr : N - 1) * K;
+  struct Rows {
+    gf_f32x4_t x[LX], w[LW];
   };
-  auto put = [&](int s) __attribute__((always_inline)) {
+  constexpr int D = !SHORT && MT * NT == 1 ? 4 : 2;        // steps under way (blocks this small stand alone: 32 rows of 6144 x 2048 24.5, 22.0)
+  Rows rows[D];
+  auto load = [&](Rows& v, int k) __attribute__((always_inline)) {
+    const int from = (TAIL ? k + lk : k) < K ? k + lk : (TAIL ? 0 : lk);      // (what lies beyond K is not used)
 #pragma unroll
-    for (int i = 0; i < MT; ++i) *reinterpret_cast<gf_f32x4_t*>(&xs[s][(32 * i + lr) * LD + lk]) = xr[i];
+    for (int i = 0; i < LX; ++i) v.x[i] = gf_load<false>(xp[i], from, K);
 #pragma unroll
-    for (int j = 0; j < NT; ++j) *reinterpret_cast<gf_f32x4_t*>(&ws[s][(32 * j + lr) * LD + lk]) = wr[j];
+    for (int j = 0; j < LW; ++j) v.w[j] = gf_load<false>(wp[j], from, K);
+  };
+  // the rows at k into buffer s: zeros beyond K (told only here, where the values have to be there)
+  auto put = [&](const Rows& v, int s, int k) __attribute__((always_inline)) {
+    const bool in = !TAIL || k + lk < K;
+    const gf_f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < LX; ++i)
+      if (BM % RPL == 0 || RPL * i + lr < BM) *reinterpret_cast<gf_f32x4_t*>(&xs[s][(RPL * i + lr) * LD + lk]) = in ? v.x[i] : zero;
+#pragma unroll
+    for (int j = 0; j < LW; ++j)
+      if (BN % RPL == 0 || RPL * j + lr < BN) *reinterpret_cast<gf_f32x4_t*>(&ws[s][(RPL * j + lr) * LD + lk]) = in ? v.w[j] : zero;
   };
   gf_f32x4_t acc[MT][NT], tot[MT][NT];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int j = 0; j < NT; ++j) tot[i][j] = gf_f32x4_t{0.f, 0.f, 0.f, 0.f};
-  auto multiply = [&](int s, bool first) __attribute__((always_inline)) {
-    const float* x = &xs[s][(mw + r16) * LD + g];
-    const float* w = &ws[s][(nw + r16) * LD + g];
+    for (int j = 0; j < NT; ++j) acc[i][j] = tot[i][j] = gf_f32x4_t{0.f, 0.f, 0.f, 0.f};
+  struct Operands {
+    float x[G][MT], w[G][NT];
+  };
+  Operands held[2];
+  auto read = [&](Operands& o, int s, int q) __attribute__((always_inline)) {
+    const float* x = &xs[s][(mw + r16) * LD + g + 4 * G * q];
+    const float* w = &ws[s][(nw + r16) * LD + g + 4 * G * q];
 #pragma unroll
-    for (int q = 0; q < KS / 4; ++q) {
-      float a[MT], b[NT];
+    for (int u = 0; u < G; ++u) {
 #pragma unroll
-      for (int i = 0; i < MT; ++i) a[i] = x[16 * i * LD + 4 * q];
+      for (int i = 0; i < MT; ++i) o.x[u][i] = x[16 * i * LD + 4 * u];
 #pragma unroll
-      for (int j = 0; j < NT; ++j) b[j] = w[16 * j * LD + 4 * q];
+      for (int j = 0; j < NT; ++j) o.w[u][j] = w[16 * j * LD + 4 * u];
+    }
+  };
+  // (first: of a chunk; what the last chunk left is added before its sum begins)
+  auto multiply = [&](const Operands& o, bool first) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < G; ++u)
 #pragma unroll
       for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-          const gf_f32x4_t c = first && q == 0 ? gf_f32x4_t{0.f, 0.f, 0.f, 0.f} : acc[i][j];
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[j], a[i], c, 0, 0, 0);
+          gf_f32x4_t c = acc[i][j];
+          if (first && u == 0) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) tot[i][j][e] += c[e];
+            c = gf_f32x4_t{0.f, 0.f, 0.f, 0.f};
+          }
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.w[u][j], o.x[u][i], c, 0, 0, 0);
         }
-    }
   };
-  load(0);
-  put(0);
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (!SHORT || d * KS < K) load(rows[d], d * KS);
+  put(rows[0], 0, 0);
   __syncthreads();
-  for (int k = 0; k < K; k += GS_SUM_CHUNK) {     // a chunk: two steps of 32 k (beyond K: zeros)
-    load(TAIL || k + KS < K ? k + KS : k);
-    multiply(0, true);
-    put(1);
+  read(held[0], 0, 0);
+  // the step at k from buffer s.  Nothing of buffer s is read behind the step's barrier, where the next step's rows may replace it
+  auto step = [&](int s, int k, Rows& later, const Rows& next, bool first) __attribute__((always_inline)) {
+    if (!SHORT) load(later, k + D * KS);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < NG - 1; ++q) {
+      read(held[(q + 1) & 1], s, q + 1);
+      if (q == (NG - 1) / 2) put(next, s ^ 1, k + KS);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(held[q & 1], first && q == 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     __syncthreads();
-    load(TAIL || k + 2 * KS < K ? k + 2 * KS : k);    // (after the last chunk: loaded and not used)
-    multiply(1, false);
-    put(0);
-    __syncthreads();
+    read(held[0], s ^ 1, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(held[(NG - 1) & 1], false);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  for (int k = 0; k < K;) {
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-      for (int j = 0; j < NT; ++j)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) tot[i][j][e] += acc[i][j][e];
+    for (int d = 0; d < D && k < K; d += 2, k += GS_SUM_CHUNK) {      // a chunk: two steps of 32 k (beyond K: zeros)
+      step(0, k, rows[d], rows[d + 1], true);
+      step(1, k + KS, rows[d + 1], rows[(d + 2) % D], false);
+    }
   }
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) tot[i][j][e] += acc[i][j][e];
   // element e of lane l: row 4 (l / 16) + e of W, row l % 16 of X
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
@@ -355,14 +405,56 @@ static void run_lanes(const float* X, int ldx, const float* W, const float* bias
   gemm_f32_lanes_kernel<MB, TO><<<blocks, GF_LANES_WAVES * 64, 0, stream>>>(X, ldx, W, bias, Y, ldy, M, N, K, span);
 }
 
-template <int MT, int NT, typename TO>
+template <int WN, int MT, int NT, typename TO>
 static void run_tiles(const float* X, int ldx, const float* W, const float* bias, TO* Y, int ldy, int M, int N, int K,
                       hipStream_t stream) {
-  const unsigned grid = (unsigned)gs_ceil_div(M, 32 * MT) * (unsigned)gs_ceil_div(N, 32 * NT);
-  if (K % GS_SUM_CHUNK == 0)
-    gemm_f32_tiles_kernel<MT, NT, false, TO><<<grid, 256, 0, stream>>>(X, ldx, W, bias, Y, ldy, M, N, K);
-  else
-    gemm_f32_tiles_kernel<MT, NT, true, TO><<<grid, 256, 0, stream>>>(X, ldx, W, bias, Y, ldy, M, N, K);
+  const unsigned grid = (unsigned)gs_ceil_div(M, 32 * MT) * (unsigned)gs_ceil_div(N, 16 * NT * WN);
+  auto kernel = K <= GS_SUM_CHUNK         ? &gemm_f32_tiles_kernel<WN, MT, NT, true, true, TO>
+                : K % GS_SUM_CHUNK == 0 ? &gemm_f32_tiles_kernel<WN, MT, NT, false, false, TO>
+                                        : &gemm_f32_tiles_kernel<WN, MT, NT, true, false, TO>;
+  kernel<<<grid, WN * 128, 0, stream>>>(X, ldx, W, bias, Y, ldy, M, N, K);
+}
+
+// Which tiles: those whose rounds of blocks take the least.  A round (a block for each of the 256 compute units) of so many rows of
+// X by so many of W takes `each` tenths of a microsecond for 2,048 k, whether blocks run beside or after one another, the first
+// `first` more.  (Measured on cold weights; microseconds by this and by the rule and kernel before: 680 rows of 2048 x 2048 64 and
+// 78, 6144 x 2048 172 and 205, 16384 x 2048 380 and 425, 2048 x 8192 230 and 292; 100 rows of 2048 x 2048 20 and 41, x 8192 80 and
+// 178; 2,048 rows of 16384 x 2048 1,050 and 1,100, of 2048 x 8192 517 and 570.)
+struct Tiles {
+  int rows, cols, first, each;
+};
+static const Tiles f32_tiles[] = {{64, 128, 80, 650}, {96, 64, 80, 535}, {64, 64, 105, 345}, {32, 64, 70, 195}, {32, 32, 85, 112}};
+
+static int tiles_choice(int M, int N, int K) {
+  // (a chunk or two are over before rounds are: the largest of the smaller tiles that make two blocks a compute unit; 2,100 rows of
+  // 8192 x 64 by 64 x 128 59.8 us, by 64 x 64 49)
+  if (K <= 2 * GS_SUM_CHUNK)
+    return (long)gs_ceil_div(M, 64) * gs_ceil_div(N, 64) >= 512 ? 2 : (long)gs_ceil_div(M, 32) * gs_ceil_div(N, 64) >= 512 ? 3 : 4;
+  int best = 0;
+  long least = 0;
+  for (int i = 0; i < 5; ++i) {
+    const long blocks = (long)gs_ceil_div(M, f32_tiles[i].rows) * gs_ceil_div(N, f32_tiles[i].cols);
+    const long takes = f32_tiles[i].first + (blocks + 255) / 256 * f32_tiles[i].each;
+    if (i == 0 || takes < least) {
+      least = takes;
+      best = i;
+    }
+  }
+  return best;
+}
+
+template <typename TO>
+static void run_chosen_tiles(const float* X, int ldx, const float* W, const float* bias, TO* Y, int ldy, int M, int N, int K,
+                             hipStream_t stream) {
+#define GF_TILES(WN, MT, NT) return run_tiles<WN, MT, NT, TO>(X, ldx, W, bias, Y, ldy, M, N, K, stream)
+  switch (tiles_choice(M, N, K)) {
+    case 0: GF_TILES(4, 2, 2);
+    case 1: GF_TILES(4, 3, 1);
+    case 2: GF_TILES(2, 2, 2);
+    case 3: GF_TILES(2, 1, 2);
+    default: GF_TILES(2, 1, 1);
+  }
+#undef GF_TILES
 }
 
 // Which kernel, by sizes (microseconds on cold weights, one MI355X; the FMA kernels that ran before: 63 on average for the
@@ -371,13 +463,12 @@ static void run_tiles(const float* X, int ldx, const float* W, const float* bias
 // Up to 16 rows: blocks of 8 rows of W up to N = 8192, which then still are no more than four a compute unit (6 rows,
 //   2048 x 8192: 21.8, blocks of 16 rows 30.7; 6144 x 2048: 15.1 and 17.2); of 16 rows beyond (65536 x 2048: 118 and 121;
 //   16 rows: 129 and 135).
-// Up to 64 rows: every block of the rows kernel reads all rows of X for its few of W, so wide weights go to the tiles (40 rows,
-//   16384 x 2048: tiles of 32 x 32 70, rows 112; 65536: tiles of 64 x 64 178, rows 432), narrow ones do not fill the chip
-//   there (2048 x 8192: rows 70, tiles of 32 x 32 195).  Nor do wavefronts that share out one chunk fill a block of the rows kernel
-//   (64 rows of 8192 x 36 21.3, tiles 4.0; of 100 x 16 6.6 and 3.0).
-// More: the largest tiles that make two blocks a compute unit (680 rows: 2048 x 8192 by 64 x 64 333, 32 x 64 280; 16384 x 2048
-//   442 and 475; 300 rows, 2048 x 2048: 64 x 64 79, 32 x 64 67, 32 x 32 55; larger ones than 64 x 64 were slower everywhere,
-//   2,048 rows included).
+// Up to 64 rows: every block of the rows kernel reads all rows of X for its few of W, so wide weights go to the tiles (rows kernel and
+//   tiles; 32 rows: 4096 x 2048 14.3 and 19.1, 5120 x 2048 25.1 and 22.0, 6144 x 512 10.9 and 7.0; 64 rows: 3072 x 2048 23.0 and 19.5,
+//   8192 x 2048 51 and 30; 40 rows: 3072 x 1024 9.8 and 10.9), narrow ones do not fill the chip there (64 rows of 2048 x 2048 18.4 and 18.8, of 2048 x 8192 63 and 80).
+//   Nor do wavefronts that share out one chunk fill a block of the rows kernel (64 rows of 8192 x 36 21.3, tiles 4.0; of 100 x 16 6.6
+//   and 3.0).
+// More: tiles.
 //
 // Whether a lane a chunk.  Long K (up to 8192): one or two rows, N up to 1024, K above 2048 (one row of 1024 x 4608 on cold weights
 // 11.9, rows kernel 12.8; of 1024 x 8192 16.1 and 20.7, two rows 19.6 and 20.6; beyond 1024, one row of 1152 x 5120: 18.0 and 14.2);
@@ -410,7 +501,6 @@ template <typename TO>
 static void run(const float* X, int ldx, const float* W, const float* bias, TO* Y, int ldy, int M, int N, int K,
                 hipStream_t stream) {
 #define GF_ROWS(WR, XR) return run_rows<WR, XR, 2, TO>(X, ldx, W, bias, Y, ldy, M, N, K, stream)
-#define GF_TILES(MT, NT) return run_tiles<MT, NT, TO>(X, ldx, W, bias, Y, ldy, M, N, K, stream)
 #define GF_LANES(MB) return run_lanes<MB, TO>(X, ldx, W, bias, Y, ldy, M, N, K, stream)
   if (lanes_take(M, N, K)) {
     if (M == 1) GF_LANES(1);
@@ -419,7 +509,6 @@ static void run(const float* X, int ldx, const float* W, const float* bias, TO* 
     if (M <= 8) GF_LANES(8);
     GF_LANES(16);
   }
-  const long by64 = (long)gs_ceil_div(M, 64) * gs_ceil_div(N, 64), by32x64 = (long)gs_ceil_div(M, 32) * gs_ceil_div(N, 64);
   if (M <= 16) {
     if (N <= 8192) {
       if (M <= 4) GF_ROWS(8, 4);
@@ -431,23 +520,16 @@ static void run(const float* X, int ldx, const float* W, const float* bias, TO* 
     GF_ROWS(16, 16);
   }
   if (M <= 64) {
-    if (by64 >= 1024) GF_TILES(2, 2);
-    if (N > 8192 || K <= GS_SUM_CHUNK) GF_TILES(1, 1);
-    if (N <= 2048) {
-      if (M <= 32) GF_ROWS(8, 32);
-      if (M <= 48) GF_ROWS(8, 48);
-      GF_ROWS(8, 64);
-    }
-    if (M <= 32) GF_ROWS(16, 32);
-    if (M <= 48) GF_ROWS(16, 48);
-    GF_ROWS(16, 64);
+    const bool rows = K > GS_SUM_CHUNK && N <= (M <= 32 ? 4096 : M <= 48 && K <= 1024 ? 3072 : 2048);
+    if (rows && N > 2048 && M <= 32) GF_ROWS(16, 32);
+    if (rows && N > 2048) GF_ROWS(16, 48);
+    if (rows && M <= 32) GF_ROWS(8, 32);
+    if (rows && M <= 48) GF_ROWS(8, 48);
+    if (rows) GF_ROWS(8, 64);
   }
-  if (by64 >= 512) GF_TILES(2, 2);
-  if (by32x64 >= 512) GF_TILES(1, 2);
-  GF_TILES(1, 1);
+  run_chosen_tiles<TO>(X, ldx, W, bias, Y, ldy, M, N, K, stream);
 #undef GF_LANES
 #undef GF_ROWS
-#undef GF_TILES
 }
 
 extern "C" int gs_gemm_f32(const float* X, int ldx, const float* W, const float* bias, void* Y, int y_dtype, int ldy,
