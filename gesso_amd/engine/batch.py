@@ -70,6 +70,10 @@ class BatchContext:
     # (``recording.subtiles``) and hands it what must run anew at every replay (``recording.eager``).
     recording = None
 
+    # Set by a block while its mixer runs, where what reads the stream next takes rows weighted for their norm: of how many
+    # rows it does so (``takes_weighted(rows)``), and that the block takes a last product that is still to be computed.
+    takes_weighted = None
+
     def _set(self, storage, **fields) -> None:
         if set(fields) != set(CONTEXT_FIELDS):
             missing, unknown = set(CONTEXT_FIELDS) - set(fields), set(fields) - set(CONTEXT_FIELDS)

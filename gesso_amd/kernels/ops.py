@@ -658,7 +658,7 @@ def gemm_tiled(x: torch.Tensor, w: torch.Tensor, bias=None, out_dtype=None, out:
 
 
 @lru_cache(maxsize=4096)
-def _mid_takes(M: int, N: int, K: int, swiglu: bool) -> bool:
+def mid_takes(M: int, N: int, K: int, swiglu: bool) -> bool:
     return bool(lib().gs_gemm_mid_takes(M, N, K, 1 if swiglu else 0))
 
 
@@ -685,7 +685,7 @@ def _mid_operands(x, w: torch.Tensor, wt) -> bool:
 def mid_ok(x, w: torch.Tensor, wt, swiglu: bool = False, out: torch.Tensor = None) -> bool:
     """Whether the product of some hundred rows is the kernel's that reads the weight's tile-major copy ``wt``: operands as
     :func:`_mid_operands` has them, an ``out`` the kernel can write, and sizes for which it is the faster one."""
-    return (_mid_operands(x, w, wt) and _mid_takes(x.shape[0], w.shape[0], w.shape[1], swiglu)
+    return (_mid_operands(x, w, wt) and mid_takes(x.shape[0], w.shape[0], w.shape[1], swiglu)
             and (out is None or (out.is_cuda and out.dtype == torch.bfloat16
                                  and out.shape == (x.shape[0], w.shape[0] // 2 if swiglu else w.shape[0])
                                  and out.stride(1) == 1 and out.stride(0) >= out.shape[1] and out.stride(0) % 4 == 0

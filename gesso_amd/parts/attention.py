@@ -138,7 +138,7 @@ class Attention(Part):
                                            + s.n_kv_heads * self.value_dim, self.out_gate)
         if out_dtype is not None:
             return self.rt.linear(o, self.wo, self.bo, out_dtype=out_dtype)
-        return self.rt.project(o, self.wo, self.bo)
+        return self.rt.project(o, self.wo, self.bo, getattr(ctx, "takes_weighted", None))
 
     # ------------------------------------------------------------------ the mixer's inner steps
 

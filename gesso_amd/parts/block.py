@@ -57,10 +57,13 @@ class PreNormBlock(Part):
         # a stage per kind of mixer (the profiler's names: conv_mixer, attn_mixer, ...); a sub-layer's last product
         # runs inside push, straight into the stream, and belongs to its stage
         with rt.stage(getattr(self.mixer, "stage", "mixer")):
-            out = self.mixer.forward(x, ctx, cache)
+            ctx.takes_weighted = weighted = getattr(self.ffn, "takes_weighted", None)
+            try:
+                out = self.mixer.forward(x, ctx, cache)
+            finally:
+                ctx.takes_weighted = None
             with rt.stage(getattr(self.mixer, "out_stage", "mixer_out")):
-                stream.push(out, rt, next_norm=self.ffn_norm if self.ffn is not None else after,
-                            weighted=getattr(self.ffn, "takes_weighted", False))
+                stream.push(out, rt, next_norm=self.ffn_norm if self.ffn is not None else after, weighted=weighted)
         if self.ffn is not None:
             with rt.stage("norm"):
                 x = self.ffn_norm.add_norm(stream)

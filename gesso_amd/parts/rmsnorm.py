@@ -38,15 +38,15 @@ class ResidualStream:
         self.bias = None              # a float32 vector still to be added to every row (a last product's bias, left
                                       # for the pass that adds the product itself)
 
-    def push(self, out, rt, next_norm=None, weighted: bool = False) -> None:
-        """``weighted``: whoever reads ``next_norm``'s rows takes them weighted and not yet scaled, also for more rows than
-        the weight-streaming products take."""
+    def push(self, out, rt, next_norm=None, weighted=None) -> None:
+        """``weighted(rows)``: whether whoever reads ``next_norm``'s rows takes that many weighted and not yet scaled, more
+        than the weight-streaming products take."""
         from .runtime import DeferredLinear
         self.flush(rt)
         self.xs = self.xs_for = self.normed = self.rows = None
         if isinstance(out, DeferredLinear) and out.parts == 1:
             # some hundred rows: straight into the stream where the rows it leaves are taken as they are
-            w = getattr(next_norm, "row_weight", None) if weighted else None
+            w = getattr(next_norm, "row_weight", None) if weighted is not None and weighted(self.res.shape[0]) else None
             if w is None or w.dtype != self.res.dtype or w.shape != (self.res.shape[1],):
                 self.pending, self.ssq = rt.linear(out.x, out.w), None
             else:

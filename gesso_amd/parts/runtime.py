@@ -272,10 +272,15 @@ class Runtime:
                 return ops.gemm_mid(x, w13, wt, swiglu=True, checked=True)
         return ops.swiglu(self.linear(x, w13))
 
-    def project(self, x: torch.Tensor, w: torch.Tensor, bias=None):
+    def swiglu_takes_weighted(self, rows: int, w13: torch.Tensor) -> bool:
+        """Whether :meth:`linear_swiglu` takes that many rows (some hundred) weighted for their norm and not yet scaled."""
+        return self.tiles_of(w13) is not None and self.ops.mid_takes(rows, w13.shape[0], w13.shape[1], True)
+
+    def project(self, x: torch.Tensor, w: torch.Tensor, bias=None, weighted=None):
         """A sub-layer's last product.  It is deferred while fused kernels are on, and for some hundred rows with a K so long
-        that it comes in parts or where one kernel can add it to the stream, so that the block can compute it straight into the
-        residual stream (:meth:`dense` computes it for a block that does not); else it is computed here."""
+        that it comes in parts, so that the block can compute it straight into the residual stream (:meth:`dense` computes it for
+        a block that does not); else it is computed here.  ``weighted(rows)``: whether the block's next reader takes that many
+        rows weighted for their norm: then some hundred rows are deferred for one kernel as well."""
         if bias is None:
             if self.fused:
                 if self.ops.skinny_ok(x, w):
@@ -283,7 +288,7 @@ class Runtime:
             elif x.shape[0] > self.streaming_rows_max and self.many_rows == "auto" and not self.no_library:
                 wt = self.tiles_of(w)
                 parts = self.ops.mid_parts_pay(x, w, wt)
-                if parts or self.ops.mid_residual_ok(x, w, wt):
+                if parts or (weighted is not None and weighted(x.shape[0]) and self.ops.mid_residual_ok(x, w, wt)):
                     return DeferredLinear(x, w, parts or 1)
         return self.linear(x, w, bias)
 

@@ -43,7 +43,7 @@ class ShortConv(Part):
 
     def forward(self, x, ctx, cache):
         mixed = self.mix(x, ctx, cache.state["history"])
-        return self.rt.project(mixed, self.w_out, self.b_out)
+        return self.rt.project(mixed, self.w_out, self.b_out, getattr(ctx, "takes_weighted", None))
 
     def mix(self, x, ctx, state):
         """Input product and gated short convolution: ``(T, H)`` mixed rows; ``state`` is advanced.

@@ -16,7 +16,6 @@ class SwiGLU(Part):
     graph_safe = True
     portions_recordable = True
     stage, out_stage = "dense_ffn", "ffn_down"        # the decode profiler's names
-    takes_weighted = True                             # a lazy norm goes straight to ``linear_swiglu``
 
     @staticmethod
     def tensor_specs(spec):
@@ -30,6 +29,10 @@ class SwiGLU(Part):
             w1, w3 = w1.float(), w3.float()
         self.w13 = self.rt.prepare(torch.cat([w1, w3], 0).contiguous(), unit=w1.shape[0])
         self.w2 = self.rt.prepare(tensors["w2.weight"])
+
+    def takes_weighted(self, rows: int) -> bool:
+        """Whether that many rows may come weighted for their norm and not yet scaled."""
+        return self.rt.swiglu_takes_weighted(rows, self.w13)
 
     def forward(self, x, ctx):
         with self.rt.stage("ffn_gateup"):                # with its activation where the kernel fuses them
