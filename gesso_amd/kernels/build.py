@@ -1,7 +1,8 @@
 """Compiling and loading the HIP extension.
 
 The kernels under ``gesso_amd/csrc`` are compiled with ``hipcc`` for gfx950 into one shared
-library with a C interface and loaded through ``ctypes``.  The library lies in the tree
+library with a C interface and loaded through ``ctypes``; ``host.cpp``, the launches a step makes most
+without the interpreter between check and launch, becomes a Python module beside it.  Both lie in the tree
 (``gesso_amd/_lib``) when that folder can be written, else in a per-user temporary folder.
 A digest of the sources and flags lies beside it; a library whose digest differs is built
 again.  Nothing here falls back to another implementation: if the library cannot be built
@@ -11,14 +12,18 @@ from __future__ import annotations
 
 import ctypes
 import hashlib
+import importlib.util
 import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 import threading
 import time
 from concurrent.futures import ThreadPoolExecutor
+
+import torch
 
 from ..errors import KernelError
 
@@ -32,8 +37,17 @@ FLAGS = ["--offload-arch=" + ARCH, "-O3", "-fPIC", "-std=c++17", "-Xclang", "-ta
 # the vendor's matrix product library (products of many rows, library_gemm.hip)
 LINK = ["-lhipblaslt"]
 
+# the module of host.cpp: compiled against the interpreter and the torch that import it
+HOST_NAME = "gesso_host"
+_TORCH = os.path.dirname(torch.__file__)
+HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+              "-isystem", os.path.join(_TORCH, "include"), "-isystem", os.path.join(_TORCH, "include", "torch", "csrc", "api", "include"),
+              "-isystem", sysconfig.get_paths()["include"]]
+HOST_LINK = ["-L" + os.path.join(_TORCH, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10", "-ldl"]
+
 _lock = threading.Lock()
 _lib = None
+_host = None
 
 
 def sources():
@@ -42,9 +56,9 @@ def sources():
 
 def _digest() -> str:
     h = hashlib.sha256()
-    h.update(" ".join(FLAGS + LINK).encode())
+    h.update(" ".join(FLAGS + LINK + [torch.__version__, sys.version]).encode())
     for name in sorted(os.listdir(CSRC)):
-        if name.endswith((".hip", ".h")):
+        if name.endswith((".hip", ".h", ".cpp")):
             h.update(name.encode())
             with open(os.path.join(CSRC, name), "rb") as f:
                 h.update(f.read())
@@ -57,6 +71,13 @@ def _hipcc() -> str:
         if cand and os.path.exists(cand):
             return cand
     raise KernelError("hipcc not found: the HIP extension cannot be built (set HIPCC or ROCM_PATH)")
+
+
+def _cxx() -> str:
+    for cand in (shutil.which("g++"), os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "clang++")):
+        if cand and os.path.exists(cand):
+            return cand
+    raise KernelError("no C++ compiler found: the host module cannot be built")
 
 
 def _lib_dirs():
@@ -90,7 +111,8 @@ def build(force: bool = True, verbose: bool = True) -> str:
         raise KernelError("no writable folder for the HIP extension", tried=_lib_dirs())
     lib = os.path.join(out_dir, LIB_NAME)
     stamp = lib + ".digest"
-    if not force and os.path.exists(lib) and os.path.exists(stamp) and open(stamp).read().strip() == digest:
+    if (not force and os.path.exists(lib) and os.path.exists(_host_path(lib)) and os.path.exists(stamp)
+            and open(stamp).read().strip() == digest):
         return lib
     hipcc = _hipcc()
     obj_dir = os.path.join(out_dir, "obj")
@@ -112,9 +134,22 @@ def build(force: bool = True, verbose: bool = True) -> str:
             _say(f"  {name} done ({time.time() - t0:.0f} s)")
         return obj
 
+    def compile_host():
+        path = _host_path(lib)
+        tmp = path + f".tmp{os.getpid()}"
+        p = subprocess.run([_cxx()] + HOST_FLAGS + ["-o", tmp, os.path.join(CSRC, "host.cpp")] + HOST_LINK,
+                           stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, env=env)
+        if p.returncode != 0:
+            raise KernelError(f"compiling the host module failed:\n{p.stdout[-4000:]}")
+        os.replace(tmp, path)
+        if verbose:
+            _say(f"  host.cpp done ({time.time() - t0:.0f} s)")
+
     workers = max(1, min(len(srcs), int(os.environ.get("MAX_JOBS", "0")) or (os.cpu_count() or 4), 16))
     with ThreadPoolExecutor(workers) as pool:
+        host = pool.submit(compile_host)
         objs = list(pool.map(compile_one, srcs))
+        host.result()
     tmp = lib + f".tmp{os.getpid()}"
     p = subprocess.run([hipcc, "--offload-arch=" + ARCH, "-shared", "-fPIC", "-o", tmp] + objs + LINK,
                        stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, env=env)
@@ -128,6 +163,10 @@ def build(force: bool = True, verbose: bool = True) -> str:
     return lib
 
 
+def _host_path(lib: str) -> str:
+    return os.path.join(os.path.dirname(lib), HOST_NAME + ".so")
+
+
 def find_built():
     """Path of a library whose digest matches the sources, or None."""
     digest = _digest()
@@ -135,7 +174,7 @@ def find_built():
         lib = os.path.join(d, LIB_NAME)
         stamp = lib + ".digest"
         try:
-            if os.path.exists(lib) and open(stamp).read().strip() == digest:
+            if os.path.exists(lib) and os.path.exists(_host_path(lib)) and open(stamp).read().strip() == digest:
                 return lib
         except OSError:
             continue
@@ -170,6 +209,24 @@ def entry_points():
                     types.append(_C_TYPES[words[0]])
             out[fn] = (ctypes.c_char_p if "char" in res else (ctypes.c_long if res == "long" else ctypes.c_int), types)
     return out
+
+
+def load_host():
+    """The module of ``host.cpp``, bound to the loaded library."""
+    global _host
+    lib = load()
+    with _lock:
+        if _host is None:
+            path = _host_path(lib._name)
+            try:
+                spec = importlib.util.spec_from_file_location(HOST_NAME, path)
+                host = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(host)
+                host.bind(lib._name, KernelError)
+            except (ImportError, OSError) as err:
+                raise KernelError(f"cannot load the host module {path}: {err}") from err
+            _host = host
+        return _host
 
 
 def load() -> ctypes.CDLL:

@@ -28,6 +28,18 @@ def lib():
     return _lib
 
 
+_host = None
+
+
+def _native():
+    """The module of launches made without the interpreter (``csrc/host.cpp``): its functions return False for a call that is not
+    in their plain form, which the functions here then check, word and make themselves."""
+    global _host
+    if _host is None:
+        _host = _build.load_host()
+    return _host
+
+
 def _dt(t: torch.Tensor) -> int:
     d = t.dtype
     if d is torch.bfloat16:
@@ -72,6 +84,12 @@ def _dev(*ts):
             raise KernelError("kernel operands must live on the GPU" if not t.is_cuda else "kernel operands must be contiguous")
 
 
+def _tile_rows(tiles):
+    """The addresses of the three rows of contiguous int32 tiles ``(3, n)``."""
+    at, row = tiles.data_ptr(), 4 * tiles.shape[1]
+    return at, at + row, at + 2 * row
+
+
 def _i32(t, n=None, what="index"):
     if t.dtype != torch.int32:
         raise KernelError(f"{what} must be int32, got {t.dtype}")
@@ -111,14 +129,14 @@ class TiledRows:
         M, K = x.shape
         t = cls(M, K, x.device)
         t.buf.zero_()
-        _check(lib().gs_retile_rows(_p(x), _p(t.buf), c_int(M), c_int(K), c_int(x.stride(0) if M > 1 else K), c_int(1),
+        _check(lib().gs_retile_rows(_p(x), _p(t.buf), M, K, x.stride(0) if M > 1 else K, 1,
                                     _stream()))
         return t
 
     def rows(self) -> torch.Tensor:
         M, K = self.shape
         out = torch.empty((M, K), dtype=torch.bfloat16, device=self.device)
-        _check(lib().gs_retile_rows(_p(self.buf), _p(out), c_int(M), c_int(K), c_int(K), c_int(0), _stream()))
+        _check(lib().gs_retile_rows(_p(self.buf), _p(out), M, K, K, 0, _stream()))
         return out
 
 
@@ -155,8 +173,8 @@ def embed(ids: torch.Tensor, table: torch.Tensor, out: torch.Tensor = None, ssq:
             xs_buf, xs_tiled = xs.buf, 1
         _need(next_weight.dtype == torch.float32 and next_weight.shape == (H,) and xs.dtype == torch.bfloat16
               and tuple(xs.shape) == (T, H) and xs_buf.is_contiguous(), "embed: next_weight float32 (H,), xs bfloat16 (T, H)")
-    _check(lib().gs_embed(_p(ids), _p(table), _dt(table), _p(out), _p(ssq), _p(next_weight), _p(xs_buf), c_int(xs_tiled),
-                          c_int(T), c_int(H), c_int(V), c_float(scale), _stream()))
+    _check(lib().gs_embed(_p(ids), _p(table), _dt(table), _p(out), _p(ssq), _p(next_weight), _p(xs_buf), xs_tiled,
+                          T, H, V, scale, _stream()))
     return out
 
 
@@ -166,6 +184,10 @@ def add_rmsnorm(res: torch.Tensor, delta, weight: torch.Tensor, eps: float, out_
 
     ``rows`` (int32) picks source rows; then ``res`` is not written.
     """
+    if rows is None and out is None:
+        y = (_host or _native()).add_rmsnorm(res, delta, weight, eps, _DT.get(out_dtype), _stream())
+        if y is not False:
+            return y
     f32 = torch.float32
     if not (res.is_cuda and res.is_contiguous() and res.dtype is f32 and res.dim() == 2):
         raise KernelError("add_rmsnorm: the residual stream is float32 (T, H), contiguous, on the GPU")
@@ -194,7 +216,7 @@ def add_rmsnorm(res: torch.Tensor, delta, weight: torch.Tensor, eps: float, out_
 def residual_add(res: torch.Tensor, delta: torch.Tensor) -> torch.Tensor:
     _dev(res, delta)
     _need(res.dtype == torch.float32 and delta.shape == res.shape, "residual_add: shapes or types differ")
-    _check(lib().gs_residual_add(_p(res), _p(delta), c_int(_dt(delta)), c_long(res.numel()), _stream()))
+    _check(lib().gs_residual_add(_p(res), _p(delta), _dt(delta), res.numel(), _stream()))
     return res
 
 
@@ -228,8 +250,8 @@ def add_bias(y: torch.Tensor, bias: torch.Tensor, out_dtype=None, out: torch.Ten
         out = torch.empty((M, N), dtype=out_dtype or torch.float32, device=y.device)
     _need(out.shape == (M, N) and out.stride(1) == 1 and out.dtype in (torch.float32, torch.bfloat16),
           "add_bias: out has the wrong shape or type")
-    _check(lib().gs_add_bias(_p(y), _p(bias), _p(out), c_int(_dt(out)), c_int(M), c_int(N),
-                             c_long(out.stride(0) if M > 1 else N), _stream()))
+    _check(lib().gs_add_bias(_p(y), _p(bias), _p(out), _dt(out), M, N,
+                             out.stride(0) if M > 1 else N, _stream()))
     return out
 
 
@@ -237,7 +259,7 @@ def softcap(logits: torch.Tensor, cap: float) -> torch.Tensor:
     """``cap * tanh(logits / cap)`` in place (float32)."""
     _dev(logits)
     _need(logits.dtype == torch.float32, "softcap takes float32 logits")
-    _check(lib().gs_softcap(_p(logits), c_float(cap), c_long(logits.numel()), _stream()))
+    _check(lib().gs_softcap(_p(logits), cap, logits.numel(), _stream()))
     return logits
 
 
@@ -249,7 +271,7 @@ def stream_read(buf: torch.Tensor, blocks: int = 2048, contiguous: bool = True, 
     if sink is None:
         sink = torch.zeros(blocks, dtype=torch.int32, device=buf.device)
     _need(sink.dtype == torch.int32 and sink.numel() >= blocks, "stream_read: sink holds an int32 per block")
-    _check(lib().gs_stream_read(_p(buf), c_long(nbytes), _p(sink), c_int(blocks), c_int(1 if contiguous else 0), _stream()))
+    _check(lib().gs_stream_read(_p(buf), nbytes, _p(sink), blocks, 1 if contiguous else 0, _stream()))
 
 
 FILL_MAX = 65535
@@ -270,8 +292,8 @@ def fill_rows(pool: torch.Tensor, ids: torch.Tensor, value: float, planes: int =
     _need(outer <= FILL_MAX, f"fill_rows: {outer} planes are more than a launch takes ({FILL_MAX})")
     for at in range(0, ids.numel(), FILL_MAX):            # a launch takes 65,535 ids: many freed pages go in turns
         part = ids[at:at + FILL_MAX]
-        _check(lib().gs_fill_rows(_p(pool), c_int(_dt(pool)), _p(part), c_int(part.numel()), c_long(row), c_int(outer),
-                                  c_long(rows), c_float(value), _stream()))
+        _check(lib().gs_fill_rows(_p(pool), _dt(pool), _p(part), part.numel(), row, outer,
+                                  rows, value, _stream()))
 
 
 # ---------------------------------------------------------------------- short convolution
@@ -279,24 +301,33 @@ def fill_rows(pool: torch.Tensor, ids: torch.Tensor, value: float, planes: int =
 def short_conv(bcx, taps, bias, state, seq_of_token, q_start, slots, nseq: int, all_single: bool,
                out: torch.Tensor = None) -> torch.Tensor:
     """Gated short convolution over segments; ``state (num_slots, H, W-1)`` is read and advanced."""
+    if out is None:
+        y = (_host or _native()).short_conv(bcx, taps, bias, state, seq_of_token, q_start, slots, nseq, 1 if all_single else 0, _stream())
+        if y is not False:
+            return y
+    f32 = torch.float32
     _dev(bcx, taps, bias, state, seq_of_token, q_start, slots, out)
     T, H3 = bcx.shape
-    _need(H3 % 3 == 0, "short_conv: bcx holds B, C, X side by side")
+    if H3 % 3 != 0:
+        raise KernelError("short_conv: bcx holds B, C, X side by side")
     H = H3 // 3
     W = taps.shape[1]
-    _need(taps.dtype == torch.float32 and taps.shape == (H, W), "short_conv: taps must be float32 (H, W)")
-    _need(bias is None or (bias.dtype == torch.float32 and bias.shape == (H,)), "short_conv: bias must be float32 (H,)")
-    _need(state.dtype == torch.float32 and state.dim() == 3 and state.shape[1:] == (H, W - 1),
-          "short_conv: state must be float32 (slots, H, W-1)")
+    if not (taps.dtype is f32 and taps.shape == (H, W)):
+        raise KernelError("short_conv: taps must be float32 (H, W)")
+    if bias is not None and not (bias.dtype is f32 and bias.shape == (H,)):
+        raise KernelError("short_conv: bias must be float32 (H,)")
+    if not (state.dtype is f32 and state.dim() == 3 and state.shape[1:] == (H, W - 1)):
+        raise KernelError("short_conv: state must be float32 (slots, H, W-1)")
     _i32(seq_of_token, T, "seq_of_token")
     _i32(q_start, nseq + 1, "q_start")
     _i32(slots, nseq, "slots")
     if out is None:
         out = torch.empty((T, H), dtype=bcx.dtype, device=bcx.device)
-    _need(out.shape == (T, H) and out.dtype == bcx.dtype, "short_conv: out has the wrong shape or type")
-    _check(lib().gs_short_conv(_p(bcx), c_int(_dt(bcx)), _p(taps), _p(bias), _p(state), _p(seq_of_token),
-                               _p(q_start), _p(slots), _p(out), c_int(T), c_int(nseq), c_int(H), c_int(W),
-                               c_int(1 if all_single else 0), _stream()))
+    elif not (out.shape == (T, H) and out.dtype == bcx.dtype):
+        raise KernelError("short_conv: out has the wrong shape or type")
+    _check(lib().gs_short_conv(_p(bcx), _dt(bcx), _p(taps), _p(bias), _p(state), _p(seq_of_token),
+                               _p(q_start), _p(slots), _p(out), T, nseq, H, W,
+                               1 if all_single else 0, _stream()))
     return out
 
 
@@ -326,6 +357,11 @@ def qknorm_rope_kv(qkv, q_weight, k_weight, eps, cos, sin, rotary_dim, positions
     goes with that many keys of width ``d``, side by side in the rows and in the key cache ``(pages, nkv, page_size,
     maps d)`` (``nh`` counts every query)."""
     _need(layout in ROPE_LAYOUTS, f"qknorm_rope_kv: pairs are laid out 'half' or 'interleaved', not {layout!r}")
+    if vcos is None and vsin is None and v_first is None and mix is None and maps == 1 and not plain_norm and (vd is None or vd == d):
+        if (_host or _native()).qknorm_rope_kv(qkv, q_weight, k_weight, eps, cos, sin, rotary_dim or 0, positions, seq_of_token, block_table,
+                                               page_size, kcache, vcache, nh, nkv, d, 1 if write_kv else 0,
+                                               1 if layout == "interleaved" else 0, _stream()) is not False:
+            return
     _dev(qkv, q_weight, k_weight, cos, sin, positions, seq_of_token, block_table, kcache, vcache, mix)
     vd = d if vd is None else int(vd)
     T = qkv.shape[0]
@@ -354,13 +390,13 @@ def qknorm_rope_kv(qkv, q_weight, k_weight, eps, cos, sin, rotary_dim, positions
     _need(kcache.dtype == qkv.dtype and vcache.dtype == qkv.dtype, "cache and activations differ in type")
     _need(kcache.dim() == 4 and kcache.shape[1:] == (nkv, page_size, maps * d) and vcache.shape == kcache.shape[:3] + (vd,),
           "caches must be (pages, nkv, page_size, d) and (pages, nkv, page_size, vd)")
-    _check(lib().gs_qknorm_rope_kv(_p(qkv), c_int(_dt(qkv)), _p(q_weight), _p(k_weight), c_float(eps), _p(cos),
-                                   _p(sin), c_int(rotary_dim), c_int(1 if layout == "interleaved" else 0), c_int(max_pos),
+    _check(lib().gs_qknorm_rope_kv(_p(qkv), _dt(qkv), _p(q_weight), _p(k_weight), eps, _p(cos),
+                                   _p(sin), rotary_dim, 1 if layout == "interleaved" else 0, max_pos,
                                    _p(positions), _p(seq_of_token),
-                                   _p(block_table), c_int(block_table.shape[1]), c_int(page_size), _p(kcache),
-                                   _p(vcache), c_int(T), c_int(nh), c_int(nkv), c_int(d),
-                                   c_int(1 if write_kv else 0), c_int(vd), _p(vcos), _p(vsin), c_int(qkv.shape[1]),
-                                   c_int(1 if plain_norm else 0), _p(v_first), c_int(ldf), _p(mix), maps, _stream()))
+                                   _p(block_table), block_table.shape[1], page_size, _p(kcache),
+                                   _p(vcache), T, nh, nkv, d,
+                                   1 if write_kv else 0, vd, _p(vcos), _p(vsin), qkv.shape[1],
+                                   1 if plain_norm else 0, _p(v_first), ldf, _p(mix), maps, _stream()))
 
 
 def attention_generic(q, q_stride, kcache, vcache, positions, seq_of_token, block_table, page_size, window, scale,
@@ -388,13 +424,13 @@ def attention_generic(q, q_stride, kcache, vcache, positions, seq_of_token, bloc
     if out is None:
         out = torch.empty((ntok, nh * vd), dtype=q.dtype, device=q.device)
     _need(out.shape == (ntok, nh * vd) and out.dtype == q.dtype, "attention: out has the wrong shape or type")
-    _check(lib().gs_attention_generic(_p(q), c_int(q_stride), _p(kcache), _p(vcache), c_int(_dt(q)), _p(positions),
-                                      _p(seq_of_token), _p(block_table), c_int(block_table.shape[1]),
-                                      c_int(page_size), c_int(window or 0), c_float(scale), _p(out), c_int(ntok),
-                                      c_int(nh), c_int(nkv), c_int(d), c_int(vd), c_int(chunk or 0),
-                                      c_int(1 if sink else 0), _p(vcos), _p(vsin),
-                                      c_int(1 if layout == "interleaved" else 0), c_float(softcap or 0.0),
-                                      c_int(keep_first or 0), _p(sinks), _stream()))
+    _check(lib().gs_attention_generic(_p(q), q_stride, _p(kcache), _p(vcache), _dt(q), _p(positions),
+                                      _p(seq_of_token), _p(block_table), block_table.shape[1],
+                                      page_size, window or 0, scale, _p(out), ntok,
+                                      nh, nkv, d, vd, chunk or 0,
+                                      1 if sink else 0, _p(vcos), _p(vsin),
+                                      1 if layout == "interleaved" else 0, softcap or 0.0,
+                                      keep_first or 0, _p(sinks), _stream()))
     return out
 
 
@@ -446,8 +482,8 @@ def attention_prefill_maps(rows, kcache, vcache, positions, tiles, block_table, 
     if out is None:
         out = torch.empty((T, nh * vd), dtype=rows.dtype, device=rows.device)
     _need(out.shape == (T, nh * vd) and out.dtype == rows.dtype and out.is_contiguous(), "attention_prefill_maps: out has the wrong shape or type")
-    _check(lib().gs_attention_prefill_maps(_p(rows), rows.shape[1], _p(kcache), _p(vcache), _p(positions), _p(tiles[0]),
-                                           _p(tiles[1]), _p(tiles[2]), tiles.shape[1], _p(block_table), block_table.shape[1],
+    _check(lib().gs_attention_prefill_maps(_p(rows), rows.shape[1], _p(kcache), _p(vcache), _p(positions), *_tile_rows(tiles),
+                                           tiles.shape[1], _p(block_table), block_table.shape[1],
                                            page_size, window or 0, scale, lam, eps, out_scale, gate_col, _p(out), nh, nkv, d,
                                            vd, tile_rows, _stream()))
     return out
@@ -544,18 +580,18 @@ def linear_attention_scan(x, oq: int, ok: int, ov: int, H: int, n: int, m: int, 
             _need(segment % 32 == 0 and longest > 0, "linear_attention: segments are whole runs of 32 tokens")
             maxseg = -(-longest // segment)
             ws = torch.empty(nseq * maxseg * H * n * m, dtype=torch.float32, device=x.device)
-        _check(lib().gs_linear_attention_chunks(_p(x), c_int(ld), c_int(oq), c_int(ok), c_int(ov), c_int(_ACTS[activation]),
+        _check(lib().gs_linear_attention_chunks(_p(x), ld, oq, ok, ov, _ACTS[activation],
                                                 _p(cos) if rotary_dim else None, _p(sin) if rotary_dim else None,
-                                                c_int(rotary_dim), c_int(max_pos), c_float(key_scale), _p(decay), _p(state),
-                                                _p(q_start), _p(slots), _p(positions), _p(out), c_int(nseq), c_int(H),
-                                                c_int(n), c_int(m), c_int(chunks_from), _p(ws), c_int(maxseg),
-                                                c_int(segment), _stream()))
+                                                rotary_dim, max_pos, key_scale, _p(decay), _p(state),
+                                                _p(q_start), _p(slots), _p(positions), _p(out), nseq, H,
+                                                n, m, chunks_from, _p(ws), maxseg,
+                                                segment, _stream()))
         return out
-    _check(lib().gs_linear_attention_scan(_p(x), c_int(_dt(x)), c_int(ld), c_int(oq), c_int(ok), c_int(ov),
-                                          c_int(_ACTS[activation]), _p(cos) if rotary_dim else None,
-                                          _p(sin) if rotary_dim else None, c_int(rotary_dim), c_int(max_pos),
-                                          c_float(key_scale), _p(decay), _p(state), _p(q_start), _p(slots), _p(positions),
-                                          _p(out), c_int(nseq), c_int(H), c_int(n), c_int(m), c_int(below), _stream()))
+    _check(lib().gs_linear_attention_scan(_p(x), _dt(x), ld, oq, ok, ov,
+                                          _ACTS[activation], _p(cos) if rotary_dim else None,
+                                          _p(sin) if rotary_dim else None, rotary_dim, max_pos,
+                                          key_scale, _p(decay), _p(state), _p(q_start), _p(slots), _p(positions),
+                                          _p(out), nseq, H, n, m, below, _stream()))
     return out
 
 
@@ -571,9 +607,9 @@ def gated_outnorm(o, gate_rows, og: int, weight, eps: float, H: int, m: int, joi
     _need(weight is None or (weight.dtype == torch.float32 and weight.shape == (H * m,)), "gated_outnorm: weight must be float32 (H m,)")
     _need(gate in _GATES, f"gated_outnorm: the gate is 'sigmoid' or 'silu', not {gate!r}")
     out = torch.empty((T, H * m), dtype=out_dtype, device=o.device)
-    _check(lib().gs_gated_outnorm(_p(o), _p(gate_rows), c_int(_dt(gate_rows)), c_int(gate_rows.shape[1]), c_int(og),
-                                  _p(weight), c_float(eps), c_int(1 if joint else 0), c_int(_GATES[gate]), _p(out),
-                                  c_int(_dt(out)), c_int(T), c_int(H), c_int(m), _stream()))
+    _check(lib().gs_gated_outnorm(_p(o), _p(gate_rows), _dt(gate_rows), gate_rows.shape[1], og,
+                                  _p(weight), eps, 1 if joint else 0, _GATES[gate], _p(out),
+                                  _dt(out), T, H, m, _stream()))
     return out
 
 
@@ -592,8 +628,8 @@ def add_rmsnorm_pair(res, d1, d2, w1, w2, eps: float, out_dtype, bias=None):
     out1 = torch.empty((T, H), dtype=out_dtype, device=res.device)
     out2 = torch.empty((T, H), dtype=out_dtype, device=res.device) if w2 is not None else None
     _check(lib().gs_add_rmsnorm_pair(_p(res), _p(ds[0]) if ds else None, _p(ds[1]) if len(ds) > 1 else None,
-                                     c_int(_dt(ds[0]) if ds else _dt(out1)), _p(w1), _p(w2), c_float(eps), _p(out1),
-                                     _p(out2), c_int(_dt(out1)), c_int(T), c_int(H), _p(bias), _stream()))
+                                     _dt(ds[0]) if ds else _dt(out1), _p(w1), _p(w2), eps, _p(out1),
+                                     _p(out2), _dt(out1), T, H, _p(bias), _stream()))
     return out1, out2
 
 
@@ -602,8 +638,8 @@ def scaled_sum(a, sa: float, b, sb: float, out_dtype) -> torch.Tensor:
     _dev(a, b)
     _need(a.shape == b.shape and a.dtype == b.dtype, "scaled_sum: operands of one shape and type")
     out = torch.empty(a.shape, dtype=out_dtype, device=a.device)
-    _check(lib().gs_scaled_sum(_p(a), c_float(sa), _p(b), c_float(sb), c_int(_dt(a)), _p(out), c_int(_dt(out)),
-                               c_long(a.numel()), _stream()))
+    _check(lib().gs_scaled_sum(_p(a), sa, _p(b), sb, _dt(a), _p(out), _dt(out),
+                               a.numel(), _stream()))
     return out
 
 
@@ -616,8 +652,8 @@ def gated_act(x, bias, activation: str, out_dtype) -> torch.Tensor:
     _need(bias is None or (bias.dtype == torch.float32 and bias.shape == (F2,)), "gated_act: bias must be float32 (2F,)")
     _need(activation in GATED_ACTS, f"gated_act: the activation is one of {sorted(GATED_ACTS)}, not {activation!r}")
     out = torch.empty((T, F), dtype=out_dtype, device=x.device)
-    _check(lib().gs_gated_act(_p(x), c_int(_dt(x)), _p(bias), _p(out), c_int(_dt(out)), c_int(T), c_int(F),
-                              c_int(GATED_ACTS[activation]), _stream()))
+    _check(lib().gs_gated_act(_p(x), _dt(x), _p(bias), _p(out), _dt(out), T, F,
+                              GATED_ACTS[activation], _stream()))
     return out
 
 
@@ -646,14 +682,14 @@ def gemm_tiled(x: torch.Tensor, w: torch.Tensor, bias=None, out_dtype=None, out:
     _need(out.shape == (M, N) and out.stride(1) == 1, "gemm: out has the wrong shape")
     ldx = x.stride(0) if M > 1 else K
     if (x.dtype == torch.float32 and w.dtype == torch.float32 and w.is_contiguous()
-            and lib().gs_gemm_f32_takes(c_int(M), c_int(N), c_int(K), c_int(ldx), _p(x), _p(w))):
+            and lib().gs_gemm_f32_takes(M, N, K, ldx, _p(x), _p(w))):
         # the matrix cores, every output summed in the order of the kernel below
-        _check(lib().gs_gemm_f32(_p(x), c_int(ldx), _p(w), _p(bias), _p(out), c_int(_dt(out)),
-                                 c_int(out.stride(0) if M > 1 else N), c_int(M), c_int(N), c_int(K), _stream()))
+        _check(lib().gs_gemm_f32(_p(x), ldx, _p(w), _p(bias), _p(out), _dt(out),
+                                 out.stride(0) if M > 1 else N, M, N, K, _stream()))
         return out
-    _check(lib().gs_gemm_tiled(_p(x), c_int(_dt(x)), c_int(x.stride(0) if M > 1 else K), _p(w), c_int(_dt(w)),
-                               _p(bias), _p(out), c_int(_dt(out)), c_int(out.stride(0) if M > 1 else N), c_int(M),
-                               c_int(N), c_int(K), _stream()))
+    _check(lib().gs_gemm_tiled(_p(x), _dt(x), x.stride(0) if M > 1 else K, _p(w), _dt(w),
+                               _p(bias), _p(out), _dt(out), out.stride(0) if M > 1 else N, M,
+                               N, K, _stream()))
     return out
 
 
@@ -675,10 +711,13 @@ def _mid_parts_pay(M: int, N: int, K: int) -> int:
 def _mid_operands(x, w: torch.Tensor, wt) -> bool:
     """bfloat16 rows on the GPU, aligned, that do not overlap, and the whole weight ``wt`` was made of as it lies there (a part
     or a transposed view of it can share its address)."""
-    if wt is None or not isinstance(x, torch.Tensor) or x.dtype is not torch.bfloat16 or not x.is_cuda or x.dim() != 2:
+    if wt is None or not isinstance(x, torch.Tensor) or x.dtype is not torch.bfloat16 or not x.is_cuda:
         return False
-    K, (s0, s1) = x.shape[1], x.stride()
-    return (s1 == 1 and s0 >= K and s0 % 8 == 0 and x.data_ptr() % 16 == 0 and K == w.shape[1] and wt.shape == w.shape
+    shape = x.shape
+    if len(shape) != 2:
+        return False
+    K, (s0, s1), whole = shape[1], x.stride(), w.shape
+    return (s1 == 1 and s0 >= K and s0 % 8 == 0 and x.data_ptr() % 16 == 0 and K == whole[1] and wt.shape == whole
             and w.is_contiguous())
 
 
@@ -690,6 +729,11 @@ def mid_ok(x, w: torch.Tensor, wt, swiglu: bool = False, out: torch.Tensor = Non
                                  and out.shape == (x.shape[0], w.shape[0] // 2 if swiglu else w.shape[0])
                                  and out.stride(1) == 1 and out.stride(0) >= out.shape[1] and out.stride(0) % 4 == 0
                                  and out.data_ptr() % 8 == 0)))
+
+
+def gemm_mid_plain(x, w: torch.Tensor, wt, swiglu: bool = False):
+    """:func:`gemm_mid` into a new tensor; False where :func:`mid_ok` says no."""
+    return (_host or _native()).gemm_mid(x, w, wt, 1 if swiglu else 0, _stream())
 
 
 def gemm_mid(x, w: torch.Tensor, wt, swiglu: bool = False, out: torch.Tensor = None, checked: bool = False) -> torch.Tensor:
@@ -717,12 +761,16 @@ def mid_residual_ok(x, w: torch.Tensor, wt) -> bool:
     return _mid_operands(x, w, wt) and _mid_residual_sums(x.shape[0], w.shape[0], w.shape[1]) > 0
 
 
-def gemm_mid_residual(x, w: torch.Tensor, wt, res: torch.Tensor, next_weight: torch.Tensor):
+def gemm_mid_residual(x, w: torch.Tensor, wt, res: torch.Tensor, next_weight: torch.Tensor, checked: bool = False):
     """``res += x @ w.T`` in place (float32) for products :func:`mid_residual_ok` takes.  Returns the new rows times
-    ``next_weight`` in bfloat16 and partial sums of their squares ``(M, sums)``."""
+    ``next_weight`` in bfloat16 and partial sums of their squares ``(M, sums)``.  ``checked``: the caller has asked about these
+    operands."""
+    y = (_host or _native()).gemm_mid_residual(x, w, wt, res, next_weight, _stream())
+    if y is not False:
+        return y
     M, K = x.shape
     N = w.shape[0]
-    sums = _mid_residual_sums(M, N, K) if _mid_operands(x, w, wt) else 0
+    sums = _mid_residual_sums(M, N, K) if checked or _mid_operands(x, w, wt) else 0
     if sums <= 0:
         raise KernelError(f"gemm_mid_residual: not a product of this kernel, M={M} N={N} K={K}")
     if not (wt.dtype is torch.bfloat16 and wt.is_cuda and wt.is_contiguous()):
@@ -746,9 +794,18 @@ def mid_scaled_ok(x, w13: torch.Tensor, wt) -> bool:
             and mid_ok(x.xs, w13, wt, swiglu=True))
 
 
-def gemm_mid_swiglu_scaled(x, w13: torch.Tensor, wt) -> torch.Tensor:
-    """``silu(gate) * up`` in bfloat16 of a lazy norm whose rows come weighted, for products :func:`mid_scaled_ok` takes."""
-    if not mid_scaled_ok(x, w13, wt):
+def gemm_mid_swiglu_scaled_plain(x, w13: torch.Tensor, wt):
+    """:func:`gemm_mid_swiglu_scaled`; False where :func:`mid_scaled_ok` says no."""
+    return (_host or _native()).gemm_mid_swiglu_scaled(x.xs, x.ssq, x.eps, w13, wt, _stream())
+
+
+def gemm_mid_swiglu_scaled(x, w13: torch.Tensor, wt, checked: bool = False) -> torch.Tensor:
+    """``silu(gate) * up`` in bfloat16 of a lazy norm whose rows come weighted, for products :func:`mid_scaled_ok` takes
+    (``checked``: the caller has asked it)."""
+    y = gemm_mid_swiglu_scaled_plain(x, w13, wt)
+    if y is not False:
+        return y
+    if not (checked or mid_scaled_ok(x, w13, wt)):
         raise KernelError(f"gemm_mid_swiglu_scaled: not a product of this kernel, M={x.shape[0]} N={w13.shape[0]} K={w13.shape[1]}")
     if not (wt.dtype is torch.bfloat16 and wt.is_cuda and wt.is_contiguous()):
         raise KernelError("gemm_mid_swiglu_scaled: the weight's tile-major copy is bfloat16 on the GPU")
@@ -777,6 +834,10 @@ def gemm_mid_residual_parts(x, w: torch.Tensor, wt, res: torch.Tensor, next_weig
     """``res += x @ w.T`` for some hundred rows and a long K in two kernels: partial sums over parts of K, then one pass that adds
     them to the stream.  Returns the rows normed with ``next_weight`` and ``eps`` for the norm that reads the stream next, or None.
     ``parts``: what :func:`mid_parts` has told the caller about these operands."""
+    if parts is not None and next_weight is not None:
+        y = (_host or _native()).gemm_mid_residual_parts(x, w, wt, res, next_weight, eps, parts, _stream())
+        if y is not False:
+            return y
     M, K = x.shape
     N = w.shape[0]
     parts = mid_parts(x, w, wt) if parts is None else parts
@@ -821,9 +882,9 @@ def gemm_mfma(x: torch.Tensor, w: torch.Tensor, out_dtype=None, out: torch.Tenso
         out = torch.empty((M, cols), dtype=out_dtype or torch.bfloat16, device=w.device)
     _need(out.shape == (M, cols) and out.stride(1) == 1, "gemm_mfma: out has the wrong shape")
     _need(not swiglu or out.dtype == torch.bfloat16, "gemm_mfma: the SwiGLU epilogue stores bfloat16")
-    _check(lib().gs_gemm_mfma(_p(x), c_int(x.stride(0) if M > 1 else K), _p(w), _p(out), c_int(_dt(out)),
-                              c_int(out.stride(0) if M > 1 else cols), c_int(M), c_int(N), c_int(K),
-                              c_int(1 if swiglu else 0), _stream()))
+    _check(lib().gs_gemm_mfma(_p(x), x.stride(0) if M > 1 else K, _p(w), _p(out), _dt(out),
+                              out.stride(0) if M > 1 else cols, M, N, K,
+                              1 if swiglu else 0, _stream()))
     return out
 
 
@@ -872,7 +933,7 @@ def library_gemm_ok(x, w: torch.Tensor) -> bool:
 def library_gemm_plan(M: int, N: int, K: int):
     """``(plans kept in all, candidates measured for this shape, the best one's microseconds)``."""
     cand, best = c_int(0), c_float(0.0)
-    n = lib().gs_library_gemm_plans(c_int(M), c_int(N), c_int(K), ctypes.byref(cand), ctypes.byref(best))
+    n = lib().gs_library_gemm_plans(M, N, K, ctypes.byref(cand), ctypes.byref(best))
     return n, cand.value, best.value
 
 
@@ -885,7 +946,7 @@ def argmax_rows(logits: torch.Tensor):
     rows, V = logits.shape
     ids = torch.empty(rows, dtype=torch.int32, device=logits.device)
     bad = torch.empty(rows, dtype=torch.int32, device=logits.device)
-    _check(lib().gs_argmax_rows(_p(logits), c_int(rows), c_int(V), _p(ids), _p(bad), _stream()))
+    _check(lib().gs_argmax_rows(_p(logits), rows, V, _p(ids), _p(bad), _stream()))
     return ids, bad
 
 
@@ -927,12 +988,13 @@ SKINNY_MAX_ROWS = 64
 
 def skinny_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether the weight-streaming kernel takes this product (few rows, bfloat16, aligned rows)."""
+    shape, bf16 = x.shape, torch.bfloat16
+    if len(shape) != 2 or shape[0] > SKINNY_MAX_ROWS or w.dtype is not bf16 or not w.is_contiguous() or w.data_ptr() % 16 != 0:
+        return False
     if isinstance(x, TiledRows):
-        return (w.dtype == torch.bfloat16 and x.shape[0] <= SKINNY_MAX_ROWS and w.is_contiguous()
-                and w.data_ptr() % 16 == 0)
-    return (x.dim() == 2 and x.shape[0] <= SKINNY_MAX_ROWS and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
-            and x.shape[1] % 8 == 0 and x.stride(1) == 1 and (x.shape[0] <= 1 or x.stride(0) % 8 == 0)
-            and x.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0)
+        return True
+    s0, s1 = x.stride()
+    return (x.dtype is bf16 and shape[1] % 8 == 0 and s1 == 1 and (shape[0] <= 1 or s0 % 8 == 0) and x.data_ptr() % 16 == 0)
 
 
 class LazyNorm:
@@ -960,8 +1022,8 @@ class LazyNorm:
             return self.ready
         T, H = self.res.shape
         out = torch.empty((T, H), dtype=self.dtype, device=self.res.device)
-        _check(lib().gs_norm_from_ssq(_p(self.res), _p(self.ssq), c_int(self.ssq.shape[1]), _p(self.weight),
-                                      c_float(self.eps), _p(out), c_int(_dt(out)), c_int(T), c_int(H), _stream()))
+        _check(lib().gs_norm_from_ssq(_p(self.res), _p(self.ssq), self.ssq.shape[1], _p(self.weight),
+                                      self.eps, _p(out), _dt(out), T, H, _stream()))
         return out
 
 
@@ -974,18 +1036,18 @@ def lazy_ok(x, w: torch.Tensor) -> bool:
 def _lazy_args(x):
     if isinstance(x, LazyNorm):
         if x.xs is not None:
-            return _x_args(x.xs) + (None, _p(x.ssq), c_int(x.ssq.shape[1]), None, c_float(x.eps))
-        return (None, c_int(x.res.shape[1]), c_int(0), _p(x.res), _p(x.ssq), c_int(x.ssq.shape[1]), _p(x.weight),
-                c_float(x.eps))
-    return _x_args(x) + (None, None, c_int(0), None, c_float(0.0))
+            return _x_args(x.xs) + (None, _p(x.ssq), x.ssq.shape[1], None, x.eps)
+        return (None, x.res.shape[1], 0, _p(x.res), _p(x.ssq), x.ssq.shape[1], _p(x.weight),
+                x.eps)
+    return _x_args(x) + (None, None, 0, None, 0.0)
 
 
 def _x_args(x):
     """Pointer, row stride and layout flag of a product's rows."""
     M, K = x.shape
     if isinstance(x, TiledRows):
-        return (_p(x.buf), c_int(K), c_int(1))
-    return (_p(x), c_int(x.stride(0) if M > 1 else K), c_int(0))
+        return (_p(x.buf), K, 1)
+    return (_p(x), x.stride(0) if M > 1 else K, 0)
 
 
 def tile_major(w: torch.Tensor) -> torch.Tensor:
@@ -995,31 +1057,44 @@ def tile_major(w: torch.Tensor) -> torch.Tensor:
     N, K = w.shape
     _need(w.dtype == torch.bfloat16 and N % 16 == 0 and K % 32 == 0, "tile_major: bfloat16 (N, K), N % 16 == 0, K % 32 == 0")
     out = torch.empty_like(w)
-    _check(lib().gs_tile_major(_p(w), _p(out), c_int(N), c_int(K), _stream()))
+    _check(lib().gs_tile_major(_p(w), _p(out), N, K, _stream()))
     return out
 
 
-def gemm_skinny(x, w: torch.Tensor, out_dtype=None, out=None, swiglu: bool = False, wt=None):
+def gemm_skinny_plain(x, w: torch.Tensor, wt, out_dtype, swiglu: bool = False):
+    """:func:`gemm_skinny` of an ordinary tensor into a new one; False where it is not for that."""
+    return (_host or _native()).gemm_skinny(x, w, wt, _DT.get(out_dtype), 1 if swiglu else 0, _stream())
+
+
+def gemm_skinny(x, w: torch.Tensor, out_dtype=None, out=None, swiglu: bool = False, wt=None, checked: bool = False):
     """``x @ w.T`` for at most 64 rows, streaming the weights once; optionally ``silu(gate) * up`` of the result.
 
     ``x`` is a bfloat16 tensor, :class:`TiledRows` or a :class:`LazyNorm`.  With ``swiglu`` the weight holds gate
     rows then up rows and the output is half as wide, and ``out`` may be True or a :class:`TiledRows` for tiled rows.
+    ``checked``: the caller has asked :func:`skinny_ok` (or :func:`lazy_ok`) about these operands.
     """
+    if out is None or out is False:
+        y = gemm_skinny_plain(x, w, wt, out_dtype or torch.bfloat16, swiglu)
+        if y is not False:
+            return y
     _dev(w, out if isinstance(out, torch.Tensor) else None)
-    lazy = isinstance(x, LazyNorm)
-    _need(lazy_ok(x, w) if lazy else skinny_ok(x, w),
-          "gemm_skinny: operands must be bfloat16, at most 64 rows, K a multiple of 8, aligned")
+    if not (checked or (lazy_ok(x, w) if isinstance(x, LazyNorm) else skinny_ok(x, w))):
+        raise KernelError("gemm_skinny: operands must be bfloat16, at most 64 rows, K a multiple of 8, aligned")
     M, K = x.shape
-    N = w.shape[0]
-    if w.shape != (N, K):
+    N, Kw = w.shape
+    if K != Kw:
         raise KernelError(f"gemm_skinny: weight is {tuple(w.shape)}, expected ({N}, {K})")
     cols = N // 2 if swiglu else N
-    out, buf, tiled = _rows_out(out, M, cols, w.device, out_dtype or torch.bfloat16)
-    _need(not tiled or swiglu, "gemm_skinny: only the SwiGLU epilogue writes tiled rows")
-    _need(tiled or (out.shape == (M, cols) and out.stride(1) == 1), "gemm_skinny: out has the wrong shape")
-    _check(lib().gs_gemm_skinny(*_lazy_args(x), _p(w), _p(wt), _p(buf), c_int(_dt(out)),
-                                c_int(cols if tiled or M <= 1 else out.stride(0)), c_int(M), c_int(N), c_int(K),
-                                c_int(1 if swiglu else 0), c_int(tiled), _stream()))
+    if out is None or out is False:
+        out = buf = torch.empty((M, cols), dtype=out_dtype or torch.bfloat16, device=w.device)
+        tiled = 0
+    else:
+        out, buf, tiled = _rows_out(out, M, cols, w.device, out_dtype or torch.bfloat16)
+        _need(not tiled or swiglu, "gemm_skinny: only the SwiGLU epilogue writes tiled rows")
+        _need(tiled or (out.shape == (M, cols) and out.stride(1) == 1), "gemm_skinny: out has the wrong shape")
+    _check(lib().gs_gemm_skinny(*_lazy_args(x), _p(w), _p(wt), _p(buf), _dt(out),
+                                cols if tiled or M <= 1 else out.stride(0), M, N, K,
+                                1 if swiglu else 0, tiled, _stream()))
     return out
 
 
@@ -1048,7 +1123,7 @@ def gemm_skinny_residual(x: torch.Tensor, w: torch.Tensor, res: torch.Tensor, wt
     M, K = x.shape
     N = w.shape[0]
     _need(w.shape == (N, K) and res.shape == (M, N) and res.dtype == torch.float32, "gemm_skinny_residual: shapes")
-    nb = lib().gs_gemm_skinny_residual_blocks(c_int(N), c_int(0 if wt is None else 1))
+    nb = lib().gs_gemm_skinny_residual_blocks(N, 0 if wt is None else 1)
     ssq = torch.empty((M, nb), dtype=torch.float32, device=res.device)
     _need((next_weight is None) == (xs is None), "gemm_skinny_residual: next_weight and xs come together")
     xs_buf, xs_tiled = xs, 0
@@ -1058,7 +1133,7 @@ def gemm_skinny_residual(x: torch.Tensor, w: torch.Tensor, res: torch.Tensor, wt
         _need(next_weight.dtype == torch.float32 and next_weight.shape == (N,) and xs.dtype == torch.bfloat16
               and tuple(xs.shape) == (M, N) and xs_buf.is_contiguous(), "gemm_skinny_residual: next_weight float32 (N,), xs bfloat16 (M, N)")
     _check(lib().gs_gemm_skinny_residual(*_x_args(x), _p(w), _p(wt), _p(res), _p(ssq), _p(next_weight), _p(xs_buf),
-                                         c_int(xs_tiled), c_int(M), c_int(N), c_int(K), _stream()))
+                                         xs_tiled, M, N, K, _stream()))
     return ssq
 
 
@@ -1075,7 +1150,7 @@ def gemm_skinny_residual_parts(x, w: torch.Tensor, res: torch.Tensor, parts: int
           "gemm_skinny_residual_parts: shapes")
     _need(1 <= parts <= 64, "gemm_skinny_residual_parts: 1 to 64 parts")
     part = torch.empty((parts, M, N), dtype=torch.float32, device=res.device)
-    _check(lib().gs_gemm_skinny_parts(*_x_args(x), _p(w), _p(wt), _p(part), c_int(parts), c_int(M), c_int(N), c_int(K),
+    _check(lib().gs_gemm_skinny_parts(*_x_args(x), _p(w), _p(wt), _p(part), parts, M, N, K,
                                       _stream()))
     ssq = torch.empty((M, 1), dtype=torch.float32, device=res.device)
     normed = None
@@ -1084,9 +1159,9 @@ def gemm_skinny_residual_parts(x, w: torch.Tensor, res: torch.Tensor, parts: int
         normed, nbuf, ntiled = _rows_out(bool(tiled), M, N, res.device, out_dtype or torch.bfloat16)
     else:
         nbuf, ntiled = None, 0
-    _check(lib().gs_residual_from_parts(_p(part), c_int(parts), _p(res), _p(ssq), _p(next_weight), c_float(eps),
-                                        _p(nbuf), c_int(_dt(normed) if normed is not None else 1), c_int(ntiled),
-                                        c_int(M), c_int(N), _stream()))
+    _check(lib().gs_residual_from_parts(_p(part), parts, _p(res), _p(ssq), _p(next_weight), eps,
+                                        _p(nbuf), _dt(normed) if normed is not None else 1, ntiled,
+                                        M, N, _stream()))
     return ssq, normed
 
 
@@ -1104,14 +1179,14 @@ def gemm_skinny_conv(x, w_in, taps, bias, state, slots, wt=None, tiled: bool = F
     _need(bias is None or (bias.dtype == torch.float32 and bias.shape == (H,)), "gemm_skinny_conv: bias float32 (H,)")
     _i32(slots, M, "slots")
     out, buf, otiled = _rows_out(bool(tiled), M, H, w_in.device)
-    _check(lib().gs_gemm_skinny_conv(*_lazy_args(x), _p(w_in), _p(wt), _p(taps), _p(bias), _p(state), _p(slots), c_int(W),
-                                     _p(buf), c_int(otiled), c_int(M), c_int(H), c_int(K), _stream()))
+    _check(lib().gs_gemm_skinny_conv(*_lazy_args(x), _p(w_in), _p(wt), _p(taps), _p(bias), _p(state), _p(slots), W,
+                                     _p(buf), otiled, M, H, K, _stream()))
     return out
 
 
 def choice_parts(V: int) -> int:
     """Partial sums a row of ``V`` logits has in the many-block form of the decode loop's choice."""
-    return int(lib().gs_choice_parts(c_int(V)))
+    return int(lib().gs_choice_parts(V))
 
 
 def choice_hist() -> int:
@@ -1137,8 +1212,8 @@ def decode_choose_greedy(logits, counter, next_ids, ring, bad_ring, positions, k
     up and a live row moves one position on.  A counter at or beyond the rings' step count writes into their last row
     and marks the step bad."""
     rows, V = _choice_rows(logits, counter, next_ids, ring, bad_ring, positions, kv_len, live)
-    _check(lib().gs_decode_choose(_p(logits), c_int(rows), c_int(V), _p(counter), _p(next_ids), _p(ring), _p(bad_ring),
-                                  _p(positions), _p(kv_len), _p(live), c_int(ring.shape[0]), _stream()))
+    _check(lib().gs_decode_choose(_p(logits), rows, V, _p(counter), _p(next_ids), _p(ring), _p(bad_ring),
+                                  _p(positions), _p(kv_len), _p(live), ring.shape[0], _stream()))
 
 
 def decode_choose(logits, temperature, u, counter, next_ids, ring, bad_ring, positions, kv_len, live, wide, top_p=None,
@@ -1164,13 +1239,13 @@ def decode_choose(logits, temperature, u, counter, next_ids, ring, bad_ring, pos
     _need(hist.dtype == torch.int64 and hist.numel() >= rows * choice_hist(), "decode_choose: hist int64, rows * choice_hist() at least")
     _i32(amax, rows)
     _i32(bad0, rows)
-    _check(lib().gs_decode_choose_wide(_p(logits), c_int(rows), c_int(V), _p(temperature), _p(top_p), _p(wbuf), _p(part),
+    _check(lib().gs_decode_choose_wide(_p(logits), rows, V, _p(temperature), _p(top_p), _p(wbuf), _p(part),
                                        _p(amax), _p(bad0), _p(hist), _p(u), _p(counter), _p(next_ids), _p(ring), _p(bad_ring),
-                                       _p(positions), _p(kv_len), _p(live), c_int(u.shape[0]), _stream()))
+                                       _p(positions), _p(kv_len), _p(live), u.shape[0], _stream()))
 
 
 def attention_decode_supports(nh: int, nkv: int, d: int) -> bool:
-    return bool(lib().gs_attention_decode_supports(c_int(nh), c_int(nkv), c_int(d)))
+    return bool(lib().gs_attention_decode_supports(nh, nkv, d))
 
 
 def _decode_workspace(held, device, nseq, nh, nkv, d, nsplit):
@@ -1179,7 +1254,7 @@ def _decode_workspace(held, device, nseq, nh, nkv, d, nsplit):
     if ws is None:
         n = lib().gs_attention_decode_workspace
         n.restype = c_long
-        floats = n(c_int(nseq), c_int(nh), c_int(nkv), c_int(d), c_int(nsplit))
+        floats = n(nseq, nh, nkv, d, nsplit)
         ws = held[key] = torch.empty(max(1, floats), dtype=torch.float32, device=device)
     return ws
 
@@ -1207,29 +1282,29 @@ def attention_decode(q, q_stride, kcache, vcache, positions, block_table, page_s
     out, buf, tiled = _rows_out(out, nseq, nh * d, q.device, q.dtype)
     _need(tuple(out.shape) == (nseq, nh * d) and out.dtype == q.dtype, "attention_decode: out has the wrong shape or type")
     if softcap or keep_first or sinks is not None:
-        _check(lib().gs_attention_decode_rules(_p(q), c_int(q_stride), _p(kcache), _p(vcache), _p(positions), _p(block_table),
-                                               c_int(block_table.shape[1]), c_int(page_size), c_int(window or 0),
-                                               c_float(scale), _p(buf), c_int(tiled), _p(ws), c_int(nseq), c_int(nh),
-                                               c_int(nkv), c_int(d), c_int(nsplit), c_int(chunk or 0),
-                                               c_int(1 if sink else 0), c_float(softcap or 0.0), c_int(keep_first or 0),
+        _check(lib().gs_attention_decode_rules(_p(q), q_stride, _p(kcache), _p(vcache), _p(positions), _p(block_table),
+                                               block_table.shape[1], page_size, window or 0,
+                                               scale, _p(buf), tiled, _p(ws), nseq, nh,
+                                               nkv, d, nsplit, chunk or 0,
+                                               1 if sink else 0, softcap or 0.0, keep_first or 0,
                                                _p(sinks), _stream()))
         return out
     if chunk or sink:
-        _check(lib().gs_attention_decode_runs(_p(q), c_int(q_stride), _p(kcache), _p(vcache), _p(positions), _p(block_table),
-                                              c_int(block_table.shape[1]), c_int(page_size), c_int(window or 0),
-                                              c_float(scale), _p(buf), c_int(tiled), _p(ws), c_int(nseq), c_int(nh),
-                                              c_int(nkv), c_int(d), c_int(nsplit), c_int(chunk or 0),
-                                              c_int(1 if sink else 0), _stream()))
+        _check(lib().gs_attention_decode_runs(_p(q), q_stride, _p(kcache), _p(vcache), _p(positions), _p(block_table),
+                                              block_table.shape[1], page_size, window or 0,
+                                              scale, _p(buf), tiled, _p(ws), nseq, nh,
+                                              nkv, d, nsplit, chunk or 0,
+                                              1 if sink else 0, _stream()))
         return out
-    _check(lib().gs_attention_decode(_p(q), c_int(q_stride), _p(kcache), _p(vcache), _p(positions), _p(block_table),
-                                     c_int(block_table.shape[1]), c_int(page_size), c_int(window or 0), c_float(scale),
-                                     _p(buf), c_int(tiled), _p(ws), c_int(nseq), c_int(nh), c_int(nkv), c_int(d),
-                                     c_int(nsplit), _stream()))
+    _check(lib().gs_attention_decode(_p(q), q_stride, _p(kcache), _p(vcache), _p(positions), _p(block_table),
+                                     block_table.shape[1], page_size, window or 0, scale,
+                                     _p(buf), tiled, _p(ws), nseq, nh, nkv, d,
+                                     nsplit, _stream()))
     return out
 
 
 def attention_decode_raw_supports(nh: int, nkv: int, d: int, rotary_dim: int) -> bool:
-    return bool(lib().gs_attention_decode_raw_supports(c_int(nh), c_int(nkv), c_int(d), c_int(rotary_dim)))
+    return bool(lib().gs_attention_decode_raw_supports(nh, nkv, d, rotary_dim))
 
 
 def attention_decode_raw(qkv, q_stride, kcache, vcache, positions, block_table, page_size, window, scale, q_weight,
@@ -1254,16 +1329,16 @@ def attention_decode_raw(qkv, q_stride, kcache, vcache, positions, block_table, 
     ws = _decode_workspace(workspaces, qkv.device, nseq, nh, nkv, d, nsplit)
     out, buf, tiled = _rows_out(out, nseq, nh * d, qkv.device, qkv.dtype)
     _need(tuple(out.shape) == (nseq, nh * d) and out.dtype == qkv.dtype, "attention_decode_raw: out has the wrong shape or type")
-    _check(lib().gs_attention_decode_raw(_p(qkv), c_int(q_stride), _p(kcache), _p(vcache), _p(positions), _p(block_table),
-                                         c_int(block_table.shape[1]), c_int(page_size), c_int(window or 0),
-                                         c_float(scale), _p(q_weight), _p(k_weight), c_float(head_eps), _p(cos), _p(sin),
-                                         c_int(d), c_int(1 if write_kv else 0), _p(buf), c_int(tiled), _p(ws), c_int(nseq),
-                                         c_int(nh), c_int(nkv), c_int(d), c_int(nsplit), _stream()))
+    _check(lib().gs_attention_decode_raw(_p(qkv), q_stride, _p(kcache), _p(vcache), _p(positions), _p(block_table),
+                                         block_table.shape[1], page_size, window or 0,
+                                         scale, _p(q_weight), _p(k_weight), head_eps, _p(cos), _p(sin),
+                                         d, 1 if write_kv else 0, _p(buf), tiled, _p(ws), nseq,
+                                         nh, nkv, d, nsplit, _stream()))
     return out
 
 
 def attention_prefill_supports(nh: int, nkv: int, d: int) -> bool:
-    return bool(lib().gs_attention_prefill_supports(c_int(nh), c_int(nkv), c_int(d)))
+    return bool(lib().gs_attention_prefill_supports(nh, nkv, d))
 
 
 def turn_heads(x, cos, sin, positions, nh: int, w: int, sign: float = 1.0, layout: str = "half") -> torch.Tensor:
@@ -1276,8 +1351,8 @@ def turn_heads(x, cos, sin, positions, nh: int, w: int, sign: float = 1.0, layou
     _need(cos is not None, "turn_heads: no tables")
     _need(layout in ROPE_LAYOUTS, f"turn_heads: pairs are laid out 'half' or 'interleaved', not {layout!r}")
     _i32(positions, T, "positions")
-    _check(lib().gs_turn_heads(_p(x), c_int(_dt(x)), _p(cos), _p(sin), c_int(cos.shape[0]), _p(positions),
-                               c_int(1 if layout == "interleaved" else 0), c_float(sign), c_int(T), c_int(nh), c_int(w),
+    _check(lib().gs_turn_heads(_p(x), _dt(x), _p(cos), _p(sin), cos.shape[0], _p(positions),
+                               1 if layout == "interleaved" else 0, sign, T, nh, w,
                                _stream()))
     return x
 
@@ -1293,6 +1368,11 @@ def attention_prefill(q, q_stride, kcache, vcache, positions, tiles, block_table
     ``tiles``: int32 ``(3, ntiles)``: sequence, first row and number of rows (at most ``tile_rows``, 16 or
     32) of each tile of consecutive queries of one sequence.
     """
+    if out is None and chunk is None and not sink and softcap is None and not keep_first and sinks is None:
+        y = (_host or _native()).attention_prefill(q, q_stride, kcache, vcache, positions, tiles, block_table, page_size, window or 0, scale,
+                                                   nh, nkv, d, ntok, tile_rows, _stream())
+        if y is not False:
+            return y
     _dev(q, kcache, vcache, positions, tiles, block_table, out, sinks)
     _need(sinks is None or (sinks.dtype == torch.float32 and sinks.shape == (nh,)), "attention_prefill: sinks must be float32 (nh,)")
     _need(q.dtype == torch.bfloat16 and kcache.dtype == torch.bfloat16 and vcache.dtype == torch.bfloat16,
@@ -1307,23 +1387,22 @@ def attention_prefill(q, q_stride, kcache, vcache, positions, tiles, block_table
         out = torch.empty((ntok, nh * d), dtype=q.dtype, device=q.device)
     _need(out.shape == (ntok, nh * d) and out.dtype == q.dtype, "attention_prefill: out has the wrong shape or type")
     nt = tiles.shape[1]
-    _check(lib().gs_attention_prefill(_p(q), c_int(q_stride), _p(kcache), _p(vcache), _p(positions), _p(tiles[0]),
-                                      _p(tiles[1]), _p(tiles[2]), c_int(nt), _p(block_table),
-                                      c_int(block_table.shape[1]), c_int(page_size), c_int(window or 0), c_float(scale),
-                                      _p(out), c_int(nh), c_int(nkv), c_int(d), c_int(tile_rows), c_int(chunk or 0),
-                                      c_int(1 if sink else 0), c_float(softcap or 0.0), c_int(keep_first or 0), _p(sinks),
+    _check(lib().gs_attention_prefill(_p(q), q_stride, _p(kcache), _p(vcache), _p(positions), *_tile_rows(tiles), nt, _p(block_table),
+                                      block_table.shape[1], page_size, window or 0, scale,
+                                      _p(out), nh, nkv, d, tile_rows, chunk or 0,
+                                      1 if sink else 0, softcap or 0.0, keep_first or 0, _p(sinks),
                                       _stream()))
     return out
 
 
 def attention_prefill_wide_supports(nh: int, nkv: int, d: int) -> bool:
-    return bool(lib().gs_attention_prefill_wide_supports(c_int(nh), c_int(nkv), c_int(d)))
+    return bool(lib().gs_attention_prefill_wide_supports(nh, nkv, d))
 
 
 def attention_prefill_wide_rows(nh: int, nkv: int) -> int:
     """The most queries a block of :func:`attention_prefill_wide` holds for these head counts when it walks the keys
     whole (half as many with the keys in two halves)."""
-    return int(lib().gs_attention_prefill_wide_rows(c_int(nh), c_int(nkv)))
+    return int(lib().gs_attention_prefill_wide_rows(nh, nkv))
 
 
 def attention_prefill_wide(q, q_stride, kcache, vcache, positions, tiles, block_table, page_size, window, scale, nh, nkv,
@@ -1352,8 +1431,7 @@ def attention_prefill_wide(q, q_stride, kcache, vcache, positions, tiles, block_
         out = torch.empty((ntok, nh * d), dtype=q.dtype, device=q.device)
     _need(out.shape == (ntok, nh * d) and out.dtype == q.dtype, "attention_prefill_wide: out has the wrong shape or type")
     nt = tiles.shape[1] // wq
-    _check(lib().gs_attention_prefill_wide(_p(q), q_stride, _p(kcache), _p(vcache), _p(positions), _p(tiles[0]),
-                                           _p(tiles[1]), _p(tiles[2]), nt, _p(block_table),
+    _check(lib().gs_attention_prefill_wide(_p(q), q_stride, _p(kcache), _p(vcache), _p(positions), *_tile_rows(tiles), nt, _p(block_table),
                                            block_table.shape[1], page_size, kcache.shape[0],
                                            window or 0, scale, _p(out), nh, nkv, d, rows, key_splits, _stream()))
     return out

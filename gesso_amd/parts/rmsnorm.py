@@ -50,7 +50,7 @@ class ResidualStream:
             if w is None or w.dtype != self.res.dtype or w.shape != (self.res.shape[1],):
                 self.pending, self.ssq = rt.linear(out.x, out.w), None
             else:
-                self.xs, self.ssq = rt.ops.gemm_mid_residual(out.x, out.w, rt.tiles_of(out.w), self.res, w)
+                self.xs, self.ssq = rt.ops.gemm_mid_residual(out.x, out.w, rt.tiles_of(out.w), self.res, w, checked=True)
                 self.xs_for = next_norm
         elif isinstance(out, DeferredLinear) and out.parts:
             # some hundred rows: the same in two kernels, the rows normed by the second

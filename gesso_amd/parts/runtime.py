@@ -198,7 +198,7 @@ class Runtime:
         out_dtype = out_dtype or self.dtype
         if isinstance(x, ops.LazyNorm):
             if bias is None and self.keep_lazy(x) and ops.lazy_ok(x, w):
-                return ops.gemm_skinny(x, w, out_dtype=out_dtype, out=out, wt=self.tiles_of(w))
+                return ops.gemm_skinny(x, w, out_dtype=out_dtype, out=out, wt=self.tiles_of(w), checked=True)
             x = x.materialize()
         if isinstance(x, ops.TiledRows) and not (bias is None and ops.skinny_ok(x, w)):
             x = x.rows()
@@ -207,12 +207,20 @@ class Runtime:
             # the matrix cores' float32 sums, then the bias and one rounding
             return ops.add_bias(self.linear(x, w, out_dtype=torch.float32), bias, out_dtype, out)
         if x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and bias is None:
+            if out is None:
+                y = ops.gemm_skinny_plain(x, w, self.tiles_of(w), out_dtype)
+                if y is not False:
+                    return y
             if ops.skinny_ok(x, w):
-                return ops.gemm_skinny(x, w, out_dtype=out_dtype, out=out, wt=self.tiles_of(w))
+                return ops.gemm_skinny(x, w, out_dtype=out_dtype, out=out, wt=self.tiles_of(w), checked=True)
             library = out_dtype == torch.bfloat16 and not self.no_library and self.many_rows != "own"
             if library and self.many_rows == "auto":
                 wt = self.tiles_of(w)
-                if ops.mid_ok(x, w, wt, out=out):
+                if out is None:
+                    y = ops.gemm_mid_plain(x, w, wt)
+                    if y is not False:
+                        return y
+                elif ops.mid_ok(x, w, wt, out=out):
                     return ops.gemm_mid(x, w, wt, out=out, checked=True)
             if library:
                 return self._library_product(x, w, out)
@@ -254,22 +262,26 @@ class Runtime:
         if isinstance(x, ops.LazyNorm):
             if not self.fused and x.xs is not None:
                 # some hundred rows, weighted by the product before
-                wt = self.tiles_of(w13)
-                if ops.mid_scaled_ok(x, w13, wt):
-                    return ops.gemm_mid_swiglu_scaled(x, w13, wt)
+                y = ops.gemm_mid_swiglu_scaled_plain(x, w13, self.tiles_of(w13))
+                if y is not False:
+                    return y
             if self.keep_lazy(x) and ops.lazy_ok(x, w13):
-                return ops.gemm_skinny(x, w13, swiglu=True, wt=self.tiles_of(w13), out=tiled)
+                return ops.gemm_skinny(x, w13, swiglu=True, wt=self.tiles_of(w13), out=tiled, checked=True)
             x = x.materialize()
+        if not tiled:
+            y = ops.gemm_skinny_plain(x, w13, self.tiles_of(w13), torch.bfloat16, True)
+            if y is not False:
+                return y
         if ops.skinny_ok(x, w13):
-            return ops.gemm_skinny(x, w13, swiglu=True, wt=self.tiles_of(w13), out=tiled)
+            return ops.gemm_skinny(x, w13, swiglu=True, wt=self.tiles_of(w13), out=tiled, checked=True)
         x = self.dense(x)
         if ((self.many_rows == "own" or (self.no_library and self.many_rows != "library"))
                 and self.dtype == torch.bfloat16 and ops.mfma_ok(x, w13) and w13.shape[0] % 2 == 0):
             return ops.gemm_mfma(x, w13, swiglu=True)          # gate|up never goes to memory
         if self.many_rows == "auto" and not self.no_library:
-            wt = self.tiles_of(w13)
-            if ops.mid_ok(x, w13, wt, swiglu=True):
-                return ops.gemm_mid(x, w13, wt, swiglu=True, checked=True)
+            y = ops.gemm_mid_plain(x, w13, self.tiles_of(w13), True)
+            if y is not False:
+                return y
         return ops.swiglu(self.linear(x, w13))
 
     def swiglu_takes_weighted(self, rows: int, w13: torch.Tensor) -> bool:
