@@ -137,7 +137,7 @@ struct Crossing {
 // scales that passes 0 and 1 use here: NUC_G0 sums for the first byte (0x3B, standing for everything below 2^-63, to
 // 0x3F: a weight is at most 1), then 256 for the second byte under each first byte from 0x3C on; after these
 // NUC_GHIST sums the counts, in the same order.  Where the first byte's crossing falls below 2^-63 the passes start
-// again and read the row themselves.
+// again and read the row themselves.  (Under a first byte only the buckets are filled in which a nucleus can end.)
 // Above its low NUC_COUNT bits a count holds a bit for each span of NUC_SPAN ids that has a weight in that bucket, so that the
 // ids of a bucket are looked for where there are any.  Rows longer than NUC_SPANS spans have no marks (nuc_marked): there the
 // whole word is the count, which may itself reach beyond NUC_COUNT bits.
@@ -558,12 +558,13 @@ __global__ __launch_bounds__(SAMP_THREADS) void choose_weights_kernel(
     int nparts, unsigned long long* __restrict__ ghist) {
   __shared__ unsigned long long lm[NUC_GHIST];
   __shared__ int lc[NUC_GHIST];
+  __shared__ double scale1[4];
   const int row = blockIdx.y;
-  const double T = temperature[row];
-  if (!(T > 0.0) || bad0[row]) return;
   const float* x = logits + (size_t)row * V;
-  const double hi = (double)x[amax[row]];
   const int j0 = blockIdx.x * WIDE_SPAN + threadIdx.x * WIDE_CH;
+  // (all asked for at once, also for a row that turns out not to draw: a block is a chain of round trips otherwise)
+  const double T = temperature[row], P = top_p ? top_p[row] : 1.0;
+  const int flagged = bad0[row], best = amax[row];
   float xv[WIDE_CH];
   if (j0 + WIDE_CH <= V && ((reinterpret_cast<uintptr_t>(x + j0) & 15) == 0)) {
     const float4 v = *reinterpret_cast<const float4*>(x + j0);
@@ -572,28 +573,46 @@ __global__ __launch_bounds__(SAMP_THREADS) void choose_weights_kernel(
 #pragma unroll
     for (int k = 0; k < WIDE_CH; ++k) xv[k] = j0 + k < V ? x[j0 + k] : -INFINITY;
   }
+  const double hi = (double)x[best];
+  if (!(T > 0.0) || flagged) return;
+  // (x - max) / T by T's reciprocal, the quotient corrected by what its product with T leaves (Markstein: with the reciprocal rounded
+  // correctly the corrected quotient is the correctly rounded one, what a division gives, at three operations instead of some
+  // fifteen); temperatures so far out that the reciprocal or the quotient leaves the range are divided by.
+  const bool ordinary = T > 1e-100 && T < 1e100;
+  const double inv = 1.0 / T;
   double w[WIDE_CH], p = 0.0;
 #pragma unroll
   for (int k = 0; k < WIDE_CH; ++k) {
-    w[k] = j0 + k < V ? exp(((double)xv[k] - hi) / T) : 0.0;
+    const double a = (double)xv[k] - hi, q = a * inv;
+    w[k] = j0 + k < V ? exp(ordinary ? fma(fma(-q, T, a), inv, q) : a / T) : 0.0;
     p += w[k];
   }
   part[(size_t)row * nparts + blockIdx.x * SAMP_THREADS + threadIdx.x] = p;
-  if (wbuf && top_p && top_p[row] < 1.0) {
+  if (wbuf && P < 1.0) {
+    double* at = wbuf + (size_t)row * V + j0;
+    typedef double __attribute__((ext_vector_type(2))) pair_t;
+    if (j0 + WIDE_CH <= V && (reinterpret_cast<uintptr_t>(at) & 15) == 0) {
 #pragma unroll
-    for (int k = 0; k < WIDE_CH; ++k)
-      if (j0 + k < V) wbuf[(size_t)row * V + j0 + k] = w[k];
+      for (int k = 0; k < WIDE_CH; k += 2) *reinterpret_cast<pair_t*>(at + k) = pair_t{w[k], w[k + 1]};
+    } else {
+#pragma unroll
+      for (int k = 0; k < WIDE_CH; ++k)
+        if (j0 + k < V) at[k] = w[k];
+    }
     if (ghist) {
       // the histograms of the weights' first two bytes, as passes 0 and 1 of radix_descend make them (same scales,
       // integer sums): in LDS for this block's ids, then added to the row's
+      int lv = 1;
+      while ((1 << lv) < V && lv < 30) ++lv;
+      const double scale0 = exp2((double)(62 - lv));
       for (int i = threadIdx.x; i < NUC_GHIST; i += blockDim.x) {
         lm[i] = 0ull;
         lc[i] = 0;
       }
+      // the scales of the second byte's sums, one for each first byte (a division a weight otherwise)
+      if (threadIdx.x < 4)
+        scale1[threadIdx.x] = scale0 / __longlong_as_double((long long)(((unsigned long long)(0x3C + threadIdx.x) << 56) | ((1ull << 56) - 1ull)));
       __syncthreads();
-      int lv = 1;
-      while ((1 << lv) < V && lv < 30) ++lv;
-      const double scale0 = exp2((double)(62 - lv));
       // The first byte has five sums, and nearly all of a wavefront's weights share two of them: an atomic add a weight would
       // queue up on one address (150 rows of 65,536 drawing: 83 us a step; like this 56; 12 rows: 16 and 11).  So a wavefront adds up
       // its weights of each first byte that it holds (integers: the order does not matter) and one lane adds the sum.  In rows of two
@@ -630,14 +649,21 @@ __global__ __launch_bounds__(SAMP_THREADS) void choose_weights_kernel(
           atomicAdd(&lc[f], held);
         }
       }
+      // The second byte's sums only of weights at which the nucleus can end: the weights below (1 - P) / 2V add up to less than half
+      // of what the nucleus leaves out (the whole mass is at least the maximum's, 1), so neither its edge nor a draw within it lies
+      // among them (where (1 - P) / 2 is well above what rounding to integers can add up to; rows of 65,536: 2^-31).  (150 rows of
+      // 65,536 at P = 0.9: 57.2 us with all weights, 51.4; 47.4 with the reciprocal, the scales from LDS, stores of two weights and
+      // all loads asked for at once.)
+      const double left_out = 0.5 * (1.0 - P);
+      const unsigned long long least =
+          left_out > exp2((double)(2 * lv - 61)) ? (unsigned long long)__double_as_longlong(left_out / (double)V) >> 48 : 0ull;
 #pragma unroll
       for (int k = 0; k < WIDE_CH; ++k) {
-        if (i0[k] < 1) continue;
         const unsigned long long bits = (unsigned long long)__double_as_longlong(w[k]);
+        if (i0[k] < 1 || (bits >> 48) < least) continue;
         const int b0 = i0[k] + 0x3B;
-        const double wmax = __longlong_as_double((long long)(((unsigned long long)b0 << 56) | ((1ull << 56) - 1ull)));
         const int i1 = NUC_G0 + (b0 - 0x3C) * 256 + (int)((bits >> 48) & 0xff);
-        atomicAdd(&lm[i1], (unsigned long long)__double2ll_rn(w[k] * (scale0 / wmax)));
+        atomicAdd(&lm[i1], (unsigned long long)__double2ll_rn(w[k] * scale1[b0 - 0x3C]));
         atomicAdd(&lc[i1], 1);
       }
       __syncthreads();
