@@ -4,7 +4,7 @@
 
 void gs_skinny_run_plain(const void* X, int ldx, int x_tiled, const float* res, const float* ssq, int nb, const float* norm_w,
                          float eps, const void* W, const void* Wt, void* Y, int y_dtype, int ldy, int M, int N, int K,
-                         int epilogue, int y_tiled, hipStream_t stream);
+                         int epilogue, int y_tiled, hipStream_t stream, int squared = 0);
 bool gs_skinny_halves(int N);
 void gs_skinny_run_gated(const void* X, int ldx, int x_tiled, const void* Wt, const float* bias, int act, void* Y, int y_tiled, int M,
                          int N, int K, hipStream_t stream);

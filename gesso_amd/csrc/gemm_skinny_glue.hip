@@ -33,9 +33,10 @@ bool gs_skinny_halves(int N) { return N % 16 == 0 && N / 16 <= 160; }
 
 void gs_skinny_run_plain(const void* X, int ldx, int x_tiled, const float* res, const float* ssq, int nb, const float* norm_w,
                          float eps, const void* W, const void* Wt, void* Y, int y_dtype, int ldy, int M, int N, int K,
-                         int epilogue, int y_tiled, hipStream_t stream) {
+                         int epilogue, int y_tiled, hipStream_t stream, int squared) {
   SkinnyCall c = base(X, ldx, x_tiled, W, Wt, Y, y_dtype, ldy, M, N, K, epilogue, stream);
   c.ex.y_tiled = y_tiled;
+  c.ex.squared = squared;
   if (res || ssq) lazy(c, res, ssq, nb, norm_w, eps);
   // Half tiles (the same bits) where a block of eight weight rows still comes once to a compute unit and K is long enough for the
   // sum over the wavefronts not to bind.  Cold weights, microseconds in half and in whole tiles: 8 rows of 2048 x 8192 13.0 and

@@ -123,6 +123,8 @@ struct SkinnyExtra {
   const float* act_bias; // (N): the gate rows', then the up rows'; or null
   int act;
   int y_tiled;           // EPI 1, 3, 4: Y, EPI 2: xs_out are written as tiled rows (their width a multiple of 32)
+  // EPI 0
+  int squared;           // the first so many columns are stored as the square of their relu, of the rounded product
 };
 
 template <int R, int MT, int WAVES, int PRO, int EPI, int LAYOUT, typename TOut>
@@ -589,6 +591,13 @@ _Pragma("unroll")                                                               
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int n = rowbase[r] + kg * 4;
+      if (EPI == 0 && n < ex.squared) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float z = to_f32(f32_to_bf16(sum[r][i])), u = z > 0.f ? z : 0.f;
+          if (n + i < ex.squared) sum[r][i] = u * u;
+        }
+      }
       if (N - n > 0 && half_ok) store4<TOut>(Yp + (size_t)em * ldy + n, sum[r], N - n);
     }
   } else if (EPI == 4) {

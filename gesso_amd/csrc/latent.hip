@@ -139,6 +139,12 @@ extern "C" int gs_latent_prep(const void* down, int dtype, int ld, int q_off, in
 }
 
 // q (T, ldq): head h at [h (n + r), ...), its last r columns rotated into qa (T, H (c + r)) at [h (c + r) + c, ...).
+// A pair of features turned.  (What is fused is written out: the compiler's choice differs between kernels, and their results with it.)
+__device__ __forceinline__ void turn_pair(float u, float v, float cs, float sn, float& a, float& b) {
+  a = fmaf(u, cs, -(v * sn));
+  b = fmaf(u, sn, v * cs);
+}
+
 template <typename T>
 __global__ void latent_q_rot_kernel(const T* __restrict__ q, int ldq, int H, int n, int r, int c,
                                     const float* __restrict__ cos_t, const float* __restrict__ sin_t,
@@ -150,8 +156,10 @@ __global__ void latent_q_rot_kernel(const T* __restrict__ q, int ldq, int H, int
     const int h = idx / half, j = idx % half;
     const float u = to_f32(row[h * (n + r) + n + j]), v = to_f32(row[h * (n + r) + n + j + half]);
     const float cs = cos_t[(size_t)pos * half + j], sn = sin_t[(size_t)pos * half + j];
-    dst[h * (c + r) + c + j] = from_f32<T>(u * cs - v * sn);
-    dst[h * (c + r) + c + j + half] = from_f32<T>(v * cs + u * sn);
+    float a, b;
+    turn_pair(u, v, cs, sn, a, b);
+    dst[h * (c + r) + c + j] = from_f32<T>(a);
+    dst[h * (c + r) + c + j + half] = from_f32<T>(b);
   }
 }
 
@@ -248,6 +256,15 @@ __global__ void heads_product_kernel(const TX* __restrict__ X, int ldx, int hx, 
 // operands loaded straight from memory in operand order (lane l: row or weight row l % 16, eight consecutive k at
 // 8 (l / 16)); a head's weight is small and stays in the caches, so nothing is staged.  A wavefront owns 16 MTW rows x
 // 16 NTW columns of one head; the wavefronts of a block own such pieces of their own, and no barrier is needed.
+//
+// `rot` features that follow a head's K in X go, turned by the row's position, behind the head's N in Y: pieces beyond those of the
+// products, a wavefront for the same rows (latent attention's queries; a launch of its own took 4.4 us a layer of a step).
+struct HeadsRot {
+  int rot;
+  const float* cos_t;      // (positions, rot / 2)
+  const float* sin_t;
+  const int* positions;    // (M)
+};
 typedef __attribute__((ext_vector_type(8))) __bf16 hp_bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float hp_f32x4_t;
 typedef __attribute__((ext_vector_type(4))) unsigned hp_u32x4_t;
@@ -256,13 +273,29 @@ template <int NTW, int MTW, int DEPTH>
 __global__ __launch_bounds__(256) void heads_product_mfma_kernel(const bf16* __restrict__ X, int ldx, int hx,
                                                                  const bf16* __restrict__ W, bf16* __restrict__ Y,
                                                                  int ldy, int hy, const bf16* __restrict__ G, int ldg,
-                                                                 int gate_each, int M, int N, int K) {
+                                                                 int gate_each, int M, int N, int K, HeadsRot hr) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, g = lane >> 4;
   const int h = blockIdx.y;
   const int mtiles = (M + 16 * MTW - 1) / (16 * MTW), ngroups = (N + 16 * NTW - 1) / (16 * NTW);
   const int item = blockIdx.x * (blockDim.x >> 6) + wave;
-  if (item >= mtiles * ngroups) return;
   const int m0 = (item % mtiles) * 16 * MTW, n0 = (item / mtiles) * 16 * NTW;
+  if (item >= mtiles * ngroups) {
+    if (hr.rot == 0 || item >= mtiles * (ngroups + 1)) return;
+    const int half = hr.rot / 2, rows = M - m0 < 16 * MTW ? M - m0 : 16 * MTW;
+    for (int p = lane; p < rows * half; p += 64) {
+      const int m = m0 + p / half, j = p % half;
+      const bf16* x = X + (size_t)m * ldx + (size_t)h * hx + K + j;
+      const float u = to_f32(x[0]), v = to_f32(x[half]);
+      const size_t at = (size_t)hr.positions[m] * half + j;
+      const float cs = hr.cos_t[at], sn = hr.sin_t[at];
+      bf16* y = Y + (size_t)m * ldy + (size_t)h * hy + N + j;
+      float a, b;
+      turn_pair(u, v, cs, sn, a, b);
+      y[0] = f32_to_bf16(a);
+      y[half] = f32_to_bf16(b);
+    }
+    return;
+  }
   const bf16* xp[MTW];
 #pragma unroll
   for (int i = 0; i < MTW; ++i) {
@@ -325,9 +358,8 @@ __global__ __launch_bounds__(256) void heads_product_mfma_kernel(const bf16* __r
     }
 }
 
-extern "C" int gs_heads_product(const void* X, int x_dtype, int ldx, int hx, const void* W, int w_dtype, void* Y,
-                                int ldy, int hy, const void* G, int ldg, int gate_each, int M, int N, int K, int H,
-                                hipStream_t stream) {
+static int heads_product(const void* X, int x_dtype, int ldx, int hx, const void* W, int w_dtype, void* Y, int ldy, int hy, const void* G,
+                         int ldg, int gate_each, int M, int N, int K, int H, HeadsRot hr, hipStream_t stream) {
   GS_REQUIRE(M >= 0 && N > 0 && K > 0 && H > 0, "heads_product: bad sizes M=%d N=%d K=%d H=%d", M, N, K, H);
   GS_REQUIRE(H <= 65535 && gs_ceil_div(M, HP_TM) <= 65535, "heads_product: too many heads or rows for one launch");
   GS_REQUIRE((long)(H - 1) * hx + K <= ldx && (long)(H - 1) * hy + N <= ldy,
@@ -339,7 +371,7 @@ extern "C" int gs_heads_product(const void* X, int x_dtype, int ldx, int hx, con
     // few rows: narrow pieces, so that a head's weight is spread over more wavefronts; many: 32 x 64 a wavefront
     const int ntw = M <= 64 ? 1 : 4, mtw = M <= 64 ? 1 : 2;
     const int mtiles = gs_ceil_div(M, 16 * mtw);
-    const long items = (long)mtiles * gs_ceil_div(N, 16 * ntw);
+    const long products = (long)mtiles * gs_ceil_div(N, 16 * ntw), items = products + (hr.rot ? mtiles : 0);
     GS_REQUIRE(items + 1 < (1L << 31), "heads_product: too many tiles");
     // Up to 64 rows, all of K in flight up to 512, in forms of 2, 4 and 16 steps of 32 k (8 rows, 16 heads of 512 x 128 and 128 x 512
     // in a step: 4.7 us each in the mean, four steps at a time, each waiting for its own, 7.3).  Steps beyond K load the row's start
@@ -348,14 +380,14 @@ extern "C" int gs_heads_product(const void* X, int x_dtype, int ldx, int hx, con
     // quarter of the steps, 9.7 and 8.2; 17 rows, 512 pieces, 5.0 and 4.6; 33 rows, 16 of 128 x 384, 384 pieces, 0.86 of it).  So
     // more pieces than units go four steps at a time unless what the form adds is little.
     const int steps = gs_ceil_div(K, 32), depth = steps <= 2 ? 2 : steps <= 4 ? 4 : 16, added = gs_ceil_div(steps, depth) * depth - steps;
-    const long pieces = items * H;
+    const long pieces = products * H;
     const bool held = pieces <= 256 || pieces * added <= 170L * steps;
     // (few pieces: a wavefront a block, so that they spread over as many compute units)
     const int waves = ntw == 1 && held && pieces < 1024 ? 1 : 4;
     dim3 grid((unsigned)gs_ceil_div(items, waves), H);
 #define HP_RUN(NTW, MTW, DEPTH)                                                                                              \
   heads_product_mfma_kernel<NTW, MTW, DEPTH><<<grid, 64 * waves, 0, stream>>>((const bf16*)X, ldx, hx, (const bf16*)W, (bf16*)Y, \
-                                                                              ldy, hy, (const bf16*)G, ldg, gate_each, M, N, K)
+                                                                              ldy, hy, (const bf16*)G, ldg, gate_each, M, N, K, hr)
     // (many rows: two steps at a time, an odd number of them one at a time: 333 rows of 16 heads of 96 x 96 5.5 us, by twos 5.8)
     if (ntw == 4) { if (steps % 2) HP_RUN(4, 2, 1); else HP_RUN(4, 2, 2); }
     else if (!held) HP_RUN(1, 1, 1);
@@ -365,6 +397,11 @@ extern "C" int gs_heads_product(const void* X, int x_dtype, int ldx, int hx, con
 #undef HP_RUN
     GS_LAUNCH_CHECK("heads_product_mfma");
     return 0;
+  }
+  if (hr.rot) {
+    // (a product of its own kind for the rest: the turned features by their own kernel)
+    const int rc = gs_latent_q_rot(X, x_dtype, ldx, H, K, hr.rot, N, hr.cos_t, hr.sin_t, hr.positions, Y, M, stream);
+    if (rc) return rc;
   }
   dim3 grid(gs_ceil_div(N, HP_TN), gs_ceil_div(M, HP_TM), H);
   if (x_dtype == GS_F32 && w_dtype == GS_F32)
@@ -380,6 +417,22 @@ extern "C" int gs_heads_product(const void* X, int x_dtype, int ldx, int hx, con
     GS_REQUIRE(false, "heads_product: unsupported types %d %d", x_dtype, w_dtype);
   GS_LAUNCH_CHECK("heads_product");
   return 0;
+}
+
+extern "C" int gs_heads_product(const void* X, int x_dtype, int ldx, int hx, const void* W, int w_dtype, void* Y,
+                                int ldy, int hy, const void* G, int ldg, int gate_each, int M, int N, int K, int H,
+                                hipStream_t stream) {
+  return heads_product(X, x_dtype, ldx, hx, W, w_dtype, Y, ldy, hy, G, ldg, gate_each, M, N, K, H, HeadsRot{}, stream);
+}
+
+// The same without gates and, in the same launch where the matrix cores take it, gs_latent_q_rot: X's rows are H heads of K + rot
+// features, Y's H heads of N + rot.
+extern "C" int gs_heads_product_rot(const void* X, int x_dtype, int ldx, const void* W, int w_dtype, void* Y, int M, int N, int K, int H,
+                                    int rot, const float* cos_t, const float* sin_t, const int* positions, hipStream_t stream) {
+  GS_REQUIRE(rot > 0 && rot % 2 == 0 && cos_t && sin_t && positions, "heads_product_rot: %d features to turn, tables and positions", rot);
+  GS_REQUIRE(H > 0 && (long)H * (K + rot) <= ldx, "heads_product_rot: rows of %d hold no %d heads of %d", ldx, H, K + rot);
+  return heads_product(X, x_dtype, ldx, K + rot, W, w_dtype, Y, H * (N + rot), N + rot, nullptr, 0, 0, M, N, K, H,
+                       HeadsRot{rot, cos_t, sin_t, positions}, stream);
 }
 
 // ---------------------------------------------------------------------------------------------------------------

@@ -1501,6 +1501,21 @@ def latent_q_rot(q, H, n, r, c, cos, sin, positions, qa) -> None:
                                  _stream()))
 
 
+def heads_product_rot(q, w, qa, r: int, cos, sin, positions) -> None:
+    """:func:`heads_product` of the first ``K`` features of every head of ``q (T, H (K + r))`` into the first ``N`` columns of every
+    head of ``qa (T, H (N + r))``, ``w (H, N, K)``, and :func:`latent_q_rot` of the others: in one launch where it can."""
+    _dev(q, w, positions, qa, cos, sin)
+    H, N, K = w.shape
+    T = q.shape[0]
+    _need(r > 0 and q.shape == (T, H * (K + r)) and qa.shape == (T, H * (N + r)) and qa.dtype == q.dtype,
+          "heads_product_rot: q is (T, H (K + r)), qa (T, H (N + r)) of one type")
+    _i32(positions, T, "positions")
+    _need(cos.dtype == torch.float32 and sin.shape == cos.shape and cos.dim() == 2 and cos.shape[1] == r // 2,
+          "heads_product_rot: cos and sin are float32 (positions, r / 2)")
+    _check(lib().gs_heads_product_rot(_p(q), _dt(q), q.stride(0), _p(w), _dt(w), _p(qa), T, N, K, H, r, _p(cos), _p(sin),
+                                      _p(positions), _stream()))
+
+
 def heads_product(x, hx: int, w, y, hy: int, K: int, gate=None, gate_each: bool = False) -> torch.Tensor:
     """``y[t, h hy : h hy + N] = w[h] @ x[t, h hx : h hx + K]`` for every head ``h`` of ``w (H, N, K)``, float32 sums in
     a fixed order; with ``gate (T, >= H)`` the result of head ``h`` is multiplied by ``sigmoid(gate[t, h])``, with
@@ -1544,6 +1559,19 @@ def attention_latent(qa, cache, positions, seq_of_token, block_table, page_size,
 
 
 # ---------------------------------------------------------------------- feed-forwards routed by a table
+
+def gemm_skinny_squared(x: torch.Tensor, w: torch.Tensor, squared: int, wt=None) -> torch.Tensor:
+    """``x @ w.T`` in bfloat16 for products :func:`skinny_ok` takes, the first ``squared`` columns as the square of their relu
+    (what :func:`relu_squared` makes of them)."""
+    _dev(w, wt)
+    M, K = x.shape
+    N = w.shape[0]
+    _need(isinstance(x, torch.Tensor) and x.is_cuda and skinny_ok(x, w) and w.shape == (N, K) and 0 < squared <= N,
+          "gemm_skinny_squared: operands must be bfloat16, at most 64 rows, K a multiple of 8, aligned")
+    out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+    _check(lib().gs_gemm_skinny_squared(_p(x), x.stride(0) if M > 1 else K, _p(w), _p(wt), _p(out), N, M, N, K, squared, _stream()))
+    return out
+
 
 def relu_squared(x: torch.Tensor, F: int) -> torch.Tensor:
     """``relu(x[:, :F])^2`` as contiguous rows ``(T, F)``."""

@@ -113,9 +113,12 @@ class LatentAttention(Part):
                                 ctx.seq_of_token, cache.block_table, cache.page_size, cache.k, write_kv=cache.write)
             q = rt.linear(a, self.w_uq)
             qa = (torch.empty if n else torch.zeros)((T, H * (c + r)), dtype=q.dtype, device=q.device)
-            if n:
-                ops.heads_product(q, n + r, self.uk_t, qa, c + r, n)
-            ops.latent_q_rot(q, H, n, r, c, pos.cos, pos.sin, ctx.positions, qa)
+            if n and r:
+                ops.heads_product_rot(q, self.uk_t, qa, r, pos.cos, pos.sin, ctx.positions)
+            else:
+                if n:
+                    ops.heads_product(q, n + r, self.uk_t, qa, c + r, n)
+                ops.latent_q_rot(q, H, n, r, c, pos.cos, pos.sin, ctx.positions, qa)
         with rt.stage("attn_core"):
             mixed = self.attend(qa, ctx, cache)
         o = torch.empty((T, H * dv), dtype=mixed.dtype, device=mixed.device)

@@ -228,6 +228,16 @@ class Runtime:
                 return ops.gemm_mfma(x, w, out_dtype=out_dtype, out=out)
         return ops.gemm_tiled(x, w, bias, out_dtype=out_dtype, out=out)
 
+    def linear_squared(self, x: torch.Tensor, w: torch.Tensor, columns: int):
+        """``x @ w.T`` and the squares of the relus of its first ``columns`` columns.  (For few rows by the product itself: what it
+        returns holds the squares in their place then.)"""
+        ops = self.ops
+        if isinstance(x, torch.Tensor) and columns % 8 == 0 and w.shape[0] % 8 == 0 and ops.skinny_ok(x, w):
+            y = ops.gemm_skinny_squared(x, w, columns, self.tiles_of(w))
+            return y, y[:, :columns]
+        y = self.linear(x, w)
+        return y, ops.relu_squared(y, columns)
+
     def narrow_linear(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         """``x @ w.T`` in float32 for a weight of few rows (the gates of a few heads, a bottleneck): for more rows than the
         weight-streaming kernel takes, by the kernel that shares K out between a block's wavefronts."""

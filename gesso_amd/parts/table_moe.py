@@ -62,8 +62,8 @@ class TableMoE(Part):
         shared = gate = None
         if self.w_sup is not None:
             with rt.stage("ffn_shared"):
-                inner = rt.linear(x, self.w_sup)                       # [shared up | gate]
-                shared = rt.linear(ops.relu_squared(inner, s.shared_ff), self.w_sdown)
+                inner, squared = rt.linear_squared(x, self.w_sup, s.shared_ff)             # [shared up | gate]
+                shared = rt.linear(squared, self.w_sdown)
                 gate = inner[:, s.shared_ff:] if s.shared_gate else None
         if shared is not None and gate is None:
             # an ungated shared expert: sigmoid(large) = 1
