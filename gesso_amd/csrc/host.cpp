@@ -2,9 +2,10 @@
 //
 // A short prompt's step is some 115 calls, and what stands between two of them is the host: a call of the Python functions takes some
 // 10 us, of which the launch itself is 2 (LFM2-350M sizes, 13 tokens 1,690 us a step on the host, with these functions 1,090; 333
-// tokens with all logits 1,590 and 1,220, of which the device needs 1,130).  A function here takes the operands of one call in its plainest form (ordinary tensors, a result made
-// here), checks all that the Python function of the same name checks, makes the result and launches.  Whatever is in another form,
-// or wrong, comes back as False, and the Python function goes on: it handles the other forms and words the errors.
+// tokens with all logits 1,590 and 1,220, of which the device needs 1,130).  A function here takes the operands of one call in its
+// plainest form (ordinary tensors, a result made here), checks all that the Python function of the same name checks, makes the
+// result and launches.  Whatever is in another form, or wrong, comes back as False, and the Python function goes on: it handles the
+// other forms and words the errors.
 #include <Python.h>
 
 #include <ATen/ATen.h>
