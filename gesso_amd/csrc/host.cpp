@@ -3,9 +3,9 @@
 // A short prompt's step is some 115 calls, and what stands between two of them is the host: a call of the Python functions takes some
 // 10 us, of which the launch itself is 2 (LFM2-350M sizes, 13 tokens 1,690 us a step on the host, with these functions 1,090; 333
 // tokens with all logits 1,590 and 1,220, of which the device needs 1,130).  A function here takes the operands of one call in its
-// plainest form (ordinary tensors, a result made here), checks all that the Python function of the same name checks, makes the
-// result and launches.  Whatever is in another form, or wrong, comes back as False, and the Python function goes on: it handles the
-// other forms and words the errors.
+// plainest form (ordinary tensors, a result made here or room for it), checks all that the Python function of the same name checks,
+// makes the result and launches.  Whatever is in another form, or wrong, comes back as False, and the Python function goes on: it
+// handles the other forms and words the errors.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -279,22 +279,25 @@ PyObject* qknorm_rope_kv(PyObject* const* a) {
   Py_RETURN_NONE;
 }
 
-// q, q_stride, caches, positions, tiles (3, n), block_table, page_size, window or 0, scale, nh, nkv, d, tokens, rows a tile, stream
+// q, q_stride, caches, positions, tiles (3, n), block_table, page_size, window or 0, scale, nh, nkv, d, tokens, rows a tile, the result's
+// room or None, stream
 PyObject* attention_prefill(PyObject* const* a) {
   bool other = false;
   const at::Tensor &q = tensor(a[0], other), &kc = tensor(a[2], other), &vc = tensor(a[3], other), &pos = tensor(a[4], other),
-                   &tiles = tensor(a[5], other), &table = tensor(a[6], other);
+                   &tiles = tensor(a[5], other), &table = tensor(a[6], other), &room = tensor(a[15], other);
   const int ld = number(a[1]), page = number(a[7]), window = number(a[8]), nh = number(a[10]), nkv = number(a[11]), d = number(a[12]),
             tokens = number(a[13]), rows = number(a[14]);
   const float scale = real(a[9]);
-  const stream_t s = stream(a[15]);
+  const stream_t s = stream(a[16]);
   if (other || PyErr_Occurred() || !is(q, at::kBFloat16) || !q.is_contiguous() || !caches(kc, vc, at::kBFloat16, nkv, page, d)) return other_form();
   if (tokens < 1 || q.numel() < (int64_t)(tokens - 1) * ld + (int64_t)nh * d || !indices(pos, tokens) || !matrix(tiles, at::kInt) ||
       tiles.size(0) != 3 || !tiles.is_contiguous() || !matrix(table, at::kInt) || !table.is_contiguous())
     return other_form();
+  if (room.defined() && !(matrix(room, at::kBFloat16) && room.size(0) == tokens && room.size(1) == (int64_t)nh * d && room.is_contiguous()))
+    return other_form();
   const int n = (int)tiles.size(1);
   const int* at = ints(tiles);
-  at::Tensor out = make(q, {tokens, (int64_t)nh * d}, at::kBFloat16);
+  at::Tensor out = room.defined() ? room : make(q, {tokens, (int64_t)nh * d}, at::kBFloat16);
   launch([&] {
     return attention_prefill_(q.data_ptr(), ld, kc.data_ptr(), vc.data_ptr(), ints(pos), at, at + n, at + 2 * n, n, ints(table), (int)table.size(1),
                               page, window, scale, out.data_ptr(), nh, nkv, d, rows, 0, 0, 0.f, 0, nullptr, s);
@@ -339,7 +342,7 @@ PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyMethodDef methods[] = {{"bind", (PyCFunction)(void*)(&bind), METH_FASTCALL, nullptr},
                          METHOD(add_rmsnorm, 6), METHOD(gemm_skinny, 6), METHOD(gemm_mid, 5), METHOD(gemm_mid_residual, 6),
                          METHOD(gemm_mid_swiglu_scaled, 6), METHOD(gemm_mid_residual_parts, 8), METHOD(short_conv, 10),
-                         METHOD(qknorm_rope_kv, 19), METHOD(attention_prefill, 16), {nullptr, nullptr, 0, nullptr}};
+                         METHOD(qknorm_rope_kv, 19), METHOD(attention_prefill, 17), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef definition = {PyModuleDef_HEAD_INIT, "gesso_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

@@ -1368,9 +1368,9 @@ def attention_prefill(q, q_stride, kcache, vcache, positions, tiles, block_table
     ``tiles``: int32 ``(3, ntiles)``: sequence, first row and number of rows (at most ``tile_rows``, 16 or
     32) of each tile of consecutive queries of one sequence.
     """
-    if out is None and chunk is None and not sink and softcap is None and not keep_first and sinks is None:
+    if chunk is None and not sink and softcap is None and not keep_first and sinks is None:
         y = (_host or _native()).attention_prefill(q, q_stride, kcache, vcache, positions, tiles, block_table, page_size, window or 0, scale,
-                                                   nh, nkv, d, ntok, tile_rows, _stream())
+                                                   nh, nkv, d, ntok, tile_rows, out, _stream())
         if y is not False:
             return y
     _dev(q, kcache, vcache, positions, tiles, block_table, out, sinks)
