@@ -799,13 +799,12 @@ def gemm_mid_swiglu_scaled_plain(x, w13: torch.Tensor, wt):
     return (_host or _native()).gemm_mid_swiglu_scaled(x.xs, x.ssq, x.eps, w13, wt, _stream())
 
 
-def gemm_mid_swiglu_scaled(x, w13: torch.Tensor, wt, checked: bool = False) -> torch.Tensor:
-    """``silu(gate) * up`` in bfloat16 of a lazy norm whose rows come weighted, for products :func:`mid_scaled_ok` takes
-    (``checked``: the caller has asked it)."""
+def gemm_mid_swiglu_scaled(x, w13: torch.Tensor, wt) -> torch.Tensor:
+    """``silu(gate) * up`` in bfloat16 of a lazy norm whose rows come weighted, for products :func:`mid_scaled_ok` takes."""
     y = gemm_mid_swiglu_scaled_plain(x, w13, wt)
     if y is not False:
         return y
-    if not (checked or mid_scaled_ok(x, w13, wt)):
+    if not mid_scaled_ok(x, w13, wt):
         raise KernelError(f"gemm_mid_swiglu_scaled: not a product of this kernel, M={x.shape[0]} N={w13.shape[0]} K={w13.shape[1]}")
     if not (wt.dtype is torch.bfloat16 and wt.is_cuda and wt.is_contiguous()):
         raise KernelError("gemm_mid_swiglu_scaled: the weight's tile-major copy is bfloat16 on the GPU")
