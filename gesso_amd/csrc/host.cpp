@@ -10,6 +10,7 @@
 
 #include <ATen/ATen.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
 
 #include <dlfcn.h>
 
@@ -75,13 +76,30 @@ PyObject* other_form() {
   Py_RETURN_FALSE;
 }
 
+// A tensor as Python's.  It is made before the launch: nothing may fail behind one, or the Python function would make it once more.
+THPObjectPtr result(const at::Tensor& t) {
+  THPObjectPtr y(THPVariable_Wrap(t));
+  if (!y) throw std::bad_alloc();
+  return y;
+}
+
 struct Failed {};                       // an entry point refused: its message is the error
-template <typename F>
-void launch(F&& f) {
+
+// The interpreter's lock let go of, and taken back however the block ends.
+struct Unlocked {
+  PyThreadState* const held = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(held); }
+};
+
+// A launch without the lock.  The operands' addresses are this function's arguments: asking for one can throw (a tensor that has no
+// memory), and does so while the lock is still held.
+template <typename... P, typename... A>
+void launch(int (*entry)(P...), A... a) {
   int rc;
-  Py_BEGIN_ALLOW_THREADS;
-  rc = f();
-  Py_END_ALLOW_THREADS;
+  {
+    const Unlocked unlocked;
+    rc = entry(a...);
+  }
   if (rc != 0) throw Failed();
 }
 
@@ -120,8 +138,9 @@ PyObject* add_rmsnorm(PyObject* const* a) {
   if (delta.defined() && !(activations(delta) && delta.is_contiguous() && delta.sizes() == res.sizes())) return other_form();
   const int T = (int)res.size(0), H = (int)res.size(1);
   at::Tensor out = make(res, {T, H}, type == BF16 ? at::kBFloat16 : at::kFloat);
-  launch([&] { return add_rmsnorm_(floats(res), at_(delta), delta.defined() ? kind(delta) : type, floats(w), eps, out.data_ptr(), type, nullptr, T, H, s); });
-  return THPVariable_Wrap(std::move(out));
+  THPObjectPtr y = result(out);
+  launch(add_rmsnorm_, floats(res), at_(delta), delta.defined() ? kind(delta) : type, floats(w), eps, out.data_ptr(), type, nullptr, T, H, s);
+  return y.release();
 }
 
 // x, w, its tile-major copy or None, whether the result is bfloat16, whether SwiGLU, stream
@@ -137,11 +156,10 @@ PyObject* gemm_skinny(PyObject* const* a) {
     return other_form();
   const int64_t cols = swiglu ? N / 2 : N;
   at::Tensor out = make(x, {M, cols}, type == BF16 ? at::kBFloat16 : at::kFloat);
-  launch([&] {
-    return gemm_skinny_(x.data_ptr(), M > 1 ? (int)x.stride(0) : (int)K, 0, nullptr, nullptr, 0, nullptr, 0.f, w.data_ptr(), at_(wt), out.data_ptr(),
-                        type, (int)cols, (int)M, (int)N, (int)K, swiglu, 0, s);
-  });
-  return THPVariable_Wrap(std::move(out));
+  THPObjectPtr y = result(out);
+  launch(gemm_skinny_, x.data_ptr(), M > 1 ? (int)x.stride(0) : (int)K, 0, nullptr, nullptr, 0, nullptr, 0.f, w.data_ptr(), at_(wt),
+         out.data_ptr(), type, (int)cols, (int)M, (int)N, (int)K, swiglu, 0, s);
+  return y.release();
 }
 
 // bfloat16 rows that do not overlap and the whole weight with its tile-major copy, as the products of some hundred rows take them
@@ -162,8 +180,9 @@ PyObject* gemm_mid(PyObject* const* a) {
   const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0), cols = swiglu ? N / 2 : N;
   if (!gemm_mid_takes_(M, N, K, swiglu)) return other_form();
   at::Tensor out = make(x, {M, cols}, at::kBFloat16);
-  launch([&] { return gemm_mid_(x.data_ptr(), (int)x.stride(0), wt.data_ptr(), out.data_ptr(), cols, M, N, K, swiglu, s); });
-  return THPVariable_Wrap(std::move(out));
+  THPObjectPtr y = result(out);
+  launch(gemm_mid_, x.data_ptr(), (int)x.stride(0), wt.data_ptr(), out.data_ptr(), cols, M, N, K, swiglu, s);
+  return y.release();
 }
 
 bool stream_of(const at::Tensor& res, const at::Tensor& x, const at::Tensor& w) {
@@ -180,10 +199,11 @@ PyObject* gemm_mid_residual(PyObject* const* a) {
   const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0), sums = gemm_mid_residual_sums_(M, N, K);
   if (sums <= 0) return other_form();
   at::Tensor rows = make(x, {M, N}, at::kBFloat16), ssq = make(x, {M, sums}, at::kFloat);
-  launch([&] {
-    return gemm_mid_residual_(x.data_ptr(), (int)x.stride(0), wt.data_ptr(), floats(res), floats(nw), rows.data_ptr(), floats(ssq), M, N, K, s);
-  });
-  return Py_BuildValue("(NN)", THPVariable_Wrap(std::move(rows)), THPVariable_Wrap(std::move(ssq)));
+  const THPObjectPtr first = result(rows), second = result(ssq);
+  THPObjectPtr y(Py_BuildValue("(OO)", first.get(), second.get()));
+  if (!y) return nullptr;
+  launch(gemm_mid_residual_, x.data_ptr(), (int)x.stride(0), wt.data_ptr(), floats(res), floats(nw), rows.data_ptr(), floats(ssq), M, N, K, s);
+  return y.release();
 }
 
 // weighted rows, their partial sums of squares, eps, gate's and up's weight, its tile-major copy, stream
@@ -196,10 +216,9 @@ PyObject* gemm_mid_swiglu_scaled(PyObject* const* a) {
   const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0), sums = (int)ssq.size(1);
   if (ssq.size(0) != M || sums > 128 || sums % 4 != 0 || !gemm_mid_takes_(M, N, K, 1)) return other_form();
   at::Tensor out = make(x, {M, N / 2}, at::kBFloat16);
-  launch([&] {
-    return gemm_mid_swiglu_scaled_(x.data_ptr(), (int)x.stride(0), floats(ssq), sums, eps, wt.data_ptr(), out.data_ptr(), N / 2, M, N, K, s);
-  });
-  return THPVariable_Wrap(std::move(out));
+  THPObjectPtr y = result(out);
+  launch(gemm_mid_swiglu_scaled_, x.data_ptr(), (int)x.stride(0), floats(ssq), sums, eps, wt.data_ptr(), out.data_ptr(), N / 2, M, N, K, s);
+  return y.release();
 }
 
 // x, w, its tile-major copy, the stream, the next norm's weight, eps, parts of K (more than none), stream: the normed rows
@@ -214,11 +233,11 @@ PyObject* gemm_mid_residual_parts(PyObject* const* a) {
   const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0);
   const int64_t sheet = (int64_t)parts * M * N;
   at::Tensor sheets = make(x, {sheet + M}, at::kFloat), normed = make(x, {M, N}, at::kBFloat16);       // (and the new rows' sums of squares)
-  launch([&] {
-    const int rc = gemm_mid_parts_(x.data_ptr(), (int)x.stride(0), wt.data_ptr(), floats(sheets), parts, M, N, K, s);
-    return rc ? rc : residual_from_parts_(floats(sheets), parts, floats(res), floats(sheets) + sheet, floats(nw), eps, normed.data_ptr(), BF16, 0, M, N, s);
-  });
-  return THPVariable_Wrap(std::move(normed));
+  THPObjectPtr y = result(normed);
+  float *part = floats(sheets), *stream_at = floats(res), *next = floats(nw);
+  launch(gemm_mid_parts_, x.data_ptr(), (int)x.stride(0), wt.data_ptr(), part, parts, M, N, K, s);
+  launch(residual_from_parts_, part, parts, stream_at, part + sheet, next, eps, normed.data_ptr(), BF16, 0, M, N, s);
+  return y.release();
 }
 
 // bcx, taps, bias or None, state, seq_of_token, q_start, slots, sequences, whether all bring one token, stream
@@ -235,11 +254,10 @@ PyObject* short_conv(PyObject* const* a) {
   if (!is(state, at::kFloat) || state.dim() != 3 || state.size(1) != H || state.size(2) != W - 1 || !state.is_contiguous()) return other_form();
   if (!indices(seq, T) || !indices(start, nseq + 1) || !indices(slots, nseq)) return other_form();
   at::Tensor out = make(bcx, {T, H}, bcx.scalar_type());
-  launch([&] {
-    return short_conv_(bcx.data_ptr(), kind(bcx), floats(taps), floats(bias), floats(state), ints(seq), ints(start), ints(slots), out.data_ptr(), T,
-                       nseq, H, W, single ? 1 : 0, s);
-  });
-  return THPVariable_Wrap(std::move(out));
+  THPObjectPtr y = result(out);
+  launch(short_conv_, bcx.data_ptr(), kind(bcx), floats(taps), floats(bias), floats(state), ints(seq), ints(start), ints(slots), out.data_ptr(),
+         T, nseq, H, W, single ? 1 : 0, s);
+  return y.release();
 }
 
 // caches (pages, nkv, page_size, d) of one type and one shape
@@ -271,11 +289,9 @@ PyObject* qknorm_rope_kv(PyObject* const* a) {
   }
   if (!indices(pos, T) || !indices(seq, T) || !matrix(table, at::kInt) || !table.is_contiguous()) return other_form();
   if (!caches(kc, vc, qkv.scalar_type(), nkv, page, d)) return other_form();
-  launch([&] {
-    return qknorm_rope_kv_(qkv.data_ptr(), kind(qkv), floats(qw), floats(kw), eps, floats(cos), floats(sin), rot, pairs ? 1 : 0, most, ints(pos),
-                           ints(seq), ints(table), (int)table.size(1), page, kc.data_ptr(), vc.data_ptr(), T, nh, nkv, d, write ? 1 : 0, d, nullptr,
-                           nullptr, (int)qkv.size(1), 0, nullptr, 0, nullptr, 1, s);
-  });
+  launch(qknorm_rope_kv_, qkv.data_ptr(), kind(qkv), floats(qw), floats(kw), eps, floats(cos), floats(sin), rot, pairs ? 1 : 0, most, ints(pos),
+         ints(seq), ints(table), (int)table.size(1), page, kc.data_ptr(), vc.data_ptr(), T, nh, nkv, d, write ? 1 : 0, d, nullptr,
+         nullptr, (int)qkv.size(1), 0, nullptr, 0, nullptr, 1, s);
   Py_RETURN_NONE;
 }
 
@@ -298,11 +314,10 @@ PyObject* attention_prefill(PyObject* const* a) {
   const int n = (int)tiles.size(1);
   const int* at = ints(tiles);
   at::Tensor out = room.defined() ? room : make(q, {tokens, (int64_t)nh * d}, at::kBFloat16);
-  launch([&] {
-    return attention_prefill_(q.data_ptr(), ld, kc.data_ptr(), vc.data_ptr(), ints(pos), at, at + n, at + 2 * n, n, ints(table), (int)table.size(1),
-                              page, window, scale, out.data_ptr(), nh, nkv, d, rows, 0, 0, 0.f, 0, nullptr, s);
-  });
-  return THPVariable_Wrap(std::move(out));
+  THPObjectPtr y = result(out);
+  launch(attention_prefill_, q.data_ptr(), ld, kc.data_ptr(), vc.data_ptr(), ints(pos), at, at + n, at + 2 * n, n, ints(table), (int)table.size(1),
+         page, window, scale, out.data_ptr(), nh, nkv, d, rows, 0, 0, 0.f, 0, nullptr, s);
+  return y.release();
 }
 
 // ------------------------------------------------------------------ the module

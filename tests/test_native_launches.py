@@ -1,0 +1,75 @@
+"""The module of native launches (``csrc/host.cpp``) where no kernel may run: operands that only look like the GPU's.
+
+No GPU is needed: nothing here gets as far as a launch.
+"""
+import os
+import subprocess
+import sys
+
+import pytest
+
+from gesso_amd.kernels import build
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+# Fake tensors on a device that need not be there; those that vmap batches have types, sizes and strides, and no memory.
+WITHOUT_MEMORY = """
+import sys
+import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+from gesso_amd.kernels import build, ops
+
+native = build.load_host()
+BF, I = torch.bfloat16, torch.int32
+with FakeTensorMode():
+    t = lambda *s, dtype=BF: torch.empty(*s, dtype=dtype, device="cuda")
+    f, i = lambda *s: t(*s, dtype=torch.float32), lambda *s: t(*s, dtype=I)
+    mid = (t(100, 512), t(1024, 512), t(1024, 512))
+    kc = t(4, 2, 4, 64)
+    calls = {
+        "add_rmsnorm": (f(3, 64), t(3, 64), f(64), 1e-5, 1),
+        "gemm_skinny": (t(3, 64), t(32, 64), t(32, 64), 1, 0),
+        "gemm_mid": mid + (0,),
+        "gemm_mid_residual": mid + (f(100, 1024), f(1024)),
+        "gemm_mid_swiglu_scaled": (mid[0], f(100, 8), 1e-5) + mid[1:],
+        "gemm_mid_residual_parts": mid + (f(100, 1024), f(1024), 1e-5, 2),
+        "short_conv": (t(9, 96), f(32, 3), f(32), f(3, 32, 2), i(9), i(3), i(2), 2, 0),
+        "qknorm_rope_kv": (t(9, 512), f(64), f(64), 1e-5, f(16, 32), f(16, 32), 64, i(9), i(9), i(2, 2), 4, kc, kc, 4, 2, 64, 1, 0),
+        "attention_prefill": (t(9, 512), 512, kc, kc, i(9), i(3, 2), i(2, 2), 4, 0, 0.125, 4, 2, 64, 9, 16, None),
+    }
+    args = list(calls[sys.argv[1]])
+    without = [int(v) for v in sys.argv[2:]] or [k for k, a in enumerate(args) if isinstance(a, torch.Tensor)]
+    said = []
+
+    def one(*batched):
+        for k, b in zip(without, batched):
+            args[k] = b
+        said.append(getattr(native, sys.argv[1])(*args, 0))
+        if sys.argv[1] == "add_rmsnorm":
+            ops._stream = lambda: 0
+            ops.add_rmsnorm(*args[:4], BF)
+        return batched[0]
+
+    try:
+        torch.vmap(one)(*[torch.empty(2, *args[k].shape, dtype=args[k].dtype, device="cuda") for k in without])
+    except RuntimeError as err:
+        assert sys.argv[1] == "add_rmsnorm" and "data pointer" in str(err), err
+    else:
+        assert sys.argv[1] != "add_rmsnorm"
+    assert said == [False], said
+print("said no")
+"""
+
+
+# All operands of a call without memory, and the one that is asked for its address last.
+@pytest.mark.parametrize("name,operand", [(n, o) for n, o in (("add_rmsnorm", 0), ("gemm_skinny", 2), ("gemm_mid", 2), ("gemm_mid_residual", 3),
+                                                             ("gemm_mid_swiglu_scaled", 1), ("gemm_mid_residual_parts", 4), ("short_conv", 3),
+                                                             ("qknorm_rope_kv", 11), ("attention_prefill", 6)) for o in (None, o)])
+def test_operands_without_memory_are_another_form(name, operand):
+    """A tensor that has no address is left to the Python function, which raises torch's own error: in a process of its own, which an
+    exception thrown where the interpreter's lock is let go of would end, and which sees no GPU."""
+    if build.find_built() is None:
+        pytest.skip("the library is not built")
+    p = subprocess.run([sys.executable, "-c", WITHOUT_MEMORY, name] + ([] if operand is None else [str(operand)]), cwd=ROOT, capture_output=True,
+                       text=True, timeout=300, env=dict(os.environ, HIP_VISIBLE_DEVICES="-1"))
+    assert p.returncode == 0 and "said no" in p.stdout, (p.returncode, p.stderr[-2000:])
