@@ -134,28 +134,36 @@ def build(force: bool = True, verbose: bool = True) -> str:
             _say(f"  {name} done ({time.time() - t0:.0f} s)")
         return obj
 
+    tmp, host_tmp = lib + f".tmp{os.getpid()}", _host_path(lib) + f".tmp{os.getpid()}"
+
     def compile_host():
-        path = _host_path(lib)
-        tmp = path + f".tmp{os.getpid()}"
-        p = subprocess.run([_cxx()] + HOST_FLAGS + ["-o", tmp, os.path.join(CSRC, "host.cpp")] + HOST_LINK,
+        p = subprocess.run([_cxx()] + HOST_FLAGS + ["-o", host_tmp, os.path.join(CSRC, "host.cpp")] + HOST_LINK,
                            stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, env=env)
         if p.returncode != 0:
             raise KernelError(f"compiling the host module failed:\n{p.stdout[-4000:]}")
-        os.replace(tmp, path)
         if verbose:
             _say(f"  host.cpp done ({time.time() - t0:.0f} s)")
 
     workers = max(1, min(len(srcs), int(os.environ.get("MAX_JOBS", "0")) or (os.cpu_count() or 4), 16))
-    with ThreadPoolExecutor(workers) as pool:
-        host = pool.submit(compile_host)
-        objs = list(pool.map(compile_one, srcs))
-        host.result()
-    tmp = lib + f".tmp{os.getpid()}"
-    p = subprocess.run([hipcc, "--offload-arch=" + ARCH, "-shared", "-fPIC", "-o", tmp] + objs + LINK,
-                       stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, env=env)
-    if p.returncode != 0:
-        raise KernelError(f"linking the HIP extension failed:\n{p.stdout[-4000:]}")
-    os.replace(tmp, lib)
+    try:
+        with ThreadPoolExecutor(workers) as pool:
+            host = pool.submit(compile_host)
+            objs = list(pool.map(compile_one, srcs))
+            host.result()
+        p = subprocess.run([hipcc, "--offload-arch=" + ARCH, "-shared", "-fPIC", "-o", tmp] + objs + LINK,
+                           stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, env=env)
+        if p.returncode != 0:
+            raise KernelError(f"linking the HIP extension failed:\n{p.stdout[-4000:]}")
+        # library, module and digest belong together: nothing is replaced before all is made, and no digest stands beside a
+        # library and a module of two builds
+        if os.path.exists(stamp):
+            os.remove(stamp)
+        os.replace(tmp, lib)
+        os.replace(host_tmp, _host_path(lib))
+    finally:
+        for left in (tmp, host_tmp):
+            if os.path.exists(left):
+                os.remove(left)
     with open(stamp, "w") as f:
         f.write(digest)
     if verbose:
