@@ -9,6 +9,8 @@
 #include <stdio.h>
 #include <string.h>
 
+#include "native_calls.h"
+
 #define GS_F32 0
 #define GS_BF16 1
 
@@ -17,7 +19,6 @@
 // The float32 products add k in chunks of this many, and then the chunks' sums, both in ascending order.
 #define GS_SUM_CHUNK 64
 
-extern "C" const char* gs_last_error();
 void gs_set_error(const char* fmt, ...);
 
 #define GS_REQUIRE(cond, ...)            \

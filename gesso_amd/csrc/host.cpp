@@ -14,30 +14,31 @@
 
 #include <dlfcn.h>
 
+#include "native_calls.h"
+
 namespace {
 
-typedef void* stream_t;
+typedef hipStream_t stream_t;
 enum { F32 = 0, BF16 = 1 };
 
-const char* (*last_error)();
 PyObject* kernel_error;
-int (*add_rmsnorm_)(float*, const void*, int, const float*, float, void*, int, const int*, int, int, stream_t);
-int (*gemm_skinny_)(const void*, int, int, const float*, const float*, int, const float*, float, const void*, const void*, void*, int,
-                    int, int, int, int, int, int, stream_t);
-int (*gemm_mid_takes_)(int, int, int, int);
-int (*gemm_mid_)(const void*, int, const void*, void*, int, int, int, int, int, stream_t);
-int (*gemm_mid_swiglu_scaled_)(const void*, int, const float*, int, float, const void*, void*, int, int, int, int, stream_t);
-int (*gemm_mid_residual_sums_)(int, int, int);
-int (*gemm_mid_residual_)(const void*, int, const void*, float*, const float*, void*, float*, int, int, int, stream_t);
-int (*gemm_mid_parts_)(const void*, int, const void*, float*, int, int, int, int, stream_t);
-int (*residual_from_parts_)(const float*, int, float*, float*, const float*, float, void*, int, int, int, int, stream_t);
-int (*short_conv_)(const void*, int, const float*, const float*, float*, const int*, const int*, const int*, void*, int, int, int, int, int,
-                   stream_t);
-int (*qknorm_rope_kv_)(void*, int, const float*, const float*, float, const float*, const float*, int, int, int, const int*, const int*,
-                       const int*, int, int, void*, void*, int, int, int, int, int, int, const float*, const float*, int, int, const void*,
-                       int, const float*, int, stream_t);
-int (*attention_prefill_)(const void*, int, const void*, const void*, const int*, const int*, const int*, const int*, int, const int*, int,
-                          int, int, float, void*, int, int, int, int, int, int, float, int, const float*, stream_t);
+
+// The library's entry points, found by name.
+decltype(&gs_last_error) last_error;
+#define ENTRY(name) decltype(&gs_##name) name##_
+ENTRY(add_rmsnorm);
+ENTRY(gemm_skinny);
+ENTRY(gemm_mid_takes);
+ENTRY(gemm_mid);
+ENTRY(gemm_mid_swiglu_scaled);
+ENTRY(gemm_mid_residual_sums);
+ENTRY(gemm_mid_residual);
+ENTRY(gemm_mid_parts);
+ENTRY(residual_from_parts);
+ENTRY(short_conv);
+ENTRY(qknorm_rope_kv);
+ENTRY(attention_prefill);
+#undef ENTRY
 
 // ------------------------------------------------------------------ arguments and results
 
@@ -69,7 +70,7 @@ at::Tensor make(const at::Tensor& like, at::IntArrayRef sizes, at::ScalarType ty
 // Numbers as the interpreter holds them (a wrong type leaves a Python error, which `call` turns into "another form").
 int number(PyObject* o) { return (int)PyLong_AsLong(o); }
 float real(PyObject* o) { return (float)PyFloat_AsDouble(o); }
-stream_t stream(PyObject* o) { return PyLong_AsVoidPtr(o); }
+stream_t stream(PyObject* o) { return (stream_t)PyLong_AsVoidPtr(o); }
 
 PyObject* other_form() {
   PyErr_Clear();
@@ -343,9 +344,10 @@ PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
   GET(add_rmsnorm); GET(gemm_skinny); GET(gemm_mid_takes); GET(gemm_mid); GET(gemm_mid_swiglu_scaled); GET(gemm_mid_residual_sums);
   GET(gemm_mid_residual); GET(gemm_mid_parts); GET(residual_from_parts); GET(short_conv); GET(qknorm_rope_kv); GET(attention_prefill);
 #undef GET
-  last_error = (const char* (*)())get("gs_last_error");
-  if (!all) {
-    PyErr_SetString(PyExc_OSError, "the kernel library lacks an entry point");
+  last_error = (decltype(last_error))get("gs_last_error");
+  const auto version = (decltype(&gs_abi_version))get("gs_abi_version");
+  if (!all || version() != GS_ABI_VERSION) {
+    PyErr_SetString(PyExc_OSError, all ? "module and kernel library have other interface versions; build them again" : "the kernel library lacks an entry point");
     return nullptr;
   }
   Py_INCREF(a[1]);

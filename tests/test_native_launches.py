@@ -3,6 +3,8 @@
 No GPU is needed: nothing here gets as far as a launch.
 """
 import os
+import re
+import shutil
 import subprocess
 import sys
 
@@ -73,3 +75,34 @@ def test_operands_without_memory_are_another_form(name, operand):
     p = subprocess.run([sys.executable, "-c", WITHOUT_MEMORY, name] + ([] if operand is None else [str(operand)]), cwd=ROOT, capture_output=True,
                        text=True, timeout=300, env=dict(os.environ, HIP_VISIBLE_DEVICES="-1"))
     assert p.returncode == 0 and "said no" in p.stdout, (p.returncode, p.stderr[-2000:])
+
+
+BINDS = """
+import importlib.util, sys
+spec = importlib.util.spec_from_file_location("gesso_host", sys.argv[1])
+host = importlib.util.module_from_spec(spec)
+spec.loader.exec_module(host)
+try:
+    host.bind(sys.argv[2], ValueError)
+except OSError as err:
+    print("refused:", err)
+"""
+
+
+@pytest.mark.parametrize("names,version,said", [("all", 14, "other interface versions"), ("all", 15, ""), ("some", 15, "lacks an entry point")])
+def test_the_module_binds_to_a_library_of_its_own_version_only(tmp_path, names, version, said):
+    """Against a library of empty functions: one that differs in version is refused, so is one without an entry point."""
+    lib, cc = build.find_built(), shutil.which("gcc") or shutil.which("cc")
+    if lib is None or cc is None:
+        pytest.skip("the library is not built, or no C compiler")
+    with open(os.path.join(build.CSRC, "native_calls.h"), encoding="utf-8") as f:
+        text = f.read()
+    assert f"GS_ABI_VERSION {15} " in text
+    entries = sorted(set(re.findall(r"\b(gs_\w+)\(", text)) - {"gs_abi_version"})
+    assert len(entries) == 13
+    with open(tmp_path / "empty.c", "w") as f:
+        f.write(f"int gs_abi_version(void) {{ return {version}; }}\n" + "".join(f"int {e}(void) {{ return 0; }}\n" for e in entries[names == "some":]))
+    subprocess.run([cc, "-shared", "-fPIC", "-o", str(tmp_path / "empty.so"), str(tmp_path / "empty.c")], check=True, timeout=60)
+    p = subprocess.run([sys.executable, "-c", "import torch\n" + BINDS, build._host_path(lib), str(tmp_path / "empty.so")], cwd=ROOT, capture_output=True,
+                       text=True, timeout=120)
+    assert p.returncode == 0 and (said in p.stdout if said else not p.stdout), (p.stdout, p.stderr[-2000:])
