@@ -39,11 +39,12 @@ LINK = ["-lhipblaslt"]
 
 # the module of host.cpp: compiled against the interpreter and the torch that import it
 HOST_NAME = "gesso_host"
+HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+HOST_LINK = ["-ltorch_python", "-ltorch_cpu", "-lc10", "-ldl"]
+# (where these lie is not part of the digest: a tree may be built on one machine and run on another)
 _TORCH = os.path.dirname(torch.__file__)
-HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-              "-isystem", os.path.join(_TORCH, "include"), "-isystem", os.path.join(_TORCH, "include", "torch", "csrc", "api", "include"),
-              "-isystem", sysconfig.get_paths()["include"]]
-HOST_LINK = ["-L" + os.path.join(_TORCH, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10", "-ldl"]
+_HOST_INCLUDE = [os.path.join(_TORCH, "include"), os.path.join(_TORCH, "include", "torch", "csrc", "api", "include"),
+                 sysconfig.get_paths()["include"]]
 
 _lock = threading.Lock()
 _lib = None
@@ -56,7 +57,7 @@ def sources():
 
 def _digest() -> str:
     h = hashlib.sha256()
-    h.update(" ".join(FLAGS + LINK + [torch.__version__, sys.version]).encode())
+    h.update(" ".join(FLAGS + LINK + HOST_FLAGS + HOST_LINK + [torch.__version__, sys.version]).encode())
     for name in sorted(os.listdir(CSRC)):
         if name.endswith((".hip", ".h", ".cpp")):
             h.update(name.encode())
@@ -137,7 +138,8 @@ def build(force: bool = True, verbose: bool = True) -> str:
     tmp, host_tmp = lib + f".tmp{os.getpid()}", _host_path(lib) + f".tmp{os.getpid()}"
 
     def compile_host():
-        p = subprocess.run([_cxx()] + HOST_FLAGS + ["-o", host_tmp, os.path.join(CSRC, "host.cpp")] + HOST_LINK,
+        where = [f for d in _HOST_INCLUDE for f in ("-isystem", d)]
+        p = subprocess.run([_cxx()] + HOST_FLAGS + where + ["-o", host_tmp, os.path.join(CSRC, "host.cpp"), "-L" + os.path.join(_TORCH, "lib")] + HOST_LINK,
                            stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, env=env)
         if p.returncode != 0:
             raise KernelError(f"compiling the host module failed:\n{p.stdout[-4000:]}")

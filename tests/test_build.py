@@ -48,3 +48,11 @@ def test_a_build_replaces_library_and_module_together(tools):
     path = build.build(verbose=False)
     assert _held(tools.folder) == {"libgesso_hip.so": "new", "gesso_host.so": "new", "libgesso_hip.so.digest": build._digest()}
     assert build.find_built() == path
+
+
+@pytest.mark.parametrize("flags", ["FLAGS", "LINK", "HOST_FLAGS", "HOST_LINK"])
+def test_other_flags_are_another_build(tools, monkeypatch, flags):
+    build.build(verbose=False)
+    assert build.find_built() is not None
+    monkeypatch.setattr(build, flags, getattr(build, flags) + ["-g"])
+    assert build.find_built() is None
