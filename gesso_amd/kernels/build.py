@@ -2,7 +2,8 @@
 
 The kernels under ``gesso_amd/csrc`` are compiled with ``hipcc`` for gfx950 into one shared
 library with a C interface and loaded through ``ctypes``; ``host.cpp``, the launches a step makes most
-without the interpreter between check and launch, becomes a Python module beside it.  Both lie in the tree
+without the interpreter between check and launch, becomes a Python module beside it where there is a C++
+compiler with Python's and torch's headers.  Both lie in the tree
 (``gesso_amd/_lib``) when that folder can be written, else in a per-user temporary folder.
 A digest of the sources and flags lies beside it; a library whose digest differs is built
 again.  Nothing here falls back to another implementation: if the library cannot be built
@@ -74,11 +75,22 @@ def _hipcc() -> str:
     raise KernelError("hipcc not found: the HIP extension cannot be built (set HIPCC or ROCM_PATH)")
 
 
-def _cxx() -> str:
+def _cxx():
+    """A C++ compiler for the host module, or None."""
     for cand in (shutil.which("g++"), os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "clang++")):
         if cand and os.path.exists(cand):
             return cand
-    raise KernelError("no C++ compiler found: the host module cannot be built")
+    return None
+
+
+def _host_lacks():
+    """What the host module cannot be compiled for want of, or None."""
+    if _cxx() is None:
+        return "a C++ compiler"
+    for header, where in (("Python.h", _HOST_INCLUDE[-1]), ("torch/csrc/autograd/python_variable.h", _HOST_INCLUDE[0])):
+        if not os.path.exists(os.path.join(where, header)):
+            return header
+    return None
 
 
 def _lib_dirs():
@@ -112,8 +124,7 @@ def build(force: bool = True, verbose: bool = True) -> str:
         raise KernelError("no writable folder for the HIP extension", tried=_lib_dirs())
     lib = os.path.join(out_dir, LIB_NAME)
     stamp = lib + ".digest"
-    if (not force and os.path.exists(lib) and os.path.exists(_host_path(lib)) and os.path.exists(stamp)
-            and open(stamp).read().strip() == digest):
+    if not force and _is_build(lib, digest):
         return lib
     hipcc = _hipcc()
     obj_dir = os.path.join(out_dir, "obj")
@@ -146,12 +157,16 @@ def build(force: bool = True, verbose: bool = True) -> str:
         if verbose:
             _say(f"  host.cpp done ({time.time() - t0:.0f} s)")
 
+    lacks = _host_lacks()
+    if lacks is not None:
+        _say(f"no {lacks}: built without the host module, every launch is made from Python (slower steps of short prompts, the same results)")
     workers = max(1, min(len(srcs), int(os.environ.get("MAX_JOBS", "0")) or (os.cpu_count() or 4), 16))
     try:
         with ThreadPoolExecutor(workers) as pool:
-            host = pool.submit(compile_host)
+            host = pool.submit(compile_host) if lacks is None else None
             objs = list(pool.map(compile_one, srcs))
-            host.result()
+            if host is not None:
+                host.result()
         p = subprocess.run([hipcc, "--offload-arch=" + ARCH, "-shared", "-fPIC", "-o", tmp] + objs + LINK,
                            stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, env=env)
         if p.returncode != 0:
@@ -161,13 +176,16 @@ def build(force: bool = True, verbose: bool = True) -> str:
         if os.path.exists(stamp):
             os.remove(stamp)
         os.replace(tmp, lib)
-        os.replace(host_tmp, _host_path(lib))
+        if host is not None:
+            os.replace(host_tmp, _host_path(lib))
+        elif os.path.exists(_host_path(lib)):
+            os.remove(_host_path(lib))
     finally:
         for left in (tmp, host_tmp):
             if os.path.exists(left):
                 os.remove(left)
     with open(stamp, "w") as f:
-        f.write(digest)
+        f.write(digest + ("" if lacks is None else "\n" + _WITHOUT_HOST + lacks))
     if verbose:
         _say(f"built {lib} in {time.time() - t0:.0f} s")
     return lib
@@ -177,18 +195,24 @@ def _host_path(lib: str) -> str:
     return os.path.join(os.path.dirname(lib), HOST_NAME + ".so")
 
 
+_WITHOUT_HOST = "without the host module for want of "           # (a digest's second line)
+
+
+def _is_build(lib: str, digest: str) -> bool:
+    """Whether the library there is of this digest, with its host module unless it was built without one."""
+    try:
+        with open(lib + ".digest") as f:
+            held = f.read().strip().split("\n")
+    except OSError:
+        return False
+    without = len(held) > 1 and held[1].startswith(_WITHOUT_HOST)
+    return held[0] == digest and os.path.exists(lib) and (without or os.path.exists(_host_path(lib)))
+
+
 def find_built():
     """Path of a library whose digest matches the sources, or None."""
     digest = _digest()
-    for d in _lib_dirs():
-        lib = os.path.join(d, LIB_NAME)
-        stamp = lib + ".digest"
-        try:
-            if os.path.exists(lib) and os.path.exists(_host_path(lib)) and open(stamp).read().strip() == digest:
-                return lib
-        except OSError:
-            continue
-    return None
+    return next((lib for lib in (os.path.join(d, LIB_NAME) for d in _lib_dirs()) if _is_build(lib, digest)), None)
 
 
 _C_TYPES = {"int": ctypes.c_int, "long": ctypes.c_long, "float": ctypes.c_float, "double": ctypes.c_double,
@@ -222,12 +246,12 @@ def entry_points():
 
 
 def load_host():
-    """The module of ``host.cpp``, bound to the loaded library."""
+    """The module of ``host.cpp``, bound to the loaded library; None where that was built without it."""
     global _host
     lib = load()
     with _lock:
-        if _host is None:
-            path = _host_path(lib._name)
+        path = _host_path(lib._name)
+        if _host is None and os.path.exists(path):
             try:
                 spec = importlib.util.spec_from_file_location(HOST_NAME, path)
                 host = importlib.util.module_from_spec(spec)

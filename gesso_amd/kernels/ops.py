@@ -36,8 +36,22 @@ def _native():
     in their plain form, which the functions here then check, word and make themselves."""
     global _host
     if _host is None:
-        _host = _build.load_host()
+        _host = _build.load_host() or _PythonForms()
     return _host
+
+
+class _PythonForms:
+    """Stands for that module where the library was built without it: nothing is in the plain form, but for the two calls whose
+    callers go on to another product then."""
+
+    def __getattr__(self, name):
+        return lambda *args: False
+
+    def gemm_mid(self, x, w, wt, swiglu, stream):
+        return gemm_mid(x, w, wt, bool(swiglu), checked=True) if mid_ok(x, w, wt, bool(swiglu)) else False
+
+    def gemm_mid_swiglu_scaled(self, xs, ssq, eps, w13, wt, stream):
+        return _mid_swiglu_scaled(xs, ssq, eps, w13, wt) if _mid_scaled_ok(xs, ssq, w13, wt) else False
 
 
 def _dt(t: torch.Tensor) -> int:
@@ -788,10 +802,14 @@ def gemm_mid_residual(x, w: torch.Tensor, wt, res: torch.Tensor, next_weight: to
     return rows, ssq
 
 
+def _mid_scaled_ok(xs, ssq, w13: torch.Tensor, wt) -> bool:
+    return (isinstance(xs, torch.Tensor) and ssq.shape[1] <= 128 and ssq.shape[1] % 4 == 0 and ssq.is_contiguous()
+            and mid_ok(xs, w13, wt, swiglu=True))
+
+
 def mid_scaled_ok(x, w13: torch.Tensor, wt) -> bool:
     """Whether :func:`gemm_mid_swiglu_scaled` takes a lazy norm's weighted rows against gate and up."""
-    return (isinstance(x.xs, torch.Tensor) and x.ssq.shape[1] <= 128 and x.ssq.shape[1] % 4 == 0 and x.ssq.is_contiguous()
-            and mid_ok(x.xs, w13, wt, swiglu=True))
+    return _mid_scaled_ok(x.xs, x.ssq, w13, wt)
 
 
 def gemm_mid_swiglu_scaled_plain(x, w13: torch.Tensor, wt):
@@ -802,19 +820,21 @@ def gemm_mid_swiglu_scaled_plain(x, w13: torch.Tensor, wt):
 def gemm_mid_swiglu_scaled(x, w13: torch.Tensor, wt) -> torch.Tensor:
     """``silu(gate) * up`` in bfloat16 of a lazy norm whose rows come weighted, for products :func:`mid_scaled_ok` takes."""
     y = gemm_mid_swiglu_scaled_plain(x, w13, wt)
-    if y is not False:
-        return y
-    if not mid_scaled_ok(x, w13, wt):
+    if y is False:
         raise KernelError(f"gemm_mid_swiglu_scaled: not a product of this kernel, M={x.shape[0]} N={w13.shape[0]} K={w13.shape[1]}")
+    return y
+
+
+def _mid_swiglu_scaled(xs, ssq, eps: float, w13: torch.Tensor, wt) -> torch.Tensor:
     if not (wt.dtype is torch.bfloat16 and wt.is_cuda and wt.is_contiguous()):
         raise KernelError("gemm_mid_swiglu_scaled: the weight's tile-major copy is bfloat16 on the GPU")
-    xs, N = x.xs, w13.shape[0]
     M, K = xs.shape
+    N = w13.shape[0]
+    if not (ssq.shape[0] == M and ssq.dtype is torch.float32 and ssq.is_cuda):
+        raise KernelError("gemm_mid_swiglu_scaled: the sums of squares are float32, some for every row")
     out = torch.empty((M, N // 2), dtype=torch.bfloat16, device=xs.device)
-    rc = lib().gs_gemm_mid_swiglu_scaled(xs.data_ptr(), xs.stride(0), x.ssq.data_ptr(), x.ssq.shape[1], x.eps, wt.data_ptr(),
-                                         out.data_ptr(), N // 2, M, N, K, _stream())
-    if rc != 0:
-        _check(rc)
+    _check(lib().gs_gemm_mid_swiglu_scaled(xs.data_ptr(), xs.stride(0), ssq.data_ptr(), ssq.shape[1], eps, wt.data_ptr(),
+                                           out.data_ptr(), N // 2, M, N, K, _stream()))
     return out
 
 

@@ -56,3 +56,23 @@ def test_other_flags_are_another_build(tools, monkeypatch, flags):
     assert build.find_built() is not None
     monkeypatch.setattr(build, flags, getattr(build, flags) + ["-g"])
     assert build.find_built() is None
+
+
+def test_a_build_with_nothing_to_compile_the_module_with_is_one_without_it(tools, monkeypatch):
+    """The kernels need hipcc alone: without a C++ compiler or Python's headers the earlier module goes, and every call is made
+    from Python."""
+    from gesso_amd.kernels import ops
+    for lacks in ("_cxx", "_HOST_INCLUDE"):
+        with monkeypatch.context() as m:
+            m.setattr(build, lacks, (lambda: None) if lacks == "_cxx" else [str(tools.folder)] * 3)
+            assert build.build(verbose=False) == build.find_built()
+            assert not (tools.folder / "gesso_host.so").exists() and (tools.folder / "libgesso_hip.so").read_text() == "new"
+            m.setattr(build, "load", lambda: SimpleNamespace(_name=build.find_built()))
+            m.setattr(build, "_host", None)
+            m.setattr(ops, "_host", None)
+            assert build.load_host() is None and ops._native().add_rmsnorm(1, 2) is False
+    assert build.build(force=False, verbose=False) == build.find_built() and not (tools.folder / "gesso_host.so").exists()
+    build.build(verbose=False)
+    assert (tools.folder / "gesso_host.so").exists()
+    (tools.folder / "gesso_host.so").unlink()                   # (gone, and not by the build's own account)
+    assert build.find_built() is None
