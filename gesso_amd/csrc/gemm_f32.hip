@@ -223,10 +223,12 @@ __global__ __launch_bounds__(WN * 128, WN == 2 ? 2 : 1) void gemm_f32_tiles_kern
   __shared__ __align__(16) float xs[2][BM * LD], ws[2][BN * LD];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, g = lane >> 4;
   // (row tiles fastest, all in x: it takes as many tiles as there can be, y only 65,535; the blocks of an XCD, every eighth, are
-  // neighbours, which share rows of W and X in its L2)
+  // neighbours, which share rows of W and X in its L2.  Not from 8,192 blocks on: an XCD meets all row tiles then over and over, and
+  // some 2,000 rows of X no longer stay in its L2; as they come it meets an eighth of them (64 x 64, 2,048 rows of 16384 x 512 317 us
+  // in neighbours, 278 as they come; x 1024 580 and 532))
   const int tiles_m = (M + BM - 1) / BM;
   const unsigned per = gridDim.x >> 3, rest = gridDim.x & 7, xcd = blockIdx.x & 7;
-  const unsigned tile = xcd * per + (xcd < rest ? xcd : rest) + (blockIdx.x >> 3);
+  const unsigned tile = gridDim.x >= 8192 ? blockIdx.x : xcd * per + (xcd < rest ? xcd : rest) + (blockIdx.x >> 3);
   const int mb = (int)(tile % tiles_m) * BM, nb = (int)(tile / tiles_m) * BN, mw = (wave & 1) * 16 * MT, nw = (wave >> 1) * 16 * NT;
   // thread t loads the four k at 4 (t % 8) of row t / 8, RPL rows a load
   const int lr = threadIdx.x >> 3, lk = 4 * (threadIdx.x & 7);
@@ -409,17 +411,22 @@ template <int WN, int MT, int NT, typename TO>
 static void run_tiles(const float* X, int ldx, const float* W, const float* bias, TO* Y, int ldy, int M, int N, int K,
                       hipStream_t stream) {
   const unsigned grid = (unsigned)gs_ceil_div(M, 32 * MT) * (unsigned)gs_ceil_div(N, 16 * NT * WN);
-  auto kernel = K <= GS_SUM_CHUNK         ? &gemm_f32_tiles_kernel<WN, MT, NT, true, true, TO>
-                : K % GS_SUM_CHUNK == 0 ? &gemm_f32_tiles_kernel<WN, MT, NT, false, false, TO>
-                                        : &gemm_f32_tiles_kernel<WN, MT, NT, true, false, TO>;
+  auto kernel = K % GS_SUM_CHUNK == 0 ? &gemm_f32_tiles_kernel<WN, MT, NT, false, false, TO> : &gemm_f32_tiles_kernel<WN, MT, NT, true, false, TO>;
+  if constexpr (WN == 2)                                     // (a short K never comes to the two largest tiles)
+    if (K <= GS_SUM_CHUNK) kernel = &gemm_f32_tiles_kernel<WN, MT, NT, true, true, TO>;
   kernel<<<grid, WN * 128, 0, stream>>>(X, ldx, W, bias, Y, ldy, M, N, K);
 }
 
 // Which tiles: those whose rounds of blocks take the least.  A round (a block for each of the 256 compute units) of so many rows of
 // X by so many of W takes `each` tenths of a microsecond for 2,048 k, whether blocks run beside or after one another, the first
-// `first` more.  (Measured on cold weights; microseconds by this and by the rule and kernel before: 680 rows of 2048 x 2048 64 and
-// 78, 6144 x 2048 172 and 205, 16384 x 2048 380 and 425, 2048 x 8192 230 and 292; 100 rows of 2048 x 2048 20 and 41, x 8192 80 and
-// 178; 2,048 rows of 16384 x 2048 1,050 and 1,100, of 2048 x 8192 517 and 570.)
+// `first` more.  (Measured on cold weights; microseconds by this and by the rule and kernel before: 680 rows of 2048 x 2048 66 and
+// 74, 6144 x 2048 172 and 197, 16384 x 2048 363 and 399, 2048 x 8192 230 and 280; 100 rows of 2048 x 2048 20 and 41, x 8192 80 and
+// 178; 1,024 rows of 16384 x 2048 529 and 563, 2,048 rows of 2048 x 8192 517 and 564.)
+// Up to a K of 1,024 blocks are over too soon for the eight wavefronts of the two largest tiles (2,048 rows of 16384 x 192 by
+// 64 x 128 156 us, by 64 x 64 138, before 140; 1,024 of 8192 x 512 82, 76, 81; 1,024 of 16384 x 1024 281, 272, 288); the others'
+// order does not change with K: over 17 to 2,048 rows of 256 to 16,384 weight rows the choice is 0.8 % above the best of the five on
+// average at a K of 192, 0.3 % at 512 and 1,024, 0.9 % at 2,048, 0.7 % at 8,192 (with `each` in proportion to K, and the fixed part
+// not, 9 % at 192 and 256, 3 % at 512).
 struct Tiles {
   int rows, cols, first, each;
 };
@@ -430,31 +437,18 @@ static int tiles_choice(int M, int N, int K) {
   // 8192 x 64 by 64 x 128 59.8 us, by 64 x 64 49)
   if (K <= 2 * GS_SUM_CHUNK)
     return (long)gs_ceil_div(M, 64) * gs_ceil_div(N, 64) >= 512 ? 2 : (long)gs_ceil_div(M, 32) * gs_ceil_div(N, 64) >= 512 ? 3 : 4;
-  int best = 0;
+  const int from = K <= 1024 ? 2 : 0;
+  int best = from;
   long least = 0;
-  for (int i = 0; i < 5; ++i) {
+  for (int i = from; i < 5; ++i) {
     const long blocks = (long)gs_ceil_div(M, f32_tiles[i].rows) * gs_ceil_div(N, f32_tiles[i].cols);
     const long takes = f32_tiles[i].first + (blocks + 255) / 256 * f32_tiles[i].each;
-    if (i == 0 || takes < least) {
+    if (i == from || takes < least) {
       least = takes;
       best = i;
     }
   }
   return best;
-}
-
-template <typename TO>
-static void run_chosen_tiles(const float* X, int ldx, const float* W, const float* bias, TO* Y, int ldy, int M, int N, int K,
-                             hipStream_t stream) {
-#define GF_TILES(WN, MT, NT) return run_tiles<WN, MT, NT, TO>(X, ldx, W, bias, Y, ldy, M, N, K, stream)
-  switch (tiles_choice(M, N, K)) {
-    case 0: GF_TILES(4, 2, 2);
-    case 1: GF_TILES(4, 3, 1);
-    case 2: GF_TILES(2, 2, 2);
-    case 3: GF_TILES(2, 1, 2);
-    default: GF_TILES(2, 1, 1);
-  }
-#undef GF_TILES
 }
 
 // Which kernel, by sizes (microseconds on cold weights, one MI355X; the FMA kernels that ran before: 63 on average for the
@@ -464,8 +458,9 @@ static void run_chosen_tiles(const float* X, int ldx, const float* W, const floa
 //   2048 x 8192: 21.8, blocks of 16 rows 30.7; 6144 x 2048: 15.1 and 17.2); of 16 rows beyond (65536 x 2048: 118 and 121;
 //   16 rows: 129 and 135).
 // Up to 64 rows: every block of the rows kernel reads all rows of X for its few of W, so wide weights go to the tiles (rows kernel and
-//   tiles; 32 rows: 4096 x 2048 14.3 and 19.1, 5120 x 2048 25.1 and 22.0, 6144 x 512 10.9 and 7.0; 64 rows: 3072 x 2048 23.0 and 19.5,
-//   8192 x 2048 51 and 30; 40 rows: 3072 x 1024 9.8 and 10.9), narrow ones do not fill the chip there (64 rows of 2048 x 2048 18.4 and 18.8, of 2048 x 8192 63 and 80).
+//   tiles; 20 rows: 4096 x 2048 13.2 and 23.6, 6144 x 512 9.3 and 7.5; 64 rows: 3072 x 1024 12.8 and 11.5, 8192 x 2048 52 and 32;
+//   33 rows: 4096 x 512 7.1 and 7.6, x 2048 22.7 and 23.9, 3072 x 2048 21.9 and 23.9, x 8192 75 and 82, but 4096 x 192 6.6 and 5.0,
+//   3072 x 256 6.6 and 5.5), narrow ones do not fill the chip there (64 rows of 2048 x 2048 18.4 and 19.2, of 2048 x 8192 63 and 81).
 //   Nor do wavefronts that share out one chunk fill a block of the rows kernel (64 rows of 8192 x 36 21.3, tiles 4.0; of 100 x 16 6.6
 //   and 3.0).
 // More: tiles.
@@ -497,39 +492,33 @@ static bool lanes_take(int M, int N, int K) {
   return rows <= 2 && chain <= (N <= 128 ? 48 : 20);
 }
 
+// Tiles 0 to 4 (f32_tiles); rows kernel: weight rows a block times 100 plus rows; a lane a chunk: 10000 plus rows.
+static int f32_choice(int M, int N, int K) {
+  const int up = M <= 1 ? 1 : M <= 2 ? 2 : M <= 4 ? 4 : M <= 8 ? 8 : M <= 16 ? 16 : M <= 32 ? 32 : M <= 48 ? 48 : 64;
+  if (lanes_take(M, N, K)) return 10000 + up;
+  if (M <= 16) return (N <= 8192 ? 800 : 1600) + (up < 4 ? 4 : up);
+  if (M <= 64 && K > GS_SUM_CHUNK && N <= (M <= 32 || (M <= 48 && K > 256) ? 4096 : 2048)) return (N <= 2048 ? 800 : 1600) + up;
+  return tiles_choice(M, N, K);
+}
+
+// The choice for these sizes, for tests of every branch.
+extern "C" int gs_gemm_f32_choice(int M, int N, int K) { return f32_choice(M, N, K); }
+
 template <typename TO>
 static void run(const float* X, int ldx, const float* W, const float* bias, TO* Y, int ldy, int M, int N, int K,
                 hipStream_t stream) {
-#define GF_ROWS(WR, XR) return run_rows<WR, XR, 2, TO>(X, ldx, W, bias, Y, ldy, M, N, K, stream)
-#define GF_LANES(MB) return run_lanes<MB, TO>(X, ldx, W, bias, Y, ldy, M, N, K, stream)
-  if (lanes_take(M, N, K)) {
-    if (M == 1) GF_LANES(1);
-    if (M == 2) GF_LANES(2);
-    if (M <= 4) GF_LANES(4);
-    if (M <= 8) GF_LANES(8);
-    GF_LANES(16);
+#define GF_TILES(I, WN, MT, NT) case I: return run_tiles<WN, MT, NT, TO>(X, ldx, W, bias, Y, ldy, M, N, K, stream)
+#define GF_ROWS(WR, XR) case 100 * WR + XR: return run_rows<WR, XR, 2, TO>(X, ldx, W, bias, Y, ldy, M, N, K, stream)
+#define GF_LANES(MB) case 10000 + MB: return run_lanes<MB, TO>(X, ldx, W, bias, Y, ldy, M, N, K, stream)
+  switch (f32_choice(M, N, K)) {
+    GF_TILES(0, 4, 2, 2); GF_TILES(1, 4, 3, 1); GF_TILES(2, 2, 2, 2); GF_TILES(3, 2, 1, 2); GF_TILES(4, 2, 1, 1);
+    GF_ROWS(8, 4); GF_ROWS(8, 8); GF_ROWS(8, 16); GF_ROWS(8, 32); GF_ROWS(8, 48); GF_ROWS(8, 64);
+    GF_ROWS(16, 4); GF_ROWS(16, 8); GF_ROWS(16, 16); GF_ROWS(16, 32); GF_ROWS(16, 48);
+    GF_LANES(1); GF_LANES(2); GF_LANES(4); GF_LANES(8); GF_LANES(16);
   }
-  if (M <= 16) {
-    if (N <= 8192) {
-      if (M <= 4) GF_ROWS(8, 4);
-      if (M <= 8) GF_ROWS(8, 8);
-      GF_ROWS(8, 16);
-    }
-    if (M <= 4) GF_ROWS(16, 4);
-    if (M <= 8) GF_ROWS(16, 8);
-    GF_ROWS(16, 16);
-  }
-  if (M <= 64) {
-    const bool rows = K > GS_SUM_CHUNK && N <= (M <= 32 ? 4096 : M <= 48 && K <= 1024 ? 3072 : 2048);
-    if (rows && N > 2048 && M <= 32) GF_ROWS(16, 32);
-    if (rows && N > 2048) GF_ROWS(16, 48);
-    if (rows && M <= 32) GF_ROWS(8, 32);
-    if (rows && M <= 48) GF_ROWS(8, 48);
-    if (rows) GF_ROWS(8, 64);
-  }
-  run_chosen_tiles<TO>(X, ldx, W, bias, Y, ldy, M, N, K, stream);
 #undef GF_LANES
 #undef GF_ROWS
+#undef GF_TILES
 }
 
 extern "C" int gs_gemm_f32(const float* X, int ldx, const float* W, const float* bias, void* Y, int y_dtype, int ldy,
