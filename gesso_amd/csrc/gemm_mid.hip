@@ -28,7 +28,8 @@
 // 27.5, 333 rows 41.3 and 40.1; 2048 wide and 8192 inside, 72 rows 47.4 and 45.9, 160 rows 56.3 and 55.6.
 //
 // The groups' sums (KG > 1) are added by two groups, half of the block's rows each: the wavefronts that add, and their loads from
-// LDS, are twice as many as with one.
+// LDS, are twice as many as with one.  (With room in LDS for all groups' sums, not for the others' alone, a K of 32 to 96 was up to
+// 5 % slower than with one group adding: 136 rows of 5472 x 32 4.23 us, so 4.44.)
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 gd_bf16x8_t;
@@ -39,7 +40,7 @@ constexpr int GD_BK = 64, GD_LDR = GD_BK + 8, GD_AHEAD = 4;
 
 // Bytes of LDS: two steps' rows of X a group, and in their place at the end the groups' sums.
 constexpr size_t mid_lds(int BM, int NT, int KG) {
-  const size_t held = (size_t)KG * 2 * BM * GD_LDR * sizeof(uint16_t), sums = KG > 1 ? (size_t)KG * BM * 64 * NT * sizeof(float) : 0;
+  const size_t held = (size_t)KG * 2 * BM * GD_LDR * sizeof(uint16_t), sums = (size_t)(KG - 1) * BM * 64 * NT * sizeof(float);
   return held > sums ? held : sums;
 }
 
@@ -239,12 +240,16 @@ __global__ __launch_bounds__(KG * 256) void gemm_mid_kernel(const bf16* __restri
   if constexpr (EPI == 3 && !ROOM) next_weights();
   gd_f32x4_t out[UM][NT];
   if constexpr (KG > 1) {
-    // the groups' sums, in group order: two groups finish half of the block's rows each
+    // the groups' sums, in group order: two groups finish half of the block's rows each.  A half's own group keeps its sums, so
+    // the others' have a place each, in order
     float* sums = reinterpret_cast<float*>(gd_lds);
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < TM; ++i) {
+      const int half = i / UM, place = kg > half ? kg - 1 : kg;
+      if (kg == half) continue;                              // (the same for the whole wavefront)
 #pragma unroll
-      for (int j = 0; j < NT; ++j) *reinterpret_cast<gd_f32x4_t*>(sums + ((kg * TM * NT + i * NT + j) * 256 + tid) * 4) = acc[i][j];
+      for (int j = 0; j < NT; ++j) *reinterpret_cast<gd_f32x4_t*>(sums + ((place * TM * NT + i * NT + j) * 256 + tid) * 4) = acc[i][j];
+    }
     __syncthreads();
     if (kg > 1) return;
 #pragma unroll
@@ -252,12 +257,15 @@ __global__ __launch_bounds__(KG * 256) void gemm_mid_kernel(const bf16* __restri
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
         const float* at = sums + (((kg * UM + i) * NT + j) * 256 + tid) * 4;
-        gd_f32x4_t each[KG];
+        const gd_f32x4_t first = acc[i][j], second = acc[UM + i][j];
+        gd_f32x4_t own, each[KG - 1];
 #pragma unroll
-        for (int q = 0; q < KG; ++q) each[q] = *reinterpret_cast<const gd_f32x4_t*>(at + q * TM * NT * 1024);
-        out[i][j] = each[0];
+        for (int e = 0; e < 4; ++e) own[e] = kg == 0 ? first[e] : second[e];       // (of values: of places it would leave the registers)
 #pragma unroll
-        for (int q = 1; q < KG; ++q) out[i][j] += each[q];
+        for (int q = 0; q < KG - 1; ++q) each[q] = *reinterpret_cast<const gd_f32x4_t*>(at + q * TM * NT * 1024);
+        out[i][j] = kg == 0 ? own + each[0] : each[0] + own;
+#pragma unroll
+        for (int q = 1; q < KG - 1; ++q) out[i][j] += each[q];
       }
   } else {
 #pragma unroll
