@@ -138,13 +138,13 @@ extern "C" int gs_latent_prep(const void* down, int dtype, int ld, int q_off, in
   return 0;
 }
 
-// q (T, ldq): head h at [h (n + r), ...), its last r columns rotated into qa (T, H (c + r)) at [h (c + r) + c, ...).
 // A pair of features turned.  (What is fused is written out: the compiler's choice differs between kernels, and their results with it.)
 __device__ __forceinline__ void turn_pair(float u, float v, float cs, float sn, float& a, float& b) {
   a = fmaf(u, cs, -(v * sn));
   b = fmaf(u, sn, v * cs);
 }
 
+// q (T, ldq): head h at [h (n + r), ...), its last r columns rotated into qa (T, H (c + r)) at [h (c + r) + c, ...).
 template <typename T>
 __global__ void latent_q_rot_kernel(const T* __restrict__ q, int ldq, int H, int n, int r, int c,
                                     const float* __restrict__ cos_t, const float* __restrict__ sin_t,
@@ -258,13 +258,17 @@ __global__ void heads_product_kernel(const TX* __restrict__ X, int ldx, int hx, 
 // 16 NTW columns of one head; the wavefronts of a block own such pieces of their own, and no barrier is needed.
 //
 // `rot` features that follow a head's K in X go, turned by the row's position, behind the head's N in Y: pieces beyond those of the
-// products, a wavefront for the same rows (latent attention's queries; a launch of its own took 4.4 us a layer of a step).
+// products, a wavefront for 256 pairs of the same rows (latent attention's queries; a launch of its own took 4.4 us a layer of a step).
+// (A wavefront for all pairs of its rows was slower than that launch where they are many beside the products: 16 heads of 128 x 64
+// with 128 turned, 256 rows, two launches 8.3 us, so 10.3, these 5.7.)
 struct HeadsRot {
   int rot;
   const float* cos_t;      // (positions, rot / 2)
   const float* sin_t;
   const int* positions;    // (M)
 };
+constexpr int HP_TURNS = 256;
+__host__ __device__ constexpr int heads_turns(int rows, int half) { return (rows * half + HP_TURNS - 1) / HP_TURNS; }
 typedef __attribute__((ext_vector_type(8))) __bf16 hp_bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float hp_f32x4_t;
 typedef __attribute__((ext_vector_type(4))) unsigned hp_u32x4_t;
@@ -280,17 +284,28 @@ __global__ __launch_bounds__(256) void heads_product_mfma_kernel(const bf16* __r
   const int item = blockIdx.x * (blockDim.x >> 6) + wave;
   const int m0 = (item % mtiles) * 16 * MTW, n0 = (item / mtiles) * 16 * NTW;
   if (item >= mtiles * ngroups) {
-    if (hr.rot == 0 || item >= mtiles * (ngroups + 1)) return;
-    const int half = hr.rot / 2, rows = M - m0 < 16 * MTW ? M - m0 : 16 * MTW;
-    for (int p = lane; p < rows * half; p += 64) {
-      const int m = m0 + p / half, j = p % half;
+    const int half = hr.rot / 2, part = item / mtiles - ngroups;
+    if (part >= heads_turns(16 * MTW, half)) return;
+    const int pairs = (M - m0 < 16 * MTW ? M - m0 : 16 * MTW) * half;
+    float u[HP_TURNS / 64], v[HP_TURNS / 64], cs[HP_TURNS / 64], sn[HP_TURNS / 64];
+    // (all asked for at once; what lies beyond the rows is loaded from the first pair and not stored)
+#pragma unroll
+    for (int t = 0; t < HP_TURNS / 64; ++t) {
+      const int p = part * HP_TURNS + 64 * t + lane, q = p < pairs ? p : 0, m = m0 + q / half, j = q % half;
       const bf16* x = X + (size_t)m * ldx + (size_t)h * hx + K + j;
-      const float u = to_f32(x[0]), v = to_f32(x[half]);
       const size_t at = (size_t)hr.positions[m] * half + j;
-      const float cs = hr.cos_t[at], sn = hr.sin_t[at];
-      bf16* y = Y + (size_t)m * ldy + (size_t)h * hy + N + j;
+      u[t] = to_f32(x[0]);
+      v[t] = to_f32(x[half]);
+      cs[t] = hr.cos_t[at];
+      sn[t] = hr.sin_t[at];
+    }
+#pragma unroll
+    for (int t = 0; t < HP_TURNS / 64; ++t) {
+      const int p = part * HP_TURNS + 64 * t + lane;
+      if (p >= pairs) return;
+      bf16* y = Y + (size_t)(m0 + p / half) * ldy + (size_t)h * hy + N + p % half;
       float a, b;
-      turn_pair(u, v, cs, sn, a, b);
+      turn_pair(u[t], v[t], cs[t], sn[t], a, b);
       y[0] = f32_to_bf16(a);
       y[half] = f32_to_bf16(b);
     }
@@ -371,7 +386,7 @@ static int heads_product(const void* X, int x_dtype, int ldx, int hx, const void
     // few rows: narrow pieces, so that a head's weight is spread over more wavefronts; many: 32 x 64 a wavefront
     const int ntw = M <= 64 ? 1 : 4, mtw = M <= 64 ? 1 : 2;
     const int mtiles = gs_ceil_div(M, 16 * mtw);
-    const long products = (long)mtiles * gs_ceil_div(N, 16 * ntw), items = products + (hr.rot ? mtiles : 0);
+    const long products = (long)mtiles * gs_ceil_div(N, 16 * ntw), items = products + (long)mtiles * heads_turns(16 * mtw, hr.rot / 2);
     GS_REQUIRE(items + 1 < (1L << 31), "heads_product: too many tiles");
     // Up to 64 rows, all of K in flight up to 512, in forms of 2, 4 and 16 steps of 32 k (8 rows, 16 heads of 512 x 128 and 128 x 512
     // in a step: 4.7 us each in the mean, four steps at a time, each waiting for its own, 7.3).  Steps beyond K load the row's start
@@ -399,7 +414,7 @@ static int heads_product(const void* X, int x_dtype, int ldx, int hx, const void
     return 0;
   }
   if (hr.rot) {
-    // (a product of its own kind for the rest: the turned features by their own kernel)
+    // (a product of another kind: the turned features by their own kernel)
     const int rc = gs_latent_q_rot(X, x_dtype, ldx, H, K, hr.rot, N, hr.cos_t, hr.sin_t, hr.positions, Y, M, stream);
     if (rc) return rc;
   }
@@ -425,14 +440,21 @@ extern "C" int gs_heads_product(const void* X, int x_dtype, int ldx, int hx, con
   return heads_product(X, x_dtype, ldx, hx, W, w_dtype, Y, ldy, hy, G, ldg, gate_each, M, N, K, H, HeadsRot{}, stream);
 }
 
-// The same without gates and, in the same launch where the matrix cores take it, gs_latent_q_rot: X's rows are H heads of K + rot
+// The same without gates and, in the same launch for up to 512 rows where the matrix cores take it, gs_latent_q_rot: X's rows are H heads of K + rot
 // features, Y's H heads of N + rot.
 extern "C" int gs_heads_product_rot(const void* X, int x_dtype, int ldx, const void* W, int w_dtype, void* Y, int M, int N, int K, int H,
                                     int rot, const float* cos_t, const float* sin_t, const int* positions, hipStream_t stream) {
   GS_REQUIRE(rot > 0 && rot % 2 == 0 && cos_t && sin_t && positions, "heads_product_rot: %d features to turn, tables and positions", rot);
   GS_REQUIRE(H > 0 && (long)H * (K + rot) <= ldx, "heads_product_rot: rows of %d hold no %d heads of %d", ldx, H, K + rot);
+  // Beyond 512 rows the pieces cost as much as the launch they save, or more: 16 heads of 512 x 128 with 64 turned, one launch and two,
+  // 512 rows 11.1 us and 13.5, 1,000 rows 21.7 and 20.9, 2,048 rows 35.2 and 33.2.
+  const bool apart = M > 512;
+  if (apart) {
+    const int rc = gs_latent_q_rot(X, x_dtype, ldx, H, K, rot, N, cos_t, sin_t, positions, Y, M, stream);
+    if (rc) return rc;
+  }
   return heads_product(X, x_dtype, ldx, K + rot, W, w_dtype, Y, H * (N + rot), N + rot, nullptr, 0, 0, M, N, K, H,
-                       HeadsRot{rot, cos_t, sin_t, positions}, stream);
+                       apart ? HeadsRot{} : HeadsRot{rot, cos_t, sin_t, positions}, stream);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
