@@ -46,8 +46,8 @@ constexpr size_t mid_lds(int BM, int NT, int KG) {
 
 constexpr int GD_SSQ_MAX = 128;         // partial sums of squares a row that a SCALED product takes
 
-// What EPI 3 writes (the stream, the next norm's weight, the rows weighted with it, their partial sums of squares; the last three
-// together or not at all) and what SCALED reads (partial sums of squares, eps).
+// What EPI 3 writes (the stream, the next norm's weight, the rows weighted with it, their partial sums of squares) and what SCALED
+// reads (partial sums of squares, eps).
 struct MidNorm {
   float* res;
   const float* weight;
@@ -159,7 +159,7 @@ __global__ __launch_bounds__(KG * 256) void gemm_mid_kernel(const bf16* __restri
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
       const int n = n0 + 16 * j + 4 * g < N ? n0 + 16 * j + 4 * g : N - 4;
-      nw[j] = *reinterpret_cast<const gd_f32x4_t*>((norm.rows ? norm.weight : norm.res) + n);
+      nw[j] = *reinterpret_cast<const gd_f32x4_t*>(norm.weight + n);
     }
   };
   if constexpr (EPI == 3) {
@@ -286,18 +286,14 @@ __global__ __launch_bounds__(KG * 256) void gemm_mid_kernel(const bf16* __restri
         const gd_f32x4_t v = held[i][j] + out[i][j];
         if (m >= M || n >= N) continue;
         *reinterpret_cast<gd_f32x4_t*>(norm.res + (size_t)m * N + n) = v;
-        if (norm.rows) {
-          squares += (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
-          uint2 o;
-          o.x = (uint32_t)f32_to_bf16(v[0] * nw[j][0]).x | ((uint32_t)f32_to_bf16(v[1] * nw[j][1]).x << 16);
-          o.y = (uint32_t)f32_to_bf16(v[2] * nw[j][2]).x | ((uint32_t)f32_to_bf16(v[3] * nw[j][3]).x << 16);
-          *reinterpret_cast<uint2*>(norm.rows + (size_t)m * N + n) = o;
-        }
+        squares += (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
+        uint2 o;
+        o.x = (uint32_t)f32_to_bf16(v[0] * nw[j][0]).x | ((uint32_t)f32_to_bf16(v[1] * nw[j][1]).x << 16);
+        o.y = (uint32_t)f32_to_bf16(v[2] * nw[j][2]).x | ((uint32_t)f32_to_bf16(v[3] * nw[j][3]).x << 16);
+        *reinterpret_cast<uint2*>(norm.rows + (size_t)m * N + n) = o;
       }
-      if (norm.rows) {
-        squares = group4_sum(squares);                     // (a row's columns lie in four lanes; a tile past the last adds zero)
-        if (g == 0 && m < M) norm.ssq_out[(size_t)m * (4 * tiles_n) + bn * 4 + wave] = squares;
-      }
+      squares = group4_sum(squares);                       // (a row's columns lie in four lanes; a tile past the last adds zero)
+      if (g == 0 && m < M) norm.ssq_out[(size_t)m * (4 * tiles_n) + bn * 4 + wave] = squares;
     }
     return;
   }
@@ -451,15 +447,14 @@ extern "C" int gs_gemm_mid_residual_sums(int M, int N, int K) {
   return sums <= GD_SSQ_MAX ? sums : 0;
 }
 
-// res (M, N) += X W^T in float32; with next_weight also rows (M, N) = res * next_weight in bfloat16 and ssq
-// (M, gs_gemm_mid_residual_sums) partial sums of the new rows' squares.
+// res (M, N) += X W^T in float32; rows (M, N) = res * next_weight in bfloat16 and ssq (M, gs_gemm_mid_residual_sums) partial sums of the
+// new rows' squares.
 extern "C" int gs_gemm_mid_residual(const void* X, int ldx, const void* Wt, float* res, const float* next_weight, void* rows, float* ssq,
                                     int M, int N, int K, hipStream_t stream) {
   GS_REQUIRE(gs_gemm_mid_residual_sums(M, N, K) > 0, "gemm_mid_residual: not a product of this kernel (M=%d N=%d K=%d)", M, N, K);
   GS_REQUIRE(ldx >= K && ldx % 8 == 0 && (((uintptr_t)X | (uintptr_t)Wt | (uintptr_t)res | (uintptr_t)next_weight) & 15) == 0 && ((uintptr_t)rows & 7) == 0,
              "gemm_mid_residual: X, W, the stream and the weight must be 16-byte aligned, the row stride of X a multiple of 8");
-  GS_REQUIRE(res && (next_weight != nullptr) == (rows != nullptr) && (rows != nullptr) == (ssq != nullptr),
-             "gemm_mid_residual: the next norm's weight, its rows and their sums come together");
+  GS_REQUIRE(res && next_weight && rows && ssq, "gemm_mid_residual: needs the stream, the next norm's weight, its rows and their sums");
   const bf16 *x = (const bf16*)X, *w = (const bf16*)Wt;
   MidNorm norm = {};
   norm.res = res;
