@@ -90,3 +90,87 @@ def test_a_last_product_of_few_rows_asks_nothing_about_parts():
     assert asked == []
     out = rt.project(torch.zeros(65, 4096), w)
     assert isinstance(out, DeferredLinear) and out.parts == 3 and asked == [65]
+
+
+def hundred_rows_runtime(takes=lambda rows: True):
+    """As much of a runtime as a last product of some hundred rows asks of it, and what was made."""
+    from gesso_amd.parts.runtime import Runtime
+    made = []
+    rt = object.__new__(Runtime)
+    rt.ops = SimpleNamespace(mid_parts_pay=lambda x, w, wt: 0, mid_residual_ok=lambda x, w, wt: takes(x.shape[0]),
+                             gemm_mid_residual=lambda x, w, wt, res, nw, checked: made.append("stream") or ("rows", "sums"))
+    rt.fused, rt.no_library, rt.many_rows, rt.streaming_rows_max, rt._tiles = False, False, "auto", 64, {}
+    rt.linear = lambda x, w, bias=None: made.append("product") or "computed"
+    rt.stage = lambda name: contextlib.nullcontext()
+    return rt, made
+
+
+def test_an_output_projection_of_some_hundred_rows_is_left_to_a_block_that_asks_for_it():
+    """Called by itself, with a bias, for a block whose next reader does not take that many rows weighted, or where no one kernel
+    adds it to the stream, it is computed at once."""
+    from gesso_amd.parts.runtime import DeferredLinear
+    w, x = torch.zeros(16, 32), torch.zeros(100, 32)
+    rt, made = hundred_rows_runtime()
+    out = rt.project(x, w, None, lambda rows: rows == 100)
+    assert isinstance(out, DeferredLinear) and out.parts == 1 and made == []
+    assert rt.project(x, w) == "computed" and rt.project(x, w, None, lambda rows: rows == 99) == "computed"
+    assert rt.project(x, w, "bias", lambda rows: True) == "computed" and rt.project(x[:64], w, None, lambda rows: True) == "computed"
+    rt, made = hundred_rows_runtime(takes=lambda rows: False)
+    assert rt.project(x, w, None, lambda rows: True) == "computed" and made == ["product"]
+
+
+@pytest.mark.parametrize("norm,weighted,into", [("fits", True, "stream"), ("fits", False, "product"), ("fits", None, "product"), ("no weight", True, "product"),
+                                                ("other width", True, "product"), ("other type", True, "product"), (None, True, "product")])
+def test_a_deferred_projection_meets_every_next_norm(norm, weighted, into):
+    """Into the stream only where the next norm's weight fits its rows and their reader takes them weighted; else the ordinary
+    product, pending for the norm's own pass."""
+    from gesso_amd.parts.rmsnorm import ResidualStream
+    from gesso_amd.parts.runtime import DeferredLinear
+    rt, made = hundred_rows_runtime()
+    weights = {"fits": torch.ones(16), "no weight": None, "other width": torch.ones(8), "other type": torch.ones(16).bfloat16()}
+    after = None if norm is None else SimpleNamespace(row_weight=weights[norm])
+    if norm == "no weight":
+        after = object()
+    stream = ResidualStream(torch.zeros(100, 16))
+    stream.push(DeferredLinear(torch.zeros(100, 32), torch.zeros(16, 32), 1), rt, next_norm=after,
+                weighted=None if weighted is None else lambda rows: weighted and rows == 100)
+    assert made == [into]
+    if into == "stream":
+        assert (stream.xs, stream.ssq, stream.xs_for, stream.pending) == ("rows", "sums", after, None)
+    else:
+        assert (stream.xs, stream.ssq, stream.xs_for, stream.pending) == (None, None, None, "computed")
+
+
+def test_a_block_says_what_reads_the_stream_next_while_its_mixer_runs_and_no_longer():
+    from gesso_amd.parts.block import PreNormBlock
+    rt, made = hundred_rows_runtime()
+    said = []
+
+    class Stream:
+        following = None
+
+        def push(self, out, rt, next_norm=None, weighted=None):
+            said.append(("push", out, next_norm, weighted))
+
+    class Mixer:
+        def forward(self, x, ctx, cache):
+            said.append(("mixer", ctx.takes_weighted))
+            if x == "raises":
+                raise RuntimeError("mixer")
+            return "mixed"
+
+    norm = lambda x: SimpleNamespace(add_norm=lambda stream: x)
+    takes = lambda rows: True
+    for ffn in (SimpleNamespace(takes_weighted=takes, forward=lambda x, ctx: said.append(("ffn", ctx.takes_weighted)) or "fed"),
+                SimpleNamespace(forward=lambda x, ctx: said.append(("ffn", ctx.takes_weighted)) or "fed"), None):
+        block = object.__new__(PreNormBlock)
+        block.rt, block.mixer, block.mixer_norm, block.ffn, block.ffn_norm = rt, Mixer(), norm("rows"), ffn, norm("normed")
+        ctx, asks = SimpleNamespace(), getattr(ffn, "takes_weighted", None)
+        said.clear()
+        block.forward(Stream(), ctx, None)
+        assert said[0] == ("mixer", asks) and said[1][1] == "mixed" and said[1][3] is asks and ctx.takes_weighted is None
+        assert said[2:] == ([("ffn", None), ("push", "fed", None, None)] if ffn is not None else [])
+        block.mixer_norm = norm("raises")
+        with pytest.raises(RuntimeError, match="mixer"):
+            block.forward(Stream(), ctx, None)
+        assert ctx.takes_weighted is None

@@ -141,6 +141,54 @@ def test_library_products_of_many_rows_are_planned_once_per_shape_and_stay_right
     assert float((y - x.double() @ w5.double().T).abs().max()) <= tol(torch.bfloat16, want)
 
 
+@pytest.mark.parametrize("rows,hidden,inside,kernels", [(65, 256, 512, True), (150, 512, 1152, True), (333, 256, 1056, True), (2000, 256, 4096, False)])
+@pytest.mark.parametrize("norm", ["rms", "rms around one", "no row weight"])
+def test_a_block_of_some_hundred_rows_from_its_projection_to_gate_and_up(fw, rows, hidden, inside, kernels, norm):
+    """Projection, add, norm, and the gated feed-forward of a pre-norm block, where the rows go weighted from kernel to kernel (an RMS
+    norm, sizes both kernels take) and where they do not (a norm that offers no row weight, rows beyond them): the same
+    numbers, and the plain implementation's."""
+    from gesso_amd.config import RMSNormSpec, SwiGLUSpec
+    from gesso_amd.kernels import ops
+    from gesso_amd.parts import ResidualStream
+    from gesso_amd.parts.block import PreNormBlock
+    from gesso_amd.parts.runtime import DeferredLinear
+    ffn = Harness("ffn", SwiGLUSpec(hidden=hidden, intermediate=inside), torch.bfloat16, seed=4, std=1 / math.sqrt(hidden))
+    rt, g = ffn.rt, gen(rows)
+    normed = Harness("norm", RMSNormSpec(size=hidden, eps=1e-5, offset=1.0 if norm == "rms around one" else 0.0), torch.bfloat16, seed=5)
+    wo = rt.prepare((torch.randn(hidden, hidden, generator=g) / math.sqrt(hidden)).bfloat16().to(DEV))
+    x = torch.randn(rows, hidden, generator=g).bfloat16().to(DEV)
+    res = torch.randn(rows, hidden, generator=g)
+
+    class Mixer:
+        def forward(self, rows_in, ctx, cache):
+            self.left = rt.project(x, wo, None, ctx.takes_weighted)
+            return self.left
+
+    class Unweighted:
+        def __init__(self, norm):
+            self.add_norm, self.spec = norm.add_norm, norm.spec
+
+    class First:
+        def add_norm(self, stream):
+            return None
+
+    block, stream = object.__new__(PreNormBlock), ResidualStream(res.clone().to(DEV))
+    normed.part.rt = rt
+    block.rt, block.mixer_norm, block.mixer, block.ffn = rt, First(), Mixer(), ffn.part
+    block.ffn_norm = normed.part if norm != "no row weight" else Unweighted(normed.part)
+    block.forward(stream, type("Context", (), {})(), None)
+    assert isinstance(block.mixer.left, DeferredLinear) == kernels and ops.mid_residual_ok(x, wo, rt.tiles_of(wo))
+    stream.flush(rt)
+    t = ffn.tensors
+    h = res.double() + x.double().cpu() @ wo.double().cpu().T
+    weight = normed.tensors["weight"] + (1.0 if norm == "rms around one" else 0.0)
+    n = P.rmsnorm(h, weight, 1e-5)
+    gate, up = n @ t["w1.weight"].T, n @ t["w3.weight"].T
+    want = h + (gate / (1 + torch.exp(-gate)) * up) @ t["w2.weight"].T
+    got = stream.res.double().cpu()
+    assert float((got - want).abs().max()) <= tol(torch.bfloat16, want)
+
+
 def test_products_of_some_hundred_rows_take_every_form_of_operands(fw):
     """What the kernel that reads the tile-major weight does not take goes the general way: an output of columns apart, a
     part or a transposed view of a prepared weight (which has the weight's address); operands on the host are refused."""
