@@ -280,11 +280,11 @@ PyObject* qknorm_rope_kv(PyObject* const* a) {
   const stream_t s = stream(a[18]);
   if (other || PyErr_Occurred() || !activations(qkv) || qkv.dim() != 2 || !qkv.is_contiguous() || qkv.size(1) < (int64_t)(nh + 2 * nkv) * d) return other_form();
   if ((qw.defined() && !vector(qw, d)) || (kw.defined() && !vector(kw, d))) return other_form();
+  if ((cos.defined() && !cos.is_contiguous()) || (sin.defined() && !sin.is_contiguous())) return other_form();
   const int T = (int)qkv.size(0);
   int most = 0;
   if (rot) {
-    if (!matrix(cos, at::kFloat) || !matrix(sin, at::kFloat) || cos.sizes() != sin.sizes() || cos.size(1) != rot / 2 || !cos.is_contiguous() ||
-        !sin.is_contiguous())
+    if (!matrix(cos, at::kFloat) || !matrix(sin, at::kFloat) || cos.sizes() != sin.sizes() || cos.size(1) != rot / 2)
       return other_form();
     most = (int)cos.size(0);
   }

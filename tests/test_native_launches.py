@@ -114,6 +114,10 @@ for name, args in calls.items():
         wrong.append((name, "an argument less"))
     except TypeError:
         pass
+# tables in another order, also where nothing is turned and they are not read
+args = calls["qknorm_rope_kv"]
+if native.qknorm_rope_kv(*args[:4], f(32, 16).T, f(32, 16).T, 0, *args[7:], 0) is not False:
+    wrong.append("tables")
 print(wrong)
 """
 
