@@ -1,8 +1,8 @@
 // The launches that a prompt's step makes most, without the interpreter between the check of an operand and the launch.
 //
 // A short prompt's step is some 115 calls, and what stands between two of them is the host: a call of the Python functions takes some
-// 10 us, of which the launch itself is 2 (LFM2-350M sizes, 13 tokens 1,690 us a step on the host, with these functions 1,090; 333
-// tokens with all logits 1,590 and 1,220, of which the device needs 1,130).  A function here takes the operands of one call in its
+// 10 us, of which the launch itself is 2 (LFM2-350M sizes, 13 tokens 1,620 us a step on the host, with these functions 880 to 980;
+// 333 tokens with all logits 1,550 and 1,100 to 1,220, of which the device needs 1,100).  A function here takes the operands of one call in its
 // plainest form (ordinary tensors, a result made here or room for it), checks all that the Python function of the same name checks,
 // makes the result and launches.  Whatever is in another form, or wrong, comes back as False, and the Python function goes on: it
 // handles the other forms and words the errors.
@@ -104,7 +104,7 @@ void launch(int (*entry)(P...), A... a) {
   if (rc != 0) throw Failed();
 }
 
-// One function as Python calls it: `n` arguments; an exception of torch's is another form too (a tensor without memory, say).
+// One function as Python calls it: `N` arguments; an exception of torch's is another form too (a tensor without memory, say).
 template <PyObject* (*BODY)(PyObject* const*), int N>
 PyObject* call(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != N) {
