@@ -25,7 +25,8 @@
 // partial sums of squares are asked for before the first weights and added while those travel, and the results are multiplied
 // by the rows' inverse root mean squares.  Between the two stands no pass: a layer's output projection, gate and up, and down product
 // (1024 wide, 4608 inside; weights in turn, a graph) take 160 rows 32.4 us with the norm's pass and 31.4 without, 72 rows 29.0 and
-// 27.5, 333 rows 41.3 and 40.1; 2048 wide and 8192 inside, 72 rows 47.4 and 45.9, 160 rows 56.3 and 55.6.
+// 27.5, 333 rows 41.3 and 40.1; 2048 wide and 8192 inside, 72 rows 47.4 and 45.9, 160 rows 56.3 and 55.6.  (Projection, norm, gate and
+// up alone, 260 sizes of 65 to 1,000 rows, 512 to 2,048 wide: 0.93 of the three launches in the mean, none more than 1 % above them.)
 //
 // The groups' sums (KG > 1) are added by two groups, half of the block's rows each: the wavefronts that add, and their loads from
 // LDS, are twice as many as with one.  (With room in LDS for all groups' sums, not for the others' alone, a K of 32 to 96 was up to
