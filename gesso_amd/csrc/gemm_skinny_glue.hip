@@ -15,6 +15,12 @@ void gs_skinny_parts_rows(const SkinnyCall& c, int parts);
 void gs_skinny_parts_tiles(const SkinnyCall& c, int parts);
 void gs_skinny_conv_half_tiles(const SkinnyCall& c);
 
+// Up to 16 rows of the tile-major weight (gemm_few.hip); false: left to the kernels above.
+bool gs_few_plain(const SkinnyCall& c, const void* Wt, bool half);
+bool gs_few_gated(const SkinnyCall& c, const void* Wt);
+bool gs_few_residual(const SkinnyCall& c, const void* Wt);
+bool gs_few_conv(const SkinnyCall& c, const void* Wt);
+
 static SkinnyCall base(const void* X, int ldx, int x_tiled, const void* W, const void* Wt, void* Y, int y_dtype, int ldy, int M,
                        int N, int K, int epilogue, hipStream_t stream) {
   SkinnyCall c = {};
@@ -39,12 +45,14 @@ void gs_skinny_run_plain(const void* X, int ldx, int x_tiled, const float* res, 
   c.ex.squared = squared;
   if (res || ssq) lazy(c, res, ssq, nb, norm_w, eps);
   // Half tiles (the same bits) where a block of eight weight rows still comes once to a compute unit and K is long enough for the
-  // sum over the wavefronts not to bind.  Cold weights, microseconds in half and in whole tiles: 8 rows of 2048 x 8192 13.0 and
-  // 14.5, of 1024 x 4608 8.2 and 9.1, of 2048 x 2048 5.4 and 5.7; 32 rows 24.4 and 24.9, 15.4 and 15.6, 8.8 and 8.8; beyond 32 the
-  // blocks' reading of X outweighs the rest.  In whole tiles one to three rows (one of 1024 x 1024 5.28 and 5.11, of 1024 x 3072
-  // 7.3 and 7.1), K below 2048 (8 rows of 2048 x 1024 5.4 and 5.2), more than 256 blocks (8 rows of 2560 x 2560 9.4 and 7.6, 32 of
-  // 2304 x 4608 26.8 and 16.9).
-  if (Wt && epilogue == 0 && N % 16 == 0 && N <= 2048 && K >= 2048 && M >= 4 && M <= 32) gs_skinny_plain_half_tiles(c);
+  // sum over the wavefronts not to bind.  Cold weights, microseconds in half and in whole tiles: 1 row of 2048 x 8192 8.2 and 10.4,
+  // of 1024 x 4608 5.3 and 6.75, of 2048 x 2048 3.9 and 4.3, of 1360 x 2048 3.7 and 4.1; 8 rows the same, 16 10.3 and 11.9, 6.8 and
+  // 7.7, 4.4 and 4.8, 4.2 and 4.6; 32 rows 24.4 and 24.9, 15.4 and 15.6, 8.8 and 8.8; beyond 32 the blocks' reading of X outweighs
+  // the rest.  In whole tiles K below 2048 (2048 x 1024 2.9 both, 1024 x 1024 2.7 both) and more than 256 blocks (8 rows of 2560 x 2560
+  // 5.9 and 5.3, of 3072 x 1024 3.9 and 3.6; 32 of 2304 x 4608 26.8 and 16.9).
+  const bool half = Wt && epilogue == 0 && N % 16 == 0 && N <= 2048 && K >= 2048 && M <= 32;
+  if (gs_few_plain(c, Wt, half)) return;
+  if (half && M >= 4) gs_skinny_plain_half_tiles(c);
   else Wt ? gs_skinny_plain_tiles(c) : gs_skinny_plain_rows(c);
 }
 
@@ -54,7 +62,7 @@ void gs_skinny_run_gated(const void* X, int ldx, int x_tiled, const void* Wt, co
   c.ex.y_tiled = y_tiled;
   c.ex.act_bias = bias;
   c.ex.act = act;
-  gs_skinny_gated_tiles(c);
+  if (!gs_few_gated(c, Wt)) gs_skinny_gated_tiles(c);
 }
 
 void gs_skinny_run_residual(const void* X, int ldx, int x_tiled, const void* W, const void* Wt, float* res, float* ssq_out,
@@ -62,6 +70,7 @@ void gs_skinny_run_residual(const void* X, int ldx, int x_tiled, const void* W, 
   SkinnyCall c = base(X, ldx, x_tiled, W, Wt, nullptr, GS_F32, N, M, N, K, 2, stream);
   c.ex.y_tiled = xs_tiled;
   c.ex.res_out = res; c.ex.ssq_out = ssq_out; c.ex.next_w = next_w; c.ex.xs_out = (bf16*)xs_out;
+  if (gs_few_residual(c, Wt)) return;
   if (Wt && gs_skinny_halves(N)) gs_skinny_residual_half_tiles(c);
   else Wt ? gs_skinny_residual_tiles(c) : gs_skinny_residual_rows(c);
 }
@@ -75,6 +84,7 @@ void gs_skinny_run_conv(const void* X, int ldx, int x_tiled, const float* res, c
   c.ex.taps = taps; c.ex.conv_bias = conv_bias; c.ex.state = state; c.ex.slots = slots; c.ex.conv_w = conv_w;
   c.ex.conv_vec = conv_w >= 2 && conv_w <= 4 && H % 4 == 0 && H >= 4 &&
                   (((uintptr_t)taps | (uintptr_t)conv_bias | (uintptr_t)state) & 15) == 0;
+  if (gs_few_conv(c, Wt)) return;
   // c.N / 3 channels, as few as a narrow weight's rows (6144 x 2048, in whole and in half tiles: 8 rows 9.5 and 8.4 us, 40 10.9 and
   // 10.1, 64 12.7 and 11.9)
   if (Wt && gs_skinny_halves(c.N / 3)) gs_skinny_conv_half_tiles(c);
