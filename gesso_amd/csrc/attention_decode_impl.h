@@ -20,6 +20,11 @@ __device__ __forceinline__ size_t out_index(int seq, int c, int width, int out_t
   return out_tiles ? tiled_index(seq, c, out_tiles) : (size_t)seq * width + c;
 }
 
+// A value that is the same for every lane and that the kernel does not write, by the scalar unit.
+__device__ __forceinline__ int scalar_load(const int* p) {
+  return *reinterpret_cast<const __attribute__((address_space(4))) int*>(reinterpret_cast<uintptr_t>(p));
+}
+
 struct DecodeRaw {
   const float* qw;       // (D) head norm weights, or null for no norm
   const float* kw;
@@ -132,82 +137,24 @@ __global__ __launch_bounds__(W * 64) void attention_decode_kernel(
   __shared__ float wacc[W][G][DV];
 
   const int split = blockIdx.x, nsplit = gridDim.x, kvh = blockIdx.y, seq = blockIdx.z;
+  // All arguments at once: each line of them asked for later would be a round trip of its own in the chain.
+  if constexpr (RAW != 0)
+    asm volatile("" ::"s"(q), "s"(kcache), "s"(vcache), "s"(positions), "s"(block_table), "s"(page_magic), "s"(raw.qw), "s"(raw.kw),
+                 "s"(raw.cos_t), "s"(raw.sin_t), "s"(raw.write_kv), "s"(nh), "s"(nkv), "s"(page_size), "s"(max_blocks),
+                 "s"(window), "s"(nsplit), "s"(q_stride), "s"(scale));
   const int kvc = MAPS == 1 ? kvh : kvh / dm.parts, nkc = MAPS == 1 ? nkv : nkv / dm.parts;   // the cache's key head, and their number
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r16 = lane & 15, kg = lane >> 4;
-  const int pos = positions[seq];
-  int lo_real = window > 0 ? (pos - window + 1 > 0 ? pos - window + 1 : 0) : 0;
-  if (raw.chunk > 0 && pos - pos % raw.chunk > lo_real) lo_real = pos - pos % raw.chunk;
-  // The kept first positions that the window has passed stand before the window's keys in one row of places: place
-  // lo + i is key i for the `kept` first places, and key lo + i (itself) from there on.
-  const int kept = (raw.keep_first > 0 && window > 0 && raw.chunk == 0) ? (raw.keep_first < lo_real ? raw.keep_first : lo_real) : 0;
-  const int lo = lo_real - kept;
-  const int nkeys = pos - lo + 1;
-  // this block's share of the keys, in whole tiles of 64
-  const int tiles = (nkeys + 63) >> 6;
-  const int tper = (tiles + nsplit - 1) / nsplit;
-  const int t0 = split * tper, t1 = (t0 + tper < tiles) ? t0 + tper : tiles;
   const int* bt = block_table + (size_t)seq * max_blocks;
-  const int kq = lane / DL;
-  const bool dlive = DL == DC || lane % DL < DC;       // (a spare lane loads and sums what its neighbours do, and stores nothing)
-  const int dc = dlive ? lane % DL : DC - 1;
-
-  // which row of the caches is key u's (u <= pos)
-  // (u / page_size as one multiplication, page_magic = floor(2^32 / page_size) + 1, exact while u page_size < 2^32:
-  // no branch near the loads, which would make the compiler wait for every load in flight)
-  auto row_off = [&](int u) -> long {
-    u = u < lo_real ? u - lo : u;          // a place before the window's first key holds a kept first position
-    const int pg = (int)__umulhi((unsigned)u, page_magic);
-    const int r = u - pg * page_size;
-    return ((long)bt[pg] * nkc + kvc) * page_size + r;
-  };
-  // The loads of tile t.  Keys, as the first operand of the score products: lane (r16, kg) holds, of the four
-  // keys 4 r16 + kt, features 32 s + 8 kg .. + 8.  Values: the lane's chunk of eight features of the value rows
-  // of its NI keys.  Keys beyond pos are read from key pos (they are masked, their probabilities are zero).
-  auto issue = [&](int t, bf16x8_t (*kreg)[KS], uint4* vreg) {
-    const int base = lo + (t << 6);
-    long ko[4], vo[NI];
-    // The tile's pages follow one another in the table (RAW: no kept first positions): lane i asks for the i-th of them, and
-    // every row's page comes from the lane that has it.  (A load a row was twelve, for whose 64 addresses each eight wavefronts
-    // queue up: 8 sequences of 530 keys 11.1 against 10.7 us, heads of 128 and 24 of 800 23.9 against 21.4.  Blocks of four
-    // wavefronts lose by the exchange: 64 of 230 11.6 against 11.8.)
-    int tile_page = 0, page0 = 0;
-    if constexpr (PAGES) {
-      page0 = (int)__umulhi((unsigned)base, page_magic);
-      const int last = (int)__umulhi((unsigned)pos, page_magic);
-      tile_page = bt[page0 + lane < last ? page0 + lane : last];
-    }
-    auto row_of = [&](int u) -> long {
-      if constexpr (PAGES) {
-        const int pg = (int)__umulhi((unsigned)u, page_magic);
-        // (rows are counted in 32 bits: 2^32 rows of 64 features are more than the card holds)
-        return (long)(((unsigned)__shfl(tile_page, pg - page0, 64) * (unsigned)nkc + (unsigned)kvc) * (unsigned)page_size + (unsigned)(u - pg * page_size));
-      } else
-        return row_off(u);
-    };
-#pragma unroll
-    for (int kt = 0; kt < 4; ++kt) {
-      const int u = base + 4 * r16 + kt;
-      ko[kt] = row_of(u <= pos ? u : pos) * D + kg * 8;
-    }
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int uu = base + kq + i * KG;
-      vo[i] = row_of(uu <= pos ? uu : pos) * DV + dc * 8;
-    }
-#pragma unroll
-    for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-      for (int st = 0; st < KS; ++st) {
-        if (32 * st + 8 * kg < D)
-          kreg[kt][st] = *reinterpret_cast<const bf16x8_t*>(kcache + ko[kt] + 32 * st);
-        else
-          kreg[kt][st] = bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
-      }
-#pragma unroll
-    for (int i = 0; i < NI; ++i) vreg[i] = *reinterpret_cast<const uint4*>(vcache + vo[i]);
-  };
-
+  // Without a window and with one split a wavefront's first tile does not depend on the position: its page numbers are asked for
+  // beside the position, not after it.  (Entries past the sequence's last page are loaded and not used.)
+  const bool known = PAGES && window == 0 && nsplit == 1;
+  int first_pages = 0;
+  if (known) {
+    const int at = (int)__umulhi((unsigned)wave << 6, page_magic) + lane;
+    first_pages = bt[at < max_blocks ? at : max_blocks - 1];
+  }
+  const int pos = scalar_load(positions + seq);
   // Loads in the order of what they wait for: the queries, the norm weights and the step's own key and value
   // (they wait for nothing), the rotation factors and the page numbers (for the position), the key and value rows
   // (for the page numbers).  Loads return in order, so the queries are normed and rotated while the rows are on
@@ -227,15 +174,19 @@ __global__ __launch_bounds__(W * 64) void attention_decode_kernel(
       qreg[st] = bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
     if (!RAW && r16 >= G) qreg[st] = bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
   }
+  // (The position beside the page numbers, the rotation's factors before the rows, the compiler kept to that order, the arguments in one
+  // piece and the new key's places chosen without branches: one sequence of 21 keys 6.6, now 5.5 us, of 400 8.3 and 7.1, of 530 9.8 and
+  // 8.65; 8 of 430 8.95 and 7.95; 64 of 180 10.2 and 9.3; groups of two heads, 24 of 700 12.15 and 10.9.  Value products by 16 blocks
+  // of 4 x 4 x 1 in float32: 0.4 us longer.  Two tiles' rows asked for at once: 64 of 180 13.)
   // Every wavefront keeps a copy of its own of the step's key and value in LDS (the wavefront whose tile holds the
   // new key reads them there: the cache's rows were loaded before they were written), so no wavefront waits for
   // another; wavefront 0 of the block whose keys end with the new one also writes them to the cache.
   __shared__ __align__(16) uint16_t knew[RAW ? W : 1][RAW ? D : 8], vnew[RAW ? W : 1][RAW ? D : 8];
-  const bool has_new = RAW && raw.write_kv && t0 < t1 && t1 == tiles;   // this block's keys end with the new one
   constexpr int E = D >= 64 ? D / 64 : 1;
   float qw8[RAW ? KS : 1][8], c8[RAW ? KS / 2 : 1][8], s8[RAW ? KS / 2 : 1][8];
   float kraw_f[E], kw_f[E], kc_f = 1.f, ks_f = 0.f;
   bf16 vraw_b[E];
+  int new_page = 0;
   if constexpr (RAW != 0) {
     if (raw.qw) {
 #pragma unroll
@@ -249,22 +200,116 @@ __global__ __launch_bounds__(W * 64) void attention_decode_kernel(
       vraw_b[e] = vraw[lane + 64 * e];
       kw_f[e] = raw.kw ? raw.kw[lane + 64 * e] : 1.f;
     }
+    __builtin_amdgcn_sched_barrier(0);                   // (all of these asked for before the position is waited for)
+  }
+  int lo_real = window > 0 ? (pos - window + 1 > 0 ? pos - window + 1 : 0) : 0;
+  if (!RAW && raw.chunk > 0 && pos - pos % raw.chunk > lo_real) lo_real = pos - pos % raw.chunk;
+  // The kept first positions that the window has passed stand before the window's keys in one row of places: place
+  // lo + i is key i for the `kept` first places, and key lo + i (itself) from there on.
+  const int kept = (!RAW && raw.keep_first > 0 && window > 0 && raw.chunk == 0) ? (raw.keep_first < lo_real ? raw.keep_first : lo_real) : 0;
+  const int lo = lo_real - kept;
+  const int nkeys = pos - lo + 1;
+  // this block's share of the keys, in whole tiles of 64
+  const int tiles = (nkeys + 63) >> 6;
+  const int tper = (tiles + nsplit - 1) / nsplit;
+  const int t0 = split * tper, t1 = (t0 + tper < tiles) ? t0 + tper : tiles;
+  const int kq = lane / DL;
+  const bool dlive = DL == DC || lane % DL < DC;       // (a spare lane loads and sums what its neighbours do, and stores nothing)
+  const int dc = dlive ? lane % DL : DC - 1;
+
+  // which row of the caches is key u's (u <= pos)
+  // (u / page_size as one multiplication, page_magic = floor(2^32 / page_size) + 1, exact while u page_size < 2^32:
+  // no branch near the loads, which would make the compiler wait for every load in flight)
+  auto row_off = [&](int u) -> long {
+    u = u < lo_real ? u - lo : u;          // a place before the window's first key holds a kept first position
+    const int pg = (int)__umulhi((unsigned)u, page_magic);
+    const int r = u - pg * page_size;
+    return ((long)bt[pg] * nkc + kvc) * page_size + r;
+  };
+  // The loads of tile t.  Keys, as the first operand of the score products: lane (r16, kg) holds, of the four
+  // keys 4 r16 + kt, features 32 s + 8 kg .. + 8.  Values: the lane's chunk of eight features of the value rows
+  // of its NI keys.  Keys beyond pos are read from key pos (they are masked, their probabilities are zero).
+  // PAGES: the tile's pages follow one another in the table (no kept first positions): lane i asks for the i-th of them, and
+  // every row's page comes from the lane that has it.  (A load a row was twelve, for whose 64 addresses each eight wavefronts
+  // queue up: 8 sequences of 530 keys 11.1 against 10.7 us, heads of 128 and 24 of 800 23.9 against 21.4.  Blocks of four
+  // wavefronts lose by the exchange: 64 of 230 11.6 against 11.8.)
+  auto pages_of = [&](int t) -> int {
+    const int at = (int)__umulhi((unsigned)(lo + (t << 6)), page_magic) + lane, last = (int)__umulhi((unsigned)pos, page_magic);
+    return bt[at < last ? at : last];
+  };
+  // (some: all ones, or zero for a tile that does not exist: the caches' first row then)
+  auto issue = [&](int t, int tile_page, unsigned some, bf16x8_t (*kreg)[KS], uint4* vreg) {
+    const int base = lo + (t << 6);
+    long ko[4], vo[NI];
+    if constexpr (PAGES) {
+      // (rows are counted in 32 bits: 2^32 rows of 64 features are more than the card holds)
+      const int page0 = (int)__umulhi((unsigned)base, page_magic);
+      unsigned kp[4], vp[NI], kr[4], vr[NI];
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt) {
+        const int u = base + 4 * r16 + kt <= pos ? base + 4 * r16 + kt : pos, pg = (int)__umulhi((unsigned)u, page_magic);
+        kp[kt] = (unsigned)__shfl(tile_page, pg - page0, 64);
+        kr[kt] = (unsigned)(u - pg * page_size);
+      }
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int u = base + kq + i * KG <= pos ? base + kq + i * KG : pos, pg = (int)__umulhi((unsigned)u, page_magic);
+        vp[i] = (unsigned)__shfl(tile_page, pg - page0, 64);
+        vr[i] = (unsigned)(u - pg * page_size);
+      }
+      __builtin_amdgcn_sched_barrier(0);                 // (all exchanges under way before the first is waited for)
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt) ko[kt] = (long)(((kp[kt] * (unsigned)nkc + (unsigned)kvc) * (unsigned)page_size + kr[kt]) & some) * D + kg * 8;
+#pragma unroll
+      for (int i = 0; i < NI; ++i) vo[i] = (long)(((vp[i] * (unsigned)nkc + (unsigned)kvc) * (unsigned)page_size + vr[i]) & some) * DV + dc * 8;
+    } else {
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt) {
+        const int u = base + 4 * r16 + kt;
+        ko[kt] = row_off(u <= pos ? u : pos) * D + kg * 8;
+      }
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int uu = base + kq + i * KG;
+        vo[i] = row_off(uu <= pos ? uu : pos) * DV + dc * 8;
+      }
+    }
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+      for (int st = 0; st < KS; ++st) {
+        if (32 * st + 8 * kg < D)
+          kreg[kt][st] = *reinterpret_cast<const bf16x8_t*>(kcache + ko[kt] + 32 * st);
+        else
+          kreg[kt][st] = bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
+      }
+#pragma unroll
+    for (int i = 0; i < NI; ++i) vreg[i] = *reinterpret_cast<const uint4*>(vcache + vo[i]);
+  };
+
+  int t = t0 + wave;
+  const int first = known || t < t1 ? t : (t0 < tiles ? t0 : 0);
+  const bool has_new = RAW && raw.write_kv && t0 < t1 && t1 == tiles;   // this block's keys end with the new one
+  if constexpr (RAW != 0) {
+    if (PAGES && !known) first_pages = pages_of(first);
     // (weights and rotation factors in 16-byte loads: the tables' rows and this lane's offsets are multiples of 8)
 #pragma unroll
     for (int st = 0; st < KS / 2; ++st) {
       load8f(raw.cos_t + (size_t)pos * (D / 2) + 32 * st + 8 * kg, c8[st]);
       load8f(raw.sin_t + (size_t)pos * (D / 2) + 32 * st + 8 * kg, s8[st]);
     }
+    new_page = scalar_load(bt + __umulhi((unsigned)pos, page_magic));
     const int pi = E == 2 ? lane : (lane & 31);          // index of this lane's pair of the key
     kc_f = raw.cos_t[(size_t)pos * (D / 2) + pi];
     ks_f = raw.sin_t[(size_t)pos * (D / 2) + pi];
+    __builtin_amdgcn_sched_barrier(0);                   // (else the compiler asks for these last, and the queries wait for every row)
   }
   bf16x8_t kn[4][KS];
   uint4 vn[NI];
-  int t = t0 + wave;
   // (a wavefront without a tile asks for the block's first one: its address is a valid one, and a load behind a
   // branch would make the compiler wait for every load in flight where it needs the queries)
-  issue(t < t1 ? t : (t0 < tiles ? t0 : 0), kn, vn);
+  issue(first, first_pages, !known || t < t1 ? ~0u : 0u, kn, vn);
+  if constexpr (RAW != 0) __builtin_amdgcn_sched_barrier(0);
 
   if constexpr (RAW != 0) {
     // head norm and rotation of this lane's part of its query: float32 arithmetic on the product's bfloat16
@@ -320,7 +365,7 @@ __global__ __launch_bounds__(W * 64) void attention_decode_kernel(
         const float other = __shfl_xor(kf[0], 32, 64);
         kf[0] = lane < 32 ? kf[0] * kc_f - other * ks_f : other * ks_f + kf[0] * kc_f;
       }
-      const long row = row_off(pos) * D;
+      const long row = ((long)(new_page * nkc + kvc) * page_size + (pos - (int)__umulhi((unsigned)pos, page_magic) * page_size)) * D;
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         const bf16 kb = f32_to_bf16(kf[e]);
@@ -344,7 +389,6 @@ __global__ __launch_bounds__(W * 64) void attention_decode_kernel(
   for (int g = 0; g < G; ++g)
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[g][j] = 0.f;
-
   // one tile: scores, online softmax, values
   auto compute = [&](int t, bf16x8_t (*kc)[KS], uint4* vc) {
     const int base = lo + (t << 6);
@@ -353,15 +397,19 @@ __global__ __launch_bounds__(W * 64) void attention_decode_kernel(
       // So do the places past it, which were loaded from the same row of the cache: their probabilities are zero, but
       // what that row held before this step (anything: the page may have been another request's) must not meet them
       const int rel = pos - base;
+      bf16x8_t nk[KS];
+#pragma unroll
+      for (int st = 0; st < KS; ++st) nk[st] = *reinterpret_cast<const bf16x8_t*>(&knew[wave][32 * st + 8 * kg]);
+      const uint4 nv = *reinterpret_cast<const uint4*>(&vnew[wave][dc * 8]);
 #pragma unroll
       for (int kt = 0; kt < 4; ++kt)
-        if (4 * r16 + kt >= rel) {
 #pragma unroll
-          for (int st = 0; st < KS; ++st) kc[kt][st] = *reinterpret_cast<const bf16x8_t*>(&knew[wave][32 * st + 8 * kg]);
-        }
+        for (int st = 0; st < KS; ++st) kc[kt][st] = 4 * r16 + kt >= rel ? nk[st] : kc[kt][st];
 #pragma unroll
-      for (int i = 0; i < NI; ++i)
-        if (kq + i * KG >= rel) vc[i] = *reinterpret_cast<const uint4*>(&vnew[wave][dc * 8]);
+      for (int i = 0; i < NI; ++i) {
+        const bool from = kq + i * KG >= rel;
+        vc[i] = uint4{from ? nv.x : vc[i].x, from ? nv.y : vc[i].y, from ? nv.z : vc[i].z, from ? nv.w : vc[i].w};
+      }
     }
     // sc[kt][i]: head r16, key base + 4 (4 kg + i) + kt
     f32x4_t sc[4];
@@ -378,7 +426,7 @@ __global__ __launch_bounds__(W * 64) void attention_decode_kernel(
       for (int i = 0; i < 4; ++i) {
         const bool valid = base + 4 * (4 * kg + i) + kt <= pos;
         float sv = sc[kt][i] * qscale;
-        if (raw.softcap > 0.f) {
+        if (!RAW && raw.softcap > 0.f) {
           // cap tanh(x / cap) = cap (1 - 2 / (1 + e^(2 x / cap))), in the base-2 units the scores are held in
           const float e2 = __builtin_amdgcn_exp2f(sv * (2.f / raw.softcap));
           sv = raw.softcap * DEC_LOG2E * (1.f - 2.f * __builtin_amdgcn_rcpf(1.f + e2));
@@ -442,7 +490,7 @@ __global__ __launch_bounds__(W * 64) void attention_decode_kernel(
         for (int st = 0; st < KS; ++st) kc[kt][st] = kn[kt][st];
 #pragma unroll
       for (int i = 0; i < NI; ++i) vc[i] = vn[i];
-      if (t + W < t1) issue(t + W, kn, vn);
+      if (t + W < t1) issue(t + W, PAGES ? pages_of(t + W) : 0, ~0u, kn, vn);
       compute(t, kc, vc);
     }
   } else {
@@ -452,7 +500,7 @@ __global__ __launch_bounds__(W * 64) void attention_decode_kernel(
       t += W;
     }
     for (; t < t1; t += W) {
-      issue(t, kn, vn);
+      issue(t, PAGES ? pages_of(t) : 0, ~0u, kn, vn);
       compute(t, kn, vn);
     }
   }
@@ -496,7 +544,7 @@ __global__ __launch_bounds__(W * 64) void attention_decode_kernel(
       wacc[0][g][j] = o / L;                // (nobody else reads this place)
     } else if (nsplit == 1) {
       // (a sink's score is 0; the maxima are in base-2 units of the scaled scores)
-      if (raw.sink || raw.sinks)
+      if (!RAW && (raw.sink || raw.sinks))
         L += M > -INFINITY ? __builtin_amdgcn_exp2f((raw.sinks ? raw.sinks[kvh * G + g] * DEC_LOG2E : 0.f) - M) : 1.f;
       out[out_index(seq, (kvh * G + g) * DV + j, nh * DV, out_tiles)] = f32_to_bf16(o / L);
     } else {
