@@ -1,59 +1,71 @@
-// Which products of up to 16 rows go to the kernels of gemm_few_impl.h, and the launches of the plain ones.
+// Which products go to the kernels of gemm_few_impl.h, and the launches of the plain ones.
 #include "gemm_few_impl.h"
 
-// Whether a wavefront's share of K is whole loads: the same number for each of a block's eight.
-static bool few_takes(const SkinnyCall& c, const void* Wt, bool half) {
-  return Wt && c.M <= 16 && c.K % (FEW_WAVES * 32 * (half ? 2 : 1)) == 0 && !c.ex.res;
+// Whether a wavefront's share of K is whole loads, the same number for each of a block's `waves` (and for each part).  Rows weighted for
+// their norm come up to 32 at a time: beyond, every block's reading of their partial sums is more than a pass.
+static bool few_takes(const SkinnyCall& c, const void* Wt, int waves, bool half, int parts = 1) {
+  return Wt && c.M <= 64 && c.K % (waves * 32 * (half ? 2 : 1) * parts) == 0 && !c.ex.res && !(c.ex.ssq && c.M > 32);
 }
 
 FewArgs few_args(const SkinnyCall& c) {
   FewArgs g = {};
+  const int tiles = gs_ceil_div(c.M, 16);
   g.W = c.w; g.X = c.x; g.M = c.M; g.N = c.N; g.K = c.K;
-  g.xrow = c.ex.x_tiled ? 8 : c.ldx; g.xgroup = c.ex.x_tiled ? 128 : 8; g.xstep = c.ex.x_tiled ? 512 : 32;
+  g.xrow = c.ex.x_tiled ? 8 : c.ldx; g.xgroup = c.ex.x_tiled ? 128 : 8; g.xstep = c.ex.x_tiled ? 512 * tiles : 32; g.xtile = c.ex.x_tiled ? 512 : 16 * c.ldx;
   g.ssq = c.ex.ssq; g.nb = c.ex.nb; g.eps = c.ex.eps;
   g.Y = c.Y; g.ldy = c.ldy; g.tiled = c.ex.y_tiled; g.extra = c.ex.squared;
   return g;
 }
 
-template <int R, bool HALF, bool SCALED, bool ONCE>
+template <int R, int W34, int MOST, bool HALF, bool SCALED, bool ONCE>
 static void few_plain_out(const SkinnyCall& c, int blocks) {
-  if (c.y_dtype == GS_F32) launch_few<R, HALF, SCALED, 0, 1, ONCE, float>(blocks, few_args(c), c.stream);
-  else launch_few<R, HALF, SCALED, 0, 1, ONCE, bf16>(blocks, few_args(c), c.stream);
+  if (c.y_dtype == GS_F32) launch_few_rows<R, 8, W34, MOST, HALF, SCALED, 0, 1, ONCE, float>(blocks, few_args(c), c.stream);
+  else launch_few_rows<R, 8, W34, MOST, HALF, SCALED, 0, 1, ONCE, bf16>(blocks, few_args(c), c.stream);
 }
-template <int R, bool HALF>
+template <int R, int W34, int MOST, bool HALF>
 static void few_plain(const SkinnyCall& c, int blocks) {
-  if (skinny_once(c.N, c.K)) c.ex.ssq ? few_plain_out<R, HALF, true, true>(c, blocks) : few_plain_out<R, HALF, false, true>(c, blocks);
-  else c.ex.ssq ? few_plain_out<R, HALF, true, false>(c, blocks) : few_plain_out<R, HALF, false, false>(c, blocks);
+  if (skinny_once(c.N, c.K)) c.ex.ssq ? few_plain_out<R, W34, 2, HALF, true, true>(c, blocks) : few_plain_out<R, W34, MOST, HALF, false, true>(c, blocks);
+  else c.ex.ssq ? few_plain_out<R, W34, 2, HALF, true, false>(c, blocks) : few_plain_out<R, W34, MOST, HALF, false, false>(c, blocks);
 }
 
-// A plain product (`half`: of a weight of few rows, half a tile a block), or gate and up with SwiGLU; false: not for these kernels.
+// A plain product (`half`: of a weight of few rows and up to 32 of X, half a tile a block), or gate and up with SwiGLU; false: not for
+// these kernels.
 bool gs_few_plain(const SkinnyCall& c, const void* Wt, bool half) {
-  if (!few_takes(c, Wt, half)) return false;
   if (c.epilogue == 1) {
-    if (c.y_dtype != GS_BF16) return false;
+    if (c.y_dtype != GS_BF16 || !few_takes(c, Wt, few_glu_waves(c), false)) return false;
     gs_few_swiglu(c);
-  } else if (half) few_plain<1, true>(c, c.N / 8);
-  else if (c.N <= 8192) few_plain<1, false>(c, c.N / 16);
-  else few_plain<2, false>(c, gs_ceil_div(c.N, 32));
+    return true;
+  }
+  const bool wide = !half && c.N > 8192;
+  if (!few_takes(c, Wt, wide && c.M > 32 ? 4 : 8, half)) return false;
+  if (half) few_plain<1, 8, 2, true>(c, c.N / 8);
+  else if (!wide) few_plain<1, 8, 4, false>(c, c.N / 16);
+  else few_plain<2, 4, 4, false>(c, gs_ceil_div(c.N, 32));
   return true;
 }
 
 bool gs_few_gated(const SkinnyCall& c, const void* Wt) {
-  if (!few_takes(c, Wt, false)) return false;
+  if (!few_takes(c, Wt, c.M > 32 ? 4 : 8, false)) return false;
   gs_few_gated_run(c);
   return true;
 }
 
-// Into the stream: weights of few rows, half a tile a block.
+// Into the stream: weights of few rows, half a tile a block, up to 32 rows (more come in parts).
 bool gs_few_residual(const SkinnyCall& c, const void* Wt) {
-  if (!gs_skinny_halves(c.N) || !few_takes(c, Wt, true)) return false;
+  if (c.M > 32 || !gs_skinny_halves(c.N) || !few_takes(c, Wt, 8, true)) return false;
   gs_few_residual_run(c);
   return true;
 }
 
 // The convolution: where every block has a compute unit to itself (three tiles' sums leave a lane's registers no room for two).
 bool gs_few_conv(const SkinnyCall& c, const void* Wt) {
-  if (!c.ex.conv_vec || c.N / 24 > 256 || !few_takes(c, Wt, true)) return false;
+  if (!c.ex.conv_vec || c.N / 24 > 256 || !few_takes(c, Wt, 8, true)) return false;
   gs_few_conv_run(c);
+  return true;
+}
+
+bool gs_few_parts(const SkinnyCall& c, const void* Wt, int parts) {
+  if (!few_takes(c, Wt, 4, false, parts)) return false;
+  gs_few_parts_run(c, parts);
   return true;
 }

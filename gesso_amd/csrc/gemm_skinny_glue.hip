@@ -15,11 +15,12 @@ void gs_skinny_parts_rows(const SkinnyCall& c, int parts);
 void gs_skinny_parts_tiles(const SkinnyCall& c, int parts);
 void gs_skinny_conv_half_tiles(const SkinnyCall& c);
 
-// Up to 16 rows of the tile-major weight (gemm_few.hip); false: left to the kernels above.
+// The tile-major weight and a K that a block's wavefronts share evenly (gemm_few.hip); false: left to the kernels above.
 bool gs_few_plain(const SkinnyCall& c, const void* Wt, bool half);
 bool gs_few_gated(const SkinnyCall& c, const void* Wt);
 bool gs_few_residual(const SkinnyCall& c, const void* Wt);
 bool gs_few_conv(const SkinnyCall& c, const void* Wt);
+bool gs_few_parts(const SkinnyCall& c, const void* Wt, int parts);
 
 static SkinnyCall base(const void* X, int ldx, int x_tiled, const void* W, const void* Wt, void* Y, int y_dtype, int ldy, int M,
                        int N, int K, int epilogue, hipStream_t stream) {
@@ -94,5 +95,6 @@ void gs_skinny_run_conv(const void* X, int ldx, int x_tiled, const float* res, c
 void gs_skinny_run_parts(const void* X, int ldx, int x_tiled, const void* W, const void* Wt, float* part, int parts, int M, int N,
                          int K, hipStream_t stream) {
   SkinnyCall c = base(X, ldx, x_tiled, W, Wt, part, GS_F32, N, M, N, K, 5, stream);
+  if (gs_few_parts(c, Wt, parts)) return;
   Wt ? gs_skinny_parts_tiles(c, parts) : gs_skinny_parts_rows(c, parts);
 }

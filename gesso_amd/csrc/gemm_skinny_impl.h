@@ -718,6 +718,17 @@ static void launch_skinny_parts(int blocks, int parts, const bf16* X, int ldx, c
 // 1024 4.65 and 4.21).  (The decode attention's keys, whose lines two loads share, loaded like that: 2 to 3 % longer.)
 static inline bool skinny_once(int N, int K) { return (long)N * K >= 4L << 20; }
 
+// Four tiles a block where four row tiles of X are read: a block reads as much of W as of X then, not half as much.  Such a
+// block has a compute unit to itself, so the last round of them has to be nearly full, and K long enough for what a block
+// starts and ends with (64 rows, microseconds with two and with four tiles, the blocks of four in brackets: 16384 x 2048 17.9
+// and 17.1 (256), x 1024 11.6 and 12.8; 16416 x 2048 23.2 and 26.4 (257); 20480 x 2048 25.7 and 29.1 (320); 24576 x 4096 48.7 and
+// 52.4 (384); 28672 x 2048 and x 4096 0.98 and 0.89 of the time with two (448), 32768 x 2048 0.96 (512); with three row tiles
+// 16384 x 2048 16.2 and 16.5, with 144 such blocks, 9216 x 1024, 9.6 and 10.1).
+static inline bool skinny_fours(int M, int cols, int K) {
+  const int blocks = gs_ceil_div(cols, 16), fours = (blocks + 1) / 2;
+  return M > 48 && blocks >= 512 && K >= 2048 && 8 * fours >= 7 * 256 * gs_ceil_div(fours, 256);
+}
+
 // What the entry points pass on after their checks.
 struct SkinnyCall {
   const bf16* x;
@@ -742,14 +753,8 @@ static void skinny_plain_pro(const SkinnyCall& c) {
   // few output columns: more wavefronts per block split K further, so that the whole chip streams
   if (c.epilogue == 1) {
     const int blocks = gs_ceil_div(cols, 16);
-    // Four tiles a block where four row tiles of X are read: a block reads as much of W as of X then, not half as much.  Such a
-    // block has a compute unit to itself, so the last round of them has to be nearly full, and K long enough for what a block
-    // starts and ends with (64 rows, microseconds with two and with four tiles, the blocks of four in brackets: 16384 x 2048 17.9
-    // and 17.1 (256), x 1024 11.6 and 12.8; 16416 x 2048 23.2 and 26.4 (257); 20480 x 2048 25.7 and 29.1 (320); 24576 x 4096 48.7 and
-    // 52.4 (384); 28672 x 2048 and x 4096 0.98 and 0.89 of the time with two (448), 32768 x 2048 0.96 (512); with three row tiles
-    // 16384 x 2048 16.2 and 16.5, with 144 such blocks, 9216 x 1024, 9.6 and 10.1).
-    const int fours = (blocks + 1) / 2;
-    if (M > 48 && blocks >= 512 && K >= 2048 && 8 * fours >= 7 * 256 * gs_ceil_div(fours, 256)) {
+    if (skinny_fours(M, cols, K)) {
+      const int fours = (blocks + 1) / 2;
       if (f32) launch_skinny<4, 4, 8, PRO, 1, LAYOUT, float>(fours, x, ldx, w, (float*)Y, ldy, M, N, K, ex, stream);
       else launch_skinny<4, 4, 8, PRO, 1, LAYOUT, bf16>(fours, x, ldx, w, (bf16*)Y, ldy, M, N, K, ex, stream);
     } else if (f32) { GS_BY_MT4(2, 8, 8, 4, 4, PRO, 1, float, blocks) } else { GS_BY_MT4(2, 8, 8, 4, 4, PRO, 1, bf16, blocks) }
