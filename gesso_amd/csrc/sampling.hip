@@ -164,11 +164,18 @@ __device__ Crossing radix_descend(const double* __restrict__ w, int V, double ta
   const unsigned long long counts = marked ? (1ull << NUC_COUNT) - 1ull : ~0ull;
   for (int pass = 0; pass < 8; ++pass) {
     int shift = 56 - 8 * pass;
+    const bool ready = ghist != nullptr && pass < 2;
     for (int b = threadIdx.x; b < 256; b += blockDim.x) {
-      hmass[b] = 0ull;
-      hcount[b] = 0;
+      unsigned long long m = 0ull, c = 0ull;
+      const int at = !ready ? -1 : pass == 0 ? (b >= 0x3B && b < 0x40 ? b - 0x3B : -1) : NUC_G0 + ((int)(prefix >> 56) - 0x3C) * 256 + b;
+      if (at >= 0) {
+        m = ghist[at];
+        c = ghist[NUC_GHIST + at] & counts;
+      }
+      hmass[b] = m;
+      hcount[b] = (int)c;
     }
-    __syncthreads();
+    if (!ready) __syncthreads();
     unsigned long long himask = pass == 0 ? 0ull : (~0ull) << (shift + 8);
     // the largest weight this pass can meet: 1 (the row's maximum has weight exp(0)) or the largest pattern under the prefix
     const double wmax = pass == 0 ? 1.0 : __longlong_as_double((long long)(prefix | ((1ull << (shift + 8)) - 1ull)));
@@ -178,19 +185,6 @@ __device__ Crossing radix_descend(const double* __restrict__ w, int V, double ta
     // queue up; the sums are integers, so neither this nor the order of the adds changes them
     int run_b = -1, run_n = 0;
     unsigned long long run_m = 0ull;
-    const bool ready = ghist != nullptr && pass < 2;
-    if (ready && pass == 0) {
-      for (int b = threadIdx.x; b < 5; b += blockDim.x) {
-        hmass[0x3B + b] = ghist[b];
-        hcount[0x3B + b] = (int)(ghist[NUC_GHIST + b] & counts);
-      }
-    } else if (ready) {
-      const int under = (int)(prefix >> 56) - 0x3C;
-      for (int b = threadIdx.x; b < 256; b += blockDim.x) {
-        hmass[b] = ghist[NUC_G0 + under * 256 + b];
-        hcount[b] = (int)(ghist[NUC_GHIST + NUC_G0 + under * 256 + b] & counts);
-      }
-    }
     const int n = ready ? 0 : (nlist >= 0 ? nlist : V);
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
       const unsigned long long bits = nlist >= 0 ? lbits[i] : (unsigned long long)__double_as_longlong(w[i]);
@@ -687,6 +681,7 @@ __global__ __launch_bounds__(SAMP_THREADS) void choose_pick_kernel(
     const int* __restrict__ live, int max_steps, const unsigned long long* __restrict__ ghist) {
   __shared__ int sid, sbad, first_t;
   __shared__ double scan[SAMP_THREADS];
+  __shared__ unsigned long long hist[2 * NUC_GHIST];
   const int row = blockIdx.x, rows = gridDim.x, tid = threadIdx.x;
   int step = counter[row];
   const bool over = step < 0 || step >= max_steps;
@@ -703,8 +698,38 @@ __global__ __launch_bounds__(SAMP_THREADS) void choose_pick_kernel(
   } else {
     const double* pr = part + (size_t)row * nparts;
     const int per = nparts / SAMP_THREADS;
+    // (sixteen of a thread's sums asked for at a time, in loads of two; added one by one)
     double ls = 0.0;
-    for (int i = 0; i < per; ++i) ls += pr[tid * per + i];
+    typedef double __attribute__((ext_vector_type(2))) pair_t;
+    int done = 0;
+    if (per % 2 == 0 && (reinterpret_cast<uintptr_t>(part) & 15) == 0)
+      for (; done + 16 <= per; done += 16) {
+        pair_t two[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) two[i] = *reinterpret_cast<const pair_t*>(pr + tid * per + done + 2 * i);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) ls = (ls + two[i][0]) + two[i][1];
+      }
+    for (; done < per; ++done) ls += pr[tid * per + done];
+    if (P < 1.0) {
+      // The total alone, as the last of the running sums below adds it up (pairs, then pairs of pairs), and the ready-made
+      // histograms beside it: both passes over them then read LDS.
+      if (ghist)
+        for (int i = tid; i < 2 * NUC_GHIST; i += SAMP_THREADS) hist[i] = ghist[(size_t)row * 2 * NUC_GHIST + i];
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) ls += __shfl_xor(ls, off, 64);
+      if ((tid & 63) == 0) scan[tid >> 6] = ls;
+      __syncthreads();
+      double w[SAMP_THREADS / 64];
+#pragma unroll
+      for (int i = 0; i < SAMP_THREADS / 64; ++i) w[i] = scan[i];
+#pragma unroll
+      for (int off = 1; off < SAMP_THREADS / 64; off <<= 1)
+#pragma unroll
+        for (int i = 0; i < SAMP_THREADS / 64; i += 2 * off) w[i] += w[i + off];
+      row_nucleus_pick(wbuf + (size_t)row * V, V, P, uu, w[0], ghist ? hist : nullptr, &sid, &sbad);
+      goto chosen;
+    }
     scan[tid] = ls;
     if (tid == 0) first_t = SAMP_THREADS;
     __syncthreads();
@@ -713,13 +738,6 @@ __global__ __launch_bounds__(SAMP_THREADS) void choose_pick_kernel(
       __syncthreads();
       scan[tid] += v;
       __syncthreads();
-    }
-    if (P < 1.0) {
-      const double total = scan[SAMP_THREADS - 1];
-      __syncthreads();
-      row_nucleus_pick(wbuf + (size_t)row * V, V, P, uu, total,
-                       ghist ? ghist + (size_t)row * 2 * NUC_GHIST : nullptr, &sid, &sbad);
-      goto chosen;
     }
     const double r = uu * scan[SAMP_THREADS - 1];
     if (r < scan[tid]) atomicMin(&first_t, tid);
