@@ -11,7 +11,7 @@
 // lanes 256 bytes, and puts them in order through LDS (rows 4 numbers further apart than their length: no bank twice).
 //
 // Few rows (up to 64): gemm_f32_rows_kernel.  The weights bind, so each is read once: a block owns 8 or 16 rows of W and
-// its eight wavefronts take the chunks in turns, D chunks in flight each; the chunk sums go to LDS, and one thread an output
+// its eight wavefronts take the chunks in turns, one or two at a time, D turns in flight each; the chunk sums go to LDS, and one thread an output
 // adds them in order.  W is loaded non-temporally (six requests, a prompt of 150 and sixteen tokens each at LFM2-1.2B sizes: 42.7 ms against 46.1).
 //
 // A few rows where that kernel's blocks bind, or the way through LDS and sixteen products in a chain: gemm_f32_lanes_kernel, by
@@ -47,7 +47,12 @@ __global__ __launch_bounds__(GF_WAVES * 64) void gemm_f32_rows_kernel(const floa
                                                                       const float* __restrict__ bias, TO* __restrict__ Y,
                                                                       int ldy, int M, int N, int K, int room) {
   constexpr int MT = XR > 16 ? XR / 16 : 1, XT = XR < 16 ? XR : 16;       // tiles of X, rows used of each
-  constexpr int OUT = MT * 16 * WR, PER = (OUT + GF_WAVES * 64 - 1) / (GF_WAVES * 64);
+  // Half a tile of W and half a tile of X: two chunks share the instructions, the second in the tiles' other halves; its sums come out in
+  // the opposite quarter, the other two hold nothing.  (One chunk at a time is sixteen products of 32 cycles in a chain, more than the
+  // weights take: a decode step's kernels of 6 rows, microseconds one and two at a time: 2048 x 8192 and 2048 x 2048 13.0 and 10.7 in
+  // the mean, 6144 x 2048 14.1 and 12.1, 3072 x 2048 10.0 and 8.3.)
+  constexpr int CH = WR == 8 && XR <= 8 ? 2 : 1;
+  constexpr int OUT = MT * XT * WR, PER = (OUT + GF_WAVES * 64 - 1) / (GF_WAVES * 64);
   constexpr int LD = GS_SUM_CHUNK + 4;
   extern __shared__ float sums[];                                         // chunk sums of a pass: `room` of OUT numbers
   __shared__ float order[GF_WAVES][16 * LD];
@@ -65,69 +70,78 @@ __global__ __launch_bounds__(GF_WAVES * 64) void gemm_f32_rows_kernel(const floa
   const int chunks = (K + GS_SUM_CHUNK - 1) / GS_SUM_CHUNK;
 
   struct Chunk {
-    gf_f32x4_t w[WR / 4], x[MT][XT / 4];
+    gf_f32x4_t w[CH][WR / 4], x[CH][MT][XT / 4];
   };
-  auto load = [&](Chunk& b, int c) __attribute__((always_inline)) {
-    const int k = c * GS_SUM_CHUNK + 4 * r16;
+  auto load = [&](Chunk& b, int c, int last) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < WR / 4; ++j) b.w[j] = gf_load<TAIL, true>(wp[j], k, K);
+    for (int h = 0; h < CH; ++h) {
+      const int k = (c + h < last ? c + h : last) * GS_SUM_CHUNK + 4 * r16;
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+      for (int j = 0; j < WR / 4; ++j) b.w[h][j] = gf_load<TAIL, true>(wp[j], k, K);
 #pragma unroll
-      for (int j = 0; j < XT / 4; ++j) b.x[i][j] = gf_load<TAIL>(xp[i][j], k, K);
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < XT / 4; ++j) b.x[h][i][j] = gf_load<TAIL>(xp[i][j], k, K);
+    }
   };
   float* mine = order[wave];
   float* put = mine + g * LD + 4 * r16;           // where a lane leaves what it loaded, four rows a load
   const float* get = mine + r16 * LD + g;         // and where it finds its operands, four numbers apart
   // (a tile of fewer rows than sixteen leaves the others as they are: they end in outputs nobody keeps)
-  auto multiply = [&](Chunk& b, int c, bool keep) __attribute__((always_inline)) {
+  auto multiply = [&](Chunk& b, int c, int keep) __attribute__((always_inline)) {     // keep: how many of the chunks from c on are there
     float w[16];
 #pragma unroll
-    for (int j = 0; j < WR / 4; ++j) *reinterpret_cast<gf_f32x4_t*>(put + 4 * j * LD) = b.w[j];
+    for (int h = 0; h < CH; ++h)
+#pragma unroll
+      for (int j = 0; j < WR / 4; ++j) *reinterpret_cast<gf_f32x4_t*>(put + (8 * h + 4 * j) * LD) = b.w[h][j];
 #pragma unroll
     for (int q = 0; q < 16; ++q) w[q] = get[4 * q];
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
       float x[16];
 #pragma unroll
-      for (int j = 0; j < XT / 4; ++j) *reinterpret_cast<gf_f32x4_t*>(put + 4 * j * LD) = b.x[i][j];
+      for (int h = 0; h < CH; ++h)
+#pragma unroll
+        for (int j = 0; j < XT / 4; ++j) *reinterpret_cast<gf_f32x4_t*>(put + (8 * h + 4 * j) * LD) = b.x[h][i][j];
 #pragma unroll
       for (int q = 0; q < 16; ++q) x[q] = get[4 * q];
       gf_f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int q = 0; q < 16; ++q) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[q], x[q], acc, 0, 0, 0);
       // element e of lane l: row 4 (l / 16) + e of W, row l % 16 of X: X's row after X's row, WR numbers each
-      if (keep && 4 * g < WR) *reinterpret_cast<gf_f32x4_t*>(sums + c * OUT + (i * 16 + r16) * WR + 4 * g) = acc;
+      const int h = CH == 2 ? r16 >> 3 : 0, m = CH == 2 ? r16 & 7 : r16, n = CH == 2 ? 4 * g - 8 * h : 4 * g;
+      if (h < keep && n >= 0 && n < WR && m < XT) *reinterpret_cast<gf_f32x4_t*>(sums + (c + h) * OUT + (i * XT + m) * WR + n) = acc;
     }
   };
   float tot[PER];
 #pragma unroll
   for (int p = 0; p < PER; ++p) tot[p] = 0.f;
   for (int c0 = 0; c0 < chunks; c0 += room) {     // (one pass where LDS holds all chunks' sums)
-    // the wavefront's chunks: c0 + wave, + GF_WAVES, ...; as many rounds for every wavefront, D chunks in flight, no load
-    // behind a branch (a round beyond the last chunk loads that chunk again and leaves nothing)
-    const int held = chunks - c0 < room ? chunks - c0 : room, n = (held + GF_WAVES - 1) / GF_WAVES;
-    auto chunk = [&](int i) __attribute__((always_inline)) { return wave + i * GF_WAVES < held ? wave + i * GF_WAVES : held - 1; };
+    // the wavefront's turns (of CH chunks): wave, + GF_WAVES, ...; as many rounds for every wavefront, D turns in flight, no load
+    // behind a branch (a round beyond the last turn loads that turn again and leaves nothing)
+    const int held = chunks - c0 < room ? chunks - c0 : room, turns = (held + CH - 1) / CH, n = (turns + GF_WAVES - 1) / GF_WAVES;
+    auto chunk = [&](int i) __attribute__((always_inline)) { return CH * (wave + i * GF_WAVES < turns ? wave + i * GF_WAVES : turns - 1); };
+    const int last = c0 + held - 1;
     Chunk b[D];
 #pragma unroll
-    for (int d = 0; d < D; ++d) load(b[d], c0 + chunk(d));
+    for (int d = 0; d < D; ++d) load(b[d], c0 + chunk(d), last);
     int i = 0;
     for (; i + D < n; i += D)
 #pragma unroll
       for (int d = 0; d < D; ++d) {
-        multiply(b[d], chunk(i + d), true);
-        load(b[d], c0 + chunk(i + d + D));
+        multiply(b[d], chunk(i + d), CH);
+        load(b[d], c0 + chunk(i + d + D), last);
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
     for (int d = 0; d < D; ++d)
-      if (i + d < n) multiply(b[d], chunk(i + d), wave + (i + d) * GF_WAVES < held);
+      if (i + d < n) multiply(b[d], chunk(i + d), wave + (i + d) * GF_WAVES < turns ? held - chunk(i + d) : 0);
     __syncthreads();
 #pragma unroll
     for (int p = 0; p < PER; ++p) {
       const int o = threadIdx.x + p * GF_WAVES * 64;
       if (o < OUT) {
-#pragma unroll 8
+#pragma unroll 16
         for (int c = 0; c < held; ++c) tot[p] += sums[c * OUT + o];
       }
     }
@@ -383,7 +397,7 @@ static void run_rows(const float* X, int ldx, const float* W, const float* bias,
   // one a unit.  A pass that ends before K does drains every load in flight and adds up before it asks for the next
   // (28 KB for all: 6 rows of 16384 x 2048, 28 of 32 chunks, 33.3 against 27.5 us; of 2048 x 8192 21.4 against 20.5; 40 rows of it
   // 70 against 57, of 2048 x 2048 18.4 against 14.6).
-  constexpr int out = (XR > 16 ? XR : 16) * WR;
+  constexpr int out = XR * WR;
   const int blocks = gs_ceil_div(N, WR), chunks = gs_ceil_div(K, GS_SUM_CHUNK), most = (blocks <= 256 ? 16384 : 8192) / out;
   const int room = chunks < most ? chunks : most;
   const size_t lds = (size_t)room * out * sizeof(float);
