@@ -41,7 +41,10 @@ __device__ __forceinline__ gf_f32x4_t gf_load(const float* __restrict__ row, int
 }
 
 // WR: rows of W a block owns (8 or 16), XR: rows of X (4, 8, or tiles of 16), D: chunks a wavefront holds in flight.
-template <int WR, int XR, int D, bool TAIL, typename TO>
+// GLU: W holds N / 2 gate rows, then as many up rows; a block takes WR / 2 of each, a gate's sum and its up's end WR / 2 lanes apart, and
+// silu(gate) * up is stored, N / 2 wide.  (A pass of its own was a launch a layer and the 16384-wide rows
+// out and in again: a decode step of 6 requests, 16 such layers, LFM2-1.2B sizes in float32, 1.295 ms, now 1.257.)
+template <int WR, int XR, int D, bool TAIL, typename TO, bool GLU>
 __global__ __launch_bounds__(GF_WAVES * 64) void gemm_f32_rows_kernel(const float* __restrict__ X, int ldx,
                                                                       const float* __restrict__ W,
                                                                       const float* __restrict__ bias, TO* __restrict__ Y,
@@ -57,12 +60,15 @@ __global__ __launch_bounds__(GF_WAVES * 64) void gemm_f32_rows_kernel(const floa
   extern __shared__ float sums[];                                         // chunk sums of a pass: `room` of OUT numbers
   __shared__ float order[GF_WAVES][16 * LD];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * WR;
+  const int n0 = blockIdx.x * (GLU ? WR / 2 : WR), rows = GLU ? N >> 1 : N;      // the block's first output, and how many there are
   // lane l loads the four k at 4 (l % 16) of row l / 16 of four
   const float* wp[WR / 4];
   const float* xp[MT][XT / 4];
 #pragma unroll
-  for (int j = 0; j < WR / 4; ++j) wp[j] = W + (size_t)(n0 + 4 * j + g < N ? n0 + 4 * j + g : N - 1) * K;
+  for (int j = 0; j < WR / 4; ++j) {
+    const int up = GLU && j >= WR / 8, n = n0 + 4 * j + g - up * (WR / 2);
+    wp[j] = W + (size_t)(up * rows + (n < rows ? n : rows - 1)) * K;
+  }
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -152,8 +158,11 @@ __global__ __launch_bounds__(GF_WAVES * 64) void gemm_f32_rows_kernel(const floa
     const int o = threadIdx.x + p * GF_WAVES * 64;
     if (o >= OUT) continue;
     const int n = n0 + o % WR, m = o / WR;
-    if (n < N && m < M) {
-      float t = tot[p];
+    float t = tot[p];
+    if constexpr (GLU) {
+      const float up = __shfl_xor(t, WR / 2);
+      if (o % WR < WR / 2 && n < rows && m < M) Y[(size_t)m * ldy + n] = from_f32<TO>(t / (1.0f + expf(-t)) * up);
+    } else if (n < N && m < M) {
       if (bias) t += bias[n];
       Y[(size_t)m * ldy + n] = from_f32<TO>(t);
     }
@@ -390,7 +399,7 @@ extern "C" int gs_gemm_f32_takes(int M, int N, int K, int ldx, const void* X, co
   return gs_gemm_f32_supports(M, N, K, ldx, X, W) && !fma_faster(M, N, K);
 }
 
-template <int WR, int XR, int D, typename TO>
+template <int WR, int XR, int D, typename TO, bool GLU = false>
 static void run_rows(const float* X, int ldx, const float* W, const float* bias, TO* Y, int ldy, int M, int N, int K,
                      hipStream_t stream) {
   // LDS for the chunk sums, beside 34 KB: 32 KB, which leaves a compute unit room for two blocks, or 64 KB where there is no more than
@@ -398,15 +407,15 @@ static void run_rows(const float* X, int ldx, const float* W, const float* bias,
   // (28 KB for all: 6 rows of 16384 x 2048, 28 of 32 chunks, 33.3 against 27.5 us; of 2048 x 8192 21.4 against 20.5; 40 rows of it
   // 70 against 57, of 2048 x 2048 18.4 against 14.6).
   constexpr int out = XR * WR;
-  const int blocks = gs_ceil_div(N, WR), chunks = gs_ceil_div(K, GS_SUM_CHUNK), most = (blocks <= 256 ? 16384 : 8192) / out;
+  const int blocks = GLU ? gs_ceil_div(N / 2, WR / 2) : gs_ceil_div(N, WR), chunks = gs_ceil_div(K, GS_SUM_CHUNK), most = (blocks <= 256 ? 16384 : 8192) / out;
   const int room = chunks < most ? chunks : most;
   const size_t lds = (size_t)room * out * sizeof(float);
-  auto kernel = K % GS_SUM_CHUNK == 0 ? &gemm_f32_rows_kernel<WR, XR, D, false, TO> : &gemm_f32_rows_kernel<WR, XR, D, true, TO>;
+  auto kernel = K % GS_SUM_CHUNK == 0 ? &gemm_f32_rows_kernel<WR, XR, D, false, TO, GLU> : &gemm_f32_rows_kernel<WR, XR, D, true, TO, GLU>;
   if (lds + sizeof(float) * GF_WAVES * 16 * (GS_SUM_CHUNK + 4) > 64 * 1024) {
     // more than the default limit of LDS: asked for once per kernel
     static const hipError_t asked[2] = {
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_rows_kernel<WR, XR, D, false, TO>), hipFuncAttributeMaxDynamicSharedMemorySize, 65536),
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_rows_kernel<WR, XR, D, true, TO>), hipFuncAttributeMaxDynamicSharedMemorySize, 65536)};
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_rows_kernel<WR, XR, D, false, TO, GLU>), hipFuncAttributeMaxDynamicSharedMemorySize, 65536),
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_rows_kernel<WR, XR, D, true, TO, GLU>), hipFuncAttributeMaxDynamicSharedMemorySize, 65536)};
     (void)asked;
   }
   kernel<<<blocks, GF_WAVES * 64, lds, stream>>>(X, ldx, W, bias, Y, ldy, M, N, K, room);
@@ -545,5 +554,28 @@ extern "C" int gs_gemm_f32(const float* X, int ldx, const float* W, const float*
   else
     run<bf16>(X, ldx, W, bias, (bf16*)Y, ldy, M, N, K, stream);
   GS_LAUNCH_CHECK("gemm_f32");
+  return 0;
+}
+
+// Whether gate and up rows, side by side in W (N of them, half each), go through gs_gemm_f32_swiglu: what the rows kernel takes of
+// such a product.  The tiles' outputs of a gate and its up lie in blocks far apart, and of so many rows the pass between is little
+// (728 rows: 12 us beside 450).
+extern "C" int gs_gemm_f32_swiglu_takes(int M, int N, int K, int ldx, const void* X, const void* W) {
+  if (N % 2 || !gs_gemm_f32_takes(M, N, K, ldx, X, W)) return 0;
+  const int choice = f32_choice(M, N, K);
+  return choice >= 800 && choice < 10000;
+}
+
+// Y = silu(X Wg^T) * (X Wu^T), N / 2 wide: the sums of gs_gemm_f32 and the activation of gs_swiglu, bit for bit.
+extern "C" int gs_gemm_f32_swiglu(const float* X, int ldx, const float* W, float* Y, int ldy, int M, int N, int K, hipStream_t stream) {
+  GS_REQUIRE(N > 0 && K > 0 && ldy >= N / 2 && (M <= 1 || ldx >= K), "gemm_f32_swiglu: bad sizes N=%d K=%d ldx=%d ldy=%d", N, K, ldx, ldy);
+  GS_REQUIRE(gs_gemm_f32_swiglu_takes(M, N, K, ldx, X, W), "gemm_f32_swiglu: not a product of these sizes and operands (M=%d N=%d K=%d)", M, N, K);
+#define GF_GLU(WR, XR) case 100 * WR + XR: run_rows<WR, XR, 2, float, true>(X, ldx, W, nullptr, Y, ldy, M, N, K, stream); break
+  switch (f32_choice(M, N, K)) {
+    GF_GLU(8, 4); GF_GLU(8, 8); GF_GLU(8, 16); GF_GLU(8, 32); GF_GLU(8, 48); GF_GLU(8, 64);
+    GF_GLU(16, 4); GF_GLU(16, 8); GF_GLU(16, 16); GF_GLU(16, 32); GF_GLU(16, 48);
+  }
+#undef GF_GLU
+  GS_LAUNCH_CHECK("gemm_f32_swiglu");
   return 0;
 }

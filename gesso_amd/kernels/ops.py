@@ -707,6 +707,22 @@ def gemm_tiled(x: torch.Tensor, w: torch.Tensor, bias=None, out_dtype=None, out:
     return out
 
 
+def gemm_f32_swiglu(x: torch.Tensor, w13: torch.Tensor):
+    """``silu(x @ wg.T) * (x @ wu.T)`` of float32 rows and weights in one kernel, ``w13`` holding the gate's rows, then up's; False
+    where the sizes are not for it (many rows, a short K) and nothing was done."""
+    if not (x.dtype == torch.float32 and w13.dtype == torch.float32 and x.is_cuda and w13.is_cuda and x.dim() == 2
+            and x.stride(1) == 1 and w13.is_contiguous() and w13.shape[1] == x.shape[1]):
+        return False
+    M, K = x.shape
+    N = w13.shape[0]
+    ldx = x.stride(0) if M > 1 else K
+    if not lib().gs_gemm_f32_swiglu_takes(M, N, K, ldx, _p(x), _p(w13)):
+        return False
+    out = torch.empty((M, N // 2), dtype=torch.float32, device=x.device)
+    _check(lib().gs_gemm_f32_swiglu(_p(x), ldx, _p(w13), _p(out), N // 2, M, N, K, _stream()))
+    return out
+
+
 @lru_cache(maxsize=4096)
 def mid_takes(M: int, N: int, K: int, swiglu: bool) -> bool:
     return bool(lib().gs_gemm_mid_takes(M, N, K, 1 if swiglu else 0))

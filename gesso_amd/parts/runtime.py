@@ -292,6 +292,10 @@ class Runtime:
             y = ops.gemm_mid_plain(x, w13, self.tiles_of(w13), True)
             if y is not False:
                 return y
+        if self.dtype == torch.float32:
+            y = ops.gemm_f32_swiglu(x, w13)                    # few rows: the activation where the product's sums end
+            if y is not False:
+                return y
         return ops.swiglu(self.linear(x, w13))
 
     def swiglu_takes_weighted(self, rows: int, w13: torch.Tensor) -> bool:
