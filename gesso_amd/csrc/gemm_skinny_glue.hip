@@ -46,7 +46,7 @@ void gs_skinny_run_plain(const void* X, int ldx, int x_tiled, const float* res, 
   c.ex.squared = squared;
   if (res || ssq) lazy(c, res, ssq, nb, norm_w, eps);
   // Half tiles (the same bits) where a block of eight weight rows still comes once to a compute unit and K is long enough for the
-  // sum over the wavefronts not to bind.  Cold weights, microseconds in half and in whole tiles: 1 row of 2048 x 8192 8.2 and 10.4,
+  // sum over the wavefronts not to bind.  Cold weights, microseconds in half and in whole tiles of gemm_skinny_impl.h's kernel: 1 row of 2048 x 8192 8.2 and 10.4,
   // of 1024 x 4608 5.3 and 6.75, of 2048 x 2048 3.9 and 4.3, of 1360 x 2048 3.7 and 4.1; 8 rows the same, 16 10.3 and 11.9, 6.8 and
   // 7.7, 4.4 and 4.8, 4.2 and 4.6; 32 rows 24.4 and 24.9, 15.4 and 15.6, 8.8 and 8.8; beyond 32 the blocks' reading of X outweighs
   // the rest.  In whole tiles K below 2048 (2048 x 1024 2.9 both, 1024 x 1024 2.7 both) and more than 256 blocks (8 rows of 2560 x 2560

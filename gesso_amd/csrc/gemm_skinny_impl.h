@@ -25,6 +25,9 @@
 // y_tiled the epilogues that write rows for a following product (SwiGLU, convolution, pre-weighted rows) write them
 // in that order.
 //
+// A tile-major weight whose K the wavefronts share evenly, without the norm's fold (PRO 1), goes to gemm_few_impl.h's kernel, which
+// gives the same bits sooner; here is what it does not take.
+//
 // What feeds X (PRO):
 //   0  X is given, bfloat16.
 //   1  X is the RMSNorm of the float32 residual stream: x = res * inv_rms(row) * norm_weight, rounded to
