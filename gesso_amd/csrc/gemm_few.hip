@@ -1,17 +1,23 @@
 // Which products go to the kernels of gemm_few_impl.h, and the launches of the plain ones.
 #include "gemm_few_impl.h"
 
-// Whether a wavefront's share of K is whole loads, the same number for each of a block's `waves` (and for each part).  Rows weighted for
-// their norm come up to 32 at a time: beyond, every block's reading of their partial sums is more than a pass.
+// Whether a wavefront's share of K is whole loads, the same number for each of a block's `waves` (and for each part), and X's rows lie
+// within 4 GB, which a lane's 32 bits of bytes reach (rows further apart are the older kernel's, as they were).
+extern "C" int gs_gemm_few_takes(int M, int K, int ldx, int x_tiled, int waves, int half, int parts) {
+  const long reach = x_tiled ? 16L * gs_ceil_div(M, 16) * K : (long)(M - 1) * ldx + K;
+  return M <= 64 && K % (waves * 32 * (half ? 2 : 1) * parts) == 0 && reach <= 1L << 31;
+}
+
+// Rows weighted for their norm come up to 32 at a time: beyond, every block's reading of their partial sums is more than a pass.
 static bool few_takes(const SkinnyCall& c, const void* Wt, int waves, bool half, int parts = 1) {
-  return Wt && c.M <= 64 && c.K % (waves * 32 * (half ? 2 : 1) * parts) == 0 && !c.ex.res && !(c.ex.ssq && c.M > 32);
+  return Wt && !c.ex.res && !(c.ex.ssq && c.M > 32) && gs_gemm_few_takes(c.M, c.K, c.ldx, c.ex.x_tiled, waves, half, parts);
 }
 
 FewArgs few_args(const SkinnyCall& c) {
   FewArgs g = {};
   const int tiles = gs_ceil_div(c.M, 16);
   g.W = c.w; g.X = c.x; g.M = c.M; g.N = c.N; g.K = c.K;
-  g.xrow = c.ex.x_tiled ? 8 : c.ldx; g.xgroup = c.ex.x_tiled ? 128 : 8; g.xstep = c.ex.x_tiled ? 512 * tiles : 32; g.xtile = c.ex.x_tiled ? 512 : 16 * c.ldx;
+  g.xrow = c.ex.x_tiled ? 8 : c.ldx; g.xgroup = c.ex.x_tiled ? 128 : 8; g.xstep = c.ex.x_tiled ? 512 * tiles : 32; g.xtile = c.ex.x_tiled ? 512 : tiles > 1 ? 16 * c.ldx : 0;
   g.ssq = c.ex.ssq; g.nb = c.ex.nb; g.eps = c.ex.eps;
   g.Y = c.Y; g.ldy = c.ldy; g.tiled = c.ex.y_tiled; g.extra = c.ex.squared;
   return g;
