@@ -34,15 +34,30 @@ static void few_plain(const SkinnyCall& c, int blocks) {
   else c.ex.ssq ? few_plain_out<R, W34, 2, HALF, true, false>(c, blocks) : few_plain_out<R, W34, MOST, HALF, false, false>(c, blocks);
 }
 
+// Two tiles a block and 17 to 48 plain rows: up to a K of 4,096 and, of more than 32 rows, 10,240 weight rows.  Beyond, both wait for the same
+// bytes and gemm_skinny_impl.h's kernel is as fast or faster (microseconds there and here, cold weights: gate and up 24 rows of 10240 x 2560
+// 15.2 and 14.5, of 12288 x 4096 22.4 both, of 22528 x 4096 32.9 and 33.5; 48 rows of 9216 x 1024 9.0 and 8.8, of 10240 x 2560 18.2 both,
+// of 16384 x 2048 16.1 and 16.3, of 28672 x 4096 50.8 and 52.1; stored, 17 rows of 12288 x 2048 12.8 and 12.5, of 16384 x 4096 25.9 and 26.6;
+// 48 rows of 65536 x 2048 57.9 and 58.9).  Up to 16 rows, 49 and more, or rows weighted for their norm: nothing was slower.
+static bool few_pairs(const SkinnyCall& c) {
+  return c.M <= 16 || c.M > 48 || c.ex.ssq || (c.K < 4096 && (c.M <= 32 || c.N <= 10240));
+}
+
 // A plain product (`half`: of a weight of few rows and up to 32 of X, half a tile a block), or gate and up with SwiGLU; false: not for
 // these kernels.
 bool gs_few_plain(const SkinnyCall& c, const void* Wt, bool half) {
   if (c.epilogue == 1) {
-    if (c.y_dtype != GS_BF16 || !few_takes(c, Wt, few_glu_waves(c), false)) return false;
+    if (c.y_dtype != GS_BF16 || !few_pairs(c) || !few_takes(c, Wt, few_glu_waves(c), false)) return false;
     gs_few_swiglu(c);
     return true;
   }
+  // More than 32 rows and one tile a block: where every block has a compute unit to itself.  (A ring of four loads for three or four row
+  // tiles leaves a unit one block, gemm_skinny_impl.h's two.  There and here: 48 rows of 4096 x 4096 11.6 and 11.5 us, of 3072 x 2048 6.9 and
+  // 6.7, of 4112 x 2048 9.9 and 10.1, of 8192 x 1024 6.85 and 7.6, x 2048 11.7 and 12.1; 64 rows of 4096 x 2560 10.1 and 9.25, of 6144 x 2048
+  // 13.0 and 13.4, of 8192 x 2048 13.6 and 14.2.  With 32-bit offsets, 103 and 128 registers where 132 and 170 were: 64 rows of 8192 x
+  // 2048 14.5, of 4096 x 4096 13.8 for 13.1; with a ring of three and 108: 13.6 and 13.35, of 8192 x 1024 8.2 for 7.8.)
   const bool wide = !half && c.N > 8192;
+  if (wide ? !few_pairs(c) : c.M > 32 && c.N > 4096) return false;
   if (!few_takes(c, Wt, wide && c.M > 32 ? 4 : 8, half)) return false;
   if (half) few_plain<1, 8, 2, true>(c, c.N / 8);
   else if (!wide) few_plain<1, 8, 4, false>(c, c.N / 16);
@@ -51,7 +66,7 @@ bool gs_few_plain(const SkinnyCall& c, const void* Wt, bool half) {
 }
 
 bool gs_few_gated(const SkinnyCall& c, const void* Wt) {
-  if (!few_takes(c, Wt, c.M > 32 ? 4 : 8, false)) return false;
+  if (!few_pairs(c) || !few_takes(c, Wt, c.M > 32 ? 4 : 8, false)) return false;
   gs_few_gated_run(c);
   return true;
 }
