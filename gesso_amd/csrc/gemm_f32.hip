@@ -44,7 +44,7 @@ __device__ __forceinline__ gf_f32x4_t gf_load(const float* __restrict__ row, int
 // GLU: W holds N / 2 gate rows, then as many up rows; a block takes WR / 2 of each, a gate's sum and its up's end WR / 2 lanes apart, and
 // silu(gate) * up is stored, N / 2 wide.  (A pass of its own was a launch a layer and the 16384-wide rows
 // out and in again: a decode step of 6 requests, 16 such layers, LFM2-1.2B sizes in float32, 1.295 ms, now 1.257.)
-template <int WR, int XR, int D, bool TAIL, typename TO, bool GLU>
+template <int WR, int XR, int D, int CH, bool TAIL, typename TO, bool GLU>
 __global__ __launch_bounds__(GF_WAVES * 64) void gemm_f32_rows_kernel(const float* __restrict__ X, int ldx,
                                                                       const float* __restrict__ W,
                                                                       const float* __restrict__ bias, TO* __restrict__ Y,
@@ -54,7 +54,7 @@ __global__ __launch_bounds__(GF_WAVES * 64) void gemm_f32_rows_kernel(const floa
   // the opposite quarter, the other two hold nothing.  (One chunk at a time is sixteen products of 32 cycles in a chain, more than the
   // weights take: a decode step's kernels of 6 rows, microseconds one and two at a time: 2048 x 8192 and 2048 x 2048 13.0 and 10.7 in
   // the mean, 6144 x 2048 14.1 and 12.1, 3072 x 2048 10.0 and 8.3.)
-  constexpr int CH = WR == 8 && XR <= 8 ? 2 : 1;
+  static_assert(CH == 1 || (CH == 2 && WR == 8 && XR <= 8), "two chunks share the halves of a tile");
   constexpr int OUT = MT * XT * WR, PER = (OUT + GF_WAVES * 64 - 1) / (GF_WAVES * 64);
   constexpr int LD = GS_SUM_CHUNK + 4;
   extern __shared__ float sums[];                                         // chunk sums of a pass: `room` of OUT numbers
@@ -81,7 +81,7 @@ __global__ __launch_bounds__(GF_WAVES * 64) void gemm_f32_rows_kernel(const floa
   auto load = [&](Chunk& b, int c, int last) __attribute__((always_inline)) {
 #pragma unroll
     for (int h = 0; h < CH; ++h) {
-      const int k = (c + h < last ? c + h : last) * GS_SUM_CHUNK + 4 * r16;
+      const int k = (CH == 1 || c + h < last ? c + h : last) * GS_SUM_CHUNK + 4 * r16;
 #pragma unroll
       for (int j = 0; j < WR / 4; ++j) b.w[h][j] = gf_load<TAIL, true>(wp[j], k, K);
 #pragma unroll
@@ -147,8 +147,15 @@ __global__ __launch_bounds__(GF_WAVES * 64) void gemm_f32_rows_kernel(const floa
     for (int p = 0; p < PER; ++p) {
       const int o = threadIdx.x + p * GF_WAVES * 64;
       if (o < OUT) {
-#pragma unroll 16
-        for (int c = 0; c < held; ++c) tot[p] += sums[c * OUT + o];
+        // (sixteen sums asked for at a time, four where fewer are left: one by one, eight of K = 512 were 0.4 us)
+        int c = 0;
+        for (; c + 16 <= held; c += 16)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) tot[p] += sums[(c + e) * OUT + o];
+        for (; c + 4 <= held; c += 4)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) tot[p] += sums[(c + e) * OUT + o];
+        for (; c < held; ++c) tot[p] += sums[c * OUT + o];
       }
     }
     if (c0 + room < chunks) __syncthreads();
@@ -399,8 +406,8 @@ extern "C" int gs_gemm_f32_takes(int M, int N, int K, int ldx, const void* X, co
   return gs_gemm_f32_supports(M, N, K, ldx, X, W) && !fma_faster(M, N, K);
 }
 
-template <int WR, int XR, int D, typename TO, bool GLU = false>
-static void run_rows(const float* X, int ldx, const float* W, const float* bias, TO* Y, int ldy, int M, int N, int K,
+template <int WR, int XR, int D, int CH, typename TO, bool GLU>
+static void launch_rows(const float* X, int ldx, const float* W, const float* bias, TO* Y, int ldy, int M, int N, int K,
                      hipStream_t stream) {
   // LDS for the chunk sums, beside 34 KB: 32 KB, which leaves a compute unit room for two blocks, or 64 KB where there is no more than
   // one a unit.  A pass that ends before K does drains every load in flight and adds up before it asks for the next
@@ -410,15 +417,30 @@ static void run_rows(const float* X, int ldx, const float* W, const float* bias,
   const int blocks = GLU ? gs_ceil_div(N / 2, WR / 2) : gs_ceil_div(N, WR), chunks = gs_ceil_div(K, GS_SUM_CHUNK), most = (blocks <= 256 ? 16384 : 8192) / out;
   const int room = chunks < most ? chunks : most;
   const size_t lds = (size_t)room * out * sizeof(float);
-  auto kernel = K % GS_SUM_CHUNK == 0 ? &gemm_f32_rows_kernel<WR, XR, D, false, TO, GLU> : &gemm_f32_rows_kernel<WR, XR, D, true, TO, GLU>;
+  auto kernel = K % GS_SUM_CHUNK == 0 ? &gemm_f32_rows_kernel<WR, XR, D, CH, false, TO, GLU> : &gemm_f32_rows_kernel<WR, XR, D, CH, true, TO, GLU>;
   if (lds + sizeof(float) * GF_WAVES * 16 * (GS_SUM_CHUNK + 4) > 64 * 1024) {
     // more than the default limit of LDS: asked for once per kernel
     static const hipError_t asked[2] = {
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_rows_kernel<WR, XR, D, false, TO, GLU>), hipFuncAttributeMaxDynamicSharedMemorySize, 65536),
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_rows_kernel<WR, XR, D, true, TO, GLU>), hipFuncAttributeMaxDynamicSharedMemorySize, 65536)};
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_rows_kernel<WR, XR, D, CH, false, TO, GLU>), hipFuncAttributeMaxDynamicSharedMemorySize, 65536),
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_rows_kernel<WR, XR, D, CH, true, TO, GLU>), hipFuncAttributeMaxDynamicSharedMemorySize, 65536)};
     (void)asked;
   }
   kernel<<<blocks, GF_WAVES * 64, lds, stream>>>(X, ldx, W, bias, Y, ldy, M, N, K, room);
+}
+
+// Whether a wavefront takes two chunks a turn (blocks of eight weight rows, up to eight of X; the same bits).  Up to a K of 512 a chunk for
+// each of the eight wavefronts is one round either way, and two cost registers and, beside them, blocks a compute unit; more than two
+// rows of more than 2,048 weight rows stay so up to 1,024.  (Microseconds one and two at a time: 1 row of 1024 x 512 3.2 and 3.5, of
+// 8192 x 512 6.2 and 7.6, x 576 8.9 and 8.1; 4 rows of 3072 x 1024 5.7 and 5.9, x 1088 7.5 and 6.8; 8 rows of 2048 x 768 4.5 and 4.4, of
+// 6144 x 1024 8.0 and 8.8, x 1088 11.2 and 10.3; 6 rows of 8192 x 512 6.5 and 8.6.)
+static bool two_chunks(int M, int N, int K) { return K > (M > 2 && N > 2048 ? 1024 : 512); }
+
+template <int WR, int XR, int D, typename TO, bool GLU = false>
+static void run_rows(const float* X, int ldx, const float* W, const float* bias, TO* Y, int ldy, int M, int N, int K, hipStream_t stream) {
+  if constexpr (WR == 8 && XR <= 8) {
+    if (two_chunks(M, N, K)) return launch_rows<WR, XR, D, 2, TO, GLU>(X, ldx, W, bias, Y, ldy, M, N, K, stream);
+  }
+  launch_rows<WR, XR, D, 1, TO, GLU>(X, ldx, W, bias, Y, ldy, M, N, K, stream);
 }
 
 template <int MB, typename TO>
