@@ -177,7 +177,7 @@ __global__ __launch_bounds__(GF_WAVES * 64) void gemm_f32_rows_kernel(const floa
 }
 
 #define GF_LANES_WAVES 2
-#define GF_LANES_CHUNKS 128    // K up to 8192
+#define GF_LANES_CHUNKS 72     // K below 4608
 
 // A wavefront owns pairs of rows of W, 64 / span of them: the span lanes of a pair (a power of two, as many as there are chunks,
 // at most 64) take chunks l, l + span, ... each, sum a chunk of both rows from zero in ascending k and leave the sums in LDS; then
@@ -500,8 +500,9 @@ static int tiles_choice(int M, int N, int K) {
 // products of a decode step of 6 rows, 729 for those of a prompt portion of 900 tokens, 2048 x 2048 to 16384 x 2048).
 // Up to 16 rows, a lane a chunk: see lanes_take.
 // Up to 16 rows: blocks of 8 rows of W up to N = 8192, which then still are no more than four a compute unit (6 rows,
-//   2048 x 8192: 21.8, blocks of 16 rows 30.7; 6144 x 2048: 15.1 and 17.2); of 16 rows beyond (65536 x 2048: 118 and 121;
-//   16 rows: 129 and 135).
+//   2048 x 8192: 21.8, blocks of 16 rows 30.7; 6144 x 2048: 15.1 and 17.2); of 16 rows beyond (two chunks a turn in blocks of 8, and blocks of
+//   16: 6 rows of 9216 x 1024 12.6 and 10.4, x 2048 17.5 and 17.6, x 4608 36.0 and 36.2; of 16384 x 2048 27.2 and 23.9; 1 row of 10240 x 4608
+//   32.7 and 33.9, of 16384 x 4608 50.3 and 47.6).
 // Up to 64 rows: every block of the rows kernel reads all rows of X for its few of W, so wide weights go to the tiles (rows kernel and
 //   tiles; 20 rows: 4096 x 2048 13.2 and 23.6, 6144 x 512 9.3 and 7.5; 64 rows: 3072 x 1024 12.8 and 11.5, 8192 x 2048 52 and 32;
 //   33 rows: 4096 x 512 7.1 and 7.6, x 2048 22.7 and 23.9, 3072 x 2048 21.9 and 23.9, x 8192 75 and 82, but 4096 x 192 6.6 and 5.0,
@@ -510,9 +511,11 @@ static int tiles_choice(int M, int N, int K) {
 //   and 3.0).
 // More: tiles.
 //
-// Whether a lane a chunk.  Long K (up to 8192): one or two rows, N up to 1024, K above 2048 (one row of 1024 x 4608 on cold weights
-// 11.9, rows kernel 12.8; of 1024 x 8192 16.1 and 20.7, two rows 19.6 and 20.6; beyond 1024, one row of 1152 x 5120: 18.0 and 14.2);
-// three and four, N up to 256, K above 3072 (4 rows of 64 x 8192 13.8, rows kernel 16.3); one, N up to 256, K of 32 chunks (5.0, 5.5).
+// Whether a lane a chunk.  Long K: one and two rows of a weight of few, whose blocks of the rows kernel leave the chip idle either way (lanes
+// and rows; 1 row of 32 x 2560 4.4 and 5.5, x 4096 5.7 and 6.4, x 4608 8.0 and 7.4; of 64 x 2560 5.3 and 5.5, x 2816 5.8 and 5.55; of
+// 128 x 2560 5.8 and 5.4, of 1024 x 4608 10.3 and 8.3; 2 rows of 32 x 3584 5.9 and 6.55, x 4096 6.7 and 6.5, of 64 x 2304 5.45 and 5.5, x
+// 2560 6.0 and 5.6, of 1024 x 8192 16.8 and 11.8; 3 rows of 16 x 2304 6.1 and 5.4; 1 row of 32 x 2048 5.0 and 4.05;
+// 1 row of 200 x 2052 6.0 and 6.1, x 2304 5.5 and 5.3, of 64 x 4100 8.1 and 8.4, of 16 x 4100 5.7 and 8.2).
 // Short K (weights in the last-level cache): what a lane does one after the other is K, at most a chunk of it, times the rows; what
 // the rows kernel does is so many blocks.  1 row of 65536 x 4 2.4 us, rows kernel 19.8, 16 rows of 65536 x 128 25.3 and 27.9, x 192
 // 55 and 30; 16 rows of 24000 x 32 10.6 and 11.4, 8 of 24000 x 64 8.2 and 8.3; 4 rows of 8192 x 48 5.3 and 5.8, x 64 6.1 and 5.5;
@@ -520,8 +523,11 @@ static int tiles_choice(int M, int N, int K) {
 static bool lanes_take(int M, int N, int K) {
   if (M > 16) return false;
   if (K > GS_SUM_CHUNK * GF_LANES_CHUNKS) return false;
-  if (M <= 2 && N <= 1024 && K > 2048) return true;
-  if (N <= 256 && ((M <= 4 && K > 3072) || (M == 1 && K > 31 * GS_SUM_CHUNK && K <= 2048))) return true;
+  if (M <= 2 && K > 2048) {
+    const bool cut = K % GS_SUM_CHUNK != 0;                        // (a chunk cut short costs the rows kernel 0.9)
+    if (N <= 32) return K < 4608;
+    return M == 1 ? (N <= 64 && K <= 2560) || (cut && N <= 256 && K < 4608) : N <= 64 && (K <= 2304 || (cut && K < 3072));
+  }
   const int rows = M <= 2 ? M : M <= 4 ? 4 : M <= 8 ? 8 : 16, chain = (K < GS_SUM_CHUNK ? K : GS_SUM_CHUNK) * rows;
   if (K > 2 * GS_SUM_CHUNK) {
     // (rows of whole 256 bytes begin in the same channels)
