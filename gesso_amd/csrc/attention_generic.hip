@@ -153,22 +153,24 @@ __global__ void attention_generic_kernel(const T* __restrict__ q, int q_stride, 
 }
 
 #define GS_ATTN_FEW_WAVES 4
-#define GS_ATTN_FEW_D 64
 
 // Few queries (a decode step in float32) whose heads are at most 64 wide: a block of four wavefronts a (query token, query head), the
 // same sums in the same order.  One wavefront alone waits for a tile's keys, then for its values, sixteen at a time, tile after tile; here
 // each wavefront takes a tile of a round of four, asks for its keys and values at once, and leaves probabilities and values in LDS; the
 // running maximum goes through the tiles' maxima in their order, and one wavefront adds up.  Keys beyond the last are the last one's row,
-// loaded and not used.  (Microseconds by one wavefront and by
-// four, 32 heads of 64 on 8, keys and values in turn from four sets: 1 query of 20 keys 5.0 and 4.7, of 160 13.3 and 6.6, of 2,000 153 and 42; 6 queries 5.2 and 4.8,
-// 16.1 and 7.7, 154 and 45.)
+// loaded and not used.  D: the room of a row in LDS and the most a row is asked for in, the keys' or the values' width rounded up to 16, 32
+// or 64.  (Microseconds by one wavefront and by four, 32 heads of 64 on 8, keys and values cold: 1 query of 20 keys 5.4 and 5.0, of 130
+// 14.2 and 7.0, of 600 51.6 and 17.2, of 2,500 192 and 52; 8 queries 5.5 and 5.15, 14.9 and 7.35, 60 and 18.8, 225 and 57.  Heads of 32,
+// 1 query of 5 keys 4.65 and 4.35, with room for 64 4.7; of 600 51 and 14.1, and 20 where the adding up read its values two at a time.  Heads
+// of 8, 4 queries of 5 keys 4.1 and 3.9, with room for 64 4.5.)
+template <int D>
 __global__ __launch_bounds__(GS_ATTN_FEW_WAVES * 64) void attention_generic_few_kernel(
     const float* __restrict__ q, int q_stride, const float* __restrict__ kcache, const float* __restrict__ vcache,
     const int* __restrict__ positions, const int* __restrict__ seq_of_token, const int* __restrict__ block_table, int max_blocks,
     int page_size, int window, float scale, float* __restrict__ out, int nh, int nkv, int d, int vd, int chunk, int sink, float softcap,
     const float* __restrict__ sinks) {
   typedef __attribute__((ext_vector_type(4))) float f4;
-  constexpr int NW = GS_ATTN_FEW_WAVES, D = GS_ATTN_FEW_D, PIECES = D / 4;
+  constexpr int NW = GS_ATTN_FEW_WAVES, PIECES = D / 4, TOGETHER = 64 / PIECES, LOADS = 64 / TOGETHER;   // rows of values a load, loads a tile
   extern __shared__ float values[];                      // (NW, 64, D)
   __shared__ float qs[D], ps[NW][64], tops[NW], sums[NW];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -179,19 +181,19 @@ __global__ __launch_bounds__(GS_ATTN_FEW_WAVES * 64) void attention_generic_few_
   int lo = window > 0 && pos - window + 1 > 0 ? pos - window + 1 : 0;
   if (chunk > 0 && pos - pos % chunk > lo) lo = pos - pos % chunk;
   float m = sinks ? sinks[h] : (sink ? 0.f : -INFINITY), l = (sink || sinks) ? 1.f : 0.f, acc = 0.f;
-  const int piece = lane & 15, group = lane >> 4;        // of a load of values: 16 bytes, of one of four rows
+  const int piece = lane % PIECES, group = lane / PIECES;  // of a load of values: 16 bytes, of one of its rows
   float* mine = values + wave * 64 * D;
   for (int base = lo; base <= pos; base += 64 * NW) {
     const int u = base + 64 * wave + lane, there = u <= pos ? u : pos;
     const long off = ((long)bt[there / page_size] * nkv + kvh) * page_size + there % page_size;
-    f4 kr[PIECES], vr[16];
+    f4 kr[PIECES], vr[LOADS];
     const bool live = base + 64 * wave <= pos;           // (the same for the whole wavefront; a round's last tiles may hold no key)
     if (live) {
 #pragma unroll
       for (int e = 0; e < PIECES; ++e) kr[e] = *reinterpret_cast<const f4*>(kcache + off * d + (4 * e < d ? 4 * e : 0));
 #pragma unroll
-      for (int e = 0; e < 16; ++e)
-        vr[e] = *reinterpret_cast<const f4*>(vcache + __shfl(off, 4 * e + group) * vd + (4 * piece < vd ? 4 * piece : 0));
+      for (int e = 0; e < LOADS; ++e)
+        vr[e] = *reinterpret_cast<const f4*>(vcache + __shfl(off, TOGETHER * e + group) * vd + (4 * piece < vd ? 4 * piece : 0));
     }
     __builtin_amdgcn_sched_barrier(0);
     __syncthreads();                                     // the queries are there, and the round before is added up
@@ -207,7 +209,7 @@ __global__ __launch_bounds__(GS_ATTN_FEW_WAVES * 64) void attention_generic_few_
       if (softcap > 0.f) s = softcap * tanhf(s / softcap);
       if (u > pos) s = -INFINITY;
 #pragma unroll
-      for (int e = 0; e < 16; ++e) *reinterpret_cast<f4*>(mine + (4 * e + group) * D + 4 * piece) = vr[e];
+      for (int e = 0; e < LOADS; ++e) *reinterpret_cast<f4*>(mine + (TOGETHER * e + group) * D + 4 * piece) = vr[e];
     }
     const float top = wave_max(s);
     if (lane == 0) tops[wave] = top;
@@ -227,12 +229,16 @@ __global__ __launch_bounds__(GS_ATTN_FEW_WAVES * 64) void attention_generic_few_
       m = m_new;
       if (wave == 0) {
         const int nk = pos - base - 64 * w + 1 < 64 ? pos - base - 64 * w + 1 : 64;
-        const float* v = values + w * 64 * D + lane;
+        const float* v = values + w * 64 * D + (lane < D ? lane : 0);
         float a = acc * alpha;
         int k = 0;
         for (; k + 16 <= nk; k += 16) {
+          float x[16];
 #pragma unroll
-          for (int e = 0; e < 16; ++e) a = fmaf(ps[w][k + e], v[(k + e) * D], a);
+          for (int e = 0; e < 16; ++e) x[e] = v[(k + e) * D];
+          __builtin_amdgcn_sched_barrier(0);               // (all sixteen asked for, not two at a time)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) a = fmaf(ps[w][k + e], x[e], a);
         }
         for (; k < nk; ++k) a = fmaf(ps[w][k], v[k * D], a);
         acc = a;
@@ -244,9 +250,10 @@ __global__ __launch_bounds__(GS_ATTN_FEW_WAVES * 64) void attention_generic_few_
 
 // Whether the four wavefronts pay: LDS has room for two such blocks a compute unit, 512 on the chip.  (One wavefront and four, 20, 160 and
 // 600 keys: 16 queries of 32 heads 5.4, 16.4, 54 and 5.4, 9.2, 22 us; one query more 6.2, 19.5, 61 and 8.3, 15.2, 40; 32 queries 6.0, 20.2, 77
-// and 9.2, 16.0, 46; 64 queries 6.9, 26, 97 and 16.6, 31, 88.  How many keys there are the host does not know.)
+// and 9.2, 16.0, 46; 64 queries 6.9, 26, 97 and 16.6, 31, 88.  How many keys there are the host does not know: the
+// first five of 16 queries are 5.25 and 5.5.)
 static bool few_queries(int ntok, int nh, int d, int vd, const void* kcache, const void* vcache, const void* vcos, int window, int keep_first) {
-  return (long)ntok * nh <= 512 && d <= GS_ATTN_FEW_D && vd <= GS_ATTN_FEW_D && d % 4 == 0 && vd % 4 == 0 && !vcos && !(window > 0 && keep_first > 0) &&
+  return (long)ntok * nh <= 512 && d <= 64 && vd <= 64 && d % 4 == 0 && vd % 4 == 0 && !vcos && !(window > 0 && keep_first > 0) &&
          (((uintptr_t)kcache | (uintptr_t)vcache) & 15) == 0;
 }
 
@@ -276,13 +283,22 @@ extern "C" int gs_attention_generic(const void* q, int q_stride, const void* kca
                                                             vsin, interleaved, softcap, keep_first, sinks)
   const bool aligned = ((uintptr_t)kcache & 15) == 0;
   if (dtype == GS_F32 && few_queries(ntok, nh, d, vd, kcache, vcache, vcos, window, keep_first)) {
-    constexpr int lds = GS_ATTN_FEW_WAVES * 64 * GS_ATTN_FEW_D * sizeof(float);
-    // with the rest more than the default limit of LDS: asked for once
-    static const hipError_t asked = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_generic_few_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    (void)asked;
-    attention_generic_few_kernel<<<grid, GS_ATTN_FEW_WAVES * 64, lds, stream>>>(
-        (const float*)q, q_stride, (const float*)kcache, (const float*)vcache, positions, seq_of_token, block_table, max_blocks, page_size,
-        window, scale, (float*)out, nh, nkv, d, vd, chunk, sink, softcap, sinks);
+#define GS_FEW(D)                                                                                                              \
+  do {                                                                                                                         \
+    constexpr int lds = GS_ATTN_FEW_WAVES * 64 * D * sizeof(float);                                                            \
+    if (D == 64) {                                                                                                             \
+      /* with the rest more than the default limit of LDS: asked for once */                                                   \
+      static const hipError_t asked = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_generic_few_kernel<D>),     \
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, lds);                    \
+      (void)asked;                                                                                                             \
+    }                                                                                                                          \
+    attention_generic_few_kernel<D><<<grid, GS_ATTN_FEW_WAVES * 64, lds, stream>>>(                                            \
+        (const float*)q, q_stride, (const float*)kcache, (const float*)vcache, positions, seq_of_token, block_table, max_blocks, page_size, \
+        window, scale, (float*)out, nh, nkv, d, vd, chunk, sink, softcap, sinks);                                              \
+  } while (0)
+    const int wide = d > vd ? d : vd;
+    if (wide <= 16) GS_FEW(16); else if (wide <= 32) GS_FEW(32); else GS_FEW(64);
+#undef GS_FEW
   } else if (dtype == GS_F32) {
     if (aligned && d % 4 == 0) { if (d <= 16) GS_RUN(float, 4); else GS_RUN(float, 16); } else GS_RUN(float, 0);
   } else if (dtype == GS_BF16) {
