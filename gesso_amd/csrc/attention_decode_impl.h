@@ -161,19 +161,22 @@ __global__ __launch_bounds__(W * 64) void attention_decode_kernel(
   // their way.
   // the queries as the second operand: lane (r16, kg) holds head r16's features 32 s + 8 kg .. + 8
   // (lanes past the group load head 0's: every lane loads, no branch hides a load from the compiler's count)
+  // (Without RAW below, beside the page numbers: here they would be asked for before the position, and every row after the last page
+  // number: 32 heads on 8, one sequence of 180 keys 5.3 us for 5.1, 8 of 1,100 15.5 for 14.8.)
   bf16x8_t qreg[KS];
-#pragma unroll
-  for (int st = 0; st < KS; ++st) {
-    if constexpr (MAPS == 2) {
-      const int f0 = 32 * st + 8 * kg, map = f0 / (D / 2);
-      qreg[st] = *reinterpret_cast<const bf16x8_t*>(q + (size_t)seq * q_stride + (size_t)(kvh * G + (r16 < G ? r16 : 0)) * (D / 2) + (f0 < D ? f0 - map * (D / 2) : 0));
-      if (r16 >= G || map != (r16 & 1)) qreg[st] = bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
-    } else if (32 * st + 8 * kg < D)
-      qreg[st] = *reinterpret_cast<const bf16x8_t*>(q + (size_t)seq * q_stride + (size_t)(kvh * G + (r16 < G ? r16 : 0)) * D + 32 * st + 8 * kg);
-    else
-      qreg[st] = bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
-    if (!RAW && r16 >= G) qreg[st] = bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
+#define GS_DECODE_QUERIES                                                                                                      \
+  _Pragma("unroll") for (int st = 0; st < KS; ++st) {                                                                          \
+    if constexpr (MAPS == 2) {                                                                                                 \
+      const int f0 = 32 * st + 8 * kg, map = f0 / (D / 2);                                                                     \
+      qreg[st] = *reinterpret_cast<const bf16x8_t*>(q + (size_t)seq * q_stride + (size_t)(kvh * G + (r16 < G ? r16 : 0)) * (D / 2) + (f0 < D ? f0 - map * (D / 2) : 0)); \
+      if (r16 >= G || map != (r16 & 1)) qreg[st] = bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};                                           \
+    } else if (32 * st + 8 * kg < D)                                                                                           \
+      qreg[st] = *reinterpret_cast<const bf16x8_t*>(q + (size_t)seq * q_stride + (size_t)(kvh * G + (r16 < G ? r16 : 0)) * D + 32 * st + 8 * kg); \
+    else                                                                                                                       \
+      qreg[st] = bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};                                                                             \
+    if (!RAW && r16 >= G) qreg[st] = bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};                                                         \
   }
+  if constexpr (RAW != 0) { GS_DECODE_QUERIES }
   // (The position beside the page numbers, the rotation's factors before the rows, the compiler kept to that order, the arguments in one
   // piece and the new key's places chosen without branches: one sequence of 21 keys 6.6, now 5.5 us, of 400 8.3 and 7.1, of 530 9.8 and
   // 8.65; 8 of 430 8.95 and 7.95; 64 of 180 10.2 and 9.3; groups of two heads, 24 of 700 12.15 and 10.9.  Value products by 16 blocks
@@ -287,6 +290,8 @@ __global__ __launch_bounds__(W * 64) void attention_decode_kernel(
     for (int i = 0; i < NI; ++i) vreg[i] = *reinterpret_cast<const uint4*>(vcache + vo[i]);
   };
 
+  if constexpr (RAW == 0) { GS_DECODE_QUERIES }
+#undef GS_DECODE_QUERIES
   int t = t0 + wave;
   const int first = known || t < t1 ? t : (t0 < tiles ? t0 : 0);
   const bool has_new = RAW && raw.write_kv && t0 < t1 && t1 == tiles;   // this block's keys end with the new one
