@@ -137,6 +137,8 @@ static int decode_entry(const void* q, int q_stride, void* kcache, void* vcache,
   GS_REQUIRE(chunk >= 0, "attention_decode: bad chunk %d", chunk);
   GS_REQUIRE(softcap >= 0.f && keep_first >= 0 && !(sink && sinks), "attention_decode: bad cap, kept positions or sinks");
   GS_REQUIRE(keep_first == 0 || (window > 0 && chunk == 0), "attention_decode: kept first positions go with a window and no runs");
+  GS_REQUIRE(!raw || (chunk == 0 && sink == 0 && softcap == 0.f && keep_first == 0 && !sinks),
+             "attention_decode: rows of q|k|v go without runs, sinks, a cap and kept positions");
   GS_REQUIRE(!out_tiled || (nh * d) % 32 == 0, "attention_decode: tiled rows need a width that is a multiple of 32, not %d", nh * d);
   const int out_tiles = out_tiled ? gs_ceil_div(nseq, 16) : 0;
   GS_REQUIRE(gs_attention_decode_supports(nh, nkv, d), "attention_decode: sizes nh=%d nkv=%d d=%d are not taken", nh, nkv, d);
@@ -162,19 +164,13 @@ static int decode_entry(const void* q, int q_stride, void* kcache, void* vcache,
   none.softcap = softcap;
   none.keep_first = keep_first;
   none.sinks = sinks;
-  DecodeRaw with = raw ? *raw : none;
-  with.chunk = chunk;
-  with.sink = sink ? 1 : 0;
-  with.softcap = softcap;
-  with.keep_first = keep_first;
-  with.sinks = sinks;
 #define GS_ARGS                                                                                             \
   G, grid, stream, (const bf16*)q, q_stride, (bf16*)kcache, (bf16*)vcache, positions, block_table, max_blocks, \
       page_size, page_magic, window, scale, (bf16*)out, part_o, part_ml, nh, nkv, out_tiles
   if (raw) {
     switch (d) {
-      case 64: rc = launch_decode<64, 1>(GS_ARGS, with); break;
-      case 128: rc = launch_decode<128, 1>(GS_ARGS, with); break;
+      case 64: rc = launch_decode<64, 1>(GS_ARGS, *raw); break;
+      case 128: rc = launch_decode<128, 1>(GS_ARGS, *raw); break;
     }
   } else {
     switch (d) {

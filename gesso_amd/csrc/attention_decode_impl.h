@@ -32,7 +32,7 @@ struct DecodeRaw {
   const float* cos_t;    // (positions, D / 2)
   const float* sin_t;
   int write_kv;          // 0: another layer owns the cache; the new key is already in it
-  // (read with and without RAW) chunk > 0: the query sees no key before the first position of its own run of `chunk`
+  // (the rest is read without RAW only) chunk > 0: the query sees no key before the first position of its own run of `chunk`
   // positions; sink: one more term exp(0), without a value, in the softmax's denominator
   int chunk;
   int sink;
