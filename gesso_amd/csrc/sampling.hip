@@ -698,7 +698,7 @@ __global__ __launch_bounds__(SAMP_THREADS) void choose_pick_kernel(
   } else {
     const double* pr = part + (size_t)row * nparts;
     const int per = nparts / SAMP_THREADS;
-    // (sixteen of a thread's sums asked for at a time, in loads of two; added one by one)
+    // (sixteen of a thread's sums asked for at a time, in loads of two, what is left eight at a time; added one by one)
     double ls = 0.0;
     typedef double __attribute__((ext_vector_type(2))) pair_t;
     int done = 0;
@@ -710,24 +710,23 @@ __global__ __launch_bounds__(SAMP_THREADS) void choose_pick_kernel(
 #pragma unroll
         for (int i = 0; i < 8; ++i) ls = (ls + two[i][0]) + two[i][1];
       }
+#pragma unroll 8
     for (; done < per; ++done) ls += pr[tid * per + done];
     if (P < 1.0) {
       // The total alone, as the last of the running sums below adds it up (pairs, then pairs of pairs), and the ready-made
-      // histograms beside it: both passes over them then read LDS.
+      // histograms beside it: both passes over them then read LDS.  (Loops, not unrolled: their code stands before the draws from the
+      // whole row, which took 0.4 us longer behind it; 64 rows of 500 15.9 us without it, 16.3 unrolled, now 15.9; from a nucleus 30.9 with
+      // every running sum, 27.85 unrolled, now 28.0.)
       if (ghist)
         for (int i = tid; i < 2 * NUC_GHIST; i += SAMP_THREADS) hist[i] = ghist[(size_t)row * 2 * NUC_GHIST + i];
-#pragma unroll
+#pragma unroll 1
       for (int off = 1; off < 64; off <<= 1) ls += __shfl_xor(ls, off, 64);
       if ((tid & 63) == 0) scan[tid >> 6] = ls;
       __syncthreads();
-      double w[SAMP_THREADS / 64];
-#pragma unroll
-      for (int i = 0; i < SAMP_THREADS / 64; ++i) w[i] = scan[i];
-#pragma unroll
-      for (int off = 1; off < SAMP_THREADS / 64; off <<= 1)
-#pragma unroll
-        for (int i = 0; i < SAMP_THREADS / 64; i += 2 * off) w[i] += w[i + off];
-      row_nucleus_pick(wbuf + (size_t)row * V, V, P, uu, w[0], ghist ? hist : nullptr, &sid, &sbad);
+      double total = scan[tid & (SAMP_THREADS / 64 - 1)];
+#pragma unroll 1
+      for (int off = 1; off < SAMP_THREADS / 64; off <<= 1) total += __shfl_xor(total, off, 64);
+      row_nucleus_pick(wbuf + (size_t)row * V, V, P, uu, total, ghist ? hist : nullptr, &sid, &sbad);
       goto chosen;
     }
     scan[tid] = ls;
