@@ -46,11 +46,13 @@ void gs_skinny_run_plain(const void* X, int ldx, int x_tiled, const float* res, 
   c.ex.squared = squared;
   if (res || ssq) lazy(c, res, ssq, nb, norm_w, eps);
   // Half tiles (the same bits) where a block of eight weight rows still comes once to a compute unit and K is long enough for the
-  // sum over the wavefronts not to bind.  Cold weights, microseconds in half and in whole tiles of gemm_skinny_impl.h's kernel: 1 row of 2048 x 8192 8.2 and 10.4,
-  // of 1024 x 4608 5.3 and 6.75, of 2048 x 2048 3.9 and 4.3, of 1360 x 2048 3.7 and 4.1; 8 rows the same, 16 10.3 and 11.9, 6.8 and
-  // 7.7, 4.4 and 4.8, 4.2 and 4.6; 32 rows 24.4 and 24.9, 15.4 and 15.6, 8.8 and 8.8; beyond 32 the blocks' reading of X outweighs
-  // the rest.  In whole tiles K below 2048 (2048 x 1024 2.9 both, 1024 x 1024 2.7 both) and more than 256 blocks (8 rows of 2560 x 2560
-  // 5.9 and 5.3, of 3072 x 1024 3.9 and 3.6; 32 of 2304 x 4608 26.8 and 16.9).
+  // sum over the wavefronts not to bind.  Cold weights, microseconds in half and in whole tiles of gemm_few_impl.h's kernel: 1 row of 2048 x
+  // 8192 8.0 and 10.1, of 1024 x 4608 5.2 and 6.5, of 2048 x 2048 3.8 and 4.1, of 1360 x 2048 3.4 and 3.7; 8 rows the same; 16 10.0 and
+  // 11.5, 6.6 and 7.5, 4.3 and 4.6, 3.8 and 4.2; 32 13.2 and 15.0, 8.3 and 9.4, 5.2 and 5.9, 4.5 and 5.0, weighted for their norm 14.6 and
+  // 16.3, 9.4 and 10.4, 6.4 and 6.9, 5.7 and 6.1; beyond 32 the blocks' reading of X outweighs the rest.  In whole tiles K below 2048 (2048 x
+  // 1024 of 1 row 3.05 both, of 32 3.65 and 3.75, of 1024 x 1024 3.25 both) and more than 256 blocks (1 row of 2064 x 2048 4.4 and 4.1, 8 of
+  // 2560 x 2560 5.6 and 5.1, 32 of it 9.2 and 7.0, of 2304 x 4608 14.3 and 10.05).  Another K goes to gemm_skinny_impl.h's kernel, in halves
+  // from four rows on (1 row of 1024 x 3072 7.3 and 7.1).
   const bool half = Wt && epilogue == 0 && N % 16 == 0 && N <= 2048 && K >= 2048 && M <= 32;
   if (gs_few_plain(c, Wt, half)) return;
   if (half && M >= 4) gs_skinny_plain_half_tiles(c);
