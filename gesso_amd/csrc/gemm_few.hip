@@ -58,9 +58,6 @@ bool gs_few_plain(const SkinnyCall& c, const void* Wt, bool half) {
   // 2048 14.5, of 4096 x 4096 13.8 for 13.1; with a ring of three and 108: 13.6 and 13.35, of 8192 x 1024 8.2 for 7.8.)
   const bool wide = !half && c.N > 8192;
   if (wide ? !few_pairs(c) : c.M > 32 && c.N > 4096) return false;
-  // 17 to 32 plain rows and a K of 2,048: its ring of eight steps holds a wavefront's whole share, this kernel's of four does not (24 rows of
-  // 3072 x 2048 5.46 and 5.56 us, 32 of 2560 x 2048 5.75 and 6.0; of 2560 x 1792 6.4 and 5.5, x 2560 7.35 and 6.8).
-  if (!half && !wide && !c.ex.ssq && c.M > 16 && c.M <= 32 && c.N <= 4096 && c.K == 2048) return false;
   if (!few_takes(c, Wt, wide && c.M > 32 ? 4 : 8, half)) return false;
   if (half) few_plain<1, 8, 2, true>(c, c.N / 8);
   else if (!wide) few_plain<1, 8, 4, false>(c, c.N / 16);
