@@ -23,15 +23,18 @@ FewArgs few_args(const SkinnyCall& c) {
   return g;
 }
 
+// Loads a wavefront at least: halves come with a K of 2,048 (four); of one tile a block 4 M weights or more, loaded once, are a K of 512
+// (8,192 rows; two), above 32 rows of X 1,024 (4,096 rows; four).
 template <int R, int W34, int MOST, bool HALF, bool SCALED, bool ONCE>
-static void few_plain_out(const SkinnyCall& c, int blocks) {
-  if (c.y_dtype == GS_F32) launch_few_rows<R, 8, W34, MOST, HALF, SCALED, 0, 1, ONCE, float>(blocks, few_args(c), c.stream);
-  else launch_few_rows<R, 8, W34, MOST, HALF, SCALED, 0, 1, ONCE, bf16>(blocks, few_args(c), c.stream);
+static bool few_plain_out(const SkinnyCall& c, int blocks) {
+  constexpr int least = HALF ? 4 : R == 1 && ONCE ? 2 : 1, least34 = R == 1 && ONCE ? 4 : 1;
+  return c.y_dtype == GS_F32 ? launch_few_rows<R, 8, W34, MOST, HALF, SCALED, 0, 1, ONCE, float, least, least34>(blocks, few_args(c), c.stream)
+                             : launch_few_rows<R, 8, W34, MOST, HALF, SCALED, 0, 1, ONCE, bf16, least, least34>(blocks, few_args(c), c.stream);
 }
 template <int R, int W34, int MOST, bool HALF>
-static void few_plain(const SkinnyCall& c, int blocks) {
-  if (skinny_once(c.N, c.K)) c.ex.ssq ? few_plain_out<R, W34, 2, HALF, true, true>(c, blocks) : few_plain_out<R, W34, MOST, HALF, false, true>(c, blocks);
-  else c.ex.ssq ? few_plain_out<R, W34, 2, HALF, true, false>(c, blocks) : few_plain_out<R, W34, MOST, HALF, false, false>(c, blocks);
+static bool few_plain(const SkinnyCall& c, int blocks) {
+  if (skinny_once(c.N, c.K)) return c.ex.ssq ? few_plain_out<R, W34, 2, HALF, true, true>(c, blocks) : few_plain_out<R, W34, MOST, HALF, false, true>(c, blocks);
+  return c.ex.ssq ? few_plain_out<R, W34, 2, HALF, true, false>(c, blocks) : few_plain_out<R, W34, MOST, HALF, false, false>(c, blocks);
 }
 
 // Two tiles a block and 17 to 48 plain rows: up to a K of 4,096 and, of more than 32 rows, 10,240 weight rows.  Beyond, both wait for the same
@@ -46,11 +49,7 @@ static bool few_pairs(const SkinnyCall& c) {
 // A plain product (`half`: of a weight of few rows and up to 32 of X, half a tile a block), or gate and up with SwiGLU; false: not for
 // these kernels.
 bool gs_few_plain(const SkinnyCall& c, const void* Wt, bool half) {
-  if (c.epilogue == 1) {
-    if (c.y_dtype != GS_BF16 || !few_pairs(c) || !few_takes(c, Wt, few_glu_waves(c), false)) return false;
-    gs_few_swiglu(c);
-    return true;
-  }
+  if (c.epilogue == 1) return c.y_dtype == GS_BF16 && few_pairs(c) && few_takes(c, Wt, few_glu_waves(c), false) && gs_few_swiglu(c);
   // More than 32 rows and one tile a block: where every block has a compute unit to itself.  (Microseconds there and here.  A ring of four loads for three or four row
   // tiles leaves a unit one block, gemm_skinny_impl.h's two: 48 rows of 4096 x 4096 11.6 and 11.5 us, of 3072 x 2048 6.9 and
   // 6.7, of 4112 x 2048 9.9 and 10.1, of 8192 x 1024 6.85 and 7.6, x 2048 11.7 and 12.1; 64 rows of 4096 x 2560 10.1 and 9.25, of 6144 x 2048
@@ -59,34 +58,25 @@ bool gs_few_plain(const SkinnyCall& c, const void* Wt, bool half) {
   const bool wide = !half && c.N > 8192;
   if (wide ? !few_pairs(c) : c.M > 32 && c.N > 4096) return false;
   if (!few_takes(c, Wt, wide && c.M > 32 ? 4 : 8, half)) return false;
-  if (half) few_plain<1, 8, 2, true>(c, c.N / 8);
-  else if (!wide) few_plain<1, 8, 4, false>(c, c.N / 16);
-  else few_plain<2, 4, 4, false>(c, gs_ceil_div(c.N, 32));
-  return true;
+  if (half) return few_plain<1, 8, 2, true>(c, c.N / 8);
+  return wide ? few_plain<2, 4, 4, false>(c, gs_ceil_div(c.N, 32)) : few_plain<1, 8, 4, false>(c, c.N / 16);
 }
 
 bool gs_few_gated(const SkinnyCall& c, const void* Wt) {
-  if (!few_pairs(c) || !few_takes(c, Wt, c.M > 32 ? 4 : 8, false)) return false;
-  gs_few_gated_run(c);
-  return true;
+  return few_pairs(c) && few_takes(c, Wt, c.M > 32 ? 4 : 8, false) && gs_few_gated_run(c);
 }
 
 // Into the stream: weights of few rows, half a tile a block, up to 32 rows (more come in parts).
 bool gs_few_residual(const SkinnyCall& c, const void* Wt) {
-  if (c.M > 32 || !gs_skinny_halves(c.N) || !few_takes(c, Wt, 8, true)) return false;
-  gs_few_residual_run(c);
-  return true;
+  return c.M <= 32 && gs_skinny_halves(c.N) && few_takes(c, Wt, 8, true) && gs_few_residual_run(c);
 }
 
-// The convolution: where every block has a compute unit to itself (three tiles' sums leave a lane's registers no room for two).
+// The convolution: where every block has a compute unit to itself (three tiles' sums and four channels' taps are 134 registers, 128
+// would leave it room for two).
 bool gs_few_conv(const SkinnyCall& c, const void* Wt) {
-  if (!c.ex.conv_vec || c.N / 24 > 256 || !few_takes(c, Wt, 8, true)) return false;
-  gs_few_conv_run(c);
-  return true;
+  return c.ex.conv_vec && c.N / 24 <= 256 && few_takes(c, Wt, 8, true) && gs_few_conv_run(c);
 }
 
 bool gs_few_parts(const SkinnyCall& c, const void* Wt, int parts) {
-  if (!few_takes(c, Wt, 4, false, parts)) return false;
-  gs_few_parts_run(c, parts);
-  return true;
+  return few_takes(c, Wt, 4, false, parts) && gs_few_parts_run(c, parts);
 }

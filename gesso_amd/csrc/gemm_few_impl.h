@@ -359,8 +359,8 @@ __global__ __launch_bounds__(WAVES * 64, MT == 1 && R == 2 ? WAVES / 2 : 1) void
 }
 
 // Where a wavefront's loads start: in halves four, or five where one would be left over (a round trip of its own: 1024 x 4608, nine
-// loads a wavefront, 5.6 and 5.3 us), or all there are; three tiles' halves two (as good as four, and a lane's registers leave room
-// for two blocks a compute unit) or, of three, all; whole tiles eight, four, two or one.
+// loads a wavefront, 5.6 and 5.3 us), or all there are; three tiles' halves two (as good as four) or, of three, all; whole tiles eight,
+// four, two or one.
 static inline int few_first(int units, bool half, bool three) {
   if (!half) return units >= 8 ? 8 : units >= 4 ? 4 : units >= 2 ? 2 : 1;
   if (three) return units == 3 ? 3 : units >= 2 ? 2 : 1;
@@ -379,45 +379,53 @@ static void launch_few_first(dim3 grid, const FewArgs& g, hipStream_t stream) {
   kernel<<<grid, WAVES * 64, lds, stream>>>(g);
 }
 
-template <int R, int MT, int WAVES, bool HALF, bool SCALED, int EPI, int CW, bool ONCE, typename TOut>
-static void launch_few(dim3 grid, const FewArgs& g, hipStream_t stream) {
+// LEAST: what callers' rules leave of K is that many loads a wavefront or more; shorter starts are not compiled (a call that had fewer
+// would come back false, nothing launched).
+template <int R, int MT, int WAVES, bool HALF, bool SCALED, int EPI, int CW, bool ONCE, typename TOut, int LEAST = 1>
+static bool launch_few(dim3 grid, const FewArgs& g, hipStream_t stream) {
   const int units = (g.K >> 5) / (WAVES * (HALF ? 2 : 1) * (EPI == 5 ? (int)grid.x : 1));
-#define GS_FEW(F) launch_few_first<R, MT, WAVES, HALF, SCALED, EPI, CW, F, ONCE, TOut>(grid, g, stream)
+#define GS_FEW(F, COMPILED)                                                                               \
+  if constexpr (COMPILED) {                                                                               \
+    launch_few_first<R, MT, WAVES, HALF, SCALED, EPI, CW, F, ONCE, TOut>(grid, g, stream);                \
+    return true;                                                                                          \
+  }
   if constexpr (MT > 1) {
     // (a ring of four loads a weight tile, three tiles' halves and four tiles of two: what a lane's registers hold beside the sums)
-    if (units >= 4 && R < 3) { if constexpr (R < 3) GS_FEW(4); }
-    else if (units >= 2) GS_FEW(2);
-    else GS_FEW(1);
+    if (units >= 4 && R < 3) { GS_FEW(4, R < 3) }
+    else if (units >= 2) { GS_FEW(2, R >= 3 || LEAST < 4) }
+    else { GS_FEW(1, LEAST < 2) }
   } else {
     switch (few_first(units, HALF, R >= 3)) {
-      case 1: GS_FEW(1); break;
-      case 2: GS_FEW(2); break;
-      case 3: if constexpr (HALF) GS_FEW(3); break;
-      case 4: if constexpr (R < 3) GS_FEW(4); break;
-      case 5: if constexpr (HALF && R < 3) GS_FEW(5); break;
-      default: if constexpr (!HALF) GS_FEW(8); break;
+      case 1: GS_FEW(1, LEAST < 2) break;
+      case 2: GS_FEW(2, HALF ? R >= 3 || LEAST < 3 : LEAST < 4) break;
+      case 3: GS_FEW(3, HALF && LEAST < 4) break;
+      case 4: GS_FEW(4, R < 3) break;
+      case 5: GS_FEW(5, HALF && R < 3) break;
+      default: GS_FEW(8, !HALF) break;
     }
   }
+  return false;
 #undef GS_FEW
 }
 
 // By row tiles: one to MOST of them, in blocks of W12 wavefronts (one and two) and W34.
-template <int R, int W12, int W34, int MOST, bool HALF, bool SCALED, int EPI, int CW, bool ONCE, typename TOut>
-static void launch_few_rows(dim3 grid, const FewArgs& g, hipStream_t stream) {
+template <int R, int W12, int W34, int MOST, bool HALF, bool SCALED, int EPI, int CW, bool ONCE, typename TOut, int LEAST = 1, int LEAST34 = LEAST>
+static bool launch_few_rows(dim3 grid, const FewArgs& g, hipStream_t stream) {
   switch ((g.M + 15) / 16) {
-    case 1: launch_few<R, 1, W12, HALF, SCALED, EPI, CW, ONCE, TOut>(grid, g, stream); break;
-    case 2: launch_few<R, 2, W12, HALF, SCALED, EPI, CW, ONCE, TOut>(grid, g, stream); break;
-    case 3: if constexpr (MOST >= 3) launch_few<R, 3, W34, HALF, SCALED, EPI, CW, ONCE, TOut>(grid, g, stream); break;
-    default: if constexpr (MOST >= 4) launch_few<R, 4, W34, HALF, SCALED, EPI, CW, ONCE, TOut>(grid, g, stream); break;
+    case 1: return launch_few<R, 1, W12, HALF, SCALED, EPI, CW, ONCE, TOut, LEAST>(grid, g, stream);
+    case 2: return launch_few<R, 2, W12, HALF, SCALED, EPI, CW, ONCE, TOut, LEAST>(grid, g, stream);
+    case 3: if constexpr (MOST >= 3) return launch_few<R, 3, W34, HALF, SCALED, EPI, CW, ONCE, TOut, LEAST34>(grid, g, stream); break;
+    default: if constexpr (MOST >= 4) return launch_few<R, 4, W34, HALF, SCALED, EPI, CW, ONCE, TOut, LEAST34>(grid, g, stream); break;
   }
+  return false;
 }
 
 // Between the entry points (gemm_skinny_glue.hip) and the launches (gemm_few.hip, gemm_few_glu.hip, gemm_few_block.hip).
 FewArgs few_args(const SkinnyCall& c);
 bool gs_skinny_halves(int N);
 int few_glu_waves(const SkinnyCall& c);
-void gs_few_swiglu(const SkinnyCall& c);
-void gs_few_gated_run(const SkinnyCall& c);
-void gs_few_residual_run(const SkinnyCall& c);
-void gs_few_conv_run(const SkinnyCall& c);
-void gs_few_parts_run(const SkinnyCall& c, int parts);
+bool gs_few_swiglu(const SkinnyCall& c);
+bool gs_few_gated_run(const SkinnyCall& c);
+bool gs_few_residual_run(const SkinnyCall& c);
+bool gs_few_conv_run(const SkinnyCall& c);
+bool gs_few_parts_run(const SkinnyCall& c, int parts);
