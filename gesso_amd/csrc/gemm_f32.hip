@@ -40,7 +40,7 @@ __device__ __forceinline__ gf_f32x4_t gf_load(const float* __restrict__ row, int
   return k < K ? v : gf_f32x4_t{0.f, 0.f, 0.f, 0.f};
 }
 
-// WR: rows of W a block owns (8 or 16), XR: rows of X (4, 8, or tiles of 16), D: chunks a wavefront holds in flight.
+// WR: rows of W a block owns (8 or 16), XR: rows of X (4, 8, or tiles of 16), D: turns a wavefront holds in flight, of CH chunks each.
 // GLU: W holds N / 2 gate rows, then as many up rows; a block takes WR / 2 of each, a gate's sum and its up's end WR / 2 lanes apart, and
 // silu(gate) * up is stored, N / 2 wide.  (A pass of its own was a launch a layer and the 16384-wide rows
 // out and in again: a decode step of 6 requests, 16 such layers, LFM2-1.2B sizes in float32, 1.295 ms, now 1.257.)
@@ -50,7 +50,7 @@ __global__ __launch_bounds__(GF_WAVES * 64) void gemm_f32_rows_kernel(const floa
                                                                       const float* __restrict__ bias, TO* __restrict__ Y,
                                                                       int ldy, int M, int N, int K, int room) {
   constexpr int MT = XR > 16 ? XR / 16 : 1, XT = XR < 16 ? XR : 16;       // tiles of X, rows used of each
-  // Half a tile of W and half a tile of X: two chunks share the instructions, the second in the tiles' other halves; its sums come out in
+  // CH = 2, half a tile of W and half a tile of X: two chunks share the instructions, the second in the tiles' other halves; its sums come out in
   // the opposite quarter, the other two hold nothing.  (One chunk at a time is sixteen products of 32 cycles in a chain, more than the
   // weights take: a decode step's kernels of 6 rows, microseconds one and two at a time: 2048 x 8192 and 2048 x 2048 13.0 and 10.7 in
   // the mean, 6144 x 2048 14.1 and 12.1, 3072 x 2048 10.0 and 8.3.)

@@ -26,7 +26,9 @@
 // in that order.
 //
 // A tile-major weight whose K the wavefronts share evenly, without the norm's fold (PRO 1), goes to gemm_few_impl.h's kernel, which
-// gives the same bits sooner; here is what it does not take.
+// gives the same bits sooner, by the rules of gemm_few.hip (gs_few_*).  Here is what they leave: besides stored rows and other K, weighted
+// rows beyond 32, products into the stream beyond 32 rows or of weights not cut in halves, convolutions of more than 2,048 channels or
+// unaligned state, float32 results of SwiGLU, and the sizes whose figures stand there.
 //
 // What feeds X (PRO):
 //   0  X is given, bfloat16.
