@@ -42,9 +42,9 @@ __device__ __forceinline__ gf_f32x4_t gf_load(const float* __restrict__ row, int
 
 // WR: rows of W a block owns (8 or 16), XR: rows of X (4, 8, or tiles of 16), D: turns a wavefront holds in flight, of CH chunks each.
 // GLU: W holds N / 2 gate rows, then as many up rows; a block takes WR / 2 of each, a gate's sum and its up's end WR / 2 lanes apart, and
-// silu(gate) * up is stored, N / 2 wide.  (A pass of its own was a launch a layer and the 16384-wide rows
+// silu(gate) * up is stored, N / 2 wide.  SPARE: sums that nobody keeps are stored behind the others, not left out.  (A pass of its own was a launch a layer and the 16384-wide rows
 // out and in again: a decode step of 6 requests, 16 such layers, LFM2-1.2B sizes in float32, 1.295 ms, now 1.257.)
-template <int WR, int XR, int D, int CH, bool TAIL, typename TO, bool GLU>
+template <int WR, int XR, int D, int CH, bool TAIL, typename TO, bool GLU, bool SPARE = false>
 __global__ __launch_bounds__(GF_WAVES * 64) void gemm_f32_rows_kernel(const float* __restrict__ X, int ldx,
                                                                       const float* __restrict__ W,
                                                                       const float* __restrict__ bias, TO* __restrict__ Y,
@@ -116,7 +116,10 @@ __global__ __launch_bounds__(GF_WAVES * 64) void gemm_f32_rows_kernel(const floa
       for (int q = 0; q < 16; ++q) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[q], x[q], acc, 0, 0, 0);
       // element e of lane l: row 4 (l / 16) + e of W, row l % 16 of X: X's row after X's row, WR numbers each
       const int h = CH == 2 ? r16 >> 3 : 0, m = CH == 2 ? r16 & 7 : r16, n = CH == 2 ? 4 * g - 8 * h : 4 * g;
-      if (h < keep && n >= 0 && n < WR && m < XT) *reinterpret_cast<gf_f32x4_t*>(sums + (c + h) * OUT + (i * XT + m) * WR + n) = acc;
+      const bool kept = h < keep && n >= 0 && n < WR && m < XT;
+      float* at = sums + (c + h) * OUT + (i * XT + m) * WR + n;
+      if (SPARE) at = kept ? at : sums + room * OUT + 4 * lane;
+      if (SPARE || kept) *reinterpret_cast<gf_f32x4_t*>(at) = acc;
     }
   };
   float tot[PER];
@@ -418,7 +421,7 @@ static void launch_rows(const float* X, int ldx, const float* W, const float* bi
   constexpr int out = XR * WR;
   const int blocks = GLU ? gs_ceil_div(N / 2, WR / 2) : gs_ceil_div(N, WR), chunks = gs_ceil_div(K, GS_SUM_CHUNK), most = (blocks <= 256 ? 16384 : 8192) / out;
   const int room = chunks < most ? chunks : most;
-  const size_t lds = (size_t)room * out * sizeof(float);
+  size_t lds = (size_t)room * out * sizeof(float);
   auto kernel = K % GS_SUM_CHUNK == 0 ? &gemm_f32_rows_kernel<WR, XR, D, CH, false, TO, GLU> : &gemm_f32_rows_kernel<WR, XR, D, CH, true, TO, GLU>;
   if (lds + sizeof(float) * GF_WAVES * 16 * (GS_SUM_CHUNK + 4) > 64 * 1024) {
     // more than the default limit of LDS: asked for once per kernel
@@ -426,6 +429,15 @@ static void launch_rows(const float* X, int ldx, const float* W, const float* bi
         hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_rows_kernel<WR, XR, D, CH, false, TO, GLU>), hipFuncAttributeMaxDynamicSharedMemorySize, 65536),
         hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_rows_kernel<WR, XR, D, CH, true, TO, GLU>), hipFuncAttributeMaxDynamicSharedMemorySize, 65536)};
     (void)asked;
+  }
+  if constexpr (WR == 16 && XR == 8 && !GLU) {
+    // (what nobody keeps goes to a spare place: behind a branch for it the compiler asks for the operands of one instruction after the
+    // other, which up to sixteen chunks, one cut short, do not hide: 8 rows of 65536 x 132 29.0 us, with the branch 31.4, of 40000 x 964 34.1
+    // and 34.5, x 1028 54.9 and 49.0)
+    if (K % GS_SUM_CHUNK != 0 && chunks <= 16) {
+      kernel = &gemm_f32_rows_kernel<WR, XR, D, CH, true, TO, GLU, true>;
+      lds += 64 * sizeof(gf_f32x4_t);
+    }
   }
   kernel<<<blocks, GF_WAVES * 64, lds, stream>>>(X, ldx, W, bias, Y, ldy, M, N, K, room);
 }
