@@ -447,7 +447,13 @@ static void launch_rows(const float* X, int ldx, const float* W, const float* bi
 // rows of more than 2,048 weight rows stay so up to 1,024.  (Microseconds one and two at a time: 1 row of 1024 x 512 3.2 and 3.5, of
 // 8192 x 512 6.2 and 7.6, x 576 8.9 and 8.1; 4 rows of 3072 x 1024 5.7 and 5.9, x 1088 7.5 and 6.8; 8 rows of 2048 x 768 4.5 and 4.4, of
 // 6144 x 1024 8.0 and 8.8, x 1088 11.2 and 10.3; 6 rows of 8192 x 512 6.5 and 8.6.)
-static bool two_chunks(int M, int N, int K) { return K > (M > 2 && N > 2048 ? 1024 : 512); }
+// Of a K whose last chunk is cut short (84 and 106 registers for 67 and 94) one at a time also up to 1,024, but for two rows of up to 2,048,
+// and just above 2,048, but for two rows of up to 5,120: 1 row of 6144 x 900 8.1 and 9.8, x 1028 11.0 and 10.7, x 2308 16.9 and 19.0, of
+// 512 x 2052 7.1 and 6.3; 8 rows of 2048 x 2308 8.7 and 9.2.
+static bool two_chunks(int M, int N, int K) {
+  if (K % GS_SUM_CHUNK != 0 && ((K <= 1024 && (M > 2 || N > 2048)) || (K > 2048 && K <= 2560 && (M > 2 || N > 5120)))) return false;
+  return K > (M > 2 && N > 2048 ? 1024 : 512);
+}
 
 template <int WR, int XR, int D, typename TO, bool GLU = false>
 static void run_rows(const float* X, int ldx, const float* W, const float* bias, TO* Y, int ldy, int M, int N, int K, hipStream_t stream) {
