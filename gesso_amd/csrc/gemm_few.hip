@@ -41,8 +41,11 @@ static bool few_plain(const SkinnyCall& c, int blocks) {
 // bytes and gemm_skinny_impl.h's kernel is as fast or faster (microseconds there and here, cold weights: gate and up 24 rows of 10240 x 2560
 // 15.2 and 14.5, of 12288 x 4096 22.4 both, of 22528 x 4096 32.9 and 33.5; 48 rows of 9216 x 1024 9.0 and 8.8, of 10240 x 2560 18.2 both,
 // of 16384 x 2048 16.1 and 16.3, of 28672 x 4096 50.8 and 52.1; stored, 17 rows of 12288 x 2048 12.8 and 12.5, of 16384 x 4096 25.9 and 26.6;
-// 48 rows of 65536 x 2048 57.9 and 58.9).  Up to 16 rows, 49 and more, or rows weighted for their norm: nothing was slower.
+// 48 rows of 65536 x 2048 57.9 and 58.9).  Up to 16 rows, 49 and more, or rows weighted for their norm: nothing was slower.  SwiGLU of up to 32
+// rows that lie as rows, not in tiles: from 16,384 rows of 2,048 on (24 of 12288 x 2048 15.15 and 15.2, of 16384 x 2048 15.85 and 16.2, of 28672 x
+// 2048 27.5 and 28.4, of 24576 x 1536 18.5 and 18.0).
 static bool few_pairs(const SkinnyCall& c) {
+  if (c.M > 16 && c.M <= 32 && c.epilogue == 1 && !c.ex.ssq && !c.ex.x_tiled && c.N >= 16384 && c.K >= 2048) return false;
   return c.M <= 16 || c.M > 48 || c.ex.ssq || (c.K < 4096 && (c.M <= 32 || c.N <= 10240));
 }
 
