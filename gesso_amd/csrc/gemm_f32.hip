@@ -430,10 +430,11 @@ static void launch_rows(const float* X, int ldx, const float* W, const float* bi
         hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_rows_kernel<WR, XR, D, CH, true, TO, GLU>), hipFuncAttributeMaxDynamicSharedMemorySize, 65536)};
     (void)asked;
   }
-  if constexpr (WR == 16 && XR == 8 && !GLU) {
+  if constexpr (WR == 16 && XR == 8) {
     // (what nobody keeps goes to a spare place: behind a branch for it the compiler asks for the operands of one instruction after the
     // other, which up to sixteen chunks, one cut short, do not hide: 8 rows of 65536 x 132 29.0 us, with the branch 31.4, of 40000 x 964 34.1
-    // and 34.5, x 1028 54.9 and 49.0)
+    // and 34.5, x 1028 54.9 and 49.0; 5 rows of gate and
+    // up, 20352 x 676 18.1 and 19.6, 40000 x 516 27.4 and 30.5)
     if (K % GS_SUM_CHUNK != 0 && chunks <= 16) {
       kernel = &gemm_f32_rows_kernel<WR, XR, D, CH, true, TO, GLU, true>;
       lds += 64 * sizeof(gf_f32x4_t);
