@@ -41,12 +41,24 @@ static bool few_plain(const SkinnyCall& c, int blocks) {
 // bytes and gemm_skinny_impl.h's kernel is as fast or faster (microseconds there and here, cold weights: gate and up 24 rows of 10240 x 2560
 // 15.2 and 14.5, of 12288 x 4096 22.4 both, of 22528 x 4096 32.9 and 33.5; 48 rows of 9216 x 1024 9.0 and 8.8, of 10240 x 2560 18.2 both,
 // of 16384 x 2048 16.1 and 16.3, of 28672 x 4096 50.8 and 52.1; stored, 17 rows of 12288 x 2048 12.8 and 12.5, of 16384 x 4096 25.9 and 26.6;
-// 48 rows of 65536 x 2048 57.9 and 58.9).  Up to 16 rows, 49 and more, or rows weighted for their norm: nothing was slower.  SwiGLU of up to 32
+// 48 rows of 65536 x 2048 57.9 and 58.9).  49 rows and more, or more than 16 weighted for their norm: nothing was slower.  SwiGLU of up to 32
 // rows that lie as rows, not in tiles: from 16,384 rows of 2,048 on (24 of 12288 x 2048 15.15 and 15.2, of 16384 x 2048 15.85 and 16.2, of 28672 x
 // 2048 27.5 and 28.4, of 24576 x 1536 18.5 and 18.0).
+// Up to 16 rows: but for one to three of a long K, which gain nothing here or lose (1 row weighted for its norm,
+// SwiGLU of 1024 x 6144 10.5 and 10.7, x 10752 16.7 and 17.35, of 4096 x 9216 16.8 and 17.2; 2 rows, stored, of 12288 x 8192 42.3 and 43.1;
+// 4 rows of 4096 x 7168 15.3 and 14.9; of the gated activation only one row from 10,240 on: 1024 x 10752 17.35
+// and 17.6, x 8192 12.9 both), and but for 7 to 12 rows of a long K that lie a multiple of 16 KB apart (8 rows of 9216 x
+// 8192 37.8 and 39.3, of 14336 x 8192 43.9 and 46.2; of SwiGLU and gated ones those of about a block a compute unit: 8192 x 8192
+// 25.2 and 26.6, 25.6 and 26.2, but 5120 x 8192 18.5 and 18.4, 9216 x 8192 34.8 and 35.0, gated 35.4 and 35.0).
 static bool few_pairs(const SkinnyCall& c) {
-  if (c.M > 16 && c.M <= 32 && c.epilogue == 1 && !c.ex.ssq && !c.ex.x_tiled && c.N >= 16384 && c.K >= 2048) return false;
-  return c.M <= 16 || c.M > 48 || c.ex.ssq || (c.K < 4096 && (c.M <= 32 || c.N <= 10240));
+  if (c.M <= 16) {
+    const bool gated = c.epilogue == 4;
+    if (c.M <= (gated ? 1 : 3) && c.K >= (gated ? 10240 : 6144)) return false;
+    if (!c.ex.x_tiled && c.M >= 7 && c.M <= 12 && c.K >= 8192 && c.ldx % 8192 == 0 && (c.epilogue == 0 || (c.N > 6144 && c.N <= 8192))) return false;
+    return true;
+  }
+  if (c.M <= 32 && c.epilogue == 1 && !c.ex.ssq && !c.ex.x_tiled && c.N >= 16384 && c.K >= 2048) return false;
+  return c.M > 48 || c.ex.ssq || (c.K < 4096 && (c.M <= 32 || c.N <= 10240));
 }
 
 // A plain product (`half`: of a weight of few rows and up to 32 of X, half a tile a block), or gate and up with SwiGLU; false: not for
