@@ -538,7 +538,7 @@ static int tiles_choice(int M, int N, int K) {
 // 2560 6.0 and 5.6, of 1024 x 8192 16.8 and 11.8; 3 rows of 16 x 2304 6.1 and 5.4; 1 row of 32 x 2048 5.0 and 4.05;
 // 1 row of 200 x 2052 6.0 and 6.1, x 2304 5.5 and 5.3, of 64 x 4100 8.1 and 8.4, of 16 x 4100 5.7 and 8.2;
 // just above 2,048 one row takes as long by either, and by lanes less where the weight lies in a cache: of 96 x 2112 5.05 and 5.25, in a cache 4.2
-// and 5.5, of 512 x 2304 5.55 and 5.45, in a cache 5.2 and 5.7, of 768 x 2304 5.85 and 5.6; of 8 x 8192 9.3 and 9.85, of 32 x 8192 11.8 and 10.15).
+// and 5.5, of 512 x 2304 5.55 and 5.45, in a cache 5.2 and 5.7, of 768 x 2304 5.85 and 5.6; of 8 x 8192 9.3 and 9.85, of 20 x 8192 9.45 and 10.15, of 32 x 8192 11.8 and 10.15).
 // Short K (weights in the last-level cache): what a lane does one after the other is K, at most a chunk of it, times the rows; what
 // the rows kernel does is so many blocks.  1 row of 65536 x 4 2.4 us, rows kernel 19.8, 16 rows of 65536 x 128 25.3 and 27.9, x 192
 // 55 and 30; 16 rows of 24000 x 32 10.6 and 11.4, 8 of 24000 x 64 8.2 and 8.3; 4 rows of 8192 x 48 5.3 and 5.8, x 64 6.1 and 5.5;
@@ -548,7 +548,7 @@ static bool lanes_take(int M, int N, int K) {
   if (K > GS_SUM_CHUNK * GF_LANES_CHUNKS) return false;
   if (M <= 2 && K > 2048) {
     const bool cut = K % GS_SUM_CHUNK != 0;                        // (a chunk cut short costs the rows kernel 0.9)
-    if (M == 1 && (N <= 16 || (N <= 512 && K <= 2304))) return true;
+    if (M == 1 && (N <= 20 || (N <= 512 && K <= 2304))) return true;
     if (N <= 32) return K < 4608;
     return M == 1 ? (N <= 64 && K <= 2560) || (cut && N <= 256 && K < 4608) : N <= 64 && (K <= 2304 || (cut && K < 3072));
   }
