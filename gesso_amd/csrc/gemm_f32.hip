@@ -450,8 +450,10 @@ static void launch_rows(const float* X, int ldx, const float* W, const float* bi
 // 6144 x 1024 8.0 and 8.8, x 1088 11.2 and 10.3; 6 rows of 8192 x 512 6.5 and 8.6.)
 // Of a K whose last chunk is cut short (84 and 106 registers for 67 and 94) one at a time also up to 1,024, but for two rows of up to 2,048,
 // and just above 2,048, but for two rows of up to 5,120: 1 row of 6144 x 900 8.1 and 9.8, x 1028 11.0 and 10.7, x 2308 16.9 and 19.0, of
-// 512 x 2052 7.1 and 6.3; 8 rows of 2048 x 2308 8.7 and 9.2.
+// 512 x 2052 7.1 and 6.3; 8 rows of 2048 x 2308 8.7 and 9.2.  And three rows and more of 23 and 24 chunks, of 21 on for seven and eight, which one at a
+// time are three full rounds of the wavefronts: 8 rows of 2048 x 1532 6.3 and 6.85, x 1412 6.4 and 6.6, x 1540 7.1 and 6.75; 3 rows 5.8 and 6.0.
 static bool two_chunks(int M, int N, int K) {
+  if (K % GS_SUM_CHUNK != 0 && M > 2 && K > (M > 6 ? 1280 : 1408) && K < 1536) return false;
   if (K % GS_SUM_CHUNK != 0 && ((K <= 1024 && (M > 2 || N > 2048)) || (K > 2048 && K <= 2560 && (M > 2 || N > 5120)))) return false;
   return K > (M > 2 && N > 2048 ? 1024 : 512);
 }
