@@ -41,7 +41,9 @@ static bool few_plain(const SkinnyCall& c, int blocks) {
 // bytes and gemm_skinny_impl.h's kernel is as fast or faster (microseconds there and here, cold weights: gate and up 24 rows of 10240 x 2560
 // 15.2 and 14.5, of 12288 x 4096 22.4 both, of 22528 x 4096 32.9 and 33.5; 48 rows of 9216 x 1024 9.0 and 8.8, of 10240 x 2560 18.2 both,
 // of 16384 x 2048 16.1 and 16.3, of 28672 x 4096 50.8 and 52.1; stored, 17 rows of 12288 x 2048 12.8 and 12.5, of 16384 x 4096 25.9 and 26.6;
-// 48 rows of 65536 x 2048 57.9 and 58.9).  49 rows and more, or more than 16 weighted for their norm: nothing was slower.  SwiGLU of up to 32
+// 48 rows of 65536 x 2048 57.9 and 58.9).  49 rows and more: as tiled rows nothing was slower; as rows a K up
+// to 4,096 (gated ones below it; 49 rows, stored, of 9472 x 4096 36.3 and 36.2, x 4608 42.7 and 43.5, x 10752 93.6 and 96.6, gated of 25344 x
+// 2048 38.0 both, x 4096 70.3 and 71.6; 64 rows of 9472 x 4608 50.6 and 50.9).  More than 16 weighted for their norm: nothing was slower.  SwiGLU of up to 32
 // rows that lie as rows, not in tiles: from 16,384 rows of 2,048 on (24 of 12288 x 2048 15.15 and 15.2, of 16384 x 2048 15.85 and 16.2, of 28672 x
 // 2048 27.5 and 28.4, of 24576 x 1536 18.5 and 18.0).
 // Up to 16 rows: but for one to three of a long K, which gain nothing here or lose (1 row weighted for its norm,
@@ -58,6 +60,7 @@ static bool few_pairs(const SkinnyCall& c) {
     return true;
   }
   if (c.M <= 32 && c.epilogue == 1 && !c.ex.ssq && !c.ex.x_tiled && c.N >= 16384 && c.K >= 2048) return false;
+  if (c.M > 48 && !c.ex.x_tiled && (c.epilogue == 4 ? c.K >= 4096 : c.K > 4096)) return false;
   return c.M > 48 || c.ex.ssq || (c.K < 4096 && (c.M <= 32 || c.N <= 10240));
 }
 
