@@ -451,9 +451,11 @@ static void launch_rows(const float* X, int ldx, const float* W, const float* bi
 // Of a K whose last chunk is cut short (84 and 106 registers for 67 and 94) one at a time also up to 1,024, but for two rows of up to 2,048,
 // and just above 2,048, but for two rows of up to 5,120: 1 row of 6144 x 900 8.1 and 9.8, x 1028 11.0 and 10.7, x 2308 16.9 and 19.0, of
 // 512 x 2052 7.1 and 6.3; 8 rows of 2048 x 2308 8.7 and 9.2.  And three rows and more of 23 and 24 chunks, of 21 on for seven and eight, which one at a
-// time are three full rounds of the wavefronts: 8 rows of 2048 x 1532 6.3 and 6.85, x 1412 6.4 and 6.6, x 1540 7.1 and 6.75; 3 rows 5.8 and 6.0.
+// time are three full rounds of the wavefronts: 8 rows of 2048 x 1532 6.3 and 6.85, x 1412 6.4 and 6.6, x 1540 7.1 and 6.75; 3 rows 5.8 and 6.0; likewise five rows and more
+// of 39 and 40 whole ones: 8 rows of 2048 x 2560 7.3 and 7.65, 5 rows 7.2 and 7.4, 8 of 4096 x 2560 12.0 and 12.6.
 static bool two_chunks(int M, int N, int K) {
   if (K % GS_SUM_CHUNK != 0 && M > 2 && K > (M > 6 ? 1280 : 1408) && K < 1536) return false;
+  if (M > 4 && K > 2432 && K <= 2560) return false;
   if (K % GS_SUM_CHUNK != 0 && ((K <= 1024 && (M > 2 || N > 2048)) || (K > 2048 && K <= 2560 && (M > 2 || N > 5120)))) return false;
   return K > (M > 2 && N > 2048 ? 1024 : 512);
 }
